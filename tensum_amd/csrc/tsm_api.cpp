@@ -489,8 +489,8 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   AL(A.partial, (size_t)S * std::max(c->nblk_v, c->tiling.ntiles) * 4);
   if (c->tiled) AL(c->dtpart, (size_t)S * c->tiling.ntiles);
   AL(A.ctl, (size_t)S);
-  double* dg; double* dr; double* ts;
-  AL(dg, (size_t)S); AL(dr, (size_t)S);
+  double* dg; double* dr; double* dc; double* ts;
+  AL(dg, (size_t)S); AL(dr, (size_t)S); AL(dc, 2 * (size_t)S);
   // time stamps of an unsteady run (src/fv.cc:50-60); a steady run has none
   // and no final time (src/parameter.cc:250-252)
   const int n_stamps = params->unsteady ? params->n_time_stamps : 1;
@@ -505,7 +505,12 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   c->h_R.assign(S, params->gas_const);
   HIP_TRY(hipMemcpy(dg, c->h_gamma.data(), S * sizeof(double), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(dr, c->h_R.data(), S * sizeof(double), hipMemcpyHostToDevice));
-  A.gamma = dg; A.gasR = dr; A.tstamps = ts;
+  {
+    std::vector<double> gc;  // load_gas
+    for (int k = 0; k < S; ++k) { gc.push_back(1.0 / (params->gamma - 1.0)); gc.push_back(1.0 / params->gamma); }
+    HIP_TRY(hipMemcpy(dc, gc.data(), gc.size() * sizeof(double), hipMemcpyHostToDevice));
+  }
+  A.gamma = dg; A.gasR = dr; A.gasc = dc; A.tstamps = ts;
   A.log = nullptr; A.log_cap = 0;
   A.fo = tsm::FluxOpts{params->ev_alpha, params->ev_beta, params->tvb_M, params->nd_active};
   A.vp = tsm::ViscParams{params->mu_ref, params->T_ref, params->T_0, params->omega,
@@ -655,6 +660,8 @@ extern "C" int tsm_set_sample_material(tsm_ctx* c, int s, double gamma, double R
   c->h_gamma[s] = gamma; c->h_R[s] = R;
   HIP_TRY(hipMemcpy((void*)(c->A.gamma + s), &gamma, sizeof(double), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy((void*)(c->A.gasR + s), &R, sizeof(double), hipMemcpyHostToDevice));
+  const double gc[2] = {1.0 / (gamma - 1.0), 1.0 / gamma};
+  HIP_TRY(hipMemcpy((void*)(c->A.gasc + 2 * s), gc, sizeof(gc), hipMemcpyHostToDevice));
   return TSM_OK;
 }
 

@@ -285,6 +285,7 @@ struct StageArgs {
   double* W_keep;  // last stage's input state of each sample's latest step, null unless kept
   Ctl* ctl;
   const double* gamma; const double* gasR;
+  const double* gasc;  // per sample: 1/(gamma - 1), 1/gamma
   const double* tstamps;
   double* log; int log_cap;
   FluxOpts fo;
@@ -297,6 +298,10 @@ struct StageArgs {
   int heun;        // two-stage Heun (SSP-RK2) instead of SSP-RK3 in the SSP update
   int scheme;      // 0 SSP-RK3, 1 RK4, 2 Heun (the tiled stage kernel's update)
 };
+
+__device__ __forceinline__ Gas load_gas(const StageArgs& A, int s) {
+  return Gas{A.gamma[s], A.gasR[s], A.gasc[2 * s], A.gasc[2 * s + 1]};
+}
 
 // One context (a level of a multilevel run) in a packed launch: its geometry,
 // tiling, stage arguments (the stage's input and output buffers) and step

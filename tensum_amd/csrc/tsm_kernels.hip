@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void k_gradient(DevGeo G, StageArgs A, int s_o
   StageArgs As = A;
   As.off = (size_t)s * G.nv;
   As.sample = s;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   int p = G.pset[v];
   int m0, m1;
   if (p < 0) { m0 = -1; m1 = 0; } else { m0 = G.pptr[p]; m1 = G.pptr[p + 1]; }
@@ -178,11 +178,11 @@ __global__ __launch_bounds__(256) void k_flux(DevGeo G, StageArgs A) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= G.nf) return;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   int l = G.fv[2 * f], r = G.fv[2 * f + 1];
   double nx = G.fn[2 * f], ny = G.fn[2 * f + 1];
-  double area = sqrt(nx * nx + ny * ny);
-  double ia = 1.0 / area;
+  double ia;
+  const double area = face_area(nx, ny, &ia);
   double unx = nx * ia, uny = ny * ia;
   Prim Wl = load_prim(A.W_in, off + l), Wr = load_prim(A.W_in, off + r);
   Cons F;
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void k_update(DevGeo G, StageArgs A, int r, in
   StageArgs As = A;
   As.off = off;
   As.sample = s;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double part[4] = {0, 0, 0, 0};
   if (v < G.nv) {
     int p = G.pset[v];
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(256) void k_dt(DevGeo G, StageArgs A, StepParams P)
   }
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double dtv = 1.0e20;
   if (v < G.nv) {
     Prim w = load_prim(A.W_in, off + v);
@@ -483,7 +483,8 @@ __global__ __launch_bounds__(256) void k_dt(DevGeo G, StageArgs A, StepParams P)
           unsigned kind = ent >> 30, idx = ent & 0x3fffffffu;
           if (kind < 2) {
             double nx = G.fn[2 * idx], ny = G.fn[2 * idx + 1];
-            double area = sqrt(nx * nx + ny * ny);
+            double ia;
+            const double area = face_area(nx, ny, &ia);
             double vn = wm.u * nx + wm.v * ny;
             lam += (fabs(vn) + cm * area) * 1.0;
           } else {
@@ -505,7 +506,8 @@ __global__ __launch_bounds__(256) void k_dt(DevGeo G, StageArgs A, StepParams P)
             unsigned kind = ent >> 30, idx = ent & 0x3fffffffu;
             if (kind >= 2) continue;
             double nx = G.fn[2 * idx], ny = G.fn[2 * idx + 1];
-            double area = sqrt(nx * nx + ny * ny);
+            double ia;
+            const double area = face_area(nx, ny, &ia);
             int l = G.fv[2 * idx], rr = G.fv[2 * idx + 1];
             double dx = G.x[rr] * 1.0 + G.x[l] * -1.0, dy = G.y[rr] * 1.0 + G.y[l] * -1.0;
             double dl = sqrt(dx * dx + dy * dy);
@@ -629,7 +631,7 @@ __global__ __launch_bounds__(256) void k_forces(DevGeo G, StageArgs A, int s, in
                                                 const int* sel, int nsel, int ns_model,
                                                 double* terms, double* out) {
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   const int type = G.btype[bq];
   const double qx = G.bn[2 * bq], qy = G.bn[2 * bq + 1];
   for (int j = threadIdx.x; j < nsel; j += blockDim.x) {
@@ -682,7 +684,7 @@ __global__ __launch_bounds__(256) void k_surface(DevGeo G, StageArgs A, int s, c
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= nsel) return;
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   const int b = sel[j];
   const int type = G.btype[b];
   const int v0 = G.bv[2 * b], v1 = G.bv[2 * b + 1];
@@ -886,7 +888,7 @@ __global__ __launch_bounds__(256) void k_ssw(DevGeo G, StageArgs A) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= G.nf) return;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   int l = G.fv[2 * f], r = G.fv[2 * f + 1];
   double nx = G.fn[2 * f], ny = G.fn[2 * f + 1];
   Prim wl = load_prim(A.W_in, off + l), wr = load_prim(A.W_in, off + r);
@@ -906,7 +908,7 @@ __global__ void k_prim2ent(DevGeo G, StageArgs A, int s) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= G.nv) return;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   Prim w = load_prim(A.W_in, off + v);
   store_ent(A.E_in, off + v, prim2ent(gas, w));
 }
@@ -916,7 +918,7 @@ __global__ __launch_bounds__(256) void k_global(DevGeo G, StageArgs A, int s, do
   __shared__ double lds[4 * 2];
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double q[2] = {0, 0};
   if (v < G.nv) {
     Prim w = load_prim(A.W_in, off + v);
@@ -934,7 +936,7 @@ __global__ __launch_bounds__(256) void k_errnorm(DevGeo G, StageArgs A, int s, c
   __shared__ double lds[4 * 24];
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t off = (size_t)s * G.nv;
-  Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double q[24];
 #pragma unroll
   for (int k = 0; k < 24; ++k) q[k] = 0.0;
@@ -1108,7 +1110,7 @@ __global__ __launch_bounds__(256) void k_moments(DevGeo G, StageArgs A, int S, d
   if (v >= G.nv) return;
   double M[5], Q[5], Z[5];
   for (int s = 0; s < S; ++s) {
-    const Gas gas{A.gamma[s], A.gasR[s]};
+    const Gas gas = load_gas(A, s);
     const Prim w = load_prim(A.W_in, (size_t)s * G.nv + v);
     const double x[5] = {w.T, w.u, w.v, w.p, density(gas, w)};
     if (s == 0) {
@@ -1142,7 +1144,7 @@ __global__ void k_probes(StageArgs A, int nv, int np, const int* pc, const doubl
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np * S) return;
   const int s = i / np, p = i % np;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double r = 0.0;
   for (int k = 0; k < 3; ++k) {
     const Prim w = load_prim(A.W_in, (size_t)s * nv + pc[3 * p + k]);
@@ -1155,7 +1157,7 @@ __global__ void k_probes(StageArgs A, int nv, int np, const int* pc, const doubl
 __global__ __launch_bounds__(256) void k_global_all(DevGeo G, StageArgs A, double* out) {
   __shared__ double lds[4 * 2];
   const int v = blockIdx.x * blockDim.x + threadIdx.x, s = blockIdx.y;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   double q[2] = {0, 0};
   if (v < G.nv) {
     const Prim w = load_prim(A.W_in, (size_t)s * G.nv + v);

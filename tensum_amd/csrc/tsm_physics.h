@@ -17,8 +17,11 @@ enum { F_ROE = 0, F_RUS = 1, F_KEPEC = 2, F_ROEEC = 3, F_KEP = 4, F_AVG = 5 };
 enum { R_FIRST = 0, R_SECOND = 1, R_MUSCL = 2, R_ALBADA = 3, R_MINMOD = 4,
        R_TVB = 5, R_ENO2 = 6 };
 
+// Material constants of a sample: gamma, R, 1/(gamma - 1) and 1/gamma.  The
+// reciprocals are the same for every vertex and face of a sample, so they are
+// formed once per sample on the host (load_gas) and arrive as scalars.
 struct Gas {
-  double gamma, R;
+  double gamma, R, ig1, igam;
 };
 
 struct Prim { double T, u, v, p; };
@@ -55,6 +58,39 @@ __device__ __forceinline__ double fsqrt(double x) {
   g = __builtin_fma(d, h, g);
   d = __builtin_fma(-g, g, x);
   return __builtin_fma(d, h, g);
+}
+
+// Reciprocal and reciprocal square root to about an ulp: the hardware estimate
+// (measured relative error 2^-24) and one third-order step, whose remaining error
+// is the cube of the estimate's (2^-72), so only the rounding of the last
+// multiply-add is left (measured 0.5, 0.6 and 0.75 x 2^-52).  3 and 5 instructions after the estimate where fdiv and
+// fsqrt take 7 and 10; used in the edge flux, which is bounded by FP64 issue
+// and multiplies the results on.  Normal-range operands, as fdiv and fsqrt.
+__device__ __forceinline__ double frcp(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+__device__ __forceinline__ double frsq(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+// square root from the same estimate: g = x y, corrected by e = 1 - x y^2
+__device__ __forceinline__ double fsqrt3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double g = x * y;
+  const double e = __builtin_fma(-g, y, 1.0);
+  return __builtin_fma(g * e, __builtin_fma(e, 0.375, 0.5), g);
+}
+// Length of a face normal and its reciprocal from one estimate.  Every kernel
+// that needs a face's area takes it from here, so that the time step a run
+// starts with and the one its last stage forms agree to the bit.
+__device__ __forceinline__ double face_area(double nx, double ny, double* inv) {
+  const double n2 = nx * nx + ny * ny;
+  const double ia = frsq(n2);
+  *inv = ia;
+  return n2 * ia;
 }
 
 __device__ __forceinline__ double density(const Gas& g, const Prim& w) {
@@ -96,6 +132,19 @@ __device__ __forceinline__ double logavg(double a, double b) {
     F = fdiv(log(fdiv(b, a)) * 0.5, f);
   }
   return fdiv(0.5 * sum, F);
+}
+
+// logavg with reciprocals of about an ulp (the TeCNO flux)
+__device__ __forceinline__ double logavg_r(double a, double b) {
+  const double sum = a + b, d = b - a;
+  const double f = d * frcp(sum);
+  const double u = f * f;
+  if (u < 1.0e-2) {
+    const double u2 = u * u;
+    const double F = 1.0 + u * (1.0 / 3.0) + u2 * (1.0 / 5.0) + (u2 * u) * (1.0 / 7.0);
+    return (0.5 * sum) * frcp(F);
+  }
+  return fdiv(d, log(fdiv(b, a)));  // (sum / 2) / (log(b/a) / (2 f))
 }
 
 // src/material.h:501-513
@@ -339,19 +388,18 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
   const double gam = g.gamma;
   const Prim& l = L.w;
   const Prim& r = Rr.w;
-  // 1/(gamma-1) and 1/gamma are the same for every face of a sample (the
-  // compiler forms them once per thread); 1/beta serves a and the energy flux.
-  const double ig1 = fdiv(1.0, gam - 1.0), igam = fdiv(1.0, gam);
+  const double ig1 = g.ig1, igam = g.igam;
   double rhol = L.rho, rhor = Rr.rho;
-  double rho = logavg(rhol, rhor);
+  double rho = logavg_r(rhol, rhor);
   double betal = L.beta, betar = Rr.beta;
   // beta's logarithmic mean enters only through 1/beta_hat: with
   // r = 1/(beta_l + beta_r), f = (beta_r - beta_l) r and beta_hat = 1/(2 r F(f)),
   // so 1/beta_hat = 2 F(f) r, and p_hat = (rho_l + rho_r) r / 2: one division
   // where the reference's expressions take four (same values to rounding)
-  const double rb = fdiv(1.0, betal + betar);
+  const double rb = frcp(betal + betar);
   const double ib = 2.0 * logavg_F((betar - betal) * rb, betal, betar) * rb;
-  double a = fsqrt(0.5 * gam * ib);
+  const double a2 = (0.5 * gam) * ib;
+  double a = fsqrt3(a2);
   double p = (0.5 * (rhol + rhor)) * rb;
   double vx = l.u * 0.5 + r.u * 0.5, vy = l.v * 0.5 + r.v * 0.5;
   double vn = vx * unx + vy * uny;
@@ -367,7 +415,7 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
   if (!o.nd_active) return F;
 
   double vsq = vx * vx + vy * vy;
-  double H = a * a * ig1 + 0.5 * vsq;
+  double H = a2 * ig1 + 0.5 * vsq;
   double v1 = vx * uny - vy * unx;
   double Lam[4];
   if (ROE) {
@@ -450,7 +498,8 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
       proj(gdr[0], gdr[1], gdr[2], gdr[3], gr);
     }
     const double rg = rho * igam;
-    const double q[4] = {0.5 * rg, (gam - 1.0) * rg, p, 0.5 * rg};
+    // half the scalings: the flux takes -D/2
+    const double q[4] = {0.25 * rg, (0.5 * (gam - 1.0)) * rg, 0.5 * p, 0.25 * rg};
     double w[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -463,17 +512,23 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
         const double K = 1.0 / 3.0;
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - ((dl + dr) * (1.0 - K) + (2.0 * dz[i]) * (1.0 + K)) * 0.25;
+      } else if (REC == R_MINMOD) {
+        // minmod(d, dz) is d clamped to the interval between 0 and dz
+        const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
+        const double lo = fmin(dz[i], 0.0), hi = fmax(dz[i], 0.0);
+        dZi = dz[i] - 0.5 * (fmax(lo, fmin(hi, dl)) + fmax(lo, fmin(hi, dr)));
       } else {
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - limited_slope<REC>(dl, dz[i], 0.0, 0.0) - limited_slope<REC>(dr, dz[i], 0.0, 0.0);
       }
       w[i] = (q[i] * Lam[i]) * dZi;
     }
-    const double w13 = w[0] + w[1] + w[3], d30 = w[3] - w[0];
-    D[0] = w13;
-    D[1] = vx * w13 + a * unx * d30 + uny * w[2];
-    D[2] = vy * w13 + a * uny * d30 - unx * w[2];
-    D[3] = H * (w[0] + w[3]) + hv * w[1] + a * vn * d30 + v1 * w[2];
+    const double w03 = w[0] + w[3], w13 = w03 + w[1], d30 = a * (w[3] - w[0]);
+    F.m -= w13;
+    F.mx -= vx * w13 + unx * d30 + uny * w[2];
+    F.my -= vy * w13 + uny * d30 - unx * w[2];
+    F.e -= H * w03 + hv * w[1] + vn * d30 + v1 * w[2];
+    return F;
   }
   F.m -= 0.5 * D[0];
   F.mx -= 0.5 * D[1];

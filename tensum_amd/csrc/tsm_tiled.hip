@@ -245,7 +245,7 @@ __device__ __forceinline__ void grad_tile_body(const DevGeo& G, const TileGeo& T
   const int b0 = TG.vbeg[t], nown = TG.vbeg[t + 1] - b0;
   const int h0 = TG.hbeg[t], ns = nown + TG.hbeg[t + 1] - h0;
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   const int tid = threadIdx.x;
   const bool own = tid < nown;
   const int v = b0 + tid;
@@ -360,7 +360,7 @@ __device__ __forceinline__ void grad_bnd_body(const DevGeo& G, const TileGeo& TG
   const bool live = i < nbv;
   const int k0 = live ? TG.gb_ptr[i] : 0, nc = live ? TG.gb_ptr[i + 1] - k0 : 0;
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
   const int base = (threadIdx.x & 63) & ~(GB_LANES - 1);
   // the longest cell list of the lane group sets the chunk count for all its lanes
   int ncm = nc;
@@ -494,7 +494,7 @@ __device__ __forceinline__ void fu_tile_body(const DevGeo& G, const TileGeo& TG,
   const int h0 = TG.hbeg[t], ns = nown + TG.hbeg[t + 1] - h0;
   const int f0 = TG.fbeg[t], nfl = TG.fbeg[t + 1] - f0;
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
 
   if (LAST && threadIdx.x == 0) arrive = 0;  // read after the phase barriers
   // this thread's faces and its owned vertex's gather range, loaded before
@@ -558,8 +558,8 @@ __device__ __forceinline__ void fu_tile_body(const DevGeo& G, const TileGeo& TG,
     const int l = lr & 0xffff, rr = lr >> 16;
     const double nx = PREF ? fnx[q] : TG.f_n[2 * (size_t)(f0 + j)];
     const double ny = PREF ? fny[q] : TG.f_n[2 * (size_t)(f0 + j) + 1];
-    const double area = fsqrt(nx * nx + ny * ny);
-    const double ia = fdiv(1.0, area);
+    double ia;
+    const double area = face_area(nx, ny, &ia);
     Side Ls, Rs;
     Ls.w = Prim{Q[l], Q[MS + l], Q[2 * MS + l], Q[3 * MS + l]};
     Rs.w = Prim{Q[rr], Q[MS + rr], Q[2 * MS + rr], Q[3 * MS + rr]};
@@ -926,7 +926,7 @@ __global__ __launch_bounds__(512, TSM_FU_WAVES) void k_stage_fused(DevGeo G, Til
   const int k0 = TG.h2beg[t], ns = n1 + TG.h2beg[t + 1] - k0;
   const int f0 = TG.fbeg[t], nfl = TG.fbeg[t + 1] - f0;
   const size_t off = (size_t)s * G.nv;
-  const Gas gas{A.gamma[s], A.gasR[s]};
+  const Gas gas = load_gas(A, s);
 
   if (LAST && threadIdx.x == 0) arrive = 0;  // read after the phase barriers
   // ---- phase 1: slot quantities (two rings) ------------------------------
@@ -1013,8 +1013,8 @@ __global__ __launch_bounds__(512, TSM_FU_WAVES) void k_stage_fused(DevGeo G, Til
     const unsigned lr = TG.f_lr[f0 + j];
     const int l = lr & 0xffff, rr = lr >> 16;
     const double nx = TG.f_n[2 * (size_t)(f0 + j)], ny = TG.f_n[2 * (size_t)(f0 + j) + 1];
-    const double area = fsqrt(nx * nx + ny * ny);
-    const double ia = fdiv(1.0, area);
+    double ia;
+    const double area = face_area(nx, ny, &ia);
     Side Ls, Rs;
     Ls.w = Prim{Q[l], Q[MS1 + l], Q[2 * MS1 + l], Q[3 * MS1 + l]};
     Rs.w = Prim{Q[rr], Q[MS1 + rr], Q[2 * MS1 + rr], Q[3 * MS1 + rr]};
