@@ -34,18 +34,12 @@ def kernel_bytes(nv, nf, nc, tiles):
         "gradient": 124 * nv + 24 * nc,
         "flux": 112 * nv + 56 * nf,
         "update": 148 * nv + 40 * nf,
-        # tiled kernels: W + coords + 1/(6 mcarea) + cell entries (3 per cell,
-        # 4 B) + CSR offsets + halo ids, dE write
-        "grad_tile": (32 + 16 + 8 + 4 + 64) * nv + 12 * nc + 4 * halo,
-        # W, dE, coords, U_old source W^n, dcarea, weight, offsets, W write;
-        # local faces (slot pair 4 B + normal 16 B), 16-bit gather entries
-        "fu_tile": (32 + 64 + 16 + 32 + 8 + 8 + 4 + 32) * nv + 20 * fl + 4 * nf + 4 * halo,
-        # fused two-ring stage kernel: W, coords, 1/(6 mcarea), U_old source
-        # W^n, dcarea, weight, gather offsets, W write; gradient cell entries
-        # of the owned and first-ring slots (4 B + 4 B offsets per slot);
-        # local faces, gather entries, halo ids of both rings
-        "stage_fused": (32 + 16 + 8 + 32 + 8 + 8 + 4 + 32) * nv + 4 * tiles.get("grad_cells", 0)
-                       + 4 * (nv + halo) + 20 * fl + 4 * nf + 4 * (halo + tiles.get("halo2", 0)),
+        # stage kernel: W, first entropy variable, coords, U_old source W^n,
+        # dcarea, 1/(6 mcarea), 16 B of gather entries, W and entropy variable
+        # written; per gradient slot (owned and first ring) 16 B of neighbour
+        # entries; per slot its id; local faces (slot pair 4 B + normal 16 B)
+        "stage": (32 + 8 + 16 + 32 + 8 + 8 + 16 + 32 + 8) * nv + 16 * (nv + halo)
+                 + 4 * (nv + halo + tiles.get("halo2", 0)) + 20 * fl,
     }
 
 
@@ -96,8 +90,8 @@ def main():
     ap.add_argument("--tile", type=int, default=0, help="owned vertices per tile (0: 128)")
     ap.add_argument("--path", default="auto", choices=["auto", "csr"])
     ap.add_argument("--fused-gradient", action="store_true",
-                    help="gradients inside the stage kernel (two halo rings) instead of a pass "
-                         "of their own")
+                    help="accepted for older command lines: the stage kernel always forms the "
+                         "gradients itself")
     ap.add_argument("--graph", type=int, default=0, help="steps per captured HIP graph (0: none)")
     ap.add_argument("--block", type=int, default=0, help="threads per tile of the stage kernel")
     ap.add_argument("--no-cpu-baseline", action="store_true")
@@ -218,12 +212,11 @@ def main():
     print(f"bench: {args.steps} steps in {wall:.3f} s, {ms_per_step:.3f} ms/step", file=sys.stderr,
           flush=True)
 
-    tiles = T.host_tiling(mesh, prm.tile_vertices or 128, two_rings=args.fused_gradient)
+    tiles = T.host_tiling(mesh, prm.tile_vertices or 128,
+                          two_rings=args.workload == "riemann")
     kb = kernel_bytes(nv, nf, nc, tiles)
-    if ku["dt_us"] == 0.0 and tiles["two_rings"]:  # fused stage kernel
-        per_launch = {"stage_fused": ku["flux_us"]}
-    elif ku["dt_us"] == 0.0:  # tiled kernels with a gradient pass
-        per_launch = {"grad_tile": ku["gradient_us"], "fu_tile": ku["flux_us"]}
+    if ku["dt_us"] == 0.0:  # tiled path: one kernel per stage
+        per_launch = {"stage": ku["flux_us"]}
     else:
         per_launch = {"dt": ku["dt_us"], "gradient": ku["gradient_us"], "flux": ku["flux_us"],
                       "update": ku["update_us"]}

@@ -44,12 +44,14 @@ struct tsm_ctx {
   tsm::StepParams SP{};
   std::vector<void*> allocs;
   double* W[3] = {nullptr, nullptr, nullptr};
+  double* V[3] = {nullptr, nullptr, nullptr};  // first entropy variable of W[] (tiled TeCNO)
   double* E[2] = {nullptr, nullptr};
   int cur = 0;              // W[cur] / E[cur] hold the current state
   bool tiled = false;       // LDS-tiled stage kernels in use
   bool e_valid = true;      // E[cur] == prim2ent(W[cur])
   tsm::Tiling tiling;
-  tsm::TileGeo TG{};
+  tsm::StageTab ST{};
+  bool two_rings_asked = false;  // tile_fused_gradient on a mesh and scheme it applies to
   double* dtpart = nullptr;
   std::vector<int> perm;    // part-file vertex id -> device vertex id
   // input bface b, end point k (bface_v[2b+k]) -> offset of its boundary
@@ -102,6 +104,7 @@ struct tsm_ctx {
   }
   void bind_state() {
     A.W_in = W[cur]; A.W_out = W[cur ^ 1];
+    A.V_in = A.V_out = V[cur];
     A.E_in = E[cur]; A.E_out = E[cur ^ 1];
   }
   // Makes W[cur] the state of the CSR kernels' double buffer (W[0]/W[1]) and
@@ -156,6 +159,13 @@ int validate_params(const tsm_params& p) {
 
 }  // namespace
 
+namespace {
+// One attempt at a context, with tiles of tb owned vertices (0: the CSR-gather
+// kernels).  1: the tiles do not fit the stage kernel.
+int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int tb,
+                      tsm_ctx** out);
+}  // namespace
+
 extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_samples,
                           tsm_ctx** out) {
   if (!mesh || !params || !out || n_samples < 1) return fail(TSM_E_ARG, "null argument");
@@ -165,6 +175,23 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
     return fail(TSM_E_HIP, "no HIP device visible");
+  // tiled stage kernels: every scheme, Euler or Navier-Stokes, with or without
+  // the Liou fix; strong boundary conditions keep the CSR kernels.  A mesh whose
+  // two halo rings do not fit LDS at the wanted tile size (vertices with
+  // hundreds of cells) takes smaller tiles, and the CSR kernels if none fits.
+  if (params->kernel_path != 0 || params->strong_bc)
+    return create_with_tiles(mesh, params, n_samples, 0, out);
+  const int want = params->tile_vertices > 0 ? params->tile_vertices : 128;
+  for (int tb = want;; tb /= 2) {
+    rc = create_with_tiles(mesh, params, n_samples, tb < 16 && tb < want ? 0 : tb, out);
+    if (rc != 1) return rc;
+  }
+}
+
+namespace {
+int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int tb,
+                      tsm_ctx** out) {
+  int rc = TSM_OK;
   tsm_ctx* c = new tsm_ctx();
   c->P = *params;
   c->S = n_samples;
@@ -188,24 +215,20 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
     return fail(TSM_E_MESH, "mesh too large for 30-bit face ids");
   }
   // ---- path and vertex numbering -----------------------------------------
-  // tiled stage kernels: every scheme, Euler or Navier-Stokes, with or without
-  // the Liou fix; strong boundary conditions keep the CSR kernels
-  c->tiled = params->kernel_path == 0 && !params->strong_bc;
+  c->tiled = tb > 0;
   std::vector<int> perm(nv), inv(nv);
   tsm::TileGeo dev_tg{};   // device-built tile arrays (dev_tiles)
   bool dev_tiles = false;
   if (c->tiled) {
-    int tb = params->tile_vertices > 0 ? params->tile_vertices : 128;
     if (tb > 256) { delete c; return fail(TSM_E_ARG, "tile_vertices must be <= 256"); }
     if (params->graph_steps < 0 || params->graph_steps > 4096) {
       delete c;
       return fail(TSM_E_ARG, "graph_steps must be in [0, 4096]");
     }
     const bool grad = (params->flux == 0 || params->flux == 1) && params->reconstruct != 0;
-    const bool ring2 = grad && params->tile_fused_gradient && params->model == 0 &&
-                       params->time_scheme == 0;
-    // on the device where the mesh allows it (no periodic sets, one halo
-    // ring), else on the host; both give the same arrays
+    c->two_rings_asked = grad && params->tile_fused_gradient && params->model == 0 &&
+                         params->time_scheme == 0 && g.periodic.empty();
+    // on the device unless the host is asked for; both give the same arrays
     int trc = 1;
     if (!params->host_preprocess) {
       auto dalloc = [c](void** p, size_t bytes) -> int {
@@ -214,12 +237,12 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
         *p = q;
         return r;
       };
-      trc = tsm::build_tiles_device(g, tb, ring2, c->tiling, dev_tg, dalloc, msg);
+      trc = tsm::build_tiles_device(g, tb, false, c->tiling, dev_tg, dalloc, msg);
       if (trc < 0) { delete c; return fail(trc, "tiling: " + msg); }
     }
     dev_tiles = trc == 0;
     if (!dev_tiles &&
-        (!tsm::build_tiles(g, tb, c->tiling, msg, ring2) || !tsm::validate_tiles(g, c->tiling, msg))) {
+        (!tsm::build_tiles(g, tb, c->tiling, msg, false) || !tsm::validate_tiles(g, c->tiling, msg))) {
       delete c;
       return fail(TSM_E_MESH, "tiling: " + msg);
     }
@@ -421,24 +444,18 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
 #undef UP
   if (c->tiled) {
     const tsm::Tiling& T = c->tiling;
-    tsm::TileGeo& TG = c->TG;
+    tsm::TileGeo TG{};
     TG.ntiles = T.ntiles; TG.tb = T.tb; TG.max_slots = T.max_slots; TG.max_faces = T.max_faces;
     TG.n_periodic_tiles = T.n_periodic_tiles;
     TG.n_gbv = dev_tiles ? dev_tg.n_gbv : (int)T.gbv.size();
-    TG.gbv = nullptr;
-    TG.gb_ptr = nullptr;
-    TG.gb_ent = nullptr;
-    TG.fused = T.fused ? 1 : 0;
-    TG.max_slots1 = T.max_slots1;
-    TG.h2beg = TG.halo2 = TG.g1beg = TG.g1ptr = TG.g1cgid = nullptr;
-    TG.g1ent = nullptr;
-    TG.grad_block = std::max(0, params->block_grad);
     TG.fu_block = std::max(0, params->block_fu);
-    const int bf = tsm::tile_fu_block(TG), bg = tsm::tile_grad_block(TG);
-    if (bf > tsm::tile_fu_block_max() || bf % 64 || bg > 512 || bg % 64 ||
-        (params->model == 1 ? tsm::tile_fu_lds_ns(TG, params->flux, params->reconstruct)
-                            : tsm::tile_fu_lds(TG, params->flux, params->reconstruct)) > 160 * 1024 ||
-        tsm::tile_grad_lds(TG) > 160 * 1024) {
+    // block_grad has had no kernel of its own since the stage kernel forms the
+    // gradients; its range is still checked
+    const int bg = std::max(((T.tb + 63) / 64) * 64, std::max(0, params->block_grad));
+    tsm::StageTab probe{};
+    probe.tb = T.tb; probe.mf = T.max_faces; probe.fu_block = TG.fu_block;
+    const int bf = tsm::stage_block(probe);
+    if (bf > tsm::stage_block_max() || bf % 64 || bg > 512 || bg % 64) {
       delete c;
       return fail(TSM_E_ARG, "tiled kernels: block size or LDS out of range (blocks " +
                                  std::to_string(bg) + "/" + std::to_string(bf) + ")");
@@ -446,19 +463,13 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
 #define UT(field, vec) do { if ((rc = c->upload(&TG.field, vec))) { delete c; return rc; } } while (0)
     if (dev_tiles) {
       TG.vbeg = dev_tg.vbeg; TG.hbeg = dev_tg.hbeg; TG.halo = dev_tg.halo; TG.fbeg = dev_tg.fbeg;
-      TG.bbeg = dev_tg.bbeg; TG.tbf = dev_tg.tbf; TG.gptr = dev_tg.gptr; TG.cptr = dev_tg.cptr;
-      TG.cgid = dev_tg.cgid; TG.tper = dev_tg.tper; TG.pinfo = dev_tg.pinfo; TG.f_lr = dev_tg.f_lr;
-      TG.cent = dev_tg.cent; TG.f_n = dev_tg.f_n; TG.gent = dev_tg.gent;
-      if (TG.n_gbv > 0) TG.gbv = dev_tg.gbv;
+      TG.bbeg = dev_tg.bbeg; TG.tbf = dev_tg.tbf; TG.gptr = dev_tg.gptr;
+      TG.tper = dev_tg.tper; TG.pinfo = dev_tg.pinfo; TG.f_lr = dev_tg.f_lr;
+      TG.f_n = dev_tg.f_n; TG.gent = dev_tg.gent;
     } else {
       UT(vbeg, T.vbeg); UT(hbeg, T.hbeg); UT(halo, T.halo); UT(fbeg, T.fbeg); UT(bbeg, T.bbeg);
-      UT(tbf, T.tbf); UT(gptr, T.gptr); UT(cptr, T.cptr); UT(cgid, T.cgid); UT(tper, T.tper);
-      UT(pinfo, T.pinfo); UT(f_lr, T.f_lr); UT(cent, T.cent); UT(f_n, T.f_n); UT(gent, T.gent);
-      if (!T.gbv.empty()) UT(gbv, T.gbv);
-    }
-    if (T.fused) {
-      UT(h2beg, T.h2beg); UT(halo2, T.halo2); UT(g1beg, T.g1beg); UT(g1ptr, T.g1ptr);
-      UT(g1cgid, T.g1cgid); UT(g1ent, T.g1ent);
+      UT(tbf, T.tbf); UT(gptr, T.gptr); UT(tper, T.tper);
+      UT(pinfo, T.pinfo); UT(f_lr, T.f_lr); UT(f_n, T.f_n); UT(gent, T.gent);
     }
 #undef UT
     auto dalloc = [c](void** p, size_t bytes) -> int {
@@ -467,9 +478,14 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
       *p = q;
       return r;
     };
-    if ((rc = tsm::build_grad_bnd_table(c->G, TG, dalloc, c->st, msg))) {
+    rc = tsm::build_stage_tables(c->G, TG, tsm::stage_has_gradients(params->flux, params->reconstruct),
+                                 params->model == 1, wall_cells, c->ST, dalloc, c->st, msg);
+    // the static LDS of the kernel and its launches fit beside this much
+    if (rc == 0 && tsm::stage_lds(c->ST, params->flux, params->reconstruct, params->model == 1) > 156 * 1024)
+      rc = 1;
+    if (rc) {
       delete c;
-      return fail(rc, msg);
+      return rc == 1 ? 1 : fail(rc, msg);
     }
   }
   tsm::StageArgs& A = c->A;
@@ -481,6 +497,8 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   const size_t cs = A.cs;
 #define AL(ptr, n) do { if ((rc = c->alloc(&(ptr), (n)))) { delete c; return rc; } } while (0)
   AL(c->W[0], 4 * cs); AL(c->W[1], 4 * cs); AL(c->W[2], 4 * cs);
+  if (c->tiled && tsm::stage_keeps_var0(params->flux))
+    for (auto& v : c->V) AL(v, cs);
   AL(c->E[0], 4 * cs); AL(c->E[1], 4 * cs);
   AL(A.Uold, 4 * cs); AL(A.dE, 8 * cs); AL(A.F, 4 * A.fs); AL(A.R, 4 * cs);
   if (params->time_scheme == 1) AL(A.R2, 4 * cs);
@@ -514,7 +532,7 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   A.log = nullptr; A.log_cap = 0;
   A.fo = tsm::FluxOpts{params->ev_alpha, params->ev_beta, params->tvb_M, params->nd_active};
   A.vp = tsm::ViscParams{params->mu_ref, params->T_ref, params->T_0, params->omega,
-                         params->prandtl, params->mu_model, params->visc_active,
+                         params->prandtl, 1.0 / params->prandtl, params->mu_model, params->visc_active,
                          params->heat_active};
   A.ns = params->model == 1;
   A.ns_walls = wall_cells;
@@ -531,6 +549,7 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   *out = c;
   return TSM_OK;
 }
+}  // namespace
 
 extern "C" void tsm_destroy(tsm_ctx* c) { delete c; }
 
@@ -889,38 +908,31 @@ void enqueue_step(tsm_ctx* c, int log_slot, bool dt_ready = false) {
 // stages write the two other buffers and the last one writes W^{n+1} back
 // in place (each vertex reads its own W^n for U_old before overwriting it).
 void enqueue_tiled_step(tsm_ctx* c, int log_slot, hipEvent_t* ev = nullptr) {
+  const int ia = (c->cur + 1) % 3, ib = (c->cur + 2) % 3;
   double* Wn = c->W[c->cur];
-  double* Wa = c->W[(c->cur + 1) % 3];
-  double* Wb = c->W[(c->cur + 2) % 3];
   // stage buffers: every stage reads W^n for U_old, the last one writes W^{n+1}
   // over it in place; SSP-RK3 and RK4 rotate through two scratch buffers
   const int nrk = c->P.time_scheme == 0 ? 3 : (c->P.time_scheme == 1 ? 4 : 2);
-  const double* ins[4] = {Wn, Wa, Wb, Wa};
-  double* outs[4] = {Wa, Wb, Wa, Wn};
-  if (nrk == 3) outs[2] = Wn;
-  if (nrk == 2) outs[1] = Wn;
+  int ins[4] = {c->cur, ia, ib, ia}, outs[4] = {ia, ib, ia, c->cur};
+  if (nrk == 3) outs[2] = c->cur;
+  if (nrk == 2) outs[1] = c->cur;
   int e = 0;
   if (c->P.liou_fix) {  // the step's Liou sensor from W^n (src/fv.cc:2281-2285)
     c->A.W_in = Wn;
     tsm::launch_ssw(c->G, c->A, c->S, c->st);
   }
   for (int r = 0; r < nrk; ++r) {
-    c->A.W_in = ins[r];
-    c->A.W_out = outs[r];
-    if (ev) (void)hipEventRecord(ev[e++], c->st);
+    c->A.W_in = c->W[ins[r]];
+    c->A.W_out = c->W[outs[r]];
+    c->A.V_in = c->V[ins[r]];
+    c->A.V_out = c->V[outs[r]];
     tsm::launch_bc_time(c->G, c->bt, c->A, c->S, r, c->st);
-    if (tsm::tile_needs_gradient_pass(c->TG, c->P.flux, c->P.reconstruct)) {
-      // boundary vertices, then the tiles (measured: on a second stream beside the
-      // tile kernel the two compete for CU slots and the stage takes longer)
-      tsm::launch_tile_gradient_bnd(c->G, c->TG, c->A, c->S, c->st);
-      tsm::launch_tile_gradient(c->G, c->TG, c->A, c->S, c->st);
-    }
     if (ev) (void)hipEventRecord(ev[e++], c->st);
-    tsm::launch_tile_stage(c->P.flux, c->P.reconstruct, c->G, c->TG, c->A, c->SP, Wn, c->dtpart,
-                           c->S, r, r == nrk - 1, c->st);
+    tsm::launch_stage(c->P.flux, c->P.reconstruct, c->G, c->ST, c->A, c->SP, Wn, c->dtpart, c->S, r,
+                      r == nrk - 1, c->st);
   }
   if (ev) (void)hipEventRecord(ev[e++], c->st);
-  tsm::launch_step_final_tiled(c->G, c->A, c->SP, c->S, c->TG.ntiles, c->dtpart, log_slot, c->st);
+  tsm::launch_step_final_tiled(c->G, c->A, c->SP, c->S, c->ST.ntiles, c->dtpart, log_slot, c->st);
   if (ev) (void)hipEventRecord(ev[e++], c->st);
   c->bind_state();
   c->e_valid = false;
@@ -1086,7 +1098,7 @@ extern "C" int tsm_run_packed(tsm_ctx** cs, int n, long nsteps, long* done) {
   for (int i = 0; i < n; ++i) {
     const tsm_ctx* c = cs[i];
     if (!c) return fail(TSM_E_ARG, "null context in group");
-    if (!c->tiled || c->TG.fused || c->P.time_scheme != 0 || c->A.ns || c->P.liou_fix)
+    if (!c->tiled || c->two_rings_asked || c->P.time_scheme != 0 || c->A.ns || c->P.liou_fix)
       return fail(TSM_E_ARG, "packed steps need Euler SSP-RK3 contexts without the Liou fix on "
                              "the tiled kernels with a gradient pass of their own");
     if (c->P.flux != cs[0]->P.flux || c->P.reconstruct != cs[0]->P.reconstruct)
@@ -1110,19 +1122,18 @@ extern "C" int tsm_run_packed(tsm_ctx** cs, int n, long nsteps, long* done) {
   for (int r = 0; r < 3; ++r) {
     for (int i = 0; i < n; ++i) {
       tsm_ctx* c = cs[i];
-      double* Wn = c->W[c->cur];
-      double* Wa = c->W[(c->cur + 1) % 3];
-      double* Wb = c->W[(c->cur + 2) % 3];
-      const double* ins[3] = {Wn, Wa, Wb};
-      double* outs[3] = {Wa, Wb, Wn};
+      const int ia = (c->cur + 1) % 3, ib = (c->cur + 2) % 3;
+      const int ins[3] = {c->cur, ia, ib}, outs[3] = {ia, ib, c->cur};
       tsm::PackLevel& L = lv[(size_t)r * n + i];
       L.G = c->G;
-      L.TG = c->TG;
+      L.T = c->ST;
       L.A = c->A;
-      L.A.W_in = ins[r];
-      L.A.W_out = outs[r];
+      L.A.W_in = c->W[ins[r]];
+      L.A.W_out = c->W[outs[r]];
+      L.A.V_in = c->V[ins[r]];
+      L.A.V_out = c->V[outs[r]];
       L.P = c->SP;
-      L.Wn = Wn;
+      L.Wn = c->W[c->cur];
       L.dtpart = c->dtpart;
       L.S = c->S;
     }
@@ -1143,7 +1154,6 @@ extern "C" int tsm_run_packed(tsm_ctx** cs, int n, long nsteps, long* done) {
   for (long k = 0; k < nsteps; ++k) {
     for (int r = 0; r < 3; ++r) {
       const tsm::PackLevel* d = c0->pack + (size_t)r * n;
-      tsm::launch_packed_gradient(d, plan, st);
       tsm::launch_packed_stage(c0->P.flux, c0->P.reconstruct, d, plan, r, r == 2, st);
     }
     tsm::launch_packed_final(c0->pack, plan, st);
@@ -1378,15 +1388,13 @@ extern "C" int tsm_bench(tsm_ctx* c, int nsteps, double* us) {
     const int nrk = c->P.time_scheme == 0 ? 3 : (c->P.time_scheme == 1 ? 4 : 2);
     for (int k = 0; k < nsteps; ++k) {
       enqueue_tiled_step(c, -1, ev);
-      HIP_TRY(hipEventSynchronize(ev[2 * nrk + 1]));
+      HIP_TRY(hipEventSynchronize(ev[nrk + 1]));
       for (int r = 0; r < nrk; ++r) {
-        HIP_TRY(hipEventElapsedTime(&ms, ev[2 * r], ev[2 * r + 1])); acc[1] += ms;
-        HIP_TRY(hipEventElapsedTime(&ms, ev[2 * r + 1], ev[2 * r + 2])); acc[2] += ms;
+        HIP_TRY(hipEventElapsedTime(&ms, ev[r], ev[r + 1])); acc[2] += ms;
       }
-      HIP_TRY(hipEventElapsedTime(&ms, ev[2 * nrk], ev[2 * nrk + 1])); acc[3] += ms;
+      HIP_TRY(hipEventElapsedTime(&ms, ev[nrk], ev[nrk + 1])); acc[3] += ms;
     }
-    us[0] = 0.0;
-    us[1] = 1e3 * acc[1] / ((double)nrk * nsteps);
+    us[0] = us[1] = 0.0;
     us[2] = 1e3 * acc[2] / ((double)nrk * nsteps);
     us[3] = 1e3 * acc[3] / nsteps;
   } else {

@@ -59,30 +59,58 @@ struct DevGeo {
   const unsigned char* snoslip;  // nv
 };
 
-// One operand record per (vertex of k_grad_bnd, cell of that vertex), in the
-// vertex's cell order: the cell's corners (new ids), its non-periodic boundary
-// faces in bface order (-1: none) and, 2 bits each, the corner (0..2) at each
-// end of each of them (bf0 end 0, bf0 end 1, bf1 end 0, bf1 end 1).
-struct alignas(16) GbEntry {
-  int a, b, d, ends;
-  int bf0, bf1, pad0, pad1;
-};
-
-// Tile arrays of the LDS-staged kernels (device pointers, new vertex ids).
+// Tile arrays (device pointers, new vertex ids); the stage kernel's own
+// tables are made from them (StageTab).
 struct TileGeo {
   int ntiles, tb, max_slots, max_faces;
-  int grad_block, fu_block;  // requested threads per tile (0: smallest that fits)
+  int fu_block;              // requested threads per tile (0: smallest that fits)
   int n_periodic_tiles;      // tiles [0, n) hold the periodic sets
-  int n_gbv;                 // vertices of k_grad_bnd
+  int n_gbv;                 // vertices with a boundary-corrected cell
   const int* gbv;            // their ids
-  const int* gb_ptr;         // n_gbv+1: their records [gb_ptr[i], gb_ptr[i+1])
-  const GbEntry* gb_ent;
-  int fused, max_slots1;     // two-ring tiles: gradients formed inside the stage kernel
-  const int *h2beg, *halo2, *g1beg, *g1ptr, *g1cgid;
-  const unsigned* g1ent;
   const int *vbeg, *hbeg, *halo, *fbeg, *bbeg, *tbf, *gptr, *cptr, *cgid, *tper, *pinfo;
   const unsigned *f_lr, *cent;
   const double* f_n;
+  const unsigned short* gent;
+};
+
+// 16-bit items of a gradient slot (StageTab::items): bits 15..14 say what
+// it is (a neighbour; a new centre; a boundary term of the tile; the end or
+// "more in the overflow list"), bit 13 is a flag (neighbour: the cell that ends
+// in it is a wall cell; centre: it is the slot's own vertex), bit 12 marks the
+// first neighbour of a closed chain, bits 11..0 are the slot or the term.
+constexpr unsigned SI_CENTRE = 0x4000u, SI_TERM = 0x8000u, SI_END = 0xc000u, SI_MORE = 0xc001u,
+                   SI_FLAG = 0x2000u, SI_CLOSED = 0x1000u;
+constexpr int SI_MASK = 0x0fff;
+// 16-bit gather entries (StageTab::ge8): local face | bit 15 at the right end;
+// bit 14: no further entries, or further ones in gent from this position on
+constexpr unsigned GE_END = 0x7fffu, GE_MORE = 0x7ffeu;
+
+// Tables of the stage kernel (tsm_stagetab.hip), each with one stride per tile.
+struct StageTab {
+  int ntiles, tb, n_periodic_tiles, fu_block;
+  int ms, ms1, mf, mbt, mwt, mc;  // largest counts of a tile: slots, gradient slots,
+                              // local faces, boundary terms, wall terms, viscous cells
+  const int4* desc;           // first owned vertex, owned, gradient slots,
+                              // local faces | bit 30: items other than neighbours
+  const int* sid;             // ms per tile: vertex of each slot, -1 past the last
+  const unsigned* f_lr;       // mf per tile: left slot | right slot << 16
+  const double2* f_n;         // mf per tile: normals
+  const double2* xy;          // per vertex
+  const uint4* items;         // ms1 per tile: eight items per gradient slot ...
+  const uint4* items2;        // ... and eight more (tiles marked in desc)
+  const int* item_ov;         // ms1 per tile: where SI_MORE continues in ov
+  const unsigned short* ov;
+  const uint4* ge8;           // per vertex: eight gather entries
+  const unsigned* vcells;     // mc per tile: corner slots of the viscous cells (3 x 10 bits),
+                              // all ones past the last
+  const uint4* vc8;           // per vertex: its first eight viscous cells (| corner << 13)
+  const int* vccnt;           // per vertex: how many there are ...
+  const unsigned short* vcent;  // ... all of them, along DevGeo::vc
+  const int *btbeg, *bt;      // boundary terms of each tile (bfaces)
+  const int *wtbeg, *wt;      // wall terms of each tile (bfaces), null without wall cells
+  const uint2* wcell;         // their cells' corner slots
+  const unsigned short* wvent;  // along vbe: term | corner << 13 | ends the bface << 15
+  const int *tper, *pinfo, *gptr, *bbeg, *tbf;
   const unsigned short* gent;
 };
 
@@ -100,7 +128,7 @@ struct BcTime {
 };
 
 struct ViscParams {
-  double mu_ref, T_ref, T_0, omega, prandtl;
+  double mu_ref, T_ref, T_0, omega, prandtl, iprandtl;
   int mu_model, visc_active, heat_active;
 };
 
@@ -273,6 +301,7 @@ struct StepParams {
 struct StageArgs {
   size_t cs, fs, off;
   const double* W_in; double* W_out;
+  const double* V_in; double* V_out;  // first entropy variable of W_in / W_out (tiled path)
   double* E_in; double* E_out;
   double* Uold;
   double* dE;      // 8 components
@@ -308,48 +337,41 @@ __device__ __forceinline__ Gas load_gas(const StageArgs& A, int s) {
 // parameters, and where its blocks start in each packed grid.
 struct PackLevel {
   DevGeo G;
-  TileGeo TG;
+  StageTab T;
   StageArgs A;
   StepParams P;
   const double* Wn;   // W^n (read by every stage for U_old)
   double* dtpart;     // per-block dt partials
   int S;              // samples
-  int base_fu, base_gper, base_grest, base_gbnd, base_final;
+  int base_fu, base_final;
 };
 // Grid totals of a packed step over nl levels (computed by pack_plan).
 struct PackPlan {
   int nl;
-  int fu_blocks, gper_blocks, grest_blocks, gbnd_blocks, final_blocks;
-  int fu_block, grad_block;   // threads per block: the largest any level needs
-  size_t fu_lds, grad_lds;    // dynamic LDS: the largest any level needs
-  bool grad_pass;
+  int fu_blocks, final_blocks;
+  int fu_block;      // threads per block: the largest any level needs
+  size_t fu_lds;     // dynamic LDS: the largest any level needs
 };
 // Fills the block bases of lv[0..nl) and the plan (host).
 void pack_plan(PackLevel* lv, int nl, int flux, int rec, PackPlan& plan);
-void launch_packed_gradient(const PackLevel* d, const PackPlan& p, hipStream_t st);
 void launch_packed_stage(int flux, int rec, const PackLevel* d, const PackPlan& p, int r,
                          bool last, hipStream_t st);
 void launch_packed_final(const PackLevel* d, const PackPlan& p, hipStream_t st);
 
-// LDS-staged tile kernels (Euler, SSP-RK3)
-size_t tile_grad_lds(const TileGeo& T);
-int tile_grad_block(const TileGeo& T);
-int tile_fu_block(const TileGeo& T);
-int tile_fu_block_max();
-bool tile_needs_gradient_pass(const TileGeo& T, int flux, int rec);
-// Builds gb_ptr / gb_ent of T (n_gbv > 0) from its cell entries and G on the
-// stream; memory from dalloc.  TSM_OK, or TSM_E_* with msg.
-int build_grad_bnd_table(const DevGeo& G, TileGeo& T, const std::function<int(void**, size_t)>& dalloc,
-                         hipStream_t st, std::string& msg);
-void launch_tile_gradient_bnd(const DevGeo& G, const TileGeo& T, const StageArgs& A, int S,
-                              hipStream_t st);
-size_t tile_fu_lds(const TileGeo& T, int flux, int rec);
-size_t tile_fu_lds_ns(const TileGeo& T, int flux, int rec);
-void launch_tile_gradient(const DevGeo& G, const TileGeo& T, const StageArgs& A, int S,
-                          hipStream_t st);
-void launch_tile_stage(int flux, int rec, const DevGeo& G, const TileGeo& T, const StageArgs& A,
-                       const StepParams& P, const double* Wn, double* dtpart, int S, int r,
-                       bool last, hipStream_t st);
+// Stage kernel (tsm_stage.hip) and its tables (tsm_stagetab.hip).
+// build_stage_tables: 0 = built, 1 = the tiles are too large for it (msg),
+// TSM_E_* with msg; memory from dalloc.
+int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, bool walls,
+                       StageTab& S, const std::function<int(void**, size_t)>& dalloc, hipStream_t st,
+                       std::string& msg);
+int stage_block(const StageTab& T);
+int stage_block_max();
+size_t stage_lds(const StageTab& T, int flux, int rec, bool ns);
+bool stage_has_gradients(int flux, int rec);
+bool stage_keeps_var0(int flux);
+void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const StageArgs& A,
+                  const StepParams& P, const double* Wn, double* dtpart, int S, int r, bool last,
+                  hipStream_t st);
 void launch_step_final_tiled(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                              int nblk, const double* dtpart, int log_slot, hipStream_t st);
 

@@ -466,6 +466,8 @@ __global__ __launch_bounds__(256) void k_dt(DevGeo G, StageArgs A, StepParams P)
     Prim w = load_prim(A.W_in, off + v);
     Cons U = prim2con(gas, w);
     reinterpret_cast<double4*>(A.Uold)[off + v] = make_double4(U.m, U.mx, U.my, U.e);
+    // the tiled path's per-vertex entropy variable of the state it starts from
+    if (A.V_out) A.V_out[off + v] = entropy_var0(gas, w);
     if (P.time_step > 0.0) {
       dtv = P.time_step;
     } else {

@@ -1,0 +1,649 @@
+// tsm_stagetab.hip -- the tables of the stage kernel (tsm_stage.hip), built on
+// the device from a tiling and the mesh incidences.
+//
+// The stage kernel forms the gradients of a tile's owned vertices and of the
+// first halo ring itself, so a tile's slots are its owned vertices, the first
+// ring (the tiling's halo) and, for schemes with gradients, the second ring:
+// the corners of the first ring's cells.  Around each of these "gradient
+// slots" the kernel walks the neighbours in ring order, so every neighbour is
+// read once and each pair of successive neighbours is a cell (a fan).  Every
+// per-tile table has one stride for all tiles: a block finds its entries from
+// its tile number alone, without first loading an offset.
+//
+// Fans depend on the cell order and orientation only, never on the tiles, so
+// the sums taken along them are the same bit for bit whatever the tile size
+// and whichever tile forms them.
+#include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>
+
+#include <algorithm>
+#include <functional>
+#include <string>
+#include <type_traits>
+#include <vector>
+
+#include "tsm_device.h"
+
+namespace tsm {
+namespace {
+
+constexpr unsigned FAN_START = 0x80000000u, FAN_WALL = 0x40000000u, FAN_CLOSED = 0x20000000u,
+                   FAN_V = 0x1fffffffu;
+
+template <class T>
+struct Tmp {  // device array freed on scope exit
+  T* p = nullptr;
+  hipError_t alloc(size_t n) { return hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)); }
+  ~Tmp() { if (p) (void)hipFree(p); }
+};
+inline unsigned nblk(long long n) { return (unsigned)((std::max(n, 1LL) + 255) / 256); }
+
+// The fan of vertex v: chains of neighbours such that each successive pair
+// (b, d) is a cell (v, b, d) in counter-clockwise order; in a closed chain the
+// last and the first are one too.  A closed ring starts at the vertex's first
+// cell, an open one at the cell without a predecessor.  An entry's wall flag
+// belongs to the cell that ends in it (a closed chain's first entry: the cell
+// from its last).  Returns the entry count and, with out, writes the entries.
+__device__ int fan_of(const DevGeo& G, int v, unsigned char* used, unsigned* out) {
+  const int e0 = G.vc_ptr[v], e1 = G.vc_ptr[v + 1];
+  auto ends = [&](int e, int& b, int& d, int& c) {
+    c = G.vc[e] & 0x7fffffff;
+    const int a0 = G.cv[3 * (size_t)c], a1 = G.cv[3 * (size_t)c + 1], a2 = G.cv[3 * (size_t)c + 2];
+    if (a0 == v) { b = a1; d = a2; }
+    else if (a1 == v) { b = a2; d = a0; }
+    else { b = a0; d = a1; }
+  };
+  for (int e = e0; e < e1; ++e) used[e] = 0;
+  int n = 0, left = e1 - e0;
+  while (left > 0) {
+    int start = -1;
+    for (int e = e0; e < e1; ++e) {
+      if (used[e]) continue;
+      if (start < 0) start = e;
+      int b, d, c, b2, d2, c2;
+      ends(e, b, d, c);
+      bool pred = false;
+      for (int f = e0; f < e1 && !pred; ++f)
+        if (!used[f] && f != e) { ends(f, b2, d2, c2); pred = d2 == b; }
+      if (!pred) { start = e; break; }
+    }
+    int cur = start, b, d, c;
+    ends(cur, b, d, c);
+    const int first = b, n0 = n;
+    if (out) out[n] = (unsigned)b | FAN_START;
+    ++n;
+    while (cur >= 0) {
+      used[cur] = 1;
+      --left;
+      const unsigned wall = G.cnb[c] ? FAN_WALL : 0u;
+      const int from = d;
+      cur = -1;
+      if (d == first) {  // back where the chain began
+        if (out) out[n0] |= FAN_CLOSED | wall;
+        break;
+      }
+      if (out) out[n] = (unsigned)d | wall;
+      ++n;
+      for (int f = e0; f < e1; ++f) {
+        if (used[f]) continue;
+        ends(f, b, d, c);
+        if (b == from) { cur = f; break; }
+      }
+    }
+  }
+  return n;
+}
+__global__ void k_fan(DevGeo G, unsigned char* used, const int* ptr, int* cnt, unsigned* fan) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v > G.nv) return;
+  if (v == G.nv) { if (cnt) cnt[v] = 0; return; }
+  const int n = fan_of(G, v, used, fan ? fan + ptr[v] : nullptr);
+  if (cnt) cnt[v] = n;
+}
+
+struct TabIn {
+  DevGeo G;
+  int nt, grad;
+  const int *vbeg, *hbeg, *halo;   // the tiling: owned ranges, first ring
+  const int *h2beg, *halo2;        // second ring (null while it is being found)
+  const int *fan_ptr;
+  const unsigned* fan;
+  const int *btbeg, *bt;           // boundary terms (null while they are being found)
+};
+
+// gradient slots of all tiles as one range: those of tile t start at
+// vbeg[t] + hbeg[t] (owned and first ring), or at vbeg[t] without gradients
+__device__ __forceinline__ int gs_beg(const TabIn& T, int t) {
+  return T.vbeg[t] + (T.grad ? T.hbeg[t] : 0);
+}
+__device__ __forceinline__ void gs_find(const TabIn& T, int q, int& t, int& k, int& v) {
+  int lo = 0, hi = T.nt;
+  while (hi - lo > 1) {
+    const int m = (lo + hi) >> 1;
+    if (gs_beg(T, m) <= q) lo = m; else hi = m;
+  }
+  t = lo;
+  k = q - gs_beg(T, t);
+  const int nown = T.vbeg[t + 1] - T.vbeg[t];
+  v = k < nown ? T.vbeg[t] + k : T.halo[T.hbeg[t] + k - nown];
+}
+__device__ __forceinline__ int tile_of(const TabIn& T, int v) {
+  int lo = 0, hi = T.nt;
+  while (hi - lo > 1) {
+    const int m = (lo + hi) >> 1;
+    if (T.vbeg[m] <= v) lo = m; else hi = m;
+  }
+  return lo;
+}
+__device__ __forceinline__ int find32(const int* a, int lo, int hi, int k) {
+  while (lo < hi) {
+    const int m = (lo + hi) >> 1;
+    if (a[m] < k) lo = m + 1; else hi = m;
+  }
+  return lo;
+}
+// slot of vertex u in tile t, -1 if it has none (yet)
+__device__ __forceinline__ int slot_in(const TabIn& T, int t, int u) {
+  const int b0 = T.vbeg[t], b1 = T.vbeg[t + 1];
+  if (u >= b0 && u < b1) return u - b0;
+  const int h0 = T.hbeg[t], h1 = T.hbeg[t + 1];
+  int k = find32(T.halo, h0, h1, u);
+  if (k < h1 && T.halo[k] == u) return (b1 - b0) + (k - h0);
+  if (!T.h2beg) return -1;
+  const int r0 = T.h2beg[t], r1 = T.h2beg[t + 1];
+  k = find32(T.halo2, r0, r1, u);
+  return (k < r1 && T.halo2[k] == u) ? (b1 - b0) + (h1 - h0) + (k - r0) : -1;
+}
+
+// The items of a gradient slot: for each member of the vertex's periodic set
+// (the vertex alone without one), a centre entry where the centre is not the
+// slot itself from the start, then the member's fan, then the boundary terms of
+// all members' cells.  f(kind, id, flag, closed): kind 0 neighbour (flag: wall
+// cell; closed: first of a closed chain), 1 centre (flag: the slot's own vertex),
+// 2 boundary term of bface id.
+template <class F>
+__device__ void walk_items(const TabIn& T, int v, F&& f) {
+  const DevGeo& G = T.G;
+  const int p = G.pset[v];
+  const int m0 = p < 0 ? 0 : G.pptr[p], m1 = p < 0 ? 1 : G.pptr[p + 1];
+  for (int i = m0; i < m1; ++i) {
+    const int m = p < 0 ? v : G.pv[i];
+    if (!(i == m0 && m == v)) f(1, m, m == v, false);
+    for (int e = T.fan_ptr[m]; e < T.fan_ptr[m + 1]; ++e) {
+      const unsigned x = T.fan[e];
+      if ((x & FAN_START) && e > T.fan_ptr[m]) f(1, m, m == v, false);
+      f(0, (int)(x & FAN_V), (x & FAN_WALL) != 0, (x & FAN_CLOSED) != 0);
+    }
+  }
+  for (int i = m0; i < m1; ++i) {
+    const int m = p < 0 ? v : G.pv[i];
+    for (int e = G.vc_ptr[m]; e < G.vc_ptr[m + 1]; ++e) {
+      const int c = G.vc[e] & 0x7fffffff;
+      for (int z = 0; z < 2; ++z) {
+        const int b = G.cbf[2 * (size_t)c + z];
+        if (b < 0) break;
+        if (bc_sets_state(G.btype[b])) f(2, b, false, false);
+      }
+    }
+  }
+}
+
+// per gradient slot: second-ring candidates, boundary terms, items
+__global__ void k_gs_count(TabIn T, int nq, int* n2, int* nbt, int* nit) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q > nq) return;
+  int c2 = 0, cb = 0, ci = 0;
+  if (q < nq) {
+    int t, k, v;
+    gs_find(T, q, t, k, v);
+    walk_items(T, v, [&](int kind, int id, bool, bool) {
+      ++ci;
+      if (kind == 2) ++cb;
+      else if (slot_in(T, t, id) < 0) ++c2;
+    });
+  }
+  n2[q] = c2; nbt[q] = cb; nit[q] = ci;
+}
+__global__ void k_gs_emit(TabIn T, int nq, const int* o2, const int* ob, unsigned long long* k2,
+                          unsigned long long* kb) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nq) return;
+  int t, k, v;
+  gs_find(T, q, t, k, v);
+  int a = o2[q], b = ob[q];
+  walk_items(T, v, [&](int kind, int id, bool, bool) {
+    const unsigned long long key = ((unsigned long long)(unsigned)t << 32) | (unsigned)id;
+    if (kind == 2) kb[b++] = key;
+    else if (slot_in(T, t, id) < 0) k2[a++] = key;
+  });
+}
+__global__ void k_seg(int n, const unsigned long long* keys, const int* nkeys, int* ptr) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > n) return;
+  const unsigned long long k = (unsigned long long)(unsigned)i << 32;
+  int lo = 0, hi = *nkeys;
+  while (lo < hi) {
+    const int m = (lo + hi) >> 1;
+    if (keys[m] < k) lo = m + 1; else hi = m;
+  }
+  ptr[i] = lo;
+}
+__global__ void k_low(int n, const unsigned long long* keys, int* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = (int)(unsigned)(keys[i] & 0xffffffffull);
+}
+
+// descriptors and the largest counts: mx = slots, gradient slots, local
+// faces, boundary terms, wall terms, viscous cells
+__global__ void k_desc(TabIn T, const int* fbeg, const int* wtbeg, const int* tcbeg,
+                       const unsigned char* special, int4* desc, int* mx) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= T.nt) return;
+  const int nown = T.vbeg[t + 1] - T.vbeg[t], n1 = nown + T.hbeg[t + 1] - T.hbeg[t];
+  const int ns = n1 + (T.h2beg ? T.h2beg[t + 1] - T.h2beg[t] : 0);
+  const int nf = fbeg[t + 1] - fbeg[t];
+  if (desc) desc[t] = make_int4(T.vbeg[t], nown, n1, nf | (special[t] ? 0x40000000 : 0));
+  if (mx) {
+    atomicMax(mx, ns);
+    atomicMax(mx + 1, n1);
+    atomicMax(mx + 2, nf);
+    if (T.btbeg) atomicMax(mx + 3, T.btbeg[t + 1] - T.btbeg[t]);
+    if (wtbeg) atomicMax(mx + 4, wtbeg[t + 1] - wtbeg[t]);
+    if (tcbeg) atomicMax(mx + 5, tcbeg[t + 1] - tcbeg[t]);
+  }
+}
+__global__ void k_fill_sid(TabIn T, int ms, int* sid) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)T.nt * ms) return;
+  const int t = (int)(i / ms);
+  int k = (int)(i % ms);
+  const int nown = T.vbeg[t + 1] - T.vbeg[t], nh = T.hbeg[t + 1] - T.hbeg[t];
+  const int n2 = T.h2beg ? T.h2beg[t + 1] - T.h2beg[t] : 0;
+  int v = -1;
+  if (k < nown) v = T.vbeg[t] + k;
+  else if ((k -= nown) < nh) v = T.halo[T.hbeg[t] + k];
+  else if ((k -= nh) < n2) v = T.halo2[T.h2beg[t] + k];
+  sid[i] = v;
+}
+__global__ void k_fill_faces(int nt, int mf, const int* fbeg, const unsigned* f_lr,
+                             const double* f_n, unsigned* lr, double2* n) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)nt * mf) return;
+  const int t = (int)(i / mf), j = (int)(i % mf);
+  const bool in = j < fbeg[t + 1] - fbeg[t];
+  const size_t o = (size_t)fbeg[t] + j;
+  lr[i] = in ? f_lr[o] : 0u;
+  n[i] = in ? make_double2(f_n[2 * o], f_n[2 * o + 1]) : make_double2(1.0, 0.0);
+}
+__global__ void k_xy(int nv, const double* x, const double* y, double2* xy) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nv) xy[i] = make_double2(x[i], y[i]);
+}
+// entries that do not fit the slot's sixteen
+__global__ void k_ov_count(int nq, const int* nit, int* nov) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q <= nq) nov[q] = (q < nq && nit[q] > 16) ? nit[q] - 15 + 1 : 0;  // entries 15.. and an end
+}
+__device__ __forceinline__ uint4 pack8(const unsigned* w) {
+  return make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
+}
+// the items of each gradient slot (codes in tsm_device.h): eight in items, the
+// next eight in items2 (read by tiles marked special only), the rest in ov;
+// special[t] is set where a tile has anything but chains of up to eight neighbours
+__global__ void k_fill_items(TabIn T, int nq, int ms1, const int* nit, const int* ovp, uint4* items,
+                             uint4* items2, int* item_ov, unsigned short* ov,
+                             unsigned char* special, int* bad) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nq) return;
+  int t, k, v;
+  gs_find(T, q, t, k, v);
+  unsigned w[16];
+  for (int u = 0; u < 16; ++u) w[u] = SI_END;
+  const bool over = nit[q] > 16;
+  int n = 0, o = ovp[q];
+  bool sp = nit[q] > 8;
+  walk_items(T, v, [&](int kind, int id, bool flag, bool closed) {
+    unsigned e;
+    if (kind == 2) {
+      const int b0 = T.btbeg[t], b1 = T.btbeg[t + 1];
+      const int j = find32(T.bt, b0, b1, id) - b0;
+      if (j > SI_MASK) atomicOr(bad, 1);
+      e = SI_TERM | (unsigned)(j & SI_MASK);
+    } else {
+      const int s = slot_in(T, t, id);
+      if (s < 0 || s > SI_MASK) atomicOr(bad, 1);
+      e = (kind == 1 ? SI_CENTRE : 0u) | (flag ? SI_FLAG : 0u) | (closed ? SI_CLOSED : 0u) |
+          (unsigned)(s & SI_MASK);
+    }
+    sp = sp || kind != 0;
+    if (!over || n < 15) w[n] = e;
+    else ov[o++] = (unsigned short)e;
+    ++n;
+  });
+  if (over) { w[15] = SI_MORE; ov[o] = SI_END; }
+  const size_t at = (size_t)t * ms1 + k;
+  items[at] = pack8(w);
+  items2[at] = pack8(w + 8);
+  item_ov[at] = ovp[q];
+  if (sp) special[t] = 1;
+}
+__global__ void k_no_items(long long n, uint4* items, uint4* items2, int* item_ov) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const unsigned e = SI_END | (SI_END << 16);
+  items[i] = items2[i] = make_uint4(e, e, e, e);
+  item_ov[i] = 0;
+}
+// the first eight gather entries of each vertex
+__global__ void k_ge8(int nv, const int* gptr, const unsigned short* gent, uint4* ge8) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= nv) return;
+  const int k0 = gptr[v], n = gptr[v + 1] - k0;
+  int nf = 0;
+  while (nf < n && !(gent[k0 + nf] & 0x4000u)) ++nf;
+  unsigned w[8];
+  for (int u = 0; u < 8; ++u) w[u] = GE_END;
+  const int m = (n <= 8 && nf == n) ? n : min(nf, 7);
+  for (int u = 0; u < m; ++u) w[u] = gent[k0 + u];
+  if (m < n) w[m] = GE_MORE;
+  ge8[v] = pack8(w);
+}
+// viscous cells: (tile, cell) of every cell of an owned vertex that is no wall cell
+__global__ void k_vcell_keys(TabIn T, unsigned long long* keys) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int t = tile_of(T, v);
+  for (int e = T.G.vc_ptr[v]; e < T.G.vc_ptr[v + 1]; ++e) {
+    const int c = T.G.vc[e] & 0x7fffffff;
+    keys[e] = T.G.cnb[c] ? ~0ull : ((unsigned long long)(unsigned)t << 32) | (unsigned)c;
+  }
+}
+// their corners as slots, one stride per tile
+__global__ void k_vcells(TabIn T, int mc, const int* beg, const int* cells, unsigned* out, int* bad) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)T.nt * mc) return;
+  const int t = (int)(i / mc), j = (int)(i % mc);
+  unsigned x = ~0u;
+  if (j < beg[t + 1] - beg[t]) {
+    const int c = cells[beg[t] + j];
+    x = 0;
+    for (int z = 0; z < 3; ++z) {
+      const int s = slot_in(T, t, T.G.cv[3 * (size_t)c + z]);
+      if (s < 0 || s > 1023) atomicOr(bad, 1);
+      x |= (unsigned)(s & 1023) << (10 * z);
+    }
+  }
+  out[i] = x;
+}
+// per vertex, in cell order: the tile's viscous cell | the vertex's corner << 13
+// (along G.vc; wall cells leave no entry), and the first eight of them packed
+__global__ void k_vcell_entries(TabIn T, const int* beg, const int* cells, unsigned short* ent,
+                                int* cnt, uint4* vc8, int* bad) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int t = tile_of(T, v);
+  int n = 0;
+  unsigned w[8];
+  for (int u = 0; u < 8; ++u) w[u] = GE_END;
+  for (int e = T.G.vc_ptr[v]; e < T.G.vc_ptr[v + 1]; ++e) {
+    const int c = T.G.vc[e] & 0x7fffffff;
+    if (T.G.cnb[c]) continue;
+    const int j = find32(cells, beg[t], beg[t + 1], c) - beg[t];
+    const int z = T.G.cv[3 * (size_t)c] == v ? 0 : (T.G.cv[3 * (size_t)c + 1] == v ? 1 : 2);
+    if (j > 0x1fff) atomicOr(bad, 1);
+    const unsigned x = ((unsigned)z << 13) | (unsigned)(j & 0x1fff);
+    ent[T.G.vc_ptr[v] + n] = (unsigned short)x;
+    if (n < 8) w[n] = x;
+    ++n;
+  }
+  cnt[v] = n;
+  vc8[v] = pack8(w);
+}
+// wall terms: (tile, bface) of every bface whose cell holds an owned vertex
+__global__ void k_wall_keys(TabIn T, unsigned long long* keys) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int t = tile_of(T, v);
+  for (int e = T.G.vbe_ptr[v]; e < T.G.vbe_ptr[v + 1]; ++e)
+    keys[e] = ((unsigned long long)(unsigned)t << 32) | ((unsigned)T.G.vbe[e] & 0x7fffffffu);
+}
+__global__ void k_wall_cells(TabIn T, const int* wtbeg, const int* wt, uint2* wcell, int* bad) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= T.nt) return;
+  for (int j = wtbeg[t]; j < wtbeg[t + 1]; ++j) {
+    const int c = T.G.blc[wt[j]];
+    int s[3];
+    for (int z = 0; z < 3; ++z) {
+      s[z] = slot_in(T, t, T.G.cv[3 * (size_t)c + z]);
+      if (s[z] < 0 || s[z] > SI_MASK) { atomicOr(bad, 1); s[z] = 0; }
+    }
+    wcell[j] = make_uint2((unsigned)s[0] | ((unsigned)s[1] << 16), (unsigned)s[2]);
+  }
+}
+// per (vertex, bface) in bface order: the tile's wall term, the vertex's corner
+// of the cell and whether the vertex ends the bface
+__global__ void k_wall_entries(TabIn T, const int* wtbeg, const int* wt, unsigned short* wvent, int* bad) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int t = tile_of(T, v);
+  for (int e = T.G.vbe_ptr[v]; e < T.G.vbe_ptr[v + 1]; ++e) {
+    const unsigned x = (unsigned)T.G.vbe[e];
+    const int b = (int)(x & 0x7fffffffu), c = T.G.blc[b];
+    const int j = find32(wt, wtbeg[t], wtbeg[t + 1], b) - wtbeg[t];
+    const int z = T.G.cv[3 * (size_t)c] == v ? 0 : (T.G.cv[3 * (size_t)c + 1] == v ? 1 : 2);
+    if (j > SI_MASK) atomicOr(bad, 1);
+    wvent[e] = (unsigned short)((x >> 31 ? 0x8000u : 0u) | ((unsigned)z << 13) | (unsigned)(j & SI_MASK));
+  }
+}
+__global__ void k_zero(long long n, unsigned char* p) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+}  // namespace
+
+int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, bool walls,
+                       StageTab& S, const std::function<int(void**, size_t)>& dalloc, hipStream_t st,
+                       std::string& msg) {
+#define TT(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { msg = std::string("stage tables: ") + hipGetErrorString(e_); return TSM_E_HIP; } } while (0)
+#define TA(ptr, n) do { void* q_ = nullptr; int r_ = dalloc(&q_, std::max<size_t>((size_t)(n), 1) * sizeof(*(ptr))); if (r_) { msg = "stage tables: allocation"; return r_; } (ptr) = static_cast<std::remove_reference_t<decltype(ptr)>>(q_); } while (0)
+#define GO(k, n, ...) hipLaunchKernelGGL(k, dim3(nblk(n)), dim3(256), 0, st, __VA_ARGS__)
+  const int nv = G.nv, nt = TG.ntiles;
+  S = StageTab{};
+  S.ntiles = nt; S.tb = TG.tb; S.fu_block = TG.fu_block; S.n_periodic_tiles = TG.n_periodic_tiles;
+  S.tper = TG.tper; S.pinfo = TG.pinfo; S.gptr = TG.gptr; S.gent = TG.gent; S.bbeg = TG.bbeg; S.tbf = TG.tbf;
+  int nhalo = 0;
+  TT(hipMemcpyAsync(&nhalo, TG.hbeg + nt, sizeof(int), hipMemcpyDeviceToHost, st));
+  TT(hipStreamSynchronize(st));
+  const int nq = nv + (grad ? nhalo : 0);
+  TabIn T{};
+  T.G = G; T.nt = nt; T.grad = grad ? 1 : 0;
+  T.vbeg = TG.vbeg; T.hbeg = TG.hbeg; T.halo = TG.halo;
+  Tmp<char> tmp;
+  size_t tmp_bytes = 0;
+  auto scan = [&](const int* in, int* out, int n) -> hipError_t {
+    size_t b = 0;
+    hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st);
+    if (e == hipSuccess && b > tmp_bytes) {
+      if (tmp.p) (void)hipFree(tmp.p);
+      tmp.p = nullptr;
+      e = tmp.alloc(b);
+      tmp_bytes = e == hipSuccess ? b : 0;
+    }
+    return e == hipSuccess ? hipcub::DeviceScan::ExclusiveSum(tmp.p, b, in, out, n, st) : e;
+  };
+  // sorted distinct keys: list (low words) and per-tile pointers
+  auto group = [&](Tmp<unsigned long long>& k, int n, int** beg, int** list, int& count) -> int {
+    Tmp<unsigned long long> ks, ku;
+    Tmp<int> nu;
+    TT(ks.alloc(n)); TT(ku.alloc(n)); TT(nu.alloc(1));
+    count = 0;
+    if (n > 0) {
+      size_t b1 = 0, b2 = 0;
+      TT(hipcub::DeviceRadixSort::SortKeys(nullptr, b1, k.p, ks.p, n, 0, 64, st));
+      TT(hipcub::DeviceSelect::Unique(nullptr, b2, ks.p, ku.p, nu.p, n, st));
+      Tmp<char> t2;
+      TT(t2.alloc(std::max(b1, b2)));
+      TT(hipcub::DeviceRadixSort::SortKeys(t2.p, b1, k.p, ks.p, n, 0, 64, st));
+      TT(hipcub::DeviceSelect::Unique(t2.p, b2, ks.p, ku.p, nu.p, n, st));
+      TT(hipMemcpyAsync(&count, nu.p, sizeof(int), hipMemcpyDeviceToHost, st));
+      TT(hipStreamSynchronize(st));
+    } else {
+      TT(hipMemcpyAsync(nu.p, &count, sizeof(int), hipMemcpyHostToDevice, st));
+      TT(hipStreamSynchronize(st));
+    }
+    if (count > 0) {  // entries to be left out sort last as all ones
+      unsigned long long last = 0;
+      TT(hipMemcpyAsync(&last, ku.p + count - 1, sizeof(last), hipMemcpyDeviceToHost, st));
+      TT(hipStreamSynchronize(st));
+      if (last == ~0ull) {
+        --count;
+        TT(hipMemcpyAsync(nu.p, &count, sizeof(int), hipMemcpyHostToDevice, st));
+        TT(hipStreamSynchronize(st));
+      }
+    }
+    TA(*beg, nt + 1);
+    TA(*list, count);
+    GO(k_seg, nt + 1, nt, ku.p, nu.p, *beg);
+    if (count > 0) GO(k_low, count, count, ku.p, *list);
+    TT(hipStreamSynchronize(st));
+    return 0;
+  };
+  Tmp<int> mx, bad;
+  TT(mx.alloc(8)); TT(bad.alloc(1));
+  {
+    const int z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    TT(hipMemcpyAsync(mx.p, z, sizeof(z), hipMemcpyHostToDevice, st));
+    TT(hipMemcpyAsync(bad.p, z, sizeof(int), hipMemcpyHostToDevice, st));
+    TT(hipStreamSynchronize(st));
+  }
+  Tmp<unsigned char> special;
+  TT(special.alloc(nt));
+  GO(k_zero, nt, (long long)nt, special.p);
+  Tmp<int> fan_ptr, nit, ovp;
+  Tmp<unsigned> fan;
+  int *h2beg = nullptr, *halo2 = nullptr, *btbeg = nullptr, *bt = nullptr;
+  if (grad) {
+    // ---- fans ---------------------------------------------------------------
+    int n_inc = 0;
+    TT(hipMemcpyAsync(&n_inc, G.vc_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    Tmp<unsigned char> used;
+    Tmp<int> cnt;
+    TT(used.alloc(n_inc)); TT(cnt.alloc(nv + 1)); TT(fan_ptr.alloc(nv + 1));
+    GO(k_fan, nv + 1, G, used.p, (const int*)nullptr, cnt.p, (unsigned*)nullptr);
+    TT(scan(cnt.p, fan_ptr.p, nv + 1));
+    int nfan = 0;
+    TT(hipMemcpyAsync(&nfan, fan_ptr.p + nv, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    TT(fan.alloc(nfan));
+    GO(k_fan, nv + 1, G, used.p, fan_ptr.p, (int*)nullptr, fan.p);
+    T.fan_ptr = fan_ptr.p;
+    T.fan = fan.p;
+    // ---- second ring and boundary terms ---------------------------------------
+    Tmp<int> n2, nb, o2, ob;
+    TT(n2.alloc(nq + 1)); TT(nb.alloc(nq + 1)); TT(nit.alloc(nq + 1));
+    TT(o2.alloc(nq + 1)); TT(ob.alloc(nq + 1));
+    GO(k_gs_count, nq + 1, T, nq, n2.p, nb.p, nit.p);
+    TT(scan(n2.p, o2.p, nq + 1));
+    TT(scan(nb.p, ob.p, nq + 1));
+    int c2 = 0, cb = 0;
+    TT(hipMemcpyAsync(&c2, o2.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipMemcpyAsync(&cb, ob.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    if (c2 < 0 || cb < 0) { msg = "stage tables: too many entries"; return 1; }
+    Tmp<unsigned long long> k2, kb;
+    TT(k2.alloc(c2)); TT(kb.alloc(cb));
+    GO(k_gs_emit, nq, T, nq, o2.p, ob.p, k2.p, kb.p);
+    int count = 0;
+    if (int r = group(k2, c2, &h2beg, &halo2, count)) return r;
+    if (int r = group(kb, cb, &btbeg, &bt, count)) return r;
+    T.h2beg = h2beg; T.halo2 = halo2; T.btbeg = btbeg; T.bt = bt;
+    // ---- overflow of the eight item entries -----------------------------------
+    TT(ovp.alloc(nq + 1));
+    GO(k_ov_count, nq + 1, nq, nit.p, n2.p);
+    TT(scan(n2.p, ovp.p, nq + 1));
+  }
+  // ---- wall terms -------------------------------------------------------------
+  int *wtbeg = nullptr, *wt = nullptr;
+  if (walls) {
+    int nvbe = 0, count = 0;
+    TT(hipMemcpyAsync(&nvbe, G.vbe_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    Tmp<unsigned long long> k;
+    TT(k.alloc(nvbe));
+    GO(k_wall_keys, nv, T, k.p);
+    if (int r = group(k, nvbe, &wtbeg, &wt, count)) return r;
+    uint2* wcell = nullptr;
+    unsigned short* wvent = nullptr;
+    TA(wcell, count);
+    TA(wvent, nvbe);
+    GO(k_wall_cells, nt, T, wtbeg, wt, wcell, bad.p);
+    GO(k_wall_entries, nv, T, wtbeg, wt, wvent, bad.p);
+    S.wtbeg = wtbeg; S.wt = wt; S.wcell = wcell; S.wvent = wvent;
+  }
+  // ---- viscous cells ----------------------------------------------------------
+  int *tcbeg = nullptr, *tc = nullptr;
+  if (ns) {
+    int n_inc = 0, count = 0;
+    TT(hipMemcpyAsync(&n_inc, G.vc_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    Tmp<unsigned long long> k;
+    TT(k.alloc(n_inc));
+    GO(k_vcell_keys, nv, T, k.p);
+    if (int r = group(k, n_inc, &tcbeg, &tc, count)) return r;
+    unsigned short* ent = nullptr;
+    int* cnt = nullptr;
+    uint4* vc8 = nullptr;
+    TA(ent, n_inc); TA(cnt, nv); TA(vc8, nv);
+    GO(k_vcell_entries, nv, T, tcbeg, tc, ent, cnt, vc8, bad.p);
+    S.vcent = ent; S.vccnt = cnt; S.vc8 = vc8;
+  }
+  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special.p, (int4*)nullptr, mx.p);
+  int h[8];
+  TT(hipMemcpyAsync(h, mx.p, sizeof(h), hipMemcpyDeviceToHost, st));
+  TT(hipStreamSynchronize(st));
+  S.ms = h[0]; S.ms1 = h[1]; S.mf = h[2]; S.mbt = h[3]; S.mwt = h[4]; S.mc = h[5];
+  if (S.ms > SI_MASK) { msg = "stage tables: too many slots"; return 1; }
+  // ---- padded tables ------------------------------------------------------------
+  int* sid = nullptr;
+  unsigned* lr = nullptr;
+  double2 *fn = nullptr, *xy = nullptr;
+  uint4 *it = nullptr, *it2 = nullptr, *ge = nullptr;
+  int4* desc = nullptr;
+  TA(sid, (size_t)nt * S.ms); TA(lr, (size_t)nt * S.mf); TA(fn, (size_t)nt * S.mf);
+  TA(xy, nv); TA(ge, nv); TA(desc, nt);
+  GO(k_fill_sid, (long long)nt * S.ms, T, S.ms, sid);
+  GO(k_fill_faces, (long long)nt * S.mf, nt, S.mf, TG.fbeg, TG.f_lr, TG.f_n, lr, fn);
+  GO(k_xy, nv, nv, G.x, G.y, xy);
+  GO(k_ge8, nv, nv, TG.gptr, TG.gent, ge);
+  if (grad) {
+    int nov = 0, *itov = nullptr;
+    unsigned short* ov = nullptr;
+    TT(hipMemcpyAsync(&nov, ovp.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
+    TT(hipStreamSynchronize(st));
+    TA(it, (size_t)nt * S.ms1); TA(it2, (size_t)nt * S.ms1); TA(itov, (size_t)nt * S.ms1); TA(ov, nov);
+    GO(k_no_items, (long long)nt * S.ms1, (long long)nt * S.ms1, it, it2, itov);
+    GO(k_fill_items, nq, T, nq, S.ms1, nit.p, ovp.p, it, it2, itov, ov, special.p, bad.p);
+    S.items = it; S.items2 = it2; S.item_ov = itov; S.ov = ov; S.btbeg = btbeg; S.bt = bt;
+  }
+  if (ns) {
+    unsigned* vcells = nullptr;
+    TA(vcells, (size_t)nt * S.mc);
+    GO(k_vcells, (long long)nt * S.mc, T, S.mc, tcbeg, tc, vcells, bad.p);
+    S.vcells = vcells;
+  }
+  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special.p, desc, (int*)nullptr);
+  int hbad = 0;
+  TT(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  TT(hipGetLastError());
+  TT(hipStreamSynchronize(st));
+  if (hbad) { msg = "stage tables: entry out of range"; return 1; }
+  S.desc = desc; S.sid = sid; S.f_lr = lr; S.f_n = fn; S.xy = xy; S.ge8 = ge;
+#undef TT
+#undef TA
+#undef GO
+  return 0;
+}
+
+}  // namespace tsm
