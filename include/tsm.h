@@ -67,18 +67,20 @@ typedef struct tsm_params {
      option except bc_scheme strong), CSR-gather kernels otherwise; 1 = always
      the CSR-gather kernels.  Both give the reference's summation order. */
   int kernel_path;
-  int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128) */
-  int block_grad;     /* threads per tile of the tiled gradient kernel (0: auto) */
-  int block_fu;       /* threads per tile of the tiled flux/update kernel (0: auto) */
-  int tile_fused_gradient; /* 1: on meshes without periodic sets, form the
-                              gradients inside the stage kernel (two halo rings)
-                              instead of in a pass of their own */
+  int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128);
+                         smaller ones are taken where two halo rings of a tile do
+                         not fit LDS */
+  int block_grad;     /* checked against the block limits; the stage kernel forms
+                         the gradients itself, so no kernel of its own reads it */
+  int block_fu;       /* threads per tile of the stage kernel (0: auto) */
+  int tile_fused_gradient; /* the tiled path always forms the gradients inside
+                              the stage kernel; 1 only keeps the context (Euler,
+                              SSP-RK3, no periodic sets) out of packed runs */
   int graph_steps;    /* tiled path: capture this many steps in one HIP graph and
                          replay it (0: launch every kernel from the host) */
   int host_preprocess; /* 1: build the dual-mesh geometry and the tiling on the
-                          host; 0: on the device for median duals (the tiling
-                          unless the fused kernel's second halo ring is asked
-                          for; the same arrays bit for bit) */
+                          host; 0: on the device for median duals (the same
+                          arrays bit for bit) */
   int strong_bc;      /* bc_scheme (src/parameter.h:31-34): 0 weak; 1 strong: after
                          every stage update each bface, in bface order, imposes its
                          boundary condition on its end points' state (src/fv.cc:
@@ -226,7 +228,7 @@ int tsm_run_group(tsm_ctx** ctxs, int n, long nsteps, long* done);
    on the first context's stream.  Each block computes what it computes in its
    own context's launch, so the results are those of tsm_run bit for bit.
    The contexts must run the Euler equations with SSP-RK3 on the tiled kernels
-   (gradients in a pass of their own) and share the flux and reconstruction;
+   (without tile_fused_gradient) and share the flux and reconstruction;
    TSM_E_ARG otherwise.  No counterpart in the reference, which runs its
    samples one after another (src/fv.cc:2440-2459). */
 int tsm_run_packed(tsm_ctx** ctxs, int n, long nsteps, long* done);
@@ -358,8 +360,8 @@ int tsm_host_tiling(const tsm_mesh* mesh, int cell_type, int tile_vertices, int 
 /* Times nsteps full steps on the context stream with HIP events and reports
    average durations in microseconds.  CSR kernels: us[0] dt pass, us[1]
    gradient, us[2] edge flux, us[3] gather + update (per stage).  Tiled
-   kernels: us[0] 0, us[1] gradient, us[2] fused flux + gather + update (per
-   stage), us[3] step finalisation (per step).  us[4]: whole step, timed
+   kernels: us[0] and us[1] 0, us[2] the stage kernel (per stage), us[3] step
+   finalisation (per step).  us[4]: whole step, timed
    without interleaved events. */
 int tsm_bench(tsm_ctx* ctx, int nsteps, double* us);
 
@@ -392,6 +394,10 @@ int tsm_mlp_get_params(tsm_mlp* m, float* params);
 int tsm_mlp_set_params(tsm_mlp* m, const float* params);
 /* y[n x widths[L]] = net(x[n x widths[0]]), in chunks of max_batch rows */
 int tsm_mlp_forward(tsm_mlp* m, long n, const float* x, float* y);
+/* the same between standardised variables, in FP64: x = (u - mu_x) / sd_x in,
+   y sd_y + mu_y out (u[n x widths[0]], y[n x widths[L]]) */
+int tsm_mlp_forward_affine(tsm_mlp* m, long n, const double* u, const double* mu_x, const double* sd_x,
+                           const double* mu_y, const double* sd_y, double* y);
 /* loss and gradient (flat, like the parameters) of one batch, n <= max_batch */
 int tsm_mlp_gradient(tsm_mlp* m, int n, const float* x, const float* t, double* loss, float* grad);
 /* epochs of minibatch Adam over a seeded shuffle; epoch_loss[epochs] optional */

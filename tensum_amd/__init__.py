@@ -89,9 +89,10 @@ class Params:
     bc_scheme: str = "weak"        # "weak" or "strong" (boundary values imposed after each stage)
     kernel_path: str = "auto"      # "auto" (tiled where supported) or "csr"
     tile_vertices: int = 0
-    block_grad: int = 0            # threads per tile, gradient kernel (0: auto)
-    block_fu: int = 0              # threads per tile, flux/update kernel (0: auto)
-    fused_gradient: bool = False   # gradients inside the stage kernel (two halo rings)
+    block_grad: int = 0            # range-checked only (no kernel of its own)
+    block_fu: int = 0              # threads per tile, stage kernel (0: auto)
+    fused_gradient: bool = False   # the stage kernel always forms the gradients; True keeps the
+                                   # context out of packed runs
     graph_steps: int = 0           # steps per captured HIP graph (0: no graph)
     preprocess: str = "auto"       # "auto" (device geometry for median duals) or "host"
 

@@ -1,10 +1,9 @@
 """Launch-shape autotuner for the tiled stage kernels.
 
 Chooses the vertex tile size (owned vertices per workgroup, which sets the
-halo fraction and the faces each tile recomputes) and the workgroup sizes of
-the stage and gradient kernels, and whether the gradients are formed inside
-the stage kernel (two halo rings) or in a pass of their own, by timing a few steps of the actual workload
-with the solver's own event timer (tsm_bench).  Every candidate computes the
+halo fraction and the faces each tile recomputes) and the workgroup size of the
+stage kernel by timing a few steps of the actual workload with the solver's own
+event timer (tsm_bench).  Every candidate computes the
 same sums in the same order, so tuning changes only the time: the tests check
 that a tuned run is bit-identical to an untuned one.  The reference has no
 counterpart (its loop is one CPU thread per rank, src/fv.cc:2273-2368).

@@ -10,8 +10,13 @@
 //   dy = 2 (y - t) / (B n_out)            (fp32 -> bf16)
 //   dW_l = dz_l^T x_l,  db_l = column sums of dz_l   (fp32)
 //   dx_l = dz_l W_l,    dz_{l-1} = dx_l * GELU'(z_{l-1})   (-> bf16)
-// Every product is one launch of the tiled GEMM below with the operands'
-// transposes absorbed by the LDS staging.
+// Networks of layers up to FUSED_MAX wide (the surrogates are 64 to 256 wide) run
+// in three kernels: k_rows takes 32 rows of a minibatch through every layer and
+// back, k_update forms each 32 x 32 tile of the weight gradients and applies Adam
+// to it, k_infer takes rows through the layers only.  Wider ones take one launch
+// of the tiled GEMM per product, the operands' transposes absorbed by the LDS
+// staging.  Both form every sum in the same order (k ascending, 16 a product), so
+// they give the same bits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -197,6 +202,318 @@ __global__ void k_gather_rows(int rows, int cols, const int* idx, const float* s
   if (df) df[i] = x;
 }
 
+// ---------------------------------------------------------------------------
+// fused kernels
+// ---------------------------------------------------------------------------
+constexpr int FUSED_MAX = 512, MAXL = 16, RT = 32;
+inline int up(int n, int m) { return (n + m - 1) / m * m; }
+
+// Weights twice in bf16, zero-padded: Wp[l] is up(n_out, 32) x up(n_in, 16) (the
+// forward operand), Wt[l] its transpose, up(n_in, 32) x up(n_out, 16) (the
+// backward one), so a lane's eight k values are one aligned 16-byte load.
+// Activations x_l and dz_l of a minibatch are kept transposed (XT, DT: feature
+// x ldr rows, zero past the last row), which is how the weight gradients read
+// them and how the MFMA result falls out (four rows per lane at a time).
+struct Net {
+  int L, ldr, lda;  // layers, row stride of XT/DT, LDS row stride
+  int w[MAXL + 1];
+  u16 *Wp[MAXL], *Wt[MAXL];
+  float *P, *G, *Mo, *Vo;          // flat parameters, gradient, Adam moments
+  int woff[MAXL], boff[MAXL];
+  u16 *XT[MAXL], *DT[MAXL];
+  float* Z[MAXL];
+  float *Y, *T;
+};
+__host__ __device__ inline int upd(int n, int m) { return (n + m - 1) / m * m; }
+
+// One layer's product for NT row tiles of 32: C (32 x 32 per tile, columns n0 ..)
+// from LDS activations A (row stride lda) and padded weights W (row stride Kp).
+template <int NT>
+__device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W, int Kp, int n0,
+                                             f32x16* acc) {
+  const int lane = threadIdx.x & 63, c = lane & 31, ko = (lane >> 5) * 8;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+  const u16* wr = W + (size_t)(n0 + c) * Kp + ko;
+  const u16* ar = A + c * lda + ko;
+  int k0 = 0;
+  for (; k0 + 128 <= Kp; k0 += 128) {  // eight slices in flight
+    bf16x8 b[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = *reinterpret_cast<const bf16x8*>(wr + k0 + 16 * u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(ar + t * RT * lda + k0 + 16 * u);
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[u], acc[t], 0, 0, 0);
+      }
+  }
+  for (; k0 < Kp; k0 += 16) {
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(wr + k0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(ar + t * RT * lda + k0);
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[t], 0, 0, 0);
+    }
+  }
+}
+// row of result element i within a tile
+__device__ __forceinline__ int c_row(int i) { return 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
+
+// 32 rows of a minibatch (rows idx[r], or r itself) forward, dy = 2 (y - t) / n,
+// and back to dz_0; the transposed activations and dz of every layer go to XT/DT.
+// Bound by the latency of its 2 L - 1 dependent products (a layer's weights are
+// read from L2 once per 32 rows): eight waves, one or more 32-column tiles each.
+__global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, const float* Xin,
+                                              const float* Tin, float scale) {
+  extern __shared__ __attribute__((aligned(16))) u16 sm[];
+  u16 *cur = sm, *nxt = sm + RT * a.lda;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
+  const int r0 = blockIdx.x * RT, L = a.L;
+  {
+    const int K = a.w[0], Kp = upd(K, 16);
+    for (int i = tid; i < RT * Kp; i += blockDim.x) {
+      const int k = i / RT, r = i % RT;  // rows fastest: XT is written in order
+      const bool in = k < K && r0 + r < nb;
+      const u16 v = in ? f2bf(Xin[(size_t)(idx ? idx[r0 + r] : r0 + r) * K + k]) : (u16)0;
+      cur[r * a.lda + k] = v;
+      if (k < K) a.XT[0][(size_t)k * a.ldr + r0 + r] = v;
+    }
+  }
+  __syncthreads();
+  f32x16 acc[1];
+  for (int l = 0; l < L; ++l) {
+    const int K = a.w[l], N = a.w[l + 1], Kp = upd(K, 16), Np = upd(N, 32);
+    const bool last = l + 1 == L;
+    const float* bias = a.P + a.boff[l];
+    for (int n0 = 32 * wave; n0 < Np; n0 += 32 * nw) {
+      tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
+      const int n = n0 + (lane & 31);
+      const bool col = n < N;
+      const float bn = col ? bias[n] : 0.0f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        ushort4 q;
+        u16* qv = reinterpret_cast<u16*>(&q);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int i = 4 * g + u, row = c_row(i), r = r0 + row;
+          const bool in = col && r < nb;
+          const float c = acc[0][i] + bn;
+          u16 v = 0;
+          if (in) {
+            if (last) {
+              a.Y[(size_t)r * N + n] = c;
+              const float t = Tin[(size_t)(idx ? idx[r] : r) * N + n];
+              v = f2bf(2.0f * (c - t) * scale);
+            } else {
+              a.Z[l][(size_t)r * N + n] = c;
+              v = f2bf(gelu(c));
+            }
+          }
+          qv[u] = v;
+          nxt[row * a.lda + n] = v;
+        }
+        if (col) {
+          u16* o = (last ? a.DT[l] : a.XT[l + 1]) + (size_t)n * a.ldr + r0 + c_row(4 * g);
+          *reinterpret_cast<ushort4*>(o) = q;
+        }
+      }
+    }
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+  // dz_{l-1} = (dz_l W_l) * GELU'(z_{l-1}); z was stored by this very lane
+  for (int l = L - 1; l > 0; --l) {
+    const int K = a.w[l], N = a.w[l + 1], Np = upd(N, 16), Kp = upd(K, 32);
+    for (int k0 = 32 * wave; k0 < Kp; k0 += 32 * nw) {
+      const int k = k0 + (lane & 31);
+      const bool col = k < K;
+      float z[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int r = r0 + c_row(i);
+        z[i] = col && r < nb ? a.Z[l - 1][(size_t)r * K + k] : 0.0f;
+      }
+      tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        ushort4 q;
+        u16* qv = reinterpret_cast<u16*>(&q);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int i = 4 * g + u, row = c_row(i);
+          const u16 v = col && r0 + row < nb ? f2bf(acc[0][i] * gelu_d(z[i])) : (u16)0;
+          qv[u] = v;
+          nxt[row * a.lda + k] = v;
+        }
+        if (col) *reinterpret_cast<ushort4*>(a.DT[l - 1] + (size_t)k * a.ldr + r0 + c_row(4 * g)) = q;
+      }
+    }
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+}
+
+// Adam on one parameter, as k_adam
+struct Adam { float lr, b1, b2, eps, c1, c2; };
+__device__ __forceinline__ float adam_step(const Net& a, const Adam& h, int i, float gi) {
+  const float mi = h.b1 * a.Mo[i] + (1.0f - h.b1) * gi;
+  const float vi = h.b2 * a.Vo[i] + (1.0f - h.b2) * gi * gi;
+  a.Mo[i] = mi;
+  a.Vo[i] = vi;
+  const float wi = a.P[i] - h.lr * (mi / h.c1) / (sqrtf(vi / h.c2) + h.eps);
+  a.P[i] = wi;
+  return wi;
+}
+// One job per wave: a 32 x 32 tile of a layer's weight gradient (MFMA over the
+// rows), 64 bias gradients (sums in row order), or one 256-element part of the
+// loss (the tree of k_mse).  TRAIN applies Adam at once and refreshes the bf16
+// weights; else the gradient goes to G.
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void k_update(Net a, int nb, const int4* jobs, int n_jobs,
+                                                const int* idx, const float* Tin, float* part, Adam h) {
+  const int lane = threadIdx.x & 63;
+  const int job = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int no = a.w[a.L], n_el = nb * no;
+  if (job >= n_jobs) {
+    const int b = job - n_jobs;
+    if (256 * b >= n_el) return;
+    float red[4];
+    for (int w = 0; w < 4; ++w) {
+      const int i = 256 * b + 64 * w + lane;
+      float e2 = 0.0f;
+      if (i < n_el) {
+        const int r = i / no, c = i % no;
+        const float d = a.Y[i] - Tin[(size_t)(idx ? idx[r] : r) * no + c];
+        e2 = d * d;
+      }
+      for (int o = 32; o > 0; o >>= 1) e2 += __shfl_down(e2, o, 64);
+      red[w] = e2;
+    }
+    if (lane == 0) part[b] = red[0] + red[1] + red[2] + red[3];
+    return;
+  }
+  const int4 J = jobs[job];  // kind, layer, first output, first input
+  const int l = J.y, K = a.w[l], N = a.w[l + 1];
+  if (J.x == 1) {
+    const int n = J.z + lane;
+    if (n >= N) return;
+    const u16* d = a.DT[l] + (size_t)n * a.ldr;
+    float s = 0.0f;
+    int r = 0;
+    for (; r + 8 <= nb; r += 8) {
+      u16 q[8];
+      *reinterpret_cast<uint4*>(q) = *reinterpret_cast<const uint4*>(d + r);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += bf2f(q[u]);
+    }
+    for (; r < nb; ++r) s += bf2f(d[r]);
+    if (TRAIN) (void)adam_step(a, h, a.boff[l] + n, s);
+    else a.G[a.boff[l] + n] = s;
+    return;
+  }
+  const int c = lane & 31, ko = (lane >> 5) * 8;
+  const int nr = min(J.z + c, N - 1), kr = min(J.w + c, K - 1);  // rows past the layer: any, not stored
+  const u16 *dr = a.DT[l] + (size_t)nr * a.ldr + ko, *xr = a.XT[l] + (size_t)kr * a.ldr + ko;
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  for (int k0 = 0; k0 < nb; k0 += 16) {
+    const bf16x8 A = *reinterpret_cast<const bf16x8*>(dr + k0);
+    const bf16x8 B = *reinterpret_cast<const bf16x8*>(xr + k0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, acc, 0, 0, 0);
+  }
+  const int k = J.w + c, Kp = upd(K, 16), Np = upd(N, 16);
+  if (k >= K) return;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int n = J.z + c_row(i);
+    if (n >= N) continue;
+    const int p = a.woff[l] + n * K + k;
+    if (TRAIN) {
+      const u16 wb = f2bf(adam_step(a, h, p, acc[i]));
+      a.Wp[l][(size_t)n * Kp + k] = wb;
+      a.Wt[l][(size_t)k * Np + n] = wb;
+    } else {
+      a.G[p] = acc[i];
+    }
+  }
+}
+
+// bf16 copies of the weights of layer l
+__global__ void k_pack_weights(Net a, int l) {
+  const int K = a.w[l], N = a.w[l + 1];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N * K) return;
+  const int n = i / K, k = i % K;
+  const u16 v = f2bf(a.P[a.woff[l] + i]);
+  a.Wp[l][(size_t)n * upd(K, 16) + k] = v;
+  a.Wt[l][(size_t)k * upd(N, 16) + n] = v;
+}
+
+// NT x 32 rows through the layers.  AFFINE: inputs (u - mu_x) / sd_x and outputs
+// y sd_y + mu_y in FP64 (io: mu_x, sd_x, mu_y, sd_y one after another), else FP32
+// rows in and out.  Two row tiles per wave share each weight load; at 65,536 rows
+// the weights are read 1,024 times from L2 (0.3 GB) beside 20 GFLOP.
+template <int NT, bool AFFINE>
+__global__ __launch_bounds__(512) void k_infer(Net a, long rows, const void* in, const double* io,
+                                               void* out) {
+  extern __shared__ __attribute__((aligned(16))) u16 sm[];
+  u16 *cur = sm, *nxt = sm + NT * RT * a.lda;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
+  const long r0 = (long)blockIdx.x * NT * RT;
+  const int L = a.L, ni = a.w[0], no = a.w[L];
+  {
+    const int Kp = upd(ni, 16);
+    for (int i = tid; i < NT * RT * Kp; i += blockDim.x) {
+      const int r = i / Kp, k = i % Kp;
+      u16 v = 0;
+      if (k < ni && r0 + r < rows) {
+        const size_t o = (size_t)(r0 + r) * ni + k;
+        const float x = AFFINE ? (float)((static_cast<const double*>(in)[o] - io[k]) / io[ni + k])
+                               : static_cast<const float*>(in)[o];
+        v = f2bf(x);
+      }
+      cur[r * a.lda + k] = v;
+    }
+  }
+  __syncthreads();
+  f32x16 acc[NT];
+  for (int l = 0; l < L; ++l) {
+    const int N = a.w[l + 1], Kp = upd(a.w[l], 16), Np = upd(N, 32);
+    const bool last = l + 1 == L;
+    const float* bias = a.P + a.boff[l];
+    for (int n0 = 32 * wave; n0 < Np; n0 += 32 * nw) {
+      tile_product<NT>(cur, a.lda, a.Wp[l], Kp, n0, acc);
+      const int n = n0 + (lane & 31);
+      const bool col = n < N;
+      const float bn = col ? bias[n] : 0.0f;
+      const double sd = AFFINE && last && col ? io[2 * ni + no + n] : 1.0;
+      const double mu = AFFINE && last && col ? io[2 * ni + n] : 0.0;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int row = t * RT + c_row(i);
+          const float c = acc[t][i] + bn;
+          if (!last) {
+            nxt[row * a.lda + n] = col ? f2bf(gelu(c)) : (u16)0;
+          } else if (col && r0 + row < rows) {
+            const size_t o = (size_t)(r0 + row) * N + n;
+            if (AFFINE) static_cast<double*>(out)[o] = (double)c * sd + mu;
+            else static_cast<float*>(out)[o] = c;
+          }
+        }
+    }
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -207,15 +524,23 @@ struct tsm_mlp {
   std::vector<int> w;                 // widths, L + 1
   std::vector<size_t> woff, boff;     // offsets of W_l, b_l in the flat parameter vector
   size_t np = 0;
+  bool fused = false;                 // no layer wider than FUSED_MAX
   float *P = nullptr, *G = nullptr, *Mo = nullptr, *Vo = nullptr;  // fp32 params, grads, Adam
-  u16* Pb = nullptr;                  // bf16 copy of the parameters
-  std::vector<u16*> X;                // activations x_0..x_{L-1} (bf16), maxb x w_l
+  u16* Pb = nullptr;                  // bf16 copy of the parameters (not fused)
+  std::vector<u16*> X;                // activations x_0..x_{L-1} (bf16), maxb x w_l (not fused)
   std::vector<float*> Z;              // pre-activations z_0..z_{L-1} (fp32)
-  u16 *dA = nullptr, *dB = nullptr;   // backward ping-pong, maxb x max width (bf16)
+  u16 *dA = nullptr, *dB = nullptr;   // backward ping-pong, maxb x max width (bf16; not fused)
   float *Y = nullptr, *T = nullptr, *part = nullptr;
+  Net net{};                          // fused
+  int4* jobs = nullptr;
+  int n_jobs = 0;
   float *Xin = nullptr, *Tin = nullptr;  // staged training set
   int* idx = nullptr;
   size_t nin_cap = 0;
+  float* parts = nullptr;             // loss parts of every minibatch of an epoch (fused)
+  size_t parts_cap = 0;
+  char* io = nullptr;                 // rows in and out of an evaluation (fused), INFER_BYTES at most
+  size_t io_cap = 0;
   long adam_t = 0;
   hipStream_t st = nullptr;
   std::string err;
@@ -224,6 +549,22 @@ struct tsm_mlp {
   hipError_t al(T** p, size_t n) {
     hipError_t e = hipMalloc((void**)p, n * sizeof(T) + 16);
     if (e == hipSuccess) allocs.push_back((void*)*p);
+    return e;
+  }
+  // replaces a buffer by a larger one once nothing on the stream uses it
+  template <class T>
+  hipError_t grow(T** p, size_t* cap, size_t n) {
+    if (n <= *cap) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return e;
+    if (*p) {
+      allocs.erase(std::remove(allocs.begin(), allocs.end(), (void*)*p), allocs.end());
+      (void)hipFree(*p);
+      *p = nullptr;
+      *cap = 0;
+    }
+    e = al(p, n);
+    if (e == hipSuccess) *cap = n;
     return e;
   }
   ~tsm_mlp() {
@@ -290,6 +631,77 @@ void backward(tsm_mlp* m, int nb) {
   }
 }
 
+// ---- fused nets ----
+size_t rows_lds(const tsm_mlp* m) { return 2 * (size_t)RT * m->net.lda * sizeof(u16); }
+
+// bf16 weights from the fp32 ones
+void refresh_weights(tsm_mlp* m) {
+  if (!m->fused) {
+    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((m->np + 255) / 256)), dim3(256), 0, m->st,
+                       (int)m->np, m->P, m->Pb);
+    return;
+  }
+  for (int l = 0; l < m->L; ++l)
+    hipLaunchKernelGGL(k_pack_weights, dim3((m->w[l] * m->w[l + 1] + 255) / 256), dim3(256), 0, m->st,
+                       m->net, l);
+}
+
+// one minibatch of nb rows: activations and dz, then the gradient (to G) or an
+// Adam step, and the loss parts
+void minibatch(tsm_mlp* m, int nb, const int* idx, const float* X, const float* T, float* part,
+               const Adam* h) {
+  const int no = m->w[m->L], n = nb * no;
+  const size_t lds = rows_lds(m);
+  if (lds > 48 * 1024)
+    (void)hipFuncSetAttribute((const void*)k_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(k_rows, dim3((nb + RT - 1) / RT), dim3(512), lds, m->st, m->net, nb, idx, X, T,
+                     1.0f / (float)n);
+  const int jobs = m->n_jobs + (n + 255) / 256;
+  if (h)
+    hipLaunchKernelGGL((k_update<true>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, m->net, nb, m->jobs,
+                       m->n_jobs, idx, T, part, *h);
+  else
+    hipLaunchKernelGGL((k_update<false>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, m->net, nb, m->jobs,
+                       m->n_jobs, idx, T, part, Adam{});
+}
+
+// Rows through the net in chunks whose staging stays under INFER_BYTES.  affine:
+// FP64 rows with (mu_x, sd_x, mu_y, sd_y), else FP32 rows.
+constexpr size_t INFER_BYTES = 64u << 20;
+int infer(tsm_mlp* m, long n, const void* in, void* out, const double* affine) {
+  const int ni = m->w[0], no = m->w[m->L];
+  const size_t es = affine ? sizeof(double) : sizeof(float);
+  const size_t na = affine ? 2 * (size_t)(ni + no) * sizeof(double) : 0;
+  const long cap = std::max<long>(1024, (long)((INFER_BYTES - na) / (es * (ni + no))));
+  const long rows = std::min(n, cap);
+  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t oi = al(na), oo = oi + al(es * ni * rows);
+  MLP_TRY(m->grow(&m->io, &m->io_cap, oo + es * no * rows));
+  if (affine) MLP_TRY(hipMemcpyAsync(m->io, affine, na, hipMemcpyHostToDevice, m->st));
+  for (long r0 = 0; r0 < n; r0 += rows) {
+    const long nr = std::min(rows, n - r0);
+    MLP_TRY(hipMemcpyAsync(m->io + oi, static_cast<const char*>(in) + es * ni * r0, es * ni * nr,
+                           hipMemcpyHostToDevice, m->st));
+    // 64 rows per block once that still leaves two blocks per CU
+    const int nt = nr >= 64 * 512 ? 2 : 1;
+    const size_t lds = nt * rows_lds(m);
+    auto go = [&](auto k) {
+      if (lds > 48 * 1024)
+        (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL(k, dim3((unsigned)((nr + RT * nt - 1) / (RT * nt))), dim3(512), lds, m->st,
+                         m->net, nr, (const void*)(m->io + oi), (const double*)m->io,
+                         (void*)(m->io + oo));
+    };
+    if (affine) { if (nt == 2) go(k_infer<2, true>); else go(k_infer<1, true>); }
+    else { if (nt == 2) go(k_infer<2, false>); else go(k_infer<1, false>); }
+    MLP_TRY(hipGetLastError());
+    MLP_TRY(hipMemcpyAsync(static_cast<char*>(out) + es * no * r0, m->io + oo, es * no * nr,
+                           hipMemcpyDeviceToHost, m->st));
+    MLP_TRY(hipStreamSynchronize(m->st));
+  }
+  return TSM_OK;
+}
+
 int stage_rows(tsm_mlp* m, int rows, const float* x, const float* t) {
   const int ni = m->w[0], no = m->w[m->L];
   float* tmp = nullptr;
@@ -345,29 +757,70 @@ extern "C" int tsm_mlp_create(int n_layers, const int* widths, int max_batch,
     for (size_t i = 0; i < (size_t)m->w[l + 1] * m->w[l]; ++i)
       h[m->woff[l] + i] = (float)(a * (2.0 * next() - 1.0));
   }
+  m->fused = wmax <= FUSED_MAX;
   hipError_t e = hipStreamCreate(&m->st);
-  if (e == hipSuccess) e = m->al(&m->P, m->np);
-  if (e == hipSuccess) e = m->al(&m->G, m->np);
-  if (e == hipSuccess) e = m->al(&m->Mo, m->np);
-  if (e == hipSuccess) e = m->al(&m->Vo, m->np);
-  if (e == hipSuccess) e = m->al(&m->Pb, m->np);
   m->X.assign(n_layers, nullptr);
   m->Z.assign(n_layers, nullptr);
-  for (int l = 0; l < n_layers && e == hipSuccess; ++l) {
-    e = m->al(&m->X[l], (size_t)max_batch * m->w[l]);
-    if (e == hipSuccess) e = m->al(&m->Z[l], (size_t)max_batch * m->w[l + 1]);
+  // one allocation for everything of a fixed size, cleared once (the padding of
+  // the fused nets' operands stays zero)
+  struct Piece { void** p; size_t bytes; };
+  std::vector<Piece> pieces;
+  auto want = [&](auto** p, size_t n) { pieces.push_back({(void**)p, n * sizeof(**p)}); };
+  const int no = m->w[n_layers];
+  want(&m->P, m->np); want(&m->G, m->np); want(&m->Mo, m->np); want(&m->Vo, m->np);
+  for (int l = 0; l < n_layers; ++l) want(&m->Z[l], (size_t)max_batch * m->w[l + 1]);
+  want(&m->Y, (size_t)max_batch * no);
+  want(&m->T, (size_t)max_batch * no);
+  want(&m->part, (size_t)max_batch * no / 256 + 2);
+  Net& N = m->net;
+  std::vector<int4> jobs;
+  if (m->fused) {
+    N.L = n_layers;
+    N.ldr = up(max_batch, RT);
+    for (int l = 0; l <= n_layers; ++l) {
+      N.w[l] = m->w[l];
+      N.lda = std::max(N.lda, up(m->w[l], 32) + 8);
+    }
+    for (int l = 0; l < n_layers; ++l) {
+      const int ni = m->w[l], n1 = m->w[l + 1];
+      want(&N.Wp[l], (size_t)up(n1, 32) * up(ni, 16));
+      want(&N.Wt[l], (size_t)up(ni, 32) * up(n1, 16));
+      want(&N.XT[l], (size_t)ni * N.ldr);
+      want(&N.DT[l], (size_t)n1 * N.ldr);
+      N.woff[l] = (int)m->woff[l];
+      N.boff[l] = (int)m->boff[l];
+      for (int n = 0; n < n1; n += 32)
+        for (int k = 0; k < ni; k += 32) jobs.push_back(int4{0, l, n, k});
+      for (int n = 0; n < n1; n += 64) jobs.push_back(int4{1, l, n, 0});
+    }
+    m->n_jobs = (int)jobs.size();
+    want(&m->jobs, jobs.size());
+  } else {
+    want(&m->Pb, m->np);
+    for (int l = 0; l < n_layers; ++l) want(&m->X[l], (size_t)max_batch * m->w[l]);
+    want(&m->dA, (size_t)max_batch * wmax);
+    want(&m->dB, (size_t)max_batch * wmax);
   }
-  if (e == hipSuccess) e = m->al(&m->dA, (size_t)max_batch * wmax);
-  if (e == hipSuccess) e = m->al(&m->dB, (size_t)max_batch * wmax);
-  if (e == hipSuccess) e = m->al(&m->Y, (size_t)max_batch * m->w[n_layers]);
-  if (e == hipSuccess) e = m->al(&m->T, (size_t)max_batch * m->w[n_layers]);
-  if (e == hipSuccess) e = m->al(&m->part, (size_t)max_batch * m->w[n_layers] / 256 + 2);
-  if (e == hipSuccess) e = hipMemcpy(m->P, h.data(), m->np * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(m->Mo, 0, m->np * sizeof(float));
-  if (e == hipSuccess) e = hipMemset(m->Vo, 0, m->np * sizeof(float));
+  size_t total = 0;
+  for (auto& q : pieces) total += (q.bytes + 255) & ~(size_t)255;
+  char* arena = nullptr;
+  if (e == hipSuccess) e = m->al(&arena, total);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((m->np + 255) / 256)), dim3(256), 0, m->st,
-                       (int)m->np, m->P, m->Pb);
+    size_t o = 0;
+    for (auto& q : pieces) {
+      *q.p = arena + o;
+      o += (q.bytes + 255) & ~(size_t)255;
+    }
+    N.P = m->P; N.G = m->G; N.Mo = m->Mo; N.Vo = m->Vo; N.Y = m->Y; N.T = m->T;
+    if (m->fused)
+      for (int l = 0; l < n_layers; ++l) N.Z[l] = m->Z[l];
+    e = hipMemsetAsync(arena, 0, total, m->st);
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(m->P, h.data(), m->np * sizeof(float), hipMemcpyHostToDevice, m->st);
+  if (e == hipSuccess && m->fused)
+    e = hipMemcpyAsync(m->jobs, jobs.data(), jobs.size() * sizeof(int4), hipMemcpyHostToDevice, m->st);
+  if (e == hipSuccess) {
+    refresh_weights(m);
     e = hipStreamSynchronize(m->st);
   }
   if (e != hipSuccess) {
@@ -393,8 +846,7 @@ extern "C" int tsm_mlp_set_params(tsm_mlp* m, const float* p) {
   if (!m || !p) return mfail(TSM_E_ARG, "bad argument");
   MLP_TRY(hipStreamSynchronize(m->st));
   MLP_TRY(hipMemcpy(m->P, p, m->np * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((m->np + 255) / 256)), dim3(256), 0, m->st,
-                     (int)m->np, m->P, m->Pb);
+  refresh_weights(m);
   MLP_TRY(hipGetLastError());
   MLP_TRY(hipStreamSynchronize(m->st));
   return TSM_OK;
@@ -402,6 +854,7 @@ extern "C" int tsm_mlp_set_params(tsm_mlp* m, const float* p) {
 
 extern "C" int tsm_mlp_forward(tsm_mlp* m, long n, const float* x, float* y) {
   if (!m || n < 0 || (n > 0 && (!x || !y))) return mfail(TSM_E_ARG, "bad argument");
+  if (m->fused) return n ? infer(m, n, x, y, nullptr) : TSM_OK;
   const int ni = m->w[0], no = m->w[m->L];
   for (long r0 = 0; r0 < n; r0 += m->maxb) {
     const int nb = (int)std::min<long>(m->maxb, n - r0);
@@ -416,13 +869,45 @@ extern "C" int tsm_mlp_forward(tsm_mlp* m, long n, const float* x, float* y) {
   return TSM_OK;
 }
 
+extern "C" int tsm_mlp_forward_affine(tsm_mlp* m, long n, const double* u, const double* mu_x,
+                                      const double* sd_x, const double* mu_y, const double* sd_y,
+                                      double* y) {
+  if (!m || n < 0 || !mu_x || !sd_x || !mu_y || !sd_y || (n > 0 && (!u || !y)))
+    return mfail(TSM_E_ARG, "bad argument");
+  if (n == 0) return TSM_OK;
+  const int ni = m->w[0], no = m->w[m->L];
+  if (m->fused) {
+    std::vector<double> a(mu_x, mu_x + ni);
+    a.insert(a.end(), sd_x, sd_x + ni);
+    a.insert(a.end(), mu_y, mu_y + no);
+    a.insert(a.end(), sd_y, sd_y + no);
+    return infer(m, n, u, y, a.data());
+  }
+  std::vector<float> x((size_t)n * ni), z((size_t)n * no);
+  for (long r = 0; r < n; ++r)
+    for (int k = 0; k < ni; ++k) x[(size_t)r * ni + k] = (float)((u[(size_t)r * ni + k] - mu_x[k]) / sd_x[k]);
+  const int rc = tsm_mlp_forward(m, n, x.data(), z.data());
+  if (rc) return rc;
+  for (long r = 0; r < n; ++r)
+    for (int k = 0; k < no; ++k) y[(size_t)r * no + k] = (double)z[(size_t)r * no + k] * sd_y[k] + mu_y[k];
+  return TSM_OK;
+}
+
 extern "C" int tsm_mlp_gradient(tsm_mlp* m, int n, const float* x, const float* t, double* loss,
                                 float* grad) {
   if (!m || n < 1 || n > m->maxb || !x || !t) return mfail(TSM_E_ARG, "bad argument");
-  int rc = stage_rows(m, n, x, t);
-  if (rc) return rc;
-  forward(m, n, true);
-  backward(m, n);
+  if (m->fused) {
+    const size_t nx = (size_t)n * m->w[0], nt = (size_t)n * m->w[m->L];
+    MLP_TRY(m->grow(&m->io, &m->io_cap, nx * sizeof(float)));
+    MLP_TRY(hipMemcpyAsync(m->io, x, nx * sizeof(float), hipMemcpyHostToDevice, m->st));
+    MLP_TRY(hipMemcpyAsync(m->T, t, nt * sizeof(float), hipMemcpyHostToDevice, m->st));
+    minibatch(m, n, nullptr, reinterpret_cast<const float*>(m->io), m->T, m->part, nullptr);
+  } else {
+    int rc = stage_rows(m, n, x, t);
+    if (rc) return rc;
+    forward(m, n, true);
+    backward(m, n);
+  }
   MLP_TRY(hipGetLastError());
   const int nparts = (n * m->w[m->L] + 255) / 256;
   std::vector<float> part(nparts);
@@ -461,11 +946,37 @@ extern "C" int tsm_mlp_train(tsm_mlp* m, long n, const float* x, const float* t,
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const int nmb = (int)((n + batch - 1) / batch);
   std::vector<float> part;
+  const size_t mp = ((size_t)batch * no + 255) / 256;  // loss parts of a full minibatch
+  if (m->fused) MLP_TRY(m->grow(&m->parts, &m->parts_cap, mp * nmb));
   for (int ep = 0; ep < epochs; ++ep) {
     for (long i = n - 1; i > 0; --i) std::swap(perm[i], perm[next() % (uint64_t)(i + 1)]);
     MLP_TRY(hipMemcpyAsync(m->idx, perm.data(), n * sizeof(int), hipMemcpyHostToDevice, m->st));
     MLP_TRY(hipStreamSynchronize(m->st));  // perm is reused by the next epoch
     double esum = 0.0;
+    if (m->fused) {  // the loss parts stay on the device until the epoch has run
+      for (int b = 0; b < nmb; ++b) {
+        const int r0 = b * batch, nb = (int)std::min<long>(batch, n - r0);
+        ++m->adam_t;
+        const Adam h{lr, b1, b2, eps, 1.0f - std::pow(b1, (float)m->adam_t),
+                     1.0f - std::pow(b2, (float)m->adam_t)};
+        minibatch(m, nb, m->idx + r0, m->Xin, m->Tin, m->parts + mp * b, &h);
+      }
+      MLP_TRY(hipGetLastError());
+      if (epoch_loss) {
+        part.resize(mp * nmb);
+        MLP_TRY(hipMemcpyAsync(part.data(), m->parts, part.size() * sizeof(float), hipMemcpyDeviceToHost,
+                               m->st));
+        MLP_TRY(hipStreamSynchronize(m->st));
+        for (int b = 0; b < nmb; ++b) {
+          const long nb = std::min<long>(batch, n - (long)b * batch);
+          double s = 0.0;
+          for (long k = 0; k < (nb * no + 255) / 256; ++k) s += part[mp * b + k];
+          esum += s;
+        }
+        epoch_loss[ep] = esum / ((double)n * no);
+      }
+      continue;
+    }
     for (int b = 0; b < nmb; ++b) {
       const int r0 = b * batch, nb = (int)std::min<long>(batch, n - r0);
       hipLaunchKernelGGL(k_gather_rows, dim3((nb * ni + 255) / 256), dim3(256), 0, m->st, nb, ni,

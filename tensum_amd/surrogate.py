@@ -38,6 +38,7 @@ def _mlib():
         L.tsm_mlp_get_params.argtypes = [C.c_void_p, C.c_void_p]
         L.tsm_mlp_set_params.argtypes = [C.c_void_p, C.c_void_p]
         L.tsm_mlp_forward.argtypes = [C.c_void_p, C.c_long, C.c_void_p, C.c_void_p]
+        L.tsm_mlp_forward_affine.argtypes = [C.c_void_p, C.c_long] + [C.c_void_p] * 6
         L.tsm_mlp_gradient.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p,
                                        C.POINTER(C.c_double), C.c_void_p]
         L.tsm_mlp_train.argtypes = [C.c_void_p, C.c_long, C.c_void_p, C.c_void_p, C.c_int,
@@ -103,6 +104,20 @@ class MLP:
         _chk(_mlib().tsm_mlp_forward(self._h, x.shape[0], _p(x), _p(y)))
         return y
 
+    def affine(self, u, mu_x, sd_x, mu_y, sd_y):
+        """net((u - mu_x) / sd_x) * sd_y + mu_y in FP64 around the network."""
+        f64 = lambda a: np.ascontiguousarray(a, dtype=np.float64)
+        n_in, n_out = self.widths[0], self.widths[-1]
+        u = np.asarray(u, dtype=np.float64)
+        if u.ndim != 2 or u.shape[1] not in (1, n_in):
+            raise ValueError(f"inputs of shape {u.shape}, expected (n, {n_in})")
+        u = f64(np.broadcast_to(u, (u.shape[0], n_in)))
+        a = [np.ascontiguousarray(np.broadcast_to(f64(v), (k,)))
+             for v, k in ((mu_x, n_in), (sd_x, n_in), (mu_y, n_out), (sd_y, n_out))]
+        y = np.empty((u.shape[0], n_out))
+        _chk(_mlib().tsm_mlp_forward_affine(self._h, u.shape[0], _p(u), *[_p(v) for v in a], _p(y)))
+        return y
+
     def gradient(self, x, t):
         x, t = _f32(x), _f32(t)
         g = np.empty(self.n_params, np.float32)
@@ -148,9 +163,8 @@ class Surrogate:
                               batch=batch, lr=lr, seed=seed)
 
     def __call__(self, u):
-        u = np.asarray(u, np.float64)
-        y = self.net((u - self.mu_x) / self.sd_x).astype(np.float64)
-        return y * self.sd_y + self.mu_y
+        # standardisation and its inverse run beside the network, on the device
+        return self.net.affine(u, self.mu_x, self.sd_x, self.mu_y, self.sd_y)
 
 
 @dataclass
