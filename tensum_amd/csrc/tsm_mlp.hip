@@ -11,7 +11,7 @@
 //   dW_l = dz_l^T x_l,  db_l = column sums of dz_l   (fp32)
 //   dx_l = dz_l W_l,    dz_{l-1} = dx_l * GELU'(z_{l-1})   (-> bf16)
 // Networks of layers up to FUSED_MAX wide (the surrogates are 64 to 256 wide) run
-// in three kernels: k_rows takes 32 rows of a minibatch through every layer and
+// in three kernels: k_rows takes eight rows of a minibatch through every layer and
 // back, k_update forms each 32 x 32 tile of the weight gradients and applies Adam
 // to it, k_infer takes rows through the layers only.  Wider ones take one launch
 // of the tiled GEMM per product, the operands' transposes absorbed by the LDS
@@ -210,7 +210,8 @@ inline int up(int n, int m) { return (n + m - 1) / m * m; }
 
 // Weights twice in bf16, zero-padded: Wp[l] is up(n_out, 32) x up(n_in, 16) (the
 // forward operand), Wt[l] its transpose, up(n_in, 32) x up(n_out, 16) (the
-// backward one), so a lane's eight k values are one aligned 16-byte load.
+// backward one), both in the order the MFMA operand reads them (w_at): a wave's
+// load of a 32 x 16 slice is one contiguous KB instead of 32 pieces of 32 bytes.
 // Activations x_l and dz_l of a minibatch are kept transposed (XT, DT: feature
 // x ldr rows, zero past the last row), which is how the weight gradients read
 // them and how the MFMA result falls out (four rows per lane at a time).
@@ -225,9 +226,14 @@ struct Net {
   float *Y, *T;
 };
 __host__ __device__ inline int upd(int n, int m) { return (n + m - 1) / m * m; }
+// element (n, k) of a weight operand of padded depth Kp: slices of 32 n x 16 k,
+// in a slice lane (k % 16 / 8) * 32 + n % 32 holds eight k one after another
+__device__ __forceinline__ int w_at(int n, int k, int Kp) {
+  return (n >> 5) * 32 * Kp + (k >> 4) * 512 + ((k >> 3) & 1) * 256 + (n & 31) * 8 + (k & 7);
+}
 
 // One layer's product for NT row tiles of 32: C (32 x 32 per tile, columns n0 ..)
-// from LDS activations A (row stride lda) and padded weights W (row stride Kp).
+// from LDS activations A (row stride lda) and weights W (padded depth Kp).
 template <int NT>
 __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W, int Kp, int n0,
                                              f32x16* acc) {
@@ -236,13 +242,13 @@ __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
-  const u16* wr = W + (size_t)(n0 + c) * Kp + ko;
+  const u16* wr = W + n0 * Kp + lane * 8;
   const u16* ar = A + c * lda + ko;
   int k0 = 0;
   for (; k0 + 128 <= Kp; k0 += 128) {  // eight slices in flight
     bf16x8 b[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) b[u] = *reinterpret_cast<const bf16x8*>(wr + k0 + 16 * u);
+    for (int u = 0; u < 8; ++u) b[u] = *reinterpret_cast<const bf16x8*>(wr + 32 * (k0 + 16 * u));
 #pragma unroll
     for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -252,7 +258,7 @@ __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W
       }
   }
   for (; k0 < Kp; k0 += 16) {
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(wr + k0);
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(wr + 32 * k0);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const bf16x8 a = *reinterpret_cast<const bf16x8*>(ar + t * RT * lda + k0);
@@ -263,26 +269,63 @@ __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W
 // row of result element i within a tile
 __device__ __forceinline__ int c_row(int i) { return 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
 
-// 32 rows of a minibatch (rows idx[r], or r itself) forward, dy = 2 (y - t) / n,
+// Weight slices of one 32-column tile in registers (layers up to 256 deep): the
+// loads of a layer are issued before the previous one's epilogue.
+struct WReg { bf16x8 b[16]; };
+__device__ __forceinline__ void load_tile(WReg& w, const u16* W, int Kp, int n0) {
+  const u16* wr = W + n0 * Kp + (threadIdx.x & 63) * 8;
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    if (16 * u < Kp) w.b[u] = *reinterpret_cast<const bf16x8*>(wr + 512 * u);
+}
+__device__ __forceinline__ void reg_product(const u16* A, int lda, const WReg& w, int Kp, f32x16& acc) {
+  const int lane = threadIdx.x & 63;
+  const u16* ar = A + (lane & 31) * lda + (lane >> 5) * 8;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    if (16 * u < Kp) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(ar + 16 * u);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w.b[u], acc, 0, 0, 0);
+    }
+}
+
+// RB rows of a minibatch (rows idx[r], or r itself) forward, dy = 2 (y - t) / n,
 // and back to dz_0; the transposed activations and dz of every layer go to XT/DT.
-// Bound by the latency of its 2 L - 1 dependent products (a layer's weights are
-// read from L2 once per 32 rows): eight waves, one or more 32-column tiles each.
+// Bound by the latency of its 2 L - 1 dependent products: eight waves, one or more
+// 32-column tiles each.  Eight rows a block, though the MFMA tile has 32: the
+// epilogues (an error function and an exponential per element) are most of the
+// work, rows 0-7 of a tile are elements 0-3 of every lane, and a minibatch of 64
+// then spreads over eight CUs instead of two.  At 64 rows of 6-256-256-66: 32 rows a
+// block 56 us; eight, with the next product's weights asked for ahead, 36; weights
+// in operand order 25.
+// REG: no layer wider than 256, so a wave has one tile per layer and holds its
+// weights in registers.
+constexpr int RB = 8;
+template <bool REG>
 __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, const float* Xin,
                                               const float* Tin, float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 sm[];
   u16 *cur = sm, *nxt = sm + RT * a.lda;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
-  const int r0 = blockIdx.x * RT, L = a.L;
+  const int r0 = blockIdx.x * RB, L = a.L;
+  WReg wr;
+  if (REG && 32 * wave < upd(a.w[1], 32)) load_tile(wr, a.Wp[0], upd(a.w[0], 16), 32 * wave);
   {
     const int K = a.w[0], Kp = upd(K, 16);
-    for (int i = tid; i < RT * Kp; i += blockDim.x) {
-      const int k = i / RT, r = i % RT;  // rows fastest: XT is written in order
+    for (int i = tid; i < RB * Kp; i += blockDim.x) {
+      const int k = i / RB, r = i % RB;  // rows fastest: XT is written in order
       const bool in = k < K && r0 + r < nb;
       const u16 v = in ? f2bf(Xin[(size_t)(idx ? idx[r0 + r] : r0 + r) * K + k]) : (u16)0;
       cur[r * a.lda + k] = v;
       if (k < K) a.XT[0][(size_t)k * a.ldr + r0 + r] = v;
     }
   }
+  const int row0 = 4 * (lane >> 5);  // this lane's rows: row0 .. row0 + 3
+  int rows[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) rows[u] = (idx && r0 + row0 + u < nb) ? idx[r0 + row0 + u] : r0 + row0 + u;
   __syncthreads();
   f32x16 acc[1];
   for (int l = 0; l < L; ++l) {
@@ -290,37 +333,51 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
     const bool last = l + 1 == L;
     const float* bias = a.P + a.boff[l];
     for (int n0 = 32 * wave; n0 < Np; n0 += 32 * nw) {
-      tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
       const int n = n0 + (lane & 31);
       const bool col = n < N;
       const float bn = col ? bias[n] : 0.0f;
+      float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (last && col)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        ushort4 q;
-        u16* qv = reinterpret_cast<u16*>(&q);
+        for (int u = 0; u < 4; ++u)
+          if (r0 + row0 + u < nb) t[u] = Tin[(size_t)rows[u] * N + n];
+      if (REG) reg_product(cur, a.lda, wr, Kp, acc[0]);
+      else tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
+      if (REG) {  // the next product's weights: the next layer's, or the last one's transposed
+        if (!last) {
+          if (n0 < upd(a.w[l + 2], 32)) load_tile(wr, a.Wp[l + 1], upd(N, 16), n0);
+        } else if (L > 1 && n0 < upd(K, 32)) {
+          load_tile(wr, a.Wt[l], upd(N, 16), n0);
+        }
+      }
+      ushort4 q;
+      u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = 4 * g + u, row = c_row(i), r = r0 + row;
-          const bool in = col && r < nb;
-          const float c = acc[0][i] + bn;
-          u16 v = 0;
-          if (in) {
-            if (last) {
-              a.Y[(size_t)r * N + n] = c;
-              const float t = Tin[(size_t)(idx ? idx[r] : r) * N + n];
-              v = f2bf(2.0f * (c - t) * scale);
-            } else {
-              a.Z[l][(size_t)r * N + n] = c;
-              v = f2bf(gelu(c));
-            }
+      for (int u = 0; u < 4; ++u) {
+        const int row = row0 + u, r = r0 + row;
+        const bool in = col && r < nb;
+        const float c = acc[0][u] + bn;
+        u16 v = 0;
+        if (in) {
+          if (last) {
+            a.Y[(size_t)r * N + n] = c;
+            v = f2bf(2.0f * (c - t[u]) * scale);
+          } else {
+            a.Z[l][(size_t)r * N + n] = c;
+            v = f2bf(gelu(c));
           }
-          qv[u] = v;
-          nxt[row * a.lda + n] = v;
         }
-        if (col) {
-          u16* o = (last ? a.DT[l] : a.XT[l + 1]) + (size_t)n * a.ldr + r0 + c_row(4 * g);
-          *reinterpret_cast<ushort4*>(o) = q;
-        }
+        qv[u] = v;
+        nxt[row * a.lda + n] = v;
+      }
+      if (col) *reinterpret_cast<ushort4*>((last ? a.DT[l] : a.XT[l + 1]) + (size_t)n * a.ldr + r0 + row0) = q;
+    }
+    // a wave without a tile in this layer may have one in the next
+    if (REG && 32 * wave >= Np) {
+      if (!last) {
+        if (32 * wave < upd(a.w[l + 2], 32)) load_tile(wr, a.Wp[l + 1], upd(N, 16), 32 * wave);
+      } else if (L > 1 && 32 * wave < upd(K, 32)) {
+        load_tile(wr, a.Wt[l], upd(N, 16), 32 * wave);
       }
     }
     __syncthreads();
@@ -329,30 +386,30 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
   // dz_{l-1} = (dz_l W_l) * GELU'(z_{l-1}); z was stored by this very lane
   for (int l = L - 1; l > 0; --l) {
     const int K = a.w[l], N = a.w[l + 1], Np = upd(N, 16), Kp = upd(K, 32);
+    const int k1 = l > 1 ? upd(a.w[l - 1], 32) : 0;  // columns of the next product
     for (int k0 = 32 * wave; k0 < Kp; k0 += 32 * nw) {
       const int k = k0 + (lane & 31);
       const bool col = k < K;
-      float z[16];
+      float z[4];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = r0 + c_row(i);
-        z[i] = col && r < nb ? a.Z[l - 1][(size_t)r * K + k] : 0.0f;
+      for (int u = 0; u < 4; ++u) {
+        const int r = r0 + row0 + u;
+        z[u] = col && r < nb ? a.Z[l - 1][(size_t)r * K + k] : 0.0f;
       }
-      tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
+      if (REG) reg_product(cur, a.lda, wr, Np, acc[0]);
+      else tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
+      if (REG && k0 < k1) load_tile(wr, a.Wt[l - 1], upd(K, 16), k0);
+      ushort4 q;
+      u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        ushort4 q;
-        u16* qv = reinterpret_cast<u16*>(&q);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = 4 * g + u, row = c_row(i);
-          const u16 v = col && r0 + row < nb ? f2bf(acc[0][i] * gelu_d(z[i])) : (u16)0;
-          qv[u] = v;
-          nxt[row * a.lda + k] = v;
-        }
-        if (col) *reinterpret_cast<ushort4*>(a.DT[l - 1] + (size_t)k * a.ldr + r0 + c_row(4 * g)) = q;
+      for (int u = 0; u < 4; ++u) {
+        const u16 v = col && r0 + row0 + u < nb ? f2bf(acc[0][u] * gelu_d(z[u])) : (u16)0;
+        qv[u] = v;
+        nxt[(row0 + u) * a.lda + k] = v;
       }
+      if (col) *reinterpret_cast<ushort4*>(a.DT[l - 1] + (size_t)k * a.ldr + r0 + row0) = q;
     }
+    if (REG && 32 * wave >= Kp && 32 * wave < k1) load_tile(wr, a.Wt[l - 1], upd(K, 16), 32 * wave);
     __syncthreads();
     u16* x = cur; cur = nxt; nxt = x;
   }
@@ -360,19 +417,19 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
 
 // Adam on one parameter, as k_adam
 struct Adam { float lr, b1, b2, eps, c1, c2; };
-__device__ __forceinline__ float adam_step(const Net& a, const Adam& h, int i, float gi) {
-  const float mi = h.b1 * a.Mo[i] + (1.0f - h.b1) * gi;
-  const float vi = h.b2 * a.Vo[i] + (1.0f - h.b2) * gi * gi;
-  a.Mo[i] = mi;
-  a.Vo[i] = vi;
-  const float wi = a.P[i] - h.lr * (mi / h.c1) / (sqrtf(vi / h.c2) + h.eps);
-  a.P[i] = wi;
-  return wi;
+__device__ __forceinline__ float adam_step(const Adam& h, float gi, float p, float* m, float* v) {
+  const float mi = h.b1 * *m + (1.0f - h.b1) * gi;
+  const float vi = h.b2 * *v + (1.0f - h.b2) * gi * gi;
+  *m = mi;
+  *v = vi;
+  return p - h.lr * (mi / h.c1) / (sqrtf(vi / h.c2) + h.eps);
 }
 // One job per wave: a 32 x 32 tile of a layer's weight gradient (MFMA over the
 // rows), 64 bias gradients (sums in row order), or one 256-element part of the
 // loss (the tree of k_mse).  TRAIN applies Adam at once and refreshes the bf16
-// weights; else the gradient goes to G.
+// weights; else the gradient goes to G.  Bound by the latency of one pass over
+// activations and moments (85 k parameters, 2.4 MB, 0.5 us at the copy rate):
+// 13.9 us with each parameter's moments read in turn, 11.7 with all ahead.
 template <bool TRAIN>
 __global__ __launch_bounds__(256) void k_update(Net a, int nb, const int4* jobs, int n_jobs,
                                                 const int* idx, const float* Tin, float* part, Adam h) {
@@ -412,13 +469,29 @@ __global__ __launch_bounds__(256) void k_update(Net a, int nb, const int4* jobs,
       for (int u = 0; u < 8; ++u) s += bf2f(q[u]);
     }
     for (; r < nb; ++r) s += bf2f(d[r]);
-    if (TRAIN) (void)adam_step(a, h, a.boff[l] + n, s);
-    else a.G[a.boff[l] + n] = s;
+    const int q = a.boff[l] + n;
+    if (TRAIN) a.P[q] = adam_step(h, s, a.P[q], &a.Mo[q], &a.Vo[q]);
+    else a.G[q] = s;
     return;
   }
   const int c = lane & 31, ko = (lane >> 5) * 8;
   const int nr = min(J.z + c, N - 1), kr = min(J.w + c, K - 1);  // rows past the layer: any, not stored
   const u16 *dr = a.DT[l] + (size_t)nr * a.ldr + ko, *xr = a.XT[l] + (size_t)kr * a.ldr + ko;
+  const int k = J.w + c, Kp = upd(K, 16), Np = upd(N, 16);
+  const bool in = k < K;
+  // the moments and weights are asked for before the product: 48 loads in flight
+  // instead of 16 waits for three
+  float p[16], mo[16], vo[16];
+  if (TRAIN) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int n = J.z + c_row(i), q = a.woff[l] + n * K + k;
+      const bool ok = in && n < N;
+      p[i] = ok ? a.P[q] : 0.0f;
+      mo[i] = ok ? a.Mo[q] : 0.0f;
+      vo[i] = ok ? a.Vo[q] : 0.0f;
+    }
+  }
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
@@ -427,19 +500,21 @@ __global__ __launch_bounds__(256) void k_update(Net a, int nb, const int4* jobs,
     const bf16x8 B = *reinterpret_cast<const bf16x8*>(xr + k0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, acc, 0, 0, 0);
   }
-  const int k = J.w + c, Kp = upd(K, 16), Np = upd(N, 16);
-  if (k >= K) return;
+  if (!in) return;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int n = J.z + c_row(i);
+    const int n = J.z + c_row(i), q = a.woff[l] + n * K + k;
     if (n >= N) continue;
-    const int p = a.woff[l] + n * K + k;
     if (TRAIN) {
-      const u16 wb = f2bf(adam_step(a, h, p, acc[i]));
-      a.Wp[l][(size_t)n * Kp + k] = wb;
-      a.Wt[l][(size_t)k * Np + n] = wb;
+      const float w = adam_step(h, acc[i], p[i], &mo[i], &vo[i]);
+      a.Mo[q] = mo[i];
+      a.Vo[q] = vo[i];
+      a.P[q] = w;
+      const u16 wb = f2bf(w);
+      a.Wp[l][w_at(n, k, Kp)] = wb;
+      a.Wt[l][w_at(k, n, Np)] = wb;
     } else {
-      a.G[p] = acc[i];
+      a.G[q] = acc[i];
     }
   }
 }
@@ -451,8 +526,8 @@ __global__ void k_pack_weights(Net a, int l) {
   if (i >= N * K) return;
   const int n = i / K, k = i % K;
   const u16 v = f2bf(a.P[a.woff[l] + i]);
-  a.Wp[l][(size_t)n * upd(K, 16) + k] = v;
-  a.Wt[l][(size_t)k * upd(N, 16) + n] = v;
+  a.Wp[l][w_at(n, k, upd(K, 16))] = v;
+  a.Wt[l][w_at(k, n, upd(N, 16))] = v;
 }
 
 // NT x 32 rows through the layers.  AFFINE: inputs (u - mu_x) / sd_x and outputs
@@ -652,16 +727,24 @@ void minibatch(tsm_mlp* m, int nb, const int* idx, const float* X, const float* 
                const Adam* h) {
   const int no = m->w[m->L], n = nb * no;
   const size_t lds = rows_lds(m);
-  if (lds > 48 * 1024)
-    (void)hipFuncSetAttribute((const void*)k_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(k_rows, dim3((nb + RT - 1) / RT), dim3(512), lds, m->st, m->net, nb, idx, X, T,
-                     1.0f / (float)n);
+  // rows of XT/DT lie side by side for this minibatch (one stride of the largest
+  // one a page apart would put every feature into the same cache sets)
+  Net net = m->net;
+  net.ldr = up(nb, RT);
+  auto rows = [&](auto k) {
+    if (lds > 48 * 1024)
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // every row k_update reads (16 a product) is written, zero past the last
+    hipLaunchKernelGGL(k, dim3(up(nb, 16) / RB), dim3(512), lds, m->st, net, nb, idx, X, T,
+                       1.0f / (float)n);
+  };
+  if (net.lda <= 256 + 8) rows(k_rows<true>); else rows(k_rows<false>);
   const int jobs = m->n_jobs + (n + 255) / 256;
   if (h)
-    hipLaunchKernelGGL((k_update<true>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, m->net, nb, m->jobs,
+    hipLaunchKernelGGL((k_update<true>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, net, nb, m->jobs,
                        m->n_jobs, idx, T, part, *h);
   else
-    hipLaunchKernelGGL((k_update<false>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, m->net, nb, m->jobs,
+    hipLaunchKernelGGL((k_update<false>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, net, nb, m->jobs,
                        m->n_jobs, idx, T, part, Adam{});
 }
 
