@@ -67,7 +67,8 @@ typedef struct tsm_params {
      option except bc_scheme strong), CSR-gather kernels otherwise; 1 = always
      the CSR-gather kernels.  Both give the reference's summation order. */
   int kernel_path;
-  int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128);
+  int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128, or 112 with viscous
+                         terms and gradients);
                          smaller ones are taken where two halo rings of a tile do
                          not fit LDS */
   int block_grad;     /* checked against the block limits; the stage kernel forms

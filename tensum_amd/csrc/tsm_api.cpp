@@ -181,7 +181,12 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   // hundreds of cells) takes smaller tiles, and the CSR kernels if none fits.
   if (params->kernel_path != 0 || params->strong_bc)
     return create_with_tiles(mesh, params, n_samples, 0, out);
-  const int want = params->tile_vertices > 0 ? params->tile_vertices : 128;
+  // 128 vertices, or 112 where viscous cells share LDS with gradients: 50 KB then,
+  // three tiles per CU instead of two (57 KB).  A no-slip channel with KEPES-TeCNO
+  // Roe and minmod, per step: 257^2 68 us against 86, 400^2 119 against 142, 640^2
+  // 234 against 281; 96 vertices 69, 140, 269.  Euler at 513^2: 128 110 us, 112 112.
+  const bool narrow = params->model == 1 && tsm::stage_has_gradients(params->flux, params->reconstruct);
+  const int want = params->tile_vertices > 0 ? params->tile_vertices : narrow ? 112 : 128;
   for (int tb = want;; tb /= 2) {
     rc = create_with_tiles(mesh, params, n_samples, tb < 16 && tb < want ? 0 : tb, out);
     if (rc != 1) return rc;
@@ -481,7 +486,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     rc = tsm::build_stage_tables(c->G, TG, tsm::stage_has_gradients(params->flux, params->reconstruct),
                                  params->model == 1, wall_cells, c->ST, dalloc, c->st, msg);
     // the static LDS of the kernel and its launches fit beside this much
-    if (rc == 0 && tsm::stage_lds(c->ST, params->flux, params->reconstruct, params->model == 1) > 156 * 1024)
+    if (rc == 0 && tsm::stage_lds(c->ST) > 156 * 1024)
       rc = 1;
     if (rc) {
       delete c;

@@ -73,12 +73,12 @@ struct TileGeo {
   const unsigned short* gent;
 };
 
-// 16-bit items of a gradient slot (StageTab::items): bits 15..14 say what
-// it is (a neighbour; a new centre; a boundary term of the tile; the end or
-// "more in the overflow list"), bit 13 is a flag (neighbour: the cell that ends
-// in it is a wall cell; centre: it is the slot's own vertex), bit 12 marks the
-// first neighbour of a closed chain, bits 11..0 are the slot or the term.
-constexpr unsigned SI_CENTRE = 0x4000u, SI_TERM = 0x8000u, SI_END = 0xc000u, SI_MORE = 0xc001u,
+// 16-bit items of a gradient slot: neighbours (bit 12: first of a closed chain) in
+// bits 11..0 the slot, boundary terms (SI_TERM | term), SI_END past the last.
+// StageTab::items is a chain of up to eight neighbours; a group (items2, ov) is a
+// head and seven items: SI_CENTRE | centre slot and a chain (SI_FLAG: the chain goes
+// on from the group before; SI_CLOSED: it goes on in the next), or SI_TERM and terms.
+constexpr unsigned SI_CENTRE = 0x4000u, SI_TERM = 0x8000u, SI_END = 0xc000u,
                    SI_FLAG = 0x2000u, SI_CLOSED = 0x1000u;
 constexpr int SI_MASK = 0x0fff;
 // 16-bit gather entries (StageTab::ge8): local face | bit 15 at the right end;
@@ -88,29 +88,36 @@ constexpr unsigned GE_END = 0x7fffu, GE_MORE = 0x7ffeu;
 // Tables of the stage kernel (tsm_stagetab.hip), each with one stride per tile.
 struct StageTab {
   int ntiles, tb, n_periodic_tiles, fu_block;
-  int ms, ms1, mf, mbt, mwt, mc;  // largest counts of a tile: slots, gradient slots,
-                              // local faces, boundary terms, wall terms, viscous cells
+  int ms, ms1, mf, mbt, mwt, mc, mb;  // largest counts of a tile: slots, gradient slots,
+                              // local faces, boundary terms, wall terms, viscous cells,
+                              // boundary entries
+  int bf0;                    // boundary entry k of a tile is its face bf0 + k
   const int4* desc;           // first owned vertex, owned, gradient slots,
                               // local faces | bit 30: items other than neighbours
   const int* sid;             // ms per tile: vertex of each slot, -1 past the last
   const unsigned* f_lr;       // mf per tile: left slot | right slot << 16
   const double2* f_n;         // mf per tile: normals
   const double2* xy;          // per vertex
-  const uint4* items;         // ms1 per tile: eight items per gradient slot ...
-  const uint4* items2;        // ... and eight more (tiles marked in desc)
-  const int* item_ov;         // ms1 per tile: where SI_MORE continues in ov
-  const unsigned short* ov;
+  const uint4* items;         // ms1 per tile: the first chain of each gradient slot (up to eight)
+  const uint4* items2;        // tiles marked in desc: the first group of extras
+  const int2* item_x;         // ... the chain's centre | groups in ov << 12; the first of these
+  const uint4* ov;
   const uint4* ge8;           // per vertex: eight gather entries
   const unsigned* vcells;     // mc per tile: corner slots of the viscous cells (3 x 10 bits),
                               // all ones past the last
   const uint4* vc8;           // per vertex: its first eight viscous cells (| corner << 13)
   const int* vccnt;           // per vertex: how many there are ...
   const unsigned short* vcent;  // ... all of them, along DevGeo::vc
-  const int *btbeg, *bt;      // boundary terms of each tile (bfaces)
-  const int *wtbeg, *wt;      // wall terms of each tile (bfaces), null without wall cells
-  const uint2* wcell;         // their cells' corner slots
+  const int* vbp;             // per vertex: its first boundary entry
+  const int2* be;             // boundary entries: bface, owned vertex of the tile | end << 16
+  const int* btbeg;           // boundary terms of each tile:
+  const int4* bt;             // bface, its vertices
+  const int* wtbeg;           // wall terms of each tile, null without wall cells:
+  const uint4* wcell;         // three each: bface, corner slots (16 bits each, in y and z),
+                              // boundary terms of the cell (16 bits each, all ones: none);
+                              // the cell's wall faces: vertices, bface | ends << 30, face
   const unsigned short* wvent;  // along vbe: term | corner << 13 | ends the bface << 15
-  const int *tper, *pinfo, *gptr, *bbeg, *tbf;
+  const int *tper, *pinfo, *gptr;
   const unsigned short* gent;
 };
 
@@ -366,7 +373,8 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
                        std::string& msg);
 int stage_block(const StageTab& T);
 int stage_block_max();
-size_t stage_lds(const StageTab& T, int flux, int rec, bool ns);
+size_t stage_lds(const StageTab& T);
+int stage_main_records(const StageTab& T, bool grad, bool ns);
 bool stage_has_gradients(int flux, int rec);
 bool stage_keeps_var0(int flux);
 void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const StageArgs& A,

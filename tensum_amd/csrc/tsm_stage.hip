@@ -75,6 +75,7 @@ constexpr int NBT = 6;   // record per boundary term: normal | dq x4
 constexpr int NWT = 12;  // record per wall term: flux of the three corners, wall flux
 constexpr int NVC = 6;   // record per viscous cell: its flux to the first two corners
 constexpr int FPT = 2;   // faces per thread
+constexpr int SR_VERTS = 64;  // owned vertices of a tile with periodic sets: at most a quarter of 256
 
 // Cell viscous flux: stress and energy flux per unit normal from the mean
 // entropy variables (vx, vy, l) and their gradients (x, y each)
@@ -120,22 +121,48 @@ __device__ __forceinline__ void flux_vars(const Gas& gas, const Prim& w, double*
   V[1] = -w.u * V[3];
   V[2] = -w.v * V[3];
 }
+// This is end e's share of it; V0: its own first entropy variable where that is
+// kept, else null.
 __device__ __forceinline__ void boundary_dq(const DevGeo& G, const StageArgs& A, const Gas& gas,
-                                            int s, size_t off, int b, double* dq) {
-  const int type = G.btype[b];
-  const double nx = G.bn[2 * b], ny = G.bn[2 * b + 1];
+                                            int s, size_t off, int b, int e, int v,
+                                            const double* V0, double* dq) {
+  const Prim w = ld_prim(A.W_in, off + v);
+  Prim x = w;
+  bc_apply1(G.btype[b], bc_values(G, s, b, e), G.bn[2 * b], G.bn[2 * b + 1], x);
+  double V[4], Vb[4];
+  V[3] = -fdiv(1.0, gas.R * w.T);
+  V[0] = V0 ? V0[off + v] : entropy_var0(gas, w);
+  V[1] = -w.u * V[3];
+  V[2] = -w.v * V[3];
+  flux_vars(gas, x, Vb);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) dq[q] = 0.0;
-  for (int e = 0; e < 2; ++e) {
-    const Prim w = ld_prim(A.W_in, off + G.bv[2 * b + e]);
-    Prim x = w;
-    bc_apply1(type, bc_values(G, s, b, e), nx, ny, x);
-    double V[4], Vb[4];
-    flux_vars(gas, w, V);
-    flux_vars(gas, x, Vb);
+  for (int q = 0; q < 4; ++q) dq[q] = 0.5 * (Vb[q] - V[q]);
+}
+
+// The state of a wall cell (wall_cell_state) from its term's wall faces: vertices,
+// bface with the vertices' ends of it in the top bits, face.
+__device__ __forceinline__ Ent wall_state(const DevGeo& G, const double* W, size_t off, int s,
+                                          const Gas& gas, const uint4* faces) {
+  Ent e{0.0, 0.0, 0.0, 0.0};
+  int n = 0;
+  for (int t = 0; t < 2; ++t) {
+    const uint4 q = faces[t];
+    const int f = (int)q.w, b = (int)(q.z & 0x3fffffffu);
+    if (f < 0) break;
+    const int type = G.btype[b];
+    const double nx = G.fn[2 * f], ny = G.fn[2 * f + 1];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dq[q] += 0.5 * (Vb[q] - V[q]);
+    for (int k = 0; k < 2; ++k) {
+      Prim st = ld_prim(W, off + (k ? q.y : q.x));
+      bc_apply1(type, bc_values(G, s, b, (q.z >> (30 + k)) & 1), nx, ny, st);
+      const Ent x = prim2ent(gas, st);
+      e.vx += x.vx; e.vy += x.vy; e.l += x.l;
+    }
+    ++n;
   }
+  const double sc = 0.5 * 1.0 / n;
+  e.vx *= sc; e.vy *= sc; e.l *= sc;
+  return e;
 }
 
 template <int FLUX, int REC>
@@ -150,14 +177,14 @@ __device__ __forceinline__ Cons pair_flux(const Gas& gas, const FluxOpts& fo, do
   return avg_flux(gas, L.w, R.w, unx, uny);
 }
 
-// Boundary flux of bface b at a vertex with state wm (src/fv.cc:1100-1189)
+// Boundary flux of bface b, normal (nx, ny), at its end e with state wm
+// (src/fv.cc:1100-1189)
 template <int FLUX, int REC>
 __device__ __forceinline__ Cons bflux(const DevGeo& G, const FluxOpts& fo, const Gas& gas, int b,
-                                   int s, int v, const Prim& wm) {
-  int type = G.btype[b];
-  double nx = G.bn[2 * b], ny = G.bn[2 * b + 1];
+                                   int s, int e, double nx, double ny, const Prim& wm) {
+  const int type = G.btype[b];
   Prim s0 = wm, s1 = wm;
-  bc_apply2(type, bc_values(G, s, b, bc_end(G, b, v)), nx, ny, s0, s1);
+  bc_apply2(type, bc_values(G, s, b, e), nx, ny, s0, s1);
   if (type == TSM_BC_FARFIELD) {
     double area = fsqrt(nx * nx + ny * ny);
     double ia = fdiv(1.0, area);
@@ -230,59 +257,53 @@ __device__ __forceinline__ void fan_end(Fan& f, double* acc) {
   fan_share(ex - f.ax, ey - f.ay, f.p, acc);
   if (f.closed) fan_share(-f.p.x, -f.p.y, f.first, acc);
 }
-// the tile's items are one chain of at most eight neighbours for every slot
-__device__ __forceinline__ void walk_simple(Fan& f, const uint4& it, const double* SA, double* acc) {
+__device__ __forceinline__ unsigned item_at(const uint4& it, int u) {
   const unsigned w[4] = {it.x, it.y, it.z, it.w};
-  fan_first(f, fan_rel(f, SA, w[0]), w[0]);
+  return (w[u >> 1] >> (16 * (u & 1))) & 0xffffu;
+}
+// the first chain, up to eight neighbours
+__device__ __forceinline__ void walk_chain(Fan& f, const uint4& it, const double* SA, double* acc) {
+  fan_first(f, fan_rel(f, SA, item_at(it, 0)), item_at(it, 0));
 #pragma unroll
   for (int u = 1; u < 8; ++u) {
-    const unsigned e = (w[u >> 1] >> (16 * (u & 1))) & 0xffffu;
+    const unsigned e = item_at(it, u);
     if (e < SI_CENTRE) fan_next(f, fan_rel(f, SA, e), acc);
   }
   fan_end(f, acc);
 }
-// any items: further chains around the same or another centre (periodic sets),
-// boundary terms, overflow
-__device__ __forceinline__ void walk_any(Fan& f, const uint4& ia, const uint4& ib, const int* item_ov,
-                                         const unsigned short* ov, const double* SA,
-                                         const double* SBT, double* acc) {
-  unsigned long long w0 = ((unsigned long long)ia.y << 32) | ia.x, w1 = ((unsigned long long)ia.w << 32) | ia.z,
-                     w2 = ((unsigned long long)ib.y << 32) | ib.x, w3 = ((unsigned long long)ib.w << 32) | ib.z;
-  const unsigned short* more = nullptr;
-  bool any = false;
-  for (int u = 0;; ++u) {
-    unsigned e = SI_END;
-    if (more) {
-      e = *more++;
-    } else if (u < 16) {
-      e = (unsigned)(w0 & 0xffffull);
-      w0 >>= 16;
-      if ((u & 3) == 3) { w0 = w1; w1 = w2; w2 = w3; }
+// One group of a slot's extras: a further chain around its own or another centre
+// (periodic sets) or boundary terms.  Few slots of a tile have any, and those of a
+// tile are mostly alike, so a group is unrolled like the first chain: entry by
+// entry in a loop, a tile with periodic vertices took 18,600 cycles for its
+// gradients instead of 3,000.
+__device__ __forceinline__ void walk_group(Fan& f, const uint4& g, const double* SA, const double* SBT,
+                                           double* acc) {
+  const unsigned head = item_at(g, 0);
+  if (head < SI_TERM) {
+    unsigned e = item_at(g, 1);
+    if (!(head & SI_FLAG)) {
+      fan_centre(f, SA, head & SI_MASK);
+      fan_first(f, fan_rel(f, SA, e), e);
+    } else {
+      fan_next(f, fan_rel(f, SA, e), acc);
     }
-    if (e < SI_CENTRE) {
-      const Rel w = fan_rel(f, SA, e);
-      if (any) fan_next(f, w, acc);
-      else fan_first(f, w, e);
-      any = true;
-      continue;
+#pragma unroll
+    for (int u = 2; u < 8; ++u) {
+      e = item_at(g, u);
+      if (e < SI_CENTRE) fan_next(f, fan_rel(f, SA, e), acc);
     }
-    if (e == SI_MORE) {
-      more = ov + *item_ov;
-      continue;
-    }
-    if (any) fan_end(f, acc);
-    any = false;
-    if (e < SI_TERM) {
-      fan_centre(f, SA, e & SI_MASK);
-    } else if (e < SI_END) {
+    if (!(head & SI_CLOSED)) fan_end(f, acc);
+  } else {
+#pragma unroll
+    for (int u = 1; u < 8; ++u) {
+      const unsigned e = item_at(g, u);
+      if (e >= SI_END) continue;
       const double* b = SBT + NBT * (e & SI_MASK);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         acc[2 * q] = __builtin_fma(b[0], b[2 + q], acc[2 * q]);
         acc[2 * q + 1] = __builtin_fma(b[1], b[2 + q], acc[2 * q + 1]);
       }
-    } else {
-      return;
     }
   }
 }
@@ -364,9 +385,8 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
   using L = Layout<FLUX, REC>;
   extern __shared__ __attribute__((aligned(16))) double lds[];
   __shared__ double wred[8 * 5];
-  __shared__ double SR[4 * 64];  // periodic exchange: at most a quarter of 256 vertices
   __shared__ int arrive;
-  if (A.ctl[s].done) return;
+  const int finished = A.ctl[s].done;
   const int tid = threadIdx.x, nth = blockDim.x;
   const int4 D = T.desc[t];
   const int b0 = D.x, nown = D.y, n1 = D.z, nfl = D.w & 0x3fffffff;
@@ -377,10 +397,11 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
   double* SAR = SF + NFR * T.mf;     // last stage: face areas
   double* SDL = SAR + T.mf;          // ... and distances of their ends (viscous)
   double* SVC = SB + L::NB * T.ms1;  // viscous cells, consumed before the fluxes
-  const int main_sz = (max(L::NA * T.ms + L::NB * T.ms1 + (NS ? NVC * T.mc : 0),
-                           (NFR + (NS ? 2 : 1)) * T.mf) + 1) & ~1;
-  double* SBT = lds + main_sz;       // boundary terms
+  double* SBF = lds + NFR * T.bf0;   // boundary entries as faces bf0 + k, kept from phase 2 on
+  double* SBA = SBF + NFR * T.mb;    // ... and their areas
+  double* SBT = SBA + ((T.mb + 1) & ~1);  // boundary terms
   double* SWT = SBT + NBT * T.mbt;   // wall terms
+  double* SR = SWT + NWT * T.mwt;    // periodic exchange
   const size_t off = (size_t)s * G.nv;
   const Gas gas = load_gas(A, s);
   if (LAST && tid == 0) arrive = 0;  // read after the phase barriers
@@ -402,20 +423,47 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     }
   }
   uint4 it = make_uint4(0, 0, 0, 0), it2 = make_uint4(0, 0, 0, 0);
+  int2 ix = make_int2(0, 0);
   double fact = 0.0;
   if (L::GRAD && tid < n1) {
     it = T.items[(size_t)t * T.ms1 + tid];
-    if (!simple) it2 = T.items2[(size_t)t * T.ms1 + tid];
+    if (!simple) {
+      it2 = T.items2[(size_t)t * T.ms1 + tid];
+      ix = T.item_x[(size_t)t * T.ms1 + tid];
+    }
     fact = G.gfact[ga];
+  }
+  // boundary terms and viscous cells go from the last thread down: its wave has
+  // no gradient slots.  Boundary entries start at the first wave, wall terms at the
+  // second: the waves of a tile at a wall then end this phase together
+  const int back = nth - 1 - tid;
+  int e0 = 0, nbe = 0;
+  int2 be = make_int2(0, 0);
+  if (T.mb) {
+    e0 = T.vbp[b0];
+    nbe = T.vbp[b0 + nown] - e0;
+    if (tid < nbe) be = T.be[e0 + tid];
   }
   unsigned vcell = ~0u;
   uint4 vc = make_uint4(0, 0, 0, 0);
   if (NS) {
-    if (tid < T.mc) vcell = T.vcells[(size_t)t * T.mc + tid];
+    if (back < T.mc) vcell = T.vcells[(size_t)t * T.mc + back];
     if (tid < nown) vc = T.vc8[b0 + tid];
   }
 
   // ---- phase 1: slot records, boundary terms ---------------------------------
+  // the part of record B beside the gradients
+  auto slot_b = [&](int gid, const Prim& w, double rho) -> double2 {
+    if (L::PT) return make_double2(w.T, w.p);
+    // Roe: the sound speed, negated where the vertex's Liou sensor is set
+    // (liou_fix; c > 0, so the sign carries the flag)
+    double c = 0.0;
+    if (FLUX == F_ROE) {
+      c = sound_speed(gas, w);
+      if (A.ssw && A.ssw[off + gid] > 0.0) c = -c;
+    }
+    return make_double2(rho, c);
+  };
   auto put_slot = [&](int i, int gid, const Prim& w, double V0, const double2& xy) {
     const double beta = 0.5 * frcp(gas.R * w.T);
     const double rho = (2.0 * beta) * w.p;
@@ -424,21 +472,11 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     sts2(a + 2, beta, L::TEC ? V0 : rho);
     sts2(a + 4, xy.x, xy.y);
     if (L::NB && i < n1) {
-      double* b = SB + L::NB * i + (L::GRAD ? 8 : 0);
-      if (L::PT) {
-        sts2(b, w.T, w.p);
-      } else {
-        // Roe: the sound speed, negated where the vertex's Liou sensor is set
-        // (liou_fix; c > 0, so the sign carries the flag)
-        double c = 0.0;
-        if (FLUX == F_ROE) {
-          c = sound_speed(gas, w);
-          if (A.ssw && A.ssw[off + gid] > 0.0) c = -c;
-        }
-        sts2(b, rho, c);
-      }
+      const double2 q = slot_b(gid, w, rho);
+      sts2(SB + L::NB * i + (L::GRAD ? 8 : 0), q.x, q.y);
     }
   };
+  if (finished) return;  // here, so that the requests do not wait for the answer
   {
     Prim wa{1, 0, 0, 1}, wb{1, 0, 0, 1};
     double va = 0.0, vb = 0.0;
@@ -463,11 +501,15 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
   }
   if (L::GRAD && !simple) {
     const int k0 = T.btbeg[t], nbt = T.btbeg[t + 1] - k0;
-    for (int j = nth - 1 - tid; j < nbt; j += nth) {
-      const int b = T.bt[k0 + j];
+    for (int j = back; j < 2 * nbt; j += nth) {  // two lanes a term, one for each end
+      const int4 bt = T.bt[k0 + (j >> 1)];
+      const int b = bt.x;
       double dq[4];
-      boundary_dq(G, A, gas, s, off, b, dq);
-      double* o = SBT + NBT * j;
+      boundary_dq(G, A, gas, s, off, b, j & 1, (j & 1) ? bt.z : bt.y, A.V_in, dq);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dq[q] += __shfl_xor(dq[q], 1, 64);
+      if (j & 1) continue;
+      double* o = SBT + NBT * (j >> 1);
       sts2(o, G.bn[2 * b], G.bn[2 * b + 1]);
       sts2(o + 2, dq[0], dq[1]);
       sts2(o + 4, dq[2], dq[3]);
@@ -481,37 +523,68 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     for (int k = tid; k < n1; k += nth) {
       if (k != tid) {
         it = T.items[(size_t)t * T.ms1 + k];
-        if (!simple) it2 = T.items2[(size_t)t * T.ms1 + k];
+        if (!simple) {
+          it2 = T.items2[(size_t)t * T.ms1 + k];
+          ix = T.item_x[(size_t)t * T.ms1 + k];
+        }
         fact = G.gfact[sid[k]];
       }
       double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       Fan f;
-      fan_centre(f, SA, k);
-      if (simple) walk_simple(f, it, SA, acc);
-      else walk_any(f, it, it2, T.item_ov + (size_t)t * T.ms1 + k, T.ov, SA, SBT, acc);
+      if (simple) {
+        fan_centre(f, SA, k);
+        walk_chain(f, it, SA, acc);
+      } else {
+        int more = ix.x >> 12;
+        uint4 g2 = make_uint4(0, 0, 0, 0);
+        if (more > 0) g2 = T.ov[ix.y];
+        fan_centre(f, SA, ix.x & SI_MASK);
+        if (item_at(it, 0) < SI_CENTRE) walk_chain(f, it, SA, acc);
+        int at = ix.y;
+        while (item_at(it2, 0) < SI_END) {
+          walk_group(f, it2, SA, SBT, acc);
+          if (more-- == 0) break;
+          it2 = g2;
+          if (more > 0) g2 = T.ov[++at];
+        }
+      }
       double* d = SB + L::NB * k;
 #pragma unroll
       for (int q = 0; q < 8; q += 2) sts2(d + q, acc[q] * fact, acc[q + 1] * fact);
     }
   }
+  for (int j = tid; j < nbe; j += nth) {  // boundary fluxes, half a bface per end
+    if (j != tid) be = T.be[e0 + j];
+    const int b = be.x;
+    const Prim wm = ld_prim(A.W_in, off + b0 + (be.y & 0xffff));
+    const double nx = G.bn[2 * b], ny = G.bn[2 * b + 1];
+    const Cons F = bflux<FLUX, REC>(G, A.fo, gas, b, s, be.y >> 16, nx, ny, wm);
+    double* o = SBF + NFR * j;
+    sts2(o, F.m * 0.5, F.mx * 0.5);
+    sts2(o + 2, F.my * 0.5, F.e * 0.5);
+    if (LAST) {
+      sts2(o + 4, 0.5 * nx, 0.5 * ny);
+      SBA[j] = 0.5 * fsqrt(nx * nx + ny * ny);
+    }
+  }
   if (NS) {
     // every cell of the owned vertices once, then summed per vertex in cell order
-    for (int j = tid; j < T.mc; j += nth) {
-      const unsigned x = j == tid ? vcell : T.vcells[(size_t)t * T.mc + j];
+    for (int j = back; j < T.mc; j += nth) {
+      const unsigned x = j == back ? vcell : T.vcells[(size_t)t * T.mc + j];
       if (x != ~0u) viscous_cell(x, SA, gas, A.vp, SVC + NVC * j);
     }
     if (NS == 2) {
       // wall cells (src/fv.cc:1236-1312): one thread per bface forms its cell's
       // flux to the three corners and the wall flux through the bface
       const int k0 = T.wtbeg[t], nwt = T.wtbeg[t + 1] - k0;
-      for (int j = nth - 1 - tid; j < nwt; j += nth) {
-        const int b = T.wt[k0 + j], c = G.blc[b];
-        const uint2 cs = T.wcell[k0 + j];
+      for (int j = tid >= 64 ? tid - 64 : tid + nth - 64; j < nwt; j += nth) {
+        const uint4 wc = T.wcell[3 * (size_t)(k0 + j)];
+        const int b = (int)wc.x;
         Fan f;
-        fan_centre(f, SA, cs.x & 0xffffu);
+        fan_centre(f, SA, wc.y & 0xffffu);
         double q[2][4], x[2], y[2];
         for (int e = 0; e < 2; ++e) {
-          const double* a = SA + L::NA * (e ? (cs.y & 0xffffu) : (cs.x >> 16));
+          const double* a = SA + L::NA * (e ? wc.z : (wc.y >> 16));
           const double2 uv = lds2(a), bV = lds2(a + 2), xy = lds2(a + 4);
           slot_vars(uv, bV, q[e][0], q[e][1], q[e][2], q[e][3]);
           x[e] = xy.x - f.cx; y[e] = xy.y - f.cy;
@@ -523,17 +596,26 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
           d[2 * z + 1] = x[0] * q[1][z + 1] - x[1] * q[0][z + 1];
         }
         for (int z = 0; z < 2; ++z) {
-          const int bf = G.cbf[2 * (size_t)c + z];
-          if (bf < 0) break;
-          if (!bc_sets_state(G.btype[bf])) continue;
-          double dq[4];
-          boundary_dq(G, A, gas, s, off, bf, dq);
-          const double bx = G.bn[2 * bf], by = G.bn[2 * bf + 1];
+          const unsigned jt = z ? wc.w >> 16 : wc.w & 0xffffu;
+          if (jt == 0xffffu) continue;
+          double bx, by, dq[4];
+          if (L::GRAD) {
+            const double* q4 = SBT + NBT * jt;
+            bx = q4[0]; by = q4[1];
+            dq[1] = q4[3]; dq[2] = q4[4]; dq[3] = q4[5];
+          } else {  // no gradient pass: jt is the bface's place in its cell's list
+            const int bf = G.cbf[2 * (size_t)G.blc[b] + jt];
+            bx = G.bn[2 * bf]; by = G.bn[2 * bf + 1];
+            double de[4];
+            boundary_dq(G, A, gas, s, off, bf, 0, G.bv[2 * bf], nullptr, dq);
+            boundary_dq(G, A, gas, s, off, bf, 1, G.bv[2 * bf + 1], nullptr, de);
+            for (int w = 0; w < 4; ++w) dq[w] += de[w];
+          }
           for (int w = 0; w < 3; ++w) { d[2 * w] += bx * dq[w + 1]; d[2 * w + 1] += by * dq[w + 1]; }
         }
         const double ia = fdiv(1.0, x[0] * y[1] - y[0] * x[1]);
         for (int z = 0; z < 6; ++z) d[z] *= ia;
-        const Ent sw = wall_cell_state(G, A.W_in, off, s, gas, c);
+        const Ent sw = wall_state(G, A.W_in, off, s, gas, T.wcell + 3 * (size_t)(k0 + j) + 1);
         const ViscTensor v = visc_tensor(gas, A.vp, sw.vx, sw.vy, sw.l, d);
         double* o = SWT + NWT * j;
         const double nx[3] = {y[0] - y[1], y[1], -y[0]}, ny[3] = {x[1] - x[0], -x[1], x[0]};
@@ -649,9 +731,10 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
   __syncthreads();
 
   // ---- phase 4: gather, periodic sums, update ----------------------------------
-  // A vertex's entries are its faces, then its boundary faces; the first eight
-  // arrive packed, longer lists and boundary faces follow from memory, so every
-  // sum keeps the reference order (+F at a face's left end, -F at its right).
+  // A vertex's entries are its faces, then its boundary entries, which have face
+  // records of their own; the first eight arrive packed, longer lists follow from
+  // memory, so every sum keeps the reference order (+F at a face's left end, -F at
+  // its right).
   double acc[4] = {0, 0, 0, 0};
   if (LAST && own && A.W_keep)  // the last stage's input state, kept for the caller
     reinterpret_cast<double4*>(A.W_keep)[off + v] = make_double4(w0.T, w0.u, w0.v, w0.p);
@@ -666,7 +749,10 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     acc[2] = __builtin_fma(sg, b.x, acc[2]);
     acc[3] = __builtin_fma(sg, b.y, acc[3]);
   };
-  int gk0 = 0, gne = 0;
+  int gk0 = 0, gne = 0, gnf = 0, gnb = 0;  // longer lists: start, length, faces, first boundary entry
+  auto entry = [&](int k) -> unsigned {
+    return k < gnf ? (unsigned)T.gent[gk0 + k] : (unsigned)(T.bf0 + gnb + k - gnf);
+  };
   if (own) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -677,17 +763,13 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     if (rest >= 0) {
       gk0 = T.gptr[v];
       gne = T.gptr[v + 1] - gk0;
-      const int bb0 = T.bbeg[t];
-      for (int k = rest; k < gne; ++k) {
-        const unsigned e = T.gent[gk0 + k];
-        if (e & 0x4000u) {
-          const int b = T.tbf[bb0 + (e & 0x3fffu)];
-          const Cons Fb = bflux<FLUX, REC>(G, A.fo, gas, b, s, v, w0);
-          acc[0] += Fb.m * 0.5; acc[1] += Fb.mx * 0.5; acc[2] += Fb.my * 0.5; acc[3] += Fb.e * 0.5;
-        } else {
-          add_face(e);
-        }
+      if (T.mb) {
+        gnb = T.vbp[v] - e0;
+        gnf = gne - (T.vbp[v + 1] - e0 - gnb);
+      } else {
+        gnf = gne;
       }
+      for (int k = rest; k < gne; ++k) add_face(entry(k));
     }
     if (NS) {  // viscous fluxes after the faces (src/fv.cc:1197-1232), then the wall terms
       acc[1] += visc[0]; acc[2] += visc[1]; acc[3] += visc[2];
@@ -702,7 +784,7 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
     }
   }
   const bool per = T.tper[t] != 0;
-  const int TB = 64;
+  const int TB = SR_VERTS;
   if (per) {
     if (own)
 #pragma unroll
@@ -777,28 +859,15 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
         const int j = e & 0x3fffu;
         const double2 n = lds2(SF + NFR * j + 4);
         const double vn = w1.u * n.x + w1.v * n.y;
-        lam += fabs(vn) + cm * SAR[j];
+        lam += fabs(vn) + cm * (j < T.bf0 ? SAR[j] : SBA[j - T.bf0]);
       };
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const unsigned e = (gw[u >> 1] >> (16 * (u & 1))) & 0xffffu;
         if (!(e & 0x4000u)) add_lam(e);
       }
-      if (rest >= 0) {
-        const int bb0 = T.bbeg[t];
-        for (int k = rest; k < gne; ++k) {
-          const unsigned e = T.gent[gk0 + k];
-          if (e & 0x4000u) {
-            const int bf = T.tbf[bb0 + (e & 0x3fffu)];
-            const double nx = G.bn[2 * bf], ny = G.bn[2 * bf + 1];
-            const double ar = fsqrt(nx * nx + ny * ny);
-            const double vn = w1.u * nx + w1.v * ny;
-            lam += 0.5 * (fabs(vn) + cm * ar);
-          } else {
-            add_lam(e);
-          }
-        }
-      }
+      if (rest >= 0)
+        for (int k = rest; k < gne; ++k) add_lam(entry(k));
       if (NS) {  // viscous share, after every inviscid term (src/fv.cc:1555-1580)
         double mu;
         const double Tm = w1.T;
@@ -808,6 +877,7 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
         const double rho = density(gas, w1);
         auto add_visc = [&](unsigned e) {
           const int j = e & 0x3fffu;
+          if (j >= T.bf0) return;
           lam += fdiv(fdiv(mu * SAR[j], SDL[j]), rho);
         };
 #pragma unroll
@@ -816,10 +886,7 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
           if (!(e & 0x4000u)) add_visc(e);
         }
         if (rest >= 0)
-          for (int k = rest; k < gne; ++k) {
-            const unsigned e = T.gent[gk0 + k];
-            if (!(e & 0x4000u)) add_visc(e);
-          }
+          for (int k = rest; k < gnf; ++k) add_visc(entry(k));
       }
     }
   }
@@ -847,16 +914,11 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
   }
 }
 
-// Four waves per SIMD (128 VGPRs): the LDS of a 128-vertex tile allows four
-// tiles of four waves per CU.
-#ifndef TSM_ST_WAVES
-#define TSM_ST_WAVES 4
-#endif
-#ifndef TSM_ST_WAVES_NS
-#define TSM_ST_WAVES_NS 3
-#endif
+// Four waves per SIMD (128 VGPRs): the LDS of a 128-vertex tile (36 KB) allows
+// four tiles of four waves per CU.  Viscous terms with gradients need 50 KB at 112
+// vertices, three tiles.
 template <int FLUX, int REC, int LAST, int NS>
-__global__ __launch_bounds__(512, NS ? TSM_ST_WAVES_NS : TSM_ST_WAVES) void k_stage(
+__global__ __launch_bounds__(512, (NS && Layout<FLUX, REC>::GRAD ? 3 : 4)) void k_stage(
     DevGeo G, StageTab T, StageArgs A, StepParams P, const double* Wn, double* dtpart, int r) {
   stage_body<FLUX, REC, LAST, NS>(G, T, A, P, Wn, dtpart, r, xcd_tile(blockIdx.x, gridDim.x),
                                   blockIdx.y, gridDim.x);
@@ -865,7 +927,7 @@ __global__ __launch_bounds__(512, NS ? TSM_ST_WAVES_NS : TSM_ST_WAVES) void k_st
 // multilevel run): block b belongs to the level whose range [base_fu, ...)
 // holds it, tile (b - base) mod ntiles, sample (b - base) / ntiles.
 template <int FLUX, int REC, int LAST>
-__global__ __launch_bounds__(512, TSM_ST_WAVES) void k_stage_packed(const PackLevel* __restrict__ pk,
+__global__ __launch_bounds__(512, 4) void k_stage_packed(const PackLevel* __restrict__ pk,
                                                                     int nl, int r) {
   const int b = blockIdx.x;
   int l = 0;
@@ -1006,17 +1068,14 @@ int stage_block(const StageTab& T) {
 int stage_block_max() { return 512; }
 
 namespace {
-template <int FLUX, int REC>
-size_t lds_of(const StageTab& T, bool ns) {
-  using L = Layout<FLUX, REC>;
-  const size_t m = (std::max((size_t)L::NA * T.ms + (size_t)L::NB * T.ms1 + (ns ? (size_t)NVC * T.mc : 0),
-                             (size_t)(NFR + (ns ? 2 : 1)) * T.mf) + 1) & ~(size_t)1;
-  return sizeof(double) * (m + (size_t)NBT * T.mbt + (size_t)NWT * T.mwt + 2);
+size_t lds_of(const StageTab& T) {
+  return sizeof(double) * ((size_t)NFR * (T.bf0 + T.mb) + ((T.mb + 1) & ~1) + (size_t)NBT * T.mbt +
+                           (size_t)NWT * T.mwt + (T.n_periodic_tiles > 0 ? 4 * SR_VERTS : 0) + 2);
 }
 template <int FLUX, int REC>
 void go(const DevGeo& G, const StageTab& T, const StageArgs& A, const StepParams& P, const double* Wn,
         double* dtpart, int S, int r, bool last, hipStream_t st) {
-  const size_t lds = lds_of<FLUX, REC>(T, A.ns != 0);
+  const size_t lds = lds_of(T);
   const dim3 grid(T.ntiles, S), blk(stage_block(T));
   auto run = [&](auto kern) {
     if (lds > 48 * 1024)
@@ -1064,12 +1123,6 @@ void with_scheme(int flux, int rec, F&& f) {
     default: f.template operator()<F_AVG, R_FIRST>(); break;
   }
 }
-struct LdsOf {
-  const StageTab& T;
-  bool ns;
-  size_t n;
-  template <int FLUX, int REC> void operator()() { n = lds_of<FLUX, REC>(T, ns); }
-};
 struct Launch {
   const DevGeo& G; const StageTab& T; const StageArgs& A; const StepParams& P;
   const double* Wn; double* dtpart; int S, r; bool last; hipStream_t st;
@@ -1081,10 +1134,13 @@ struct LaunchPacked {
 };
 }  // namespace
 
-size_t stage_lds(const StageTab& T, int flux, int rec, bool ns) {
-  LdsOf f{T, ns, 0};
-  with_scheme(flux, rec, f);
-  return f.n;
+size_t stage_lds(const StageTab& T) { return lds_of(T); }
+// records of the main part: the widest layout of the slots, or the faces
+int stage_main_records(const StageTab& T, bool grad, bool ns) {
+  using L = Layout<F_ROE, R_MINMOD>;
+  using L1 = Layout<F_ROE, R_FIRST>;
+  const int slots = L::NA * T.ms + (grad ? L::NB : L1::NB) * T.ms1 + (ns ? NVC * T.mc : 0);
+  return (std::max(slots, (NFR + (ns ? 2 : 1)) * T.mf) + NFR - 1) / NFR;
 }
 bool stage_has_gradients(int flux, int rec) { return (flux == F_ROE || flux == F_RUS) && rec != R_FIRST; }
 bool stage_keeps_var0(int flux) { return flux == F_ROE || flux == F_RUS; }
@@ -1115,7 +1171,7 @@ void pack_plan(PackLevel* lv, int nl, int flux, int rec, PackPlan& p) {
     L.base_fu = p.fu_blocks;         p.fu_blocks += L.T.ntiles * L.S;
     L.base_final = p.final_blocks;   p.final_blocks += L.S;
     p.fu_block = std::max(p.fu_block, stage_block(L.T));
-    p.fu_lds = std::max(p.fu_lds, stage_lds(L.T, flux, rec, false));
+    p.fu_lds = std::max(p.fu_lds, stage_lds(L.T));
   }
 }
 

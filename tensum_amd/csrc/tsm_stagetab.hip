@@ -188,21 +188,20 @@ __device__ void walk_items(const TabIn& T, int v, F&& f) {
   }
 }
 
-// per gradient slot: second-ring candidates, boundary terms, items
-__global__ void k_gs_count(TabIn T, int nq, int* n2, int* nbt, int* nit) {
+// per gradient slot: second-ring candidates, boundary terms
+__global__ void k_gs_count(TabIn T, int nq, int* n2, int* nbt) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q > nq) return;
-  int c2 = 0, cb = 0, ci = 0;
+  int c2 = 0, cb = 0;
   if (q < nq) {
     int t, k, v;
     gs_find(T, q, t, k, v);
     walk_items(T, v, [&](int kind, int id, bool, bool) {
-      ++ci;
       if (kind == 2) ++cb;
       else if (slot_in(T, t, id) < 0) ++c2;
     });
   }
-  n2[q] = c2; nbt[q] = cb; nit[q] = ci;
+  n2[q] = c2; nbt[q] = cb;
 }
 __global__ void k_gs_emit(TabIn T, int nq, const int* o2, const int* ob, unsigned long long* k2,
                           unsigned long long* kb) {
@@ -279,74 +278,140 @@ __global__ void k_xy(int nv, const double* x, const double* y, double2* xy) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nv) xy[i] = make_double2(x[i], y[i]);
 }
-// entries that do not fit the slot's sixteen
-__global__ void k_ov_count(int nq, const int* nit, int* nov) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q <= nq) nov[q] = (q < nq && nit[q] > 16) ? nit[q] - 15 + 1 : 0;  // entries 15.. and an end
-}
 __device__ __forceinline__ uint4 pack8(const unsigned* w) {
   return make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
 }
-// the items of each gradient slot (codes in tsm_device.h): eight in items, the
-// next eight in items2 (read by tiles marked special only), the rest in ov;
-// special[t] is set where a tile has anything but chains of up to eight neighbours
-__global__ void k_fill_items(TabIn T, int nq, int ms1, const int* nit, const int* ovp, uint4* items,
-                             uint4* items2, int* item_ov, unsigned short* ov,
-                             unsigned char* special, int* bad) {
+// the items of each gradient slot (codes in tsm_device.h): the first chain in
+// items if it has up to eight neighbours, everything else in groups (read by tiles
+// marked special only); special[t] is set where a tile has anything but such chains
+// around the slots themselves.  Without ov the groups beyond the first are counted
+// in nov.
+__global__ void k_fill_items(TabIn T, int nq, int ms1, int* nov, const int* ovp, uint4* items,
+                             uint4* items2, int2* item_x, uint4* ov, unsigned char* special,
+                             int* bad) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
+  if (q > nq) return;
+  if (q == nq) { if (nov) nov[q] = 0; return; }
   int t, k, v;
   gs_find(T, q, t, k, v);
-  unsigned w[16];
-  for (int u = 0; u < 16; ++u) w[u] = SI_END;
-  const bool over = nit[q] > 16;
-  int n = 0, o = ovp[q];
-  bool sp = nit[q] > 8;
-  walk_items(T, v, [&](int kind, int id, bool flag, bool closed) {
-    unsigned e;
+  int first = 0, pos = 0;  // neighbours of the first chain
+  bool open = true;
+  walk_items(T, v, [&](int kind, int, bool, bool) {
+    if (kind == 0 && open) ++first;
+    else if (!(pos == 0 && kind == 1)) open = false;
+    ++pos;
+  });
+  const bool inl = first <= 8;
+  unsigned w[8], g[8];
+  for (int u = 0; u < 8; ++u) w[u] = g[u] = SI_END;
+  int n = 0, groups = 0, seen = 0, at = 0, start = k, centre = k;
+  uint4 g0 = pack8(g);
+  auto put = [&]() {  // the group is full or the next item needs another
+    if (groups == 0) g0 = pack8(g);
+    else if (ov) ov[ovp[q] + groups - 1] = pack8(g);
+    ++groups;
+    n = 0;
+    for (int u = 0; u < 8; ++u) g[u] = SI_END;
+  };
+  walk_items(T, v, [&](int kind, int id, bool, bool closed) {
     if (kind == 2) {
       const int b0 = T.btbeg[t], b1 = T.btbeg[t + 1];
       const int j = find32(T.bt, b0, b1, id) - b0;
       if (j > SI_MASK) atomicOr(bad, 1);
-      e = SI_TERM | (unsigned)(j & SI_MASK);
+      if (n > 0 && ((g[0] & 0xc000u) != SI_TERM || n == 8)) put();
+      if (n == 0) g[n++] = SI_TERM;
+      g[n++] = SI_TERM | (unsigned)(j & SI_MASK);
     } else {
       const int s = slot_in(T, t, id);
       if (s < 0 || s > SI_MASK) atomicOr(bad, 1);
-      e = (kind == 1 ? SI_CENTRE : 0u) | (flag ? SI_FLAG : 0u) | (closed ? SI_CLOSED : 0u) |
-          (unsigned)(s & SI_MASK);
+      if (kind == 1) {
+        centre = s;
+        if (at == 0) start = s;
+        if (n > 0) put();
+      } else {
+        const unsigned e = (closed ? SI_CLOSED : 0u) | (unsigned)(s & SI_MASK);
+        if (inl && seen < first) {
+          w[seen] = e;
+        } else {
+          if (n == 8) {  // the chain goes on
+            g[0] |= SI_CLOSED;
+            put();
+            g[n++] = SI_CENTRE | SI_FLAG | (unsigned)(centre & SI_MASK);
+          } else if (n == 0) {
+            g[n++] = SI_CENTRE | (unsigned)(centre & SI_MASK);
+          }
+          g[n++] = e;
+        }
+        ++seen;
+      }
     }
-    sp = sp || kind != 0;
-    if (!over || n < 15) w[n] = e;
-    else ov[o++] = (unsigned short)e;
-    ++n;
+    ++at;
   });
-  if (over) { w[15] = SI_MORE; ov[o] = SI_END; }
-  const size_t at = (size_t)t * ms1 + k;
-  items[at] = pack8(w);
-  items2[at] = pack8(w + 8);
-  item_ov[at] = ovp[q];
-  if (sp) special[t] = 1;
+  if (n > 0) put();
+  if (nov) nov[q] = max(groups - 1, 0);
+  if (!ov) return;
+  const size_t o = (size_t)t * ms1 + k;
+  items[o] = pack8(w);
+  items2[o] = g0;
+  item_x[o] = make_int2((start & SI_MASK) | (max(groups - 1, 0) << 12), ovp[q]);
+  if (groups > 0 || start != k) special[t] = 1;
 }
-__global__ void k_no_items(long long n, uint4* items, uint4* items2, int* item_ov) {
+__global__ void k_no_items(long long n, uint4* items, uint4* items2, int2* item_x) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const unsigned e = SI_END | (SI_END << 16);
   items[i] = items2[i] = make_uint4(e, e, e, e);
-  item_ov[i] = 0;
+  item_x[i] = make_int2(0, 0);
 }
-// the first eight gather entries of each vertex
-__global__ void k_ge8(int nv, const int* gptr, const unsigned short* gent, uint4* ge8) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nv) return;
+// boundary entries: per vertex their count, then the entries
+__device__ __forceinline__ int vertex_faces(const int* gptr, const unsigned short* gent, int v) {
   const int k0 = gptr[v], n = gptr[v + 1] - k0;
   int nf = 0;
   while (nf < n && !(gent[k0 + nf] & 0x4000u)) ++nf;
+  return nf;
+}
+__global__ void k_be_count(int nv, const int* gptr, const unsigned short* gent, int* cnt) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v <= nv) cnt[v] = v < nv ? gptr[v + 1] - gptr[v] - vertex_faces(gptr, gent, v) : 0;
+}
+__global__ void k_be_fill(TabIn T, const int* gptr, const unsigned short* gent, const int* bbeg,
+                          const int* tbf, const int* vbp, int2* be) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int n = vbp[v + 1] - vbp[v];
+  if (n == 0) return;
+  const int t = tile_of(T, v), k0 = gptr[v + 1] - n;
+  for (int i = 0; i < n; ++i) {
+    const int b = tbf[bbeg[t] + (gent[k0 + i] & 0x3fffu)];
+    be[vbp[v] + i] = make_int2(b, (v - T.vbeg[t]) | (bc_end(T.G, b, v) << 16));
+  }
+}
+__global__ void k_be_max(TabIn T, const int* vbp, int* mx) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < T.nt) atomicMax(mx, vbp[T.vbeg[t + 1]] - vbp[T.vbeg[t]]);
+}
+// the first eight gather entries of each vertex
+__global__ void k_ge8(TabIn T, int bf0, const int* gptr, const unsigned short* gent, const int* vbp,
+                      uint4* ge8, int* bad) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= T.G.nv) return;
+  const int k0 = gptr[v], n = gptr[v + 1] - k0, nf = n - (vbp[v + 1] - vbp[v]);
+  int k = 0;  // the tile's boundary entries before this vertex's
+  if (nf < n) k = vbp[v] - vbp[T.vbeg[tile_of(T, v)]];
   unsigned w[8];
   for (int u = 0; u < 8; ++u) w[u] = GE_END;
-  const int m = (n <= 8 && nf == n) ? n : min(nf, 7);
-  for (int u = 0; u < m; ++u) w[u] = gent[k0 + u];
+  const int m = n <= 8 ? n : 7;
+  for (int u = 0; u < m; ++u) w[u] = u < nf ? gent[k0 + u] : (unsigned)(bf0 + k + u - nf);
+  if (bf0 + k + n - nf > 0x3fff) atomicOr(bad, 1);
   if (m < n) w[m] = GE_MORE;
   ge8[v] = pack8(w);
+}
+// boundary terms with their vertices
+__global__ void k_bt4(DevGeo G, int n, const int* bt, int4* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int b = bt[i];
+  out[i] = make_int4(b, G.bv[2 * b], G.bv[2 * b + 1], 0);
 }
 // viscous cells: (tile, cell) of every cell of an owned vertex that is no wall cell
 __global__ void k_vcell_keys(TabIn T, unsigned long long* keys) {
@@ -407,17 +472,44 @@ __global__ void k_wall_keys(TabIn T, unsigned long long* keys) {
   for (int e = T.G.vbe_ptr[v]; e < T.G.vbe_ptr[v + 1]; ++e)
     keys[e] = ((unsigned long long)(unsigned)t << 32) | ((unsigned)T.G.vbe[e] & 0x7fffffffu);
 }
-__global__ void k_wall_cells(TabIn T, const int* wtbeg, const int* wt, uint2* wcell, int* bad) {
+__global__ void k_wall_cells(TabIn T, const int* wtbeg, const int* wt, uint4* wcell, int* bad) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T.nt) return;
+  const DevGeo& G = T.G;
   for (int j = wtbeg[t]; j < wtbeg[t + 1]; ++j) {
-    const int c = T.G.blc[wt[j]];
+    const int c = G.blc[wt[j]];
     int s[3];
     for (int z = 0; z < 3; ++z) {
-      s[z] = slot_in(T, t, T.G.cv[3 * (size_t)c + z]);
+      s[z] = slot_in(T, t, G.cv[3 * (size_t)c + z]);
       if (s[z] < 0 || s[z] > SI_MASK) { atomicOr(bad, 1); s[z] = 0; }
     }
-    wcell[j] = make_uint2((unsigned)s[0] | ((unsigned)s[1] << 16), (unsigned)s[2]);
+    unsigned jt[2] = {0xffffu, 0xffffu};
+    for (int z = 0; z < 2; ++z) {
+      const int b = G.cbf[2 * (size_t)c + z];
+      if (b < 0) break;
+      if (!bc_sets_state(G.btype[b])) continue;
+      jt[z] = (unsigned)z;
+      if (T.grad) {
+        const int k = find32(T.bt, T.btbeg[t], T.btbeg[t + 1], b);
+        if (k >= T.btbeg[t + 1] || T.bt[k] != b) atomicOr(bad, 1);
+        jt[z] = (unsigned)(k - T.btbeg[t]) & 0xffffu;
+      }
+    }
+    uint4* o = wcell + 3 * (size_t)j;
+    o[0] = make_uint4((unsigned)wt[j], (unsigned)s[0] | ((unsigned)s[1] << 16), (unsigned)s[2],
+                      jt[0] | (jt[1] << 16));
+    for (int z = 0; z < 2; ++z) {
+      const int f = G.cwf[2 * c + z];
+      uint4 q = make_uint4(0, 0, 0, 0xffffffffu);
+      if (f >= 0) {
+        const int b = G.cwb[2 * c + z], v0 = G.fv[2 * f], v1 = G.fv[2 * f + 1];
+        if (b > 0x3fffffff) atomicOr(bad, 1);
+        q = make_uint4((unsigned)v0, (unsigned)v1,
+                       (unsigned)b | ((unsigned)bc_end(G, b, v0) << 30) | ((unsigned)bc_end(G, b, v1) << 31),
+                       (unsigned)f);
+      }
+      o[1 + z] = q;
+    }
   }
 }
 // per (vertex, bface) in bface order: the tile's wall term, the vertex's corner
@@ -451,7 +543,7 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
   const int nv = G.nv, nt = TG.ntiles;
   S = StageTab{};
   S.ntiles = nt; S.tb = TG.tb; S.fu_block = TG.fu_block; S.n_periodic_tiles = TG.n_periodic_tiles;
-  S.tper = TG.tper; S.pinfo = TG.pinfo; S.gptr = TG.gptr; S.gent = TG.gent; S.bbeg = TG.bbeg; S.tbf = TG.tbf;
+  S.tper = TG.tper; S.pinfo = TG.pinfo; S.gptr = TG.gptr; S.gent = TG.gent;
   int nhalo = 0;
   TT(hipMemcpyAsync(&nhalo, TG.hbeg + nt, sizeof(int), hipMemcpyDeviceToHost, st));
   TT(hipStreamSynchronize(st));
@@ -520,7 +612,7 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
   Tmp<unsigned char> special;
   TT(special.alloc(nt));
   GO(k_zero, nt, (long long)nt, special.p);
-  Tmp<int> fan_ptr, nit, ovp;
+  Tmp<int> fan_ptr, ovp;
   Tmp<unsigned> fan;
   int *h2beg = nullptr, *halo2 = nullptr, *btbeg = nullptr, *bt = nullptr;
   if (grad) {
@@ -542,9 +634,9 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
     T.fan = fan.p;
     // ---- second ring and boundary terms ---------------------------------------
     Tmp<int> n2, nb, o2, ob;
-    TT(n2.alloc(nq + 1)); TT(nb.alloc(nq + 1)); TT(nit.alloc(nq + 1));
+    TT(n2.alloc(nq + 1)); TT(nb.alloc(nq + 1));
     TT(o2.alloc(nq + 1)); TT(ob.alloc(nq + 1));
-    GO(k_gs_count, nq + 1, T, nq, n2.p, nb.p, nit.p);
+    GO(k_gs_count, nq + 1, T, nq, n2.p, nb.p);
     TT(scan(n2.p, o2.p, nq + 1));
     TT(scan(nb.p, ob.p, nq + 1));
     int c2 = 0, cb = 0;
@@ -559,9 +651,10 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
     if (int r = group(k2, c2, &h2beg, &halo2, count)) return r;
     if (int r = group(kb, cb, &btbeg, &bt, count)) return r;
     T.h2beg = h2beg; T.halo2 = halo2; T.btbeg = btbeg; T.bt = bt;
-    // ---- overflow of the eight item entries -----------------------------------
+    // ---- groups of items beyond each slot's first ------------------------------
     TT(ovp.alloc(nq + 1));
-    GO(k_ov_count, nq + 1, nq, nit.p, n2.p);
+    GO(k_fill_items, nq + 1, T, nq, 0, n2.p, (const int*)nullptr, (uint4*)nullptr, (uint4*)nullptr,
+       (int2*)nullptr, (uint4*)nullptr, (unsigned char*)nullptr, bad.p);
     TT(scan(n2.p, ovp.p, nq + 1));
   }
   // ---- wall terms -------------------------------------------------------------
@@ -574,13 +667,13 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
     TT(k.alloc(nvbe));
     GO(k_wall_keys, nv, T, k.p);
     if (int r = group(k, nvbe, &wtbeg, &wt, count)) return r;
-    uint2* wcell = nullptr;
+    uint4* wcell = nullptr;
     unsigned short* wvent = nullptr;
-    TA(wcell, count);
+    TA(wcell, 3 * (size_t)count);
     TA(wvent, nvbe);
     GO(k_wall_cells, nt, T, wtbeg, wt, wcell, bad.p);
     GO(k_wall_entries, nv, T, wtbeg, wt, wvent, bad.p);
-    S.wtbeg = wtbeg; S.wt = wt; S.wcell = wcell; S.wvent = wvent;
+    S.wtbeg = wtbeg; S.wcell = wcell; S.wvent = wvent;
   }
   // ---- viscous cells ----------------------------------------------------------
   int *tcbeg = nullptr, *tc = nullptr;
@@ -600,10 +693,20 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
     S.vcent = ent; S.vccnt = cnt; S.vc8 = vc8;
   }
   GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special.p, (int4*)nullptr, mx.p);
-  int h[8];
+  // ---- boundary entries ---------------------------------------------------------
+  Tmp<int> becnt;
+  int* vbp = nullptr;
+  TT(becnt.alloc(nv + 1));
+  TA(vbp, nv + 1);
+  GO(k_be_count, nv + 1, nv, TG.gptr, TG.gent, becnt.p);
+  TT(scan(becnt.p, vbp, nv + 1));
+  GO(k_be_max, nt, T, vbp, mx.p + 6);
+  int h[8], nbe = 0;
+  TT(hipMemcpyAsync(&nbe, vbp + nv, sizeof(int), hipMemcpyDeviceToHost, st));
   TT(hipMemcpyAsync(h, mx.p, sizeof(h), hipMemcpyDeviceToHost, st));
   TT(hipStreamSynchronize(st));
-  S.ms = h[0]; S.ms1 = h[1]; S.mf = h[2]; S.mbt = h[3]; S.mwt = h[4]; S.mc = h[5];
+  S.ms = h[0]; S.ms1 = h[1]; S.mf = h[2]; S.mbt = h[3]; S.mwt = h[4]; S.mc = h[5]; S.mb = h[6];
+  S.bf0 = stage_main_records(S, grad, ns);
   if (S.ms > SI_MASK) { msg = "stage tables: too many slots"; return 1; }
   // ---- padded tables ------------------------------------------------------------
   int* sid = nullptr;
@@ -616,16 +719,25 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
   GO(k_fill_sid, (long long)nt * S.ms, T, S.ms, sid);
   GO(k_fill_faces, (long long)nt * S.mf, nt, S.mf, TG.fbeg, TG.f_lr, TG.f_n, lr, fn);
   GO(k_xy, nv, nv, G.x, G.y, xy);
-  GO(k_ge8, nv, nv, TG.gptr, TG.gent, ge);
+  int2* be = nullptr;
+  TA(be, nbe);
+  GO(k_be_fill, nv, T, TG.gptr, TG.gent, TG.bbeg, TG.tbf, vbp, be);
+  GO(k_ge8, nv, T, S.bf0, TG.gptr, TG.gent, vbp, ge, bad.p);
+  S.vbp = vbp; S.be = be;
   if (grad) {
-    int nov = 0, *itov = nullptr;
-    unsigned short* ov = nullptr;
+    int nov = 0;
+    int2* itx = nullptr;
+    uint4* ov = nullptr;
+    int4* bt4 = nullptr;
+    int nbt = 0;
+    TT(hipMemcpyAsync(&nbt, btbeg + nt, sizeof(int), hipMemcpyDeviceToHost, st));
     TT(hipMemcpyAsync(&nov, ovp.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
     TT(hipStreamSynchronize(st));
-    TA(it, (size_t)nt * S.ms1); TA(it2, (size_t)nt * S.ms1); TA(itov, (size_t)nt * S.ms1); TA(ov, nov);
-    GO(k_no_items, (long long)nt * S.ms1, (long long)nt * S.ms1, it, it2, itov);
-    GO(k_fill_items, nq, T, nq, S.ms1, nit.p, ovp.p, it, it2, itov, ov, special.p, bad.p);
-    S.items = it; S.items2 = it2; S.item_ov = itov; S.ov = ov; S.btbeg = btbeg; S.bt = bt;
+    TA(it, (size_t)nt * S.ms1); TA(it2, (size_t)nt * S.ms1); TA(itx, (size_t)nt * S.ms1); TA(ov, nov); TA(bt4, nbt);
+    if (nbt > 0) GO(k_bt4, nbt, G, nbt, bt, bt4);
+    GO(k_no_items, (long long)nt * S.ms1, (long long)nt * S.ms1, it, it2, itx);
+    GO(k_fill_items, nq, T, nq, S.ms1, (int*)nullptr, ovp.p, it, it2, itx, ov, special.p, bad.p);
+    S.items = it; S.items2 = it2; S.item_x = itx; S.ov = ov; S.btbeg = btbeg; S.bt = bt4;
   }
   if (ns) {
     unsigned* vcells = nullptr;
