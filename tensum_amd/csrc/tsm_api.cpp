@@ -511,6 +511,10 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   if (params->liou_fix) AL(A.ssw, cs);
   AL(A.partial, (size_t)S * std::max(c->nblk_v, c->tiling.ntiles) * 4);
   if (c->tiled) AL(c->dtpart, (size_t)S * c->tiling.ntiles);
+  if (c->tiled && tsm::stage_ends_step(c->tiling.ntiles)) {
+    AL(A.arrive, S);
+    if (hipMemset(A.arrive, 0, S * sizeof(int)) != hipSuccess) { delete c; return fail(TSM_E_HIP, "memset"); }
+  }
   AL(A.ctl, (size_t)S);
   double* dg; double* dr; double* dc; double* ts;
   AL(dg, (size_t)S); AL(dr, (size_t)S); AL(dc, 2 * (size_t)S);
@@ -934,7 +938,7 @@ void enqueue_tiled_step(tsm_ctx* c, int log_slot, hipEvent_t* ev = nullptr) {
     tsm::launch_bc_time(c->G, c->bt, c->A, c->S, r, c->st);
     if (ev) (void)hipEventRecord(ev[e++], c->st);
     tsm::launch_stage(c->P.flux, c->P.reconstruct, c->G, c->ST, c->A, c->SP, Wn, c->dtpart, c->S, r,
-                      r == nrk - 1, c->st);
+                      r == nrk - 1, log_slot, c->st);
   }
   if (ev) (void)hipEventRecord(ev[e++], c->st);
   tsm::launch_step_final_tiled(c->G, c->A, c->SP, c->S, c->ST.ntiles, c->dtpart, log_slot, c->st);

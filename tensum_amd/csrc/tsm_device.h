@@ -317,6 +317,7 @@ struct StageArgs {
   double* R2;      // 4 components (rk4)
   double* ssw;
   double* partial; // per-block reduction scratch
+  int* arrive;     // per sample: tiles of the last stage that are done (null: a launch of its own ends a step)
   double* dtl;     // per-vertex local time step (steady mode), null in unsteady mode
   double* W_keep;  // last stage's input state of each sample's latest step, null unless kept
   Ctl* ctl;
@@ -374,12 +375,13 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
 int stage_block(const StageTab& T);
 int stage_block_max();
 size_t stage_lds(const StageTab& T);
+bool stage_ends_step(int ntiles);
 int stage_main_records(const StageTab& T, bool grad, bool ns);
 bool stage_has_gradients(int flux, int rec);
 bool stage_keeps_var0(int flux);
 void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const StageArgs& A,
                   const StepParams& P, const double* Wn, double* dtpart, int S, int r, bool last,
-                  hipStream_t st);
+                  int log_slot, hipStream_t st);
 void launch_step_final_tiled(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                              int nblk, const double* dtpart, int log_slot, hipStream_t st);
 

@@ -338,13 +338,94 @@ __device__ __forceinline__ void viscous_add(unsigned e, const double* SVC, doubl
   else { visc[0] -= a.x + b.y; visc[1] -= a.y + c.x; visc[2] -= b.x + c.y; }
 }
 
+// Residual norm, time advance, loop test and the next step's global dt
+// (src/fv.cc:1591-1618, :1801-1879, :2273-2316) from the step's sums; c: the
+// sample's control block as the step found it.
+__device__ __forceinline__ void step_ctl(const StageArgs& A, const StepParams& P, Ctl c, int nv,
+                                         const double* part, double x, int log_slot, int s) {
+  double n[4];
+  for (int k = 0; k < 4; ++k) {
+    n[k] = sqrt(part[k]) / nv;
+    c.rn[k] = n[k];
+  }
+  const double tot = sqrt((n[0] * n[0]) + (n[1] * n[1] + n[2] * n[2]) + (n[3] * n[3]));
+  if (c.iter == 0) {
+    c.res0 = tot;
+    if (c.res0 == 0.0) c.res0 = 1.0;
+  }
+  c.res_total = tot / c.res0;
+  c.iter += 1;
+  c.t += c.dt;
+  if (c.reached && P.unsteady) { c.counter += 1; c.reached = 0; }
+  if (A.log && log_slot >= 0) {
+    double* Lg = A.log + ((size_t)s * A.log_cap + log_slot) * 4;
+    Lg[0] = (double)c.iter; Lg[1] = c.dt; Lg[2] = c.t; Lg[3] = c.res_total;
+  }
+  const bool go = c.res_total > P.min_residue && (P.unsteady ? true : c.iter < P.max_iter) &&
+                  c.t < P.final_time;
+  if (!go) {
+    c.done = 1;
+  } else {
+    double dt = x;
+    if (P.unsteady && !(P.time_step > 0.0)) {
+      const double target = A.tstamps[min(c.counter, P.n_stamps)];
+      if (c.t + dt > target) { dt = target - c.t; c.reached = 1; }
+    }
+    c.dt = dt;
+  }
+  A.ctl[s] = c;
+}
+
+// The end of a step by one wave, from the partials of nblk blocks of this very
+// launch: they were written through to memory before their blocks counted
+// themselves in, and are read past the caches.
+__device__ __forceinline__ double agent_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams& P, int nblk, int nv,
+                                           const double* dtpart, int log_slot, int s) {
+  const int lane = threadIdx.x & 63;
+  const Ctl c = A.ctl[s];
+  const double* q = A.partial + (size_t)s * nblk * 4;
+  const double* dq = dtpart + (size_t)s * nblk;
+  double part[4] = {0, 0, 0, 0}, x = 1.0e20;
+  for (int i0 = 0; i0 < nblk; i0 += 8 * 64) {
+    double a[8][5];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + 64 * u + lane;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[u][k] = i < nblk ? agent_load(q + 4 * (size_t)i + k) : 0.0;
+      a[u][4] = i < nblk ? agent_load(dq + i) : 1.0e20;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) part[k] += a[u][k];
+      x = fmin(x, a[u][4]);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[k] += __shfl_down(part[k], o, 64);
+    x = fmin(x, __shfl_down(x, o, 64));
+  }
+  if (lane == 0) step_ctl(A, P, c, nv, part, x, log_slot, s);
+}
+
 // Per-block partials of the last stage without a block barrier: every wave
 // reduces its residual-norm sums and smallest local dt by shuffles, its lane 0
 // leaves them in LDS and counts itself in with an LDS integer atomic; the
 // last wave to arrive adds the waves' values in wave order and writes the
-// block's slot.  Waves that finish early leave at once.
-__device__ __forceinline__ void block_partials(double* part, double dtv, double* wred, int* arrive,
-                                               double* partial, double* dtpart, size_t slot) {
+// block's slot.  Waves that finish early leave at once.  Where the sample's
+// blocks are counted (A.arrive), the last block's wave ends the step.
+__device__ __forceinline__ void block_partials(const StageArgs& A, const StepParams& P, double* part,
+                                               double dtv, double* wred, int* arrive, double* dtpart,
+                                               int s, int t, int nt, int nv, int log_slot) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     double x = part[k];
@@ -354,24 +435,41 @@ __device__ __forceinline__ void block_partials(double* part, double dtv, double*
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) dtv = fmin(dtv, __shfl_down(dtv, o, 64));
-  if ((threadIdx.x & 63) != 0) return;
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int ends = 0;
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) wred[5 * w + k] = part[k];
-  wred[5 * w + 4] = dtv;
-  __threadfence_block();
-  if (atomicAdd(arrive, 1) != nw - 1) return;
-  __threadfence_block();
-  double sum[4] = {wred[0], wred[1], wred[2], wred[3]};
-  double m = wred[4];
-  for (int u = 1; u < nw; ++u) {
+    for (int k = 0; k < 4; ++k) wred[5 * w + k] = part[k];
+    wred[5 * w + 4] = dtv;
+    __threadfence_block();
+    if (atomicAdd(arrive, 1) == nw - 1) {
+      __threadfence_block();
+      double sum[4] = {wred[0], wred[1], wred[2], wred[3]};
+      double m = wred[4];
+      for (int u = 1; u < nw; ++u) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) sum[k] += wred[5 * u + k];
-    m = fmin(m, wred[5 * u + 4]);
+        for (int k = 0; k < 4; ++k) sum[k] += wred[5 * u + k];
+        m = fmin(m, wred[5 * u + 4]);
+      }
+      const size_t slot = (size_t)s * nt + t;
+      if (A.arrive) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) agent_store(A.partial + slot * 4 + k, sum[k]);
+        agent_store(dtpart + slot, m);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // written before the block is counted
+        ends = __hip_atomic_fetch_add(A.arrive + s, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt - 1;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) A.partial[slot * 4 + k] = sum[k];
+        dtpart[slot] = m;
+      }
+    }
   }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) partial[slot * 4 + k] = sum[k];
-  dtpart[slot] = m;
+  if (!__builtin_amdgcn_readfirstlane(ends)) return;
+  asm volatile("" ::: "memory");
+  final_wave(A, P, nt, nv, dtpart, log_slot, s);
+  if ((threadIdx.x & 63) == 0)
+    __hip_atomic_store(A.arrive + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace
@@ -381,7 +479,7 @@ __device__ __forceinline__ void block_partials(double* part, double dtv, double*
 template <int FLUX, int REC, int LAST, int NS>
 __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, const StageArgs& A,
                                            const StepParams& P, const double* Wn, double* dtpart,
-                                           int r, int t, int s, int nbx) {
+                                           int r, int t, int s, int nbx, int log_slot) {
   using L = Layout<FLUX, REC>;
   extern __shared__ __attribute__((aligned(16))) double lds[];
   __shared__ double wred[8 * 5];
@@ -910,7 +1008,7 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
       dtv = (P.time_step > 0.0) ? P.time_step : fdiv(P.cfl * area_v, lam);
       if (A.dtl) A.dtl[off + v] = dtv;  // steady mode: read by this vertex only, next step
     }
-    block_partials(part, dtv, wred, &arrive, A.partial, dtpart, (size_t)s * nbx + t);
+    block_partials(A, P, part, dtv, wred, &arrive, dtpart, s, t, nbx, G.nv, log_slot);
   }
 }
 
@@ -919,9 +1017,10 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
 // vertices, three tiles.
 template <int FLUX, int REC, int LAST, int NS>
 __global__ __launch_bounds__(512, (NS && Layout<FLUX, REC>::GRAD ? 3 : 4)) void k_stage(
-    DevGeo G, StageTab T, StageArgs A, StepParams P, const double* Wn, double* dtpart, int r) {
+    DevGeo G, StageTab T, StageArgs A, StepParams P, const double* Wn, double* dtpart, int r,
+    int log_slot) {
   stage_body<FLUX, REC, LAST, NS>(G, T, A, P, Wn, dtpart, r, xcd_tile(blockIdx.x, gridDim.x),
-                                  blockIdx.y, gridDim.x);
+                                  blockIdx.y, gridDim.x, log_slot);
 }
 // The same over the tiles and samples of several contexts (the levels of a
 // multilevel run): block b belongs to the level whose range [base_fu, ...)
@@ -934,11 +1033,11 @@ __global__ __launch_bounds__(512, 4) void k_stage_packed(const PackLevel* __rest
   while (l + 1 < nl && b >= pk[l + 1].base_fu) ++l;
   const PackLevel& L = pk[l];
   const int nt = L.T.ntiles, local = b - L.base_fu;
-  stage_body<FLUX, REC, LAST, 0>(L.G, L.T, L.A, L.P, L.Wn, L.dtpart, r, local % nt, local / nt, nt);
+  stage_body<FLUX, REC, LAST, 0>(L.G, L.T, L.A, L.P, L.Wn, L.dtpart, r, local % nt, local / nt, nt, -1);
 }
 
 // ---------------------------------------------------------------------------
-// end of a step
+// end of a step of meshes with more tiles than the stage kernel folds
 // ---------------------------------------------------------------------------
 namespace {
 template <int NV>
@@ -977,15 +1076,11 @@ __device__ __forceinline__ double bmin(double x, double* red) {
   }
   return x;
 }
-}  // namespace
-
-// Residual norm, time advance, loop test and the next step's global dt
-// (src/fv.cc:1591-1618, :1801-1879, :2273-2316).
 __device__ __forceinline__ void step_final_body(const StageArgs& A, const StepParams& P, int nblk,
                                                 int nv, const double* dtpart, int log_slot,
                                                 int s) {
   __shared__ double red[64];
-  Ctl& c = A.ctl[s];
+  const Ctl c = A.ctl[s];
   if (c.done) return;
   double part[4] = {0, 0, 0, 0};
   double x = 1.0e20;
@@ -1011,39 +1106,9 @@ __device__ __forceinline__ void step_final_body(const StageArgs& A, const StepPa
   bsum<4>(part, red);
   __syncthreads();
   x = bmin(x, red);
-  if (threadIdx.x == 0) {
-    double n[4];
-    for (int k = 0; k < 4; ++k) {
-      n[k] = sqrt(part[k]) / nv;
-      c.rn[k] = n[k];
-    }
-    const double tot = sqrt((n[0] * n[0]) + (n[1] * n[1] + n[2] * n[2]) + (n[3] * n[3]));
-    if (c.iter == 0) {
-      c.res0 = tot;
-      if (c.res0 == 0.0) c.res0 = 1.0;
-    }
-    c.res_total = tot / c.res0;
-    c.iter += 1;
-    c.t += c.dt;
-    if (c.reached && P.unsteady) { c.counter += 1; c.reached = 0; }
-    if (A.log && log_slot >= 0) {
-      double* Lg = A.log + ((size_t)s * A.log_cap + log_slot) * 4;
-      Lg[0] = (double)c.iter; Lg[1] = c.dt; Lg[2] = c.t; Lg[3] = c.res_total;
-    }
-    const bool go = c.res_total > P.min_residue && (P.unsteady ? true : c.iter < P.max_iter) &&
-                    c.t < P.final_time;
-    if (!go) {
-      c.done = 1;
-    } else {
-      double dt = x;
-      if (P.unsteady && !(P.time_step > 0.0)) {
-        const double target = A.tstamps[min(c.counter, P.n_stamps)];
-        if (c.t + dt > target) { dt = target - c.t; c.reached = 1; }
-      }
-      c.dt = dt;
-    }
-  }
+  if (threadIdx.x == 0) step_ctl(A, P, c, nv, part, x, log_slot, s);
 }
+}  // namespace
 __global__ __launch_bounds__(1024) void k_step_final_tiled(StageArgs A, StepParams P, int nblk,
                                                           int nv, const double* dtpart,
                                                           int log_slot) {
@@ -1057,6 +1122,12 @@ __global__ __launch_bounds__(1024) void k_step_final_packed(const PackLevel* __r
   step_final_body(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
 }
 
+// The last stage ends the step of a mesh with up to this many tiles, eight partials
+// a lane of the wave that does it.  A step of the vortex (Roe, minmod) against a
+// launch of its own: 129^2 (150 tiles) 37.7 us against 41.8, 200^2 43.0 / 45.7,
+// 257^2 (541) 53.9 / 54.3, 350^2 63.2 / 62.7.
+constexpr int FOLD_TILES = 512;
+
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -1066,6 +1137,7 @@ int stage_block(const StageTab& T) {
   return std::max(b, T.fu_block);
 }
 int stage_block_max() { return 512; }
+bool stage_ends_step(int ntiles) { return ntiles <= FOLD_TILES; }
 
 namespace {
 size_t lds_of(const StageTab& T) {
@@ -1074,13 +1146,13 @@ size_t lds_of(const StageTab& T) {
 }
 template <int FLUX, int REC>
 void go(const DevGeo& G, const StageTab& T, const StageArgs& A, const StepParams& P, const double* Wn,
-        double* dtpart, int S, int r, bool last, hipStream_t st) {
+        double* dtpart, int S, int r, bool last, int log_slot, hipStream_t st) {
   const size_t lds = lds_of(T);
   const dim3 grid(T.ntiles, S), blk(stage_block(T));
   auto run = [&](auto kern) {
     if (lds > 48 * 1024)
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(kern, grid, blk, lds, st, G, T, A, P, Wn, dtpart, r);
+    hipLaunchKernelGGL(kern, grid, blk, lds, st, G, T, A, P, Wn, dtpart, r, log_slot);
   };
   if (A.ns && A.ns_walls) {
     if (last) run(k_stage<FLUX, REC, 1, 2>); else run(k_stage<FLUX, REC, 0, 2>);
@@ -1125,8 +1197,8 @@ void with_scheme(int flux, int rec, F&& f) {
 }
 struct Launch {
   const DevGeo& G; const StageTab& T; const StageArgs& A; const StepParams& P;
-  const double* Wn; double* dtpart; int S, r; bool last; hipStream_t st;
-  template <int FLUX, int REC> void operator()() { go<FLUX, REC>(G, T, A, P, Wn, dtpart, S, r, last, st); }
+  const double* Wn; double* dtpart; int S, r; bool last; int log_slot; hipStream_t st;
+  template <int FLUX, int REC> void operator()() { go<FLUX, REC>(G, T, A, P, Wn, dtpart, S, r, last, log_slot, st); }
 };
 struct LaunchPacked {
   const PackLevel* d; const PackPlan& p; int r; bool last; hipStream_t st;
@@ -1147,13 +1219,14 @@ bool stage_keeps_var0(int flux) { return flux == F_ROE || flux == F_RUS; }
 
 void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const StageArgs& A,
                   const StepParams& P, const double* Wn, double* dtpart, int S, int r, bool last,
-                  hipStream_t st) {
-  Launch f{G, T, A, P, Wn, dtpart, S, r, last, st};
+                  int log_slot, hipStream_t st) {
+  Launch f{G, T, A, P, Wn, dtpart, S, r, last, log_slot, st};
   with_scheme(flux, rec, f);
 }
 
 void launch_step_final_tiled(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                              int nblk, const double* dtpart, int log_slot, hipStream_t st) {
+  if (A.arrive) return;  // ended by the last stage
   hipLaunchKernelGGL(k_step_final_tiled, dim3(S), dim3(1024), 0, st, A, P, nblk, G.nv, dtpart,
                      log_slot);
 }
@@ -1169,7 +1242,7 @@ void pack_plan(PackLevel* lv, int nl, int flux, int rec, PackPlan& p) {
   for (int l = 0; l < nl; ++l) {
     PackLevel& L = lv[l];
     L.base_fu = p.fu_blocks;         p.fu_blocks += L.T.ntiles * L.S;
-    L.base_final = p.final_blocks;   p.final_blocks += L.S;
+    L.base_final = p.final_blocks;   p.final_blocks += L.A.arrive ? 0 : L.S;
     p.fu_block = std::max(p.fu_block, stage_block(L.T));
     p.fu_lds = std::max(p.fu_lds, stage_lds(L.T));
   }
@@ -1182,6 +1255,7 @@ void launch_packed_stage(int flux, int rec, const PackLevel* d, const PackPlan& 
 }
 
 void launch_packed_final(const PackLevel* d, const PackPlan& p, hipStream_t st) {
+  if (p.final_blocks == 0) return;
   hipLaunchKernelGGL(k_step_final_packed, dim3(p.final_blocks), dim3(1024), 0, st, d, p.nl);
 }
 

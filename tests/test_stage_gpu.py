@@ -87,3 +87,27 @@ def test_launch_shapes_and_cut_runs_agree_bitwise(kind):
             s.run(k)
         out.append(s.get_state())
         assert np.array_equal(out[0], out[-1]), (kw, cuts)
+
+
+@pytest.mark.parametrize("tile", [4, 5, 6, 16])
+def test_steps_end_alike_whoever_ends_them(tile):
+    """Meshes of up to 512 tiles end their steps in the last stage, larger ones in
+    a launch of its own (2401 vertices: 600 tiles or more at 4, 480 or more at 5).
+    The time steps are minima and equal to the bit; a norm is the root of a sum of
+    2401 positive terms taken in another order (2401 eps / 2 = 3e-13 relative)."""
+    m = T.jittered_mesh(49, seed=2, bc={t: ("outlet",) for t in (1, 2, 3, 4)})
+    base = dict(flux="kepes_tecno_rusanov", reconstruct="minmod", cfl=0.4, final_time=10.0)
+    logs = []
+    for kw in (dict(), dict(tile_vertices=tile), dict(tile_vertices=tile)):
+        s = T.Solver(m, T.Params(**base, **kw), n_samples=3)
+        for k in range(3):
+            w = _wave(m)
+            w[:, 1] += 0.1 * k
+            s.set_state(w, k)
+        print(tile, kw, T.host_tiling(m, kw.get("tile_vertices", 128))["tiles"], flush=True)
+        done, log = s.run(8, want_log=True)
+        assert np.all(np.asarray(done) == 8)
+        logs.append(np.asarray(log).reshape(3, 8, 4).copy())
+    assert np.array_equal(logs[1], logs[2])
+    assert np.array_equal(logs[0][..., :3], logs[1][..., :3])
+    np.testing.assert_allclose(logs[1][..., 3], logs[0][..., 3], rtol=6e-13, atol=0)
