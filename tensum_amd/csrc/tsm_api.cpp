@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -48,12 +49,19 @@ struct tsm_ctx {
   double* E[2] = {nullptr, nullptr};
   int cur = 0;              // W[cur] / E[cur] hold the current state
   bool tiled = false;       // LDS-tiled stage kernels in use
+  int* bad = nullptr;       // first refused vertex of a state
   bool e_valid = true;      // E[cur] == prim2ent(W[cur])
   tsm::Tiling tiling;
   tsm::StageTab ST{};
   bool two_rings_asked = false;  // tile_fused_gradient on a mesh and scheme it applies to
   double* dtpart = nullptr;
   std::vector<int> perm;    // part-file vertex id -> device vertex id
+  const int* d_perm = nullptr;
+  // Host memory that kernels write: what a call returns of a few KB arrives with
+  // the call's one synchronisation, without copy commands.  Larger answers go
+  // through device memory.
+  static constexpr size_t PIN = 64 * 1024;
+  char* pin = nullptr;
   // input bface b, end point k (bface_v[2b+k]) -> offset of its boundary
   // values in a sample's block of G.bstate; device boundary codes
   std::vector<long long> bmap;
@@ -61,7 +69,6 @@ struct tsm_ctx {
   int* force_sel = nullptr;
   size_t force_cap = 0;
   double* W_keep = nullptr;     // last stage's input states (tsm_keep_stage_state)
-  double* bounds_buf = nullptr; // per-block minima and maxima (tsm_bounds)
   std::vector<int> h_btype;
   double* red = nullptr;   // reduction partials for global / error norms
   size_t red_cap = 0;
@@ -79,6 +86,8 @@ struct tsm_ctx {
   tsm::BcTime bt{};
 
   ~tsm_ctx() {
+    if (st) (void)hipStreamSynchronize(st);
+    if (pin) (void)hipHostFree(pin);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     for (void* p : allocs) (void)hipFree(p);
     if (st) (void)hipStreamDestroy(st);
@@ -101,6 +110,20 @@ struct tsm_ctx {
     if (!src.empty()) HIP_TRY(hipMemcpy(d, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice));
     *dst = d;
     return TSM_OK;
+  }
+  // the samples' control blocks on the host
+  hipError_t read_ctl(std::vector<tsm::Ctl>& q) {
+    const size_t n = S * sizeof(tsm::Ctl);
+    hipError_t e;
+    if (n <= PIN) {
+      tsm::launch_words((long)n, A.ctl, pin, st);
+      e = hipStreamSynchronize(st);
+      if (e == hipSuccess) std::memcpy(q.data(), pin, n);
+    } else {
+      e = hipStreamSynchronize(st);
+      if (e == hipSuccess) e = hipMemcpy(q.data(), A.ctl, n, hipMemcpyDeviceToHost);
+    }
+    return e;
   }
   void bind_state() {
     A.W_in = W[cur]; A.W_out = W[cur ^ 1];
@@ -257,6 +280,11 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     for (int i = 0; i < nv; ++i) perm[i] = inv[i] = i;
   }
   c->perm = perm;
+  if (int e = c->upload(&c->d_perm, perm)) { delete c; return e; }
+  if (hipHostMalloc((void**)&c->pin, tsm_ctx::PIN, hipHostMallocDefault) != hipSuccess) {
+    delete c;
+    return fail(TSM_E_HIP, "hipHostMalloc");
+  }
   // ---- host layout (device vertex ids) -----------------------------------
   std::vector<int> fv(2 * (size_t)nf);
   std::vector<double> fn(2 * (size_t)nf);
@@ -516,6 +544,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     if (hipMemset(A.arrive, 0, S * sizeof(int)) != hipSuccess) { delete c; return fail(TSM_E_HIP, "memset"); }
   }
   AL(A.ctl, (size_t)S);
+  AL(c->bad, 1);
   double* dg; double* dr; double* dc; double* ts;
   AL(dg, (size_t)S); AL(dr, (size_t)S); AL(dc, 2 * (size_t)S);
   // time stamps of an unsteady run (src/fv.cc:50-60); a steady run has none
@@ -696,32 +725,30 @@ extern "C" int tsm_set_sample_material(tsm_ctx* c, int s, double gamma, double R
 extern "C" int tsm_set_state(tsm_ctx* c, int s, const double* prim) {
   if (!c || !prim || s < 0 || s >= c->S) return fail(TSM_E_ARG, "bad argument");
   const int nv = c->G.nv;
-  for (int i = 0; i < nv; ++i) {
-    if (!(prim[4 * i] > 0.0) || !(prim[4 * i + 3] > 0.0) || !std::isfinite(prim[4 * i]) ||
-        !std::isfinite(prim[4 * i + 3]))
+  const size_t off = (size_t)s * nv;
+  if (c->tiled) {
+    c->state_ready();
+    c->e_valid = false;
+  } else {
+    c->csr_ready();
+  }
+  double* in = c->W[c->cur == 2 ? 0 : 2];  // free between steps
+  int* bad = reinterpret_cast<int*>(c->pin);
+  HIP_TRY(hipMemcpyAsync(in, prim, 4 * (size_t)nv * sizeof(double), hipMemcpyHostToDevice, c->st));
+  tsm::launch_state_put(nv, c->d_perm, in, c->bad, c->W[c->cur] + 4 * off,
+                        c->A.W_keep ? c->A.W_keep + 4 * off : nullptr, c->A.ctl + s, c->st);
+  tsm::launch_words(sizeof(int), c->bad, bad, c->st);
+  if (!c->tiled) tsm::launch_prim2ent(c->G, c->A, s, c->st);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(c->st));
+  const int i = *bad;
+  if (i != INT_MAX) {
+    if (!(prim[4 * (size_t)i] > 0.0) || !(prim[4 * (size_t)i + 3] > 0.0) || !std::isfinite(prim[4 * (size_t)i]) ||
+        !std::isfinite(prim[4 * (size_t)i + 3]))
       return fail(TSM_E_STATE, "initial temperature and pressure must be positive and finite "
                                "(vertex " + std::to_string(i) + ")");
-    if (!std::isfinite(prim[4 * i + 1]) || !std::isfinite(prim[4 * i + 2]))
-      return fail(TSM_E_STATE, "initial velocity is not finite (vertex " + std::to_string(i) + ")");
+    return fail(TSM_E_STATE, "initial velocity is not finite (vertex " + std::to_string(i) + ")");
   }
-  std::vector<double> aos(4 * (size_t)nv);
-  for (int i = 0; i < nv; ++i)
-    for (int k = 0; k < 4; ++k) aos[4 * (size_t)c->perm[i] + k] = prim[4 * i + k];
-  const size_t off = (size_t)s * nv;
-  HIP_TRY(hipStreamSynchronize(c->st));
-  c->csr_ready();
-  HIP_TRY(hipMemcpy(c->W[c->cur] + 4 * off, aos.data(), aos.size() * sizeof(double),
-                    hipMemcpyHostToDevice));
-  c->bind_state();
-  tsm::launch_prim2ent(c->G, c->A, s, c->st);
-  HIP_TRY(hipGetLastError());
-  if (c->A.W_keep)  // before any step the kept state is the current one
-    HIP_TRY(hipMemcpyAsync(c->A.W_keep + 4 * off, c->W[c->cur] + 4 * off, aos.size() * sizeof(double),
-                           hipMemcpyDeviceToDevice, c->st));
-  tsm::Ctl q{};
-  q.res_total = 1e20; q.counter = 1; q.done = 0;
-  HIP_TRY(hipMemcpyAsync(c->A.ctl + s, &q, sizeof(q), hipMemcpyHostToDevice, c->st));
-  HIP_TRY(hipStreamSynchronize(c->st));
   return TSM_OK;
 }
 
@@ -742,7 +769,12 @@ int download_vec(tsm_ctx* c, const double* base, int ncomp, int s, double* out) 
 
 extern "C" int tsm_get_state(tsm_ctx* c, int s, double* prim) {
   if (!c || !prim || s < 0 || s >= c->S) return fail(TSM_E_ARG, "bad argument");
-  return download_vec(c, c->W[c->cur], 4, s, prim);
+  double* out = c->W[c->cur == 2 ? 0 : 2];  // free between steps
+  tsm::launch_state_get(c->G.nv, c->d_perm, c->W[c->cur] + 4 * (size_t)s * c->G.nv, out, c->st);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(prim, out, 4 * (size_t)c->G.nv * sizeof(double), hipMemcpyDeviceToHost, c->st));
+  HIP_TRY(hipStreamSynchronize(c->st));
+  return TSM_OK;
 }
 
 extern "C" int tsm_gradients(tsm_ctx* c, int s, double* dE) {
@@ -990,8 +1022,7 @@ extern "C" int tsm_run(tsm_ctx* c, long nsteps, long* done, double* log) {
   if (!c || nsteps < 0) return fail(TSM_E_ARG, "bad argument");
   const int S = c->S;
   std::vector<tsm::Ctl> before(S), after(S);
-  HIP_TRY(hipStreamSynchronize(c->st));
-  HIP_TRY(hipMemcpy(before.data(), c->A.ctl, S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
+  HIP_TRY(c->read_ctl(before));
   if (log && nsteps > 0) {
     if (c->A.log_cap < nsteps) {
       double* p = nullptr;
@@ -1003,8 +1034,7 @@ extern "C" int tsm_run(tsm_ctx* c, long nsteps, long* done, double* log) {
   }
   enqueue_steps(c, nsteps, log != nullptr);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipStreamSynchronize(c->st));
-  HIP_TRY(hipMemcpy(after.data(), c->A.ctl, S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
+  HIP_TRY(c->read_ctl(after));
   if (done)
     for (int s = 0; s < S; ++s) done[s] = (long)(after[s].iter - before[s].iter);
   if (log && nsteps > 0) {
@@ -1026,9 +1056,8 @@ extern "C" int tsm_step(tsm_ctx* c, double t_target, double* dt_out, double* res
   if (t_target > 0.0 && !c->P.unsteady)
     return fail(TSM_E_ARG, "t_target needs an unsteady run (steady steps use local time steps)");
   const int S = c->S;
+  const size_t nc = S * sizeof(tsm::Ctl);
   std::vector<tsm::Ctl> before(S), after(S);
-  HIP_TRY(hipStreamSynchronize(c->st));
-  HIP_TRY(hipMemcpy(before.data(), c->A.ctl, S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
   if (c->A.log_cap < 1) {  // the step's (iter, dt, t, res) rows
     double* p = nullptr;
     int rc = c->alloc(&p, (size_t)S * 4);
@@ -1036,6 +1065,11 @@ extern "C" int tsm_step(tsm_ctx* c, double t_target, double* dt_out, double* res
     c->A.log = p;
     c->A.log_cap = 1;
   }
+  // the control blocks before and after and the rows, in one go if they fit
+  const size_t nl = (size_t)S * c->A.log_cap * 4 * sizeof(double);
+  const bool small = 2 * nc + nl <= tsm_ctx::PIN;
+  if (small) tsm::launch_words((long)nc, c->A.ctl, c->pin, c->st);
+  else HIP_TRY(c->read_ctl(before));
   if (c->tiled) {
     c->bind_state();
     tsm::launch_dt(c->G, c->A, c->SP, S, c->st);
@@ -1049,10 +1083,19 @@ extern "C" int tsm_step(tsm_ctx* c, double t_target, double* dt_out, double* res
     enqueue_step(c, 0, /*dt_ready=*/true);
   }
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipStreamSynchronize(c->st));
-  HIP_TRY(hipMemcpy(after.data(), c->A.ctl, S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
-  std::vector<double> rows((size_t)S * c->A.log_cap * 4);
-  HIP_TRY(hipMemcpy(rows.data(), c->A.log, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
+  std::vector<double> rows(nl / sizeof(double));
+  if (small) {
+    tsm::launch_words((long)nc, c->A.ctl, c->pin + nc, c->st);
+    tsm::launch_words((long)nl, c->A.log, c->pin + 2 * nc, c->st);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->st));
+    std::memcpy(before.data(), c->pin, nc);
+    std::memcpy(after.data(), c->pin + nc, nc);
+    std::memcpy(rows.data(), c->pin + 2 * nc, nl);
+  } else {
+    HIP_TRY(c->read_ctl(after));
+    HIP_TRY(hipMemcpy(rows.data(), c->A.log, nl, hipMemcpyDeviceToHost));
+  }
   for (int s = 0; s < S; ++s) {
     const bool ran = after[s].iter > before[s].iter;
     const double* r = &rows[(size_t)s * c->A.log_cap * 4];
@@ -1069,8 +1112,27 @@ extern "C" int tsm_run_group(tsm_ctx** cs, int n, long nsteps, long* done) {
     tsm_ctx* c = cs[i];
     if (!c) return fail(TSM_E_ARG, "null context in group");
     before[i].resize(c->S);
-    HIP_TRY(hipStreamSynchronize(c->st));
-    HIP_TRY(hipMemcpy(before[i].data(), c->A.ctl, c->S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
+    HIP_TRY(c->read_ctl(before[i]));
+  }
+  // A context whose samples are all done takes no further launches: it is looked
+  // at after every POLL steps, one look behind so that its stream does not run dry
+  // (the launches of a step of finished samples cost 30 us at 64 samples of 129^2).
+  constexpr long POLL = 16;
+  std::vector<char> idle(n, 0);
+  std::vector<int> looks(n, 0);
+  struct Events {
+    std::vector<hipEvent_t> e;
+    ~Events() { for (auto x : e) (void)hipEventDestroy(x); }
+  } ev;
+  for (int i = 0; i < n; ++i) {
+    bool all = true;
+    for (const auto& q : before[i]) all = all && q.done;
+    idle[i] = all;
+    for (int k = 0; k < 2; ++k) {
+      hipEvent_t x;
+      HIP_TRY(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+      ev.e.push_back(x);
+    }
   }
   // Interleave the contexts' launches in chunks so every stream has work queued
   // while the others run: levels of different sizes share the GPU.
@@ -1079,6 +1141,20 @@ extern "C" int tsm_run_group(tsm_ctx** cs, int n, long nsteps, long* done) {
     const long m = std::min(chunk, nsteps - k0);
     for (int i = 0; i < n; ++i) {
       tsm_ctx* c = cs[i];
+      if (idle[i]) continue;
+      int* flag = reinterpret_cast<int*>(c->pin);
+      if (k0 > 0 && k0 % POLL == 0) {
+        const int look = looks[i]++;
+        if (look > 0) {
+          HIP_TRY(hipEventSynchronize(ev.e[2 * i + (look - 1) % 2]));
+          if (*static_cast<volatile int*>(flag + (look - 1) % 2)) {
+            idle[i] = 1;
+            continue;
+          }
+        }
+        tsm::launch_all_done(c->S, c->A.ctl, flag + look % 2, c->st);
+        HIP_TRY(hipEventRecord(ev.e[2 * i + look % 2], c->st));
+      }
       if (c->tiled) {
         c->bind_state();
         if (k0 == 0) tsm::launch_dt(c->G, c->A, c->SP, c->S, c->st);
@@ -1093,8 +1169,7 @@ extern "C" int tsm_run_group(tsm_ctx** cs, int n, long nsteps, long* done) {
   for (int i = 0; i < n; ++i) {
     tsm_ctx* c = cs[i];
     std::vector<tsm::Ctl> after(c->S);
-    HIP_TRY(hipStreamSynchronize(c->st));
-    HIP_TRY(hipMemcpy(after.data(), c->A.ctl, c->S * sizeof(tsm::Ctl), hipMemcpyDeviceToHost));
+    HIP_TRY(c->read_ctl(after));
     long tot = 0;
     for (int s = 0; s < c->S; ++s) tot += (long)(after[s].iter - before[i][s].iter);
     if (done) done[i] = tot;
@@ -1195,16 +1270,11 @@ extern "C" int tsm_time(tsm_ctx* c, int s, double* t, long* iter) {
 extern "C" int tsm_bounds(tsm_ctx* c, int s, double* out) {
   if (!c || !out || s < 0 || s >= c->S) return fail(TSM_E_ARG, "bad argument");
   const int nblk = std::max(1, std::min(1024, (c->G.nv + 255) / 256));
-  if (!c->bounds_buf) {
-    int rc = c->alloc(&c->bounds_buf, 8 * 1024);
-    if (rc) return rc;
-  }
   c->state_ready();
-  tsm::launch_bounds(c->G, c->A, s, c->bounds_buf, nblk, c->st);
+  static_assert(8 * 1024 * sizeof(double) <= tsm_ctx::PIN, "the blocks' bounds fit");
+  const double* part = reinterpret_cast<const double*>(c->pin);
+  tsm::launch_bounds(c->G, c->A, s, reinterpret_cast<double*>(c->pin), nblk, c->st);
   HIP_TRY(hipGetLastError());
-  std::vector<double> part(8 * (size_t)nblk);
-  HIP_TRY(hipMemcpyAsync(part.data(), c->bounds_buf, part.size() * sizeof(double),
-                         hipMemcpyDeviceToHost, c->st));
   HIP_TRY(hipStreamSynchronize(c->st));
   // T, p, u, v as (min, max); w is zero in two dimensions
   double r[8] = {1.0e20, -1.0e20, 1.0e20, -1.0e20, 1.0e20, -1.0e20, 1.0e20, -1.0e20};
@@ -1592,14 +1662,17 @@ extern "C" int tsm_check_arith(long n, const double* a, const double* b, double*
 extern "C" int tsm_global_all(tsm_ctx* c, double* ke, double* ent) {
   if (!c) return fail(TSM_E_ARG, "bad argument");
   const int nb = c->nblk_v, S = c->S;
-  int rc = ensure_red(c, (size_t)nb * S * 2);  // the context's reduction buffer: no allocation per call
-  if (rc) return rc;
+  const size_t n = (size_t)nb * S * 2;
+  const bool small = n * sizeof(double) <= tsm_ctx::PIN;
+  if (!small)
+    if (int rc = ensure_red(c, n)) return rc;  // the context's reduction buffer: no allocation per call
   c->bind_state();
-  tsm::launch_global_all(c->G, c->A, S, c->red, c->st);
+  tsm::launch_global_all(c->G, c->A, S, small ? reinterpret_cast<double*>(c->pin) : c->red, c->st);
   HIP_TRY(hipGetLastError());
-  std::vector<double> h((size_t)nb * S * 2);
   HIP_TRY(hipStreamSynchronize(c->st));
-  HIP_TRY(hipMemcpy(h.data(), c->red, h.size() * sizeof(double), hipMemcpyDeviceToHost));
+  std::vector<double> big(small ? 0 : n);
+  if (!small) HIP_TRY(hipMemcpy(big.data(), c->red, n * sizeof(double), hipMemcpyDeviceToHost));
+  const double* h = small ? reinterpret_cast<const double*>(c->pin) : big.data();
   for (int s = 0; s < S; ++s) {
     double K = 0, E = 0;
     for (int b = 0; b < nb; ++b) { K += h[((size_t)s * nb + b) * 2]; E += h[((size_t)s * nb + b) * 2 + 1]; }

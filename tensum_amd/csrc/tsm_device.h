@@ -408,6 +408,11 @@ void launch_step_final(const DevGeo& G, const StageArgs& A, const StepParams& P,
                        int log_slot, hipStream_t st);
 void launch_ssw(const DevGeo& G, const StageArgs& A, int S, hipStream_t st);
 void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st);
+void launch_state_put(int nv, const int* perm, const double* in, int* bad, double* W, double* keep,
+                      Ctl* ctl, hipStream_t st);
+void launch_state_get(int nv, const int* perm, const double* W, double* out, hipStream_t st);
+void launch_words(long bytes, const void* in, void* out, hipStream_t st);
+void launch_all_done(int S, const Ctl* ctl, int* out, hipStream_t st);
 void launch_global(const DevGeo& G, const StageArgs& A, int s, double* out, hipStream_t st);
 void launch_enstrophy(const DevGeo& G, const StageArgs& A, int s, double* out, hipStream_t st);
 void launch_errnorm(const DevGeo& G, const StageArgs& A, int s, const double* ex, double* out,
