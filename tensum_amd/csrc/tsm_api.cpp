@@ -539,7 +539,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   if (params->liou_fix) AL(A.ssw, cs);
   AL(A.partial, (size_t)S * std::max(c->nblk_v, c->tiling.ntiles) * 4);
   if (c->tiled) AL(c->dtpart, (size_t)S * c->tiling.ntiles);
-  if (c->tiled && tsm::stage_ends_step(c->tiling.ntiles)) {
+  if (c->tiled && tsm::stage_ends_step(c->tiling.ntiles, S)) {
     AL(A.arrive, S);
     if (hipMemset(A.arrive, 0, S * sizeof(int)) != hipSuccess) { delete c; return fail(TSM_E_HIP, "memset"); }
   }

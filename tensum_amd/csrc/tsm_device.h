@@ -375,7 +375,7 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
 int stage_block(const StageTab& T);
 int stage_block_max();
 size_t stage_lds(const StageTab& T);
-bool stage_ends_step(int ntiles);
+bool stage_ends_step(int ntiles, int samples);
 int stage_main_records(const StageTab& T, bool grad, bool ns);
 bool stage_has_gradients(int flux, int rec);
 bool stage_keeps_var0(int flux);

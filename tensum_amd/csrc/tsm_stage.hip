@@ -1122,11 +1122,13 @@ __global__ __launch_bounds__(1024) void k_step_final_packed(const PackLevel* __r
   step_final_body(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
 }
 
-// The last stage ends the step of a mesh with up to this many tiles, eight partials
-// a lane of the wave that does it.  A step of the vortex (Roe, minmod) against a
-// launch of its own: 129^2 (150 tiles) 37.7 us against 41.8, 200^2 43.0 / 45.7,
-// 257^2 (541) 53.9 / 54.3, 350^2 63.2 / 62.7.
-constexpr int FOLD_TILES = 512;
+// The last stage ends the steps of a context with up to this many tiles over all its
+// samples, which run at once: eight partials a lane of the wave that does it.  A step
+// of the vortex (Roe, minmod) against a launch of its own: 129^2 (150 tiles) 37.7 us
+// against 41.8, 200^2 43.0 / 45.7, 257^2 (541) 53.9 / 54.3, 350^2 63.2 / 62.7.  Where
+// tiles queue for a CU each is held up by the wait for its partials: 32 samples of
+// 257^2 took 1.15 times as long.
+constexpr long FOLD_TILES = 512;
 
 // ---------------------------------------------------------------------------
 // launchers
@@ -1137,7 +1139,7 @@ int stage_block(const StageTab& T) {
   return std::max(b, T.fu_block);
 }
 int stage_block_max() { return 512; }
-bool stage_ends_step(int ntiles) { return ntiles <= FOLD_TILES; }
+bool stage_ends_step(int ntiles, int samples) { return (long)ntiles * samples <= FOLD_TILES; }
 
 namespace {
 size_t lds_of(const StageTab& T) {

@@ -91,8 +91,9 @@ def test_launch_shapes_and_cut_runs_agree_bitwise(kind):
 
 @pytest.mark.parametrize("tile", [4, 5, 6, 16])
 def test_steps_end_alike_whoever_ends_them(tile):
-    """Meshes of up to 512 tiles end their steps in the last stage, larger ones in
-    a launch of its own (2401 vertices: 600 tiles or more at 4, 480 or more at 5).
+    """Contexts of up to 512 tiles end their steps in the last stage, larger ones in
+    a launch of its own (2401 vertices, three samples: 1800 tiles or more at 4, 450
+    at 16, 57 by default).
     The time steps are minima and equal to the bit; a norm is the root of a sum of
     2401 positive terms taken in another order (2401 eps / 2 = 3e-13 relative)."""
     m = T.jittered_mesh(49, seed=2, bc={t: ("outlet",) for t in (1, 2, 3, 4)})
