@@ -376,6 +376,32 @@ __device__ __forceinline__ void step_ctl(const StageArgs& A, const StepParams& P
   A.ctl[s] = c;
 }
 
+// A wave's sum or minimum in its lane 63 by data-parallel primitives: shifts within
+// rows of 16 lanes, then a row's last lane to the next row and the first half's to the
+// second.  Lanes without a source take the neutral element z.
+template <int CTRL, int ROWS, class F>
+__device__ __forceinline__ double dpp_step(double x, double z, F f) {
+  const long long xb = __double_as_longlong(x), zb = __double_as_longlong(z);
+  const int lo = __builtin_amdgcn_update_dpp((int)zb, (int)xb, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(zb >> 32), (int)(xb >> 32), CTRL, ROWS, 0xf, false);
+  return f(x, __longlong_as_double(((long long)hi << 32) | (unsigned)lo));
+}
+template <class F>
+__device__ __forceinline__ double wave_fold(double x, double z, F f) {
+  x = dpp_step<0x111, 0xf>(x, z, f);
+  x = dpp_step<0x112, 0xf>(x, z, f);
+  x = dpp_step<0x114, 0xf>(x, z, f);
+  x = dpp_step<0x118, 0xf>(x, z, f);
+  x = dpp_step<0x142, 0xa>(x, z, f);
+  return dpp_step<0x143, 0xc>(x, z, f);
+}
+__device__ __forceinline__ double wave_sum(double x) {
+  return wave_fold(x, 0.0, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_min(double x) {  // of values up to 1e20
+  return wave_fold(x, 1.0e20, [](double a, double b) { return fmin(a, b); });
+}
+
 // The end of a step by one wave, from the partials of nblk blocks of this very
 // launch: they were written through to memory before their blocks counted
 // themselves in, and are read past the caches.
@@ -409,35 +435,27 @@ __device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams&
     }
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) part[k] += __shfl_down(part[k], o, 64);
-    x = fmin(x, __shfl_down(x, o, 64));
-  }
-  if (lane == 0) step_ctl(A, P, c, nv, part, x, log_slot, s);
+  for (int k = 0; k < 4; ++k) part[k] = wave_sum(part[k]);
+  x = wave_min(x);
+  if (lane == 63) step_ctl(A, P, c, nv, part, x, log_slot, s);
 }
 
-// Per-block partials of the last stage without a block barrier: every wave
-// reduces its residual-norm sums and smallest local dt by shuffles, its lane 0
+// Per-block partials of the last stage without a block barrier: every wave with
+// owned vertices reduces its residual-norm sums and smallest local dt, its lane 63
 // leaves them in LDS and counts itself in with an LDS integer atomic; the
 // last wave to arrive adds the waves' values in wave order and writes the
 // block's slot.  Waves that finish early leave at once.  Where the sample's
 // blocks are counted (A.arrive), the last block's wave ends the step.
 __device__ __forceinline__ void block_partials(const StageArgs& A, const StepParams& P, double* part,
                                                double dtv, double* wred, int* arrive, double* dtpart,
-                                               int s, int t, int nt, int nv, int log_slot) {
+                                               int s, int t, int nt, int nv, int nw, int log_slot) {
+  const int w = threadIdx.x >> 6;
+  if (w >= nw) return;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    double x = part[k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-    part[k] = x;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) dtv = fmin(dtv, __shfl_down(dtv, o, 64));
+  for (int k = 0; k < 4; ++k) part[k] = wave_sum(part[k]);
+  dtv = wave_min(dtv);
   int ends = 0;
-  if ((threadIdx.x & 63) == 0) {
-    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if ((threadIdx.x & 63) == 63) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) wred[5 * w + k] = part[k];
     wred[5 * w + 4] = dtv;
@@ -465,7 +483,7 @@ __device__ __forceinline__ void block_partials(const StageArgs& A, const StepPar
       }
     }
   }
-  if (!__builtin_amdgcn_readfirstlane(ends)) return;
+  if (!__builtin_amdgcn_readlane(ends, 63)) return;
   asm volatile("" ::: "memory");
   final_wave(A, P, nt, nv, dtpart, log_slot, s);
   if ((threadIdx.x & 63) == 0)
@@ -1008,7 +1026,7 @@ __device__ __forceinline__ void stage_body(const DevGeo& G, const StageTab& T, c
       dtv = (P.time_step > 0.0) ? P.time_step : fdiv(P.cfl * area_v, lam);
       if (A.dtl) A.dtl[off + v] = dtv;  // steady mode: read by this vertex only, next step
     }
-    block_partials(A, P, part, dtv, wred, &arrive, dtpart, s, t, nbx, G.nv, log_slot);
+    block_partials(A, P, part, dtv, wred, &arrive, dtpart, s, t, nbx, G.nv, (nown + 63) >> 6, log_slot);
   }
 }
 
@@ -1043,14 +1061,9 @@ namespace {
 template <int NV>
 __device__ __forceinline__ void bsum(double* v, double* red) {
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    double x = v[k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-    v[k] = x;
-  }
+  for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0)
+  if (lane == 63)
 #pragma unroll
     for (int k = 0; k < NV; ++k) red[wid * NV + k] = v[k];
   __syncthreads();
@@ -1065,13 +1078,13 @@ __device__ __forceinline__ void bsum(double* v, double* red) {
   }
 }
 __device__ __forceinline__ double bmin(double x, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmin(x, __shfl_down(x, o, 64));
+  x = wave_min(x);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) red[wid] = x;
+  if (lane == 63) red[wid] = x;
   __syncthreads();
   if (threadIdx.x == 0) {
     const int nw = blockDim.x >> 6;
+    x = red[0];
     for (int w = 1; w < nw; ++w) x = fmin(x, red[w]);
   }
   return x;
