@@ -270,7 +270,7 @@ __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W
 __device__ __forceinline__ int c_row(int i) { return 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
 
 // Weight slices of one 32-column tile in registers (layers up to 256 deep): the
-// loads of a layer are issued before the previous one's epilogue.
+// loads of a layer are issued before the previous one's product.
 struct WReg { bf16x8 b[16]; };
 __device__ __forceinline__ void load_tile(WReg& w, const u16* W, int Kp, int n0) {
   const u16* wr = W + n0 * Kp + (threadIdx.x & 63) * 8;
@@ -298,8 +298,8 @@ __device__ __forceinline__ void reg_product(const u16* A, int lda, const WReg& w
 // epilogues (an error function and an exponential per element) are most of the
 // work, rows 0-7 of a tile are elements 0-3 of every lane, and a minibatch of 64
 // then spreads over eight CUs instead of two.  At 64 rows of 6-256-256-66: 32 rows a
-// block 56 us; eight, with the next product's weights asked for ahead, 36; weights
-// in operand order 25.
+// block 56 us; eight, with the next product's weights asked for after this one's, 36;
+// weights in operand order 25; asked for before this one's product 22.
 // REG: no layer wider than 256, so a wave has one tile per layer and holds its
 // weights in registers.
 constexpr int RB = 8;
@@ -310,8 +310,16 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
   u16 *cur = sm, *nxt = sm + RT * a.lda;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   const int r0 = blockIdx.x * RB, L = a.L;
-  WReg wr;
-  if (REG && 32 * wave < upd(a.w[1], 32)) load_tile(wr, a.Wp[0], upd(a.w[0], 16), 32 * wave);
+  // products in order: forward through the layers, back from the last to the second
+  WReg wr, wn;
+  auto fetch = [&](int p, WReg& w) {
+    if (!REG || p > 2 * L - 2) return;
+    const bool f = p < L;
+    const int l = f ? p : 2 * L - 1 - p;
+    const int cols = upd(f ? a.w[l + 1] : a.w[l], 32), depth = upd(f ? a.w[l] : a.w[l + 1], 16);
+    if (32 * wave < cols) load_tile(w, f ? a.Wp[l] : a.Wt[l], depth, 32 * wave);
+  };
+  fetch(0, wr);
   {
     const int K = a.w[0], Kp = upd(K, 16);
     for (int i = tid; i < RB * Kp; i += blockDim.x) {
@@ -332,6 +340,7 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
     const int K = a.w[l], N = a.w[l + 1], Kp = upd(K, 16), Np = upd(N, 32);
     const bool last = l + 1 == L;
     const float* bias = a.P + a.boff[l];
+    if (REG && 32 * wave >= Np) fetch(l + 1, wn);
     for (int n0 = 32 * wave; n0 < Np; n0 += 32 * nw) {
       const int n = n0 + (lane & 31);
       const bool col = n < N;
@@ -341,15 +350,9 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
 #pragma unroll
         for (int u = 0; u < 4; ++u)
           if (r0 + row0 + u < nb) t[u] = Tin[(size_t)rows[u] * N + n];
+      fetch(l + 1, wn);  // after this product's own loads: waits are in order
       if (REG) reg_product(cur, a.lda, wr, Kp, acc[0]);
       else tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
-      if (REG) {  // the next product's weights: the next layer's, or the last one's transposed
-        if (!last) {
-          if (n0 < upd(a.w[l + 2], 32)) load_tile(wr, a.Wp[l + 1], upd(N, 16), n0);
-        } else if (L > 1 && n0 < upd(K, 32)) {
-          load_tile(wr, a.Wt[l], upd(N, 16), n0);
-        }
-      }
       ushort4 q;
       u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
@@ -372,21 +375,14 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
       }
       if (col) *reinterpret_cast<ushort4*>((last ? a.DT[l] : a.XT[l + 1]) + (size_t)n * a.ldr + r0 + row0) = q;
     }
-    // a wave without a tile in this layer may have one in the next
-    if (REG && 32 * wave >= Np) {
-      if (!last) {
-        if (32 * wave < upd(a.w[l + 2], 32)) load_tile(wr, a.Wp[l + 1], upd(N, 16), 32 * wave);
-      } else if (L > 1 && 32 * wave < upd(K, 32)) {
-        load_tile(wr, a.Wt[l], upd(N, 16), 32 * wave);
-      }
-    }
+    if (REG) wr = wn;
     __syncthreads();
     u16* x = cur; cur = nxt; nxt = x;
   }
   // dz_{l-1} = (dz_l W_l) * GELU'(z_{l-1}); z was stored by this very lane
   for (int l = L - 1; l > 0; --l) {
     const int K = a.w[l], N = a.w[l + 1], Np = upd(N, 16), Kp = upd(K, 32);
-    const int k1 = l > 1 ? upd(a.w[l - 1], 32) : 0;  // columns of the next product
+    if (REG && 32 * wave >= Kp) fetch(2 * L - l, wn);
     for (int k0 = 32 * wave; k0 < Kp; k0 += 32 * nw) {
       const int k = k0 + (lane & 31);
       const bool col = k < K;
@@ -396,9 +392,9 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
         const int r = r0 + row0 + u;
         z[u] = col && r < nb ? a.Z[l - 1][(size_t)r * K + k] : 0.0f;
       }
+      fetch(2 * L - l, wn);
       if (REG) reg_product(cur, a.lda, wr, Np, acc[0]);
       else tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
-      if (REG && k0 < k1) load_tile(wr, a.Wt[l - 1], upd(K, 16), k0);
       ushort4 q;
       u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
@@ -409,7 +405,7 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
       }
       if (col) *reinterpret_cast<ushort4*>(a.DT[l - 1] + (size_t)k * a.ldr + r0 + row0) = q;
     }
-    if (REG && 32 * wave >= Kp && 32 * wave < k1) load_tile(wr, a.Wt[l - 1], upd(K, 16), 32 * wave);
+    if (REG) wr = wn;
     __syncthreads();
     u16* x = cur; cur = nxt; nxt = x;
   }
