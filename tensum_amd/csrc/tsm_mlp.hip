@@ -297,7 +297,7 @@ __device__ __forceinline__ void reg_product(const u16* A, int lda, const WReg& w
 // 32-column tiles each.  Eight rows a block, though the MFMA tile has 32: the
 // epilogues (an error function and an exponential per element) are most of the
 // work, rows 0-7 of a tile are elements 0-3 of every lane, and a minibatch of 64
-// then spreads over eight CUs instead of two.  At 64 rows of 6-256-256-66: 32 rows a
+// then spreads over eight CUs instead of two.  At 64 rows of 6-256-256-256-66: 32 rows a
 // block 56 us; eight, with the next product's weights asked for after this one's, 36;
 // weights in operand order 25; asked for before this one's product 22.
 // REG: no layer wider than 256, so a wave has one tile per layer and holds its
@@ -424,7 +424,7 @@ __device__ __forceinline__ float adam_step(const Adam& h, float gi, float p, flo
 // rows), 64 bias gradients (sums in row order), or one 256-element part of the
 // loss (the tree of k_mse).  TRAIN applies Adam at once and refreshes the bf16
 // weights; else the gradient goes to G.  Bound by the latency of one pass over
-// activations and moments (85 k parameters, 2.4 MB, 0.5 us at the copy rate):
+// activations and moments (150 k parameters, 3.6 MB, 0.7 us at the copy rate):
 // 13.9 us with each parameter's moments read in turn, 11.7 with all ahead.
 template <bool TRAIN>
 __global__ __launch_bounds__(256) void k_update(Net a, int nb, const int4* jobs, int n_jobs,

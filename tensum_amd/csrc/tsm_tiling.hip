@@ -1,6 +1,5 @@
 // tsm_tiling.hip -- the vertex tiling of the LDS-staged kernels built on the
-// device (the arrays build_tiles forms on the host, tiles.cpp, bit for bit),
-// for every mesh but those of the fused kernel's second halo ring.
+// device (the arrays build_tiles forms on the host, tiles.cpp, bit for bit).
 //
 // Every per-tile list is a sort of 64-bit keys (tile << 32 | id) followed by
 // binary searches: periodic-set members first (whole sets in set order, in

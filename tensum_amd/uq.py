@@ -170,10 +170,9 @@ def advance(solvers, chunk=64, max_chunks=100000, packed=False, log=None, log_ev
     solvers' own launches interleaved on their streams, or (packed=True) one
     launch per kernel spanning every solver where their scheme allows it
     (Euler, SSP-RK3, tiled kernels, one flux and reconstruction; the same
-    results bit for bit).  Measured on the four-level vortex batch (65^2 to
-    513^2 with 4096/1024/256/64 samples) the streams are faster: 6.2e9 against
-    5.1e9 vertex-stage updates/s, as their gradient and flux passes of
-    different levels overlap.  log: called with a progress line every
+    results bit for bit).  Measured on two levels of the vortex batch (129^2 with
+    512 samples, 257^2 with 64) the streams are faster: 1.02e10 against 9.3e9
+    vertex-stage updates/s, as one level's last tiles overlap another's first.  log: called with a progress line every
     log_every seconds."""
     step = run_packed if packed else run_group
     t_last = time.perf_counter()
