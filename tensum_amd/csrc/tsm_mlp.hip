@@ -11,7 +11,7 @@
 //   dW_l = dz_l^T x_l,  db_l = column sums of dz_l   (fp32)
 //   dx_l = dz_l W_l,    dz_{l-1} = dx_l * GELU'(z_{l-1})   (-> bf16)
 // Networks of layers up to FUSED_MAX wide (the surrogates are 64 to 256 wide) run
-// in three kernels: k_rows takes eight rows of a minibatch through every layer and
+// in three kernels: k_rows (k_rows_reg up to 256 wide) takes eight rows of a minibatch through every layer and
 // back, k_update forms each 32 x 32 tile of the weight gradients and applies Adam
 // to it, k_infer takes rows through the layers only.  Wider ones take one launch
 // of the tiled GEMM per product, the operands' transposes absorbed by the LDS
@@ -269,57 +269,154 @@ __device__ __forceinline__ void tile_product(const u16* A, int lda, const u16* W
 // row of result element i within a tile
 __device__ __forceinline__ int c_row(int i) { return 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
 
-// Weight slices of one 32-column tile in registers (layers up to 256 deep): the
-// loads of a layer are issued before the previous one's product.
-struct WReg { bf16x8 b[16]; };
-__device__ __forceinline__ void load_tile(WReg& w, const u16* W, int Kp, int n0) {
-  const u16* wr = W + n0 * Kp + (threadIdx.x & 63) * 8;
-#pragma unroll
-  for (int u = 0; u < 16; ++u)
-    if (16 * u < Kp) w.b[u] = *reinterpret_cast<const bf16x8*>(wr + 512 * u);
-}
-__device__ __forceinline__ void reg_product(const u16* A, int lda, const WReg& w, int Kp, f32x16& acc) {
-  const int lane = threadIdx.x & 63;
-  const u16* ar = A + (lane & 31) * lda + (lane >> 5) * 8;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-#pragma unroll
-  for (int u = 0; u < 16; ++u)
-    if (16 * u < Kp) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(ar + 16 * u);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w.b[u], acc, 0, 0, 0);
-    }
-}
-
 // RB rows of a minibatch (rows idx[r], or r itself) forward, dy = 2 (y - t) / n,
 // and back to dz_0; the transposed activations and dz of every layer go to XT/DT.
 // Bound by the latency of its 2 L - 1 dependent products: eight waves, one or more
 // 32-column tiles each.  Eight rows a block, though the MFMA tile has 32: the
 // epilogues (an error function and an exponential per element) are most of the
 // work, rows 0-7 of a tile are elements 0-3 of every lane, and a minibatch of 64
-// then spreads over eight CUs instead of two.  At 64 rows of 6-256-256-256-66: 32 rows a
-// block 56 us; eight, with the next product's weights asked for after this one's, 36;
-// weights in operand order 25; asked for before this one's product 22.
-// REG: no layer wider than 256, so a wave has one tile per layer and holds its
-// weights in registers.
+// then spreads over eight CUs instead of two.
 constexpr int RB = 8;
-template <bool REG>
+
+// The product of a wave's tile with the weight slices in w (up to 16 of 16 deep),
+// each slice's registers taking the next product's as soon as it is used.
+struct WReg { bf16x8 b[16]; };
+__device__ __forceinline__ void reg_load(WReg& w, const u16* W, int Kp) {
+  const u16* p = W + (threadIdx.x & 63) * 8;
+  const int last = (Kp >> 4) - 1;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) w.b[u] = *reinterpret_cast<const bf16x8*>(p + 512 * min(u, last));
+}
+__device__ __forceinline__ f32x16 reg_product(const u16* A, int lda, WReg& w, int Kp, const u16* Wn,
+                                              int Kpn) {
+  const int lane = threadIdx.x & 63, lastn = (Kpn >> 4) - 1;
+  const u16* ar = A + (lane & 31) * lda + (lane >> 5) * 8;
+  const u16* p = Wn + lane * 8;
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    if (16 * u < Kp) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(ar + 16 * u);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w.b[u], acc, 0, 0, 0);
+    }
+    w.b[u] = *reinterpret_cast<const bf16x8*>(p + 512 * min(u, lastn));
+  }
+  return acc;
+}
+
+// For nets with no layer wider than 256: one tile per wave (waves beyond a layer's
+// tiles repeat the last one, with the same results), its weights in registers.
+// Nothing but the loss's row depends on a branch and pre-activations stay in LDS, so
+// that a layer waits for its own weights only, which were asked for a product ago.
+// At 64 rows of 6-256-256-256-66: 32 rows a block 56 us; eight, with the next
+// weights asked for after a product, 36; weights in operand order 25; asked for
+// before it 22; as now 18.
+__global__ __launch_bounds__(512) void k_rows_reg(Net a, int nb, const int* idx, const float* Xin,
+                                                  const float* Tin, float scale) {
+  extern __shared__ __attribute__((aligned(16))) u16 sm[];
+  u16 *cur = sm, *nxt = sm + RT * a.lda;
+  float4* zs = reinterpret_cast<float4*>(sm + 2 * RT * a.lda);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = blockIdx.x * RB, L = a.L;
+  const int row0 = 4 * (lane >> 5);  // this lane's rows: row0 .. row0 + 3
+  auto tile = [&](int n) { return min(32 * wave, upd(n, 32) - 32); };  // of a layer n wide
+  auto fwd = [&](int l) { return a.Wp[l] + tile(a.w[l + 1]) * upd(a.w[l], 16); };
+  auto bwd = [&](int l) { return a.Wt[l] + tile(a.w[l]) * upd(a.w[l + 1], 16); };
+  auto bias = [&](int l) {
+    return a.P[a.boff[l] + min(tile(a.w[l + 1]) + (lane & 31), a.w[l + 1] - 1)];
+  };
+  WReg w;
+  reg_load(w, fwd(0), upd(a.w[0], 16));
+  float bn = bias(0);
+  const int no = a.w[L], ny = tile(no) + (lane & 31);
+  float t[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = min(r0 + row0 + u, nb - 1);
+    t[u] = Tin[(size_t)(idx ? idx[r] : r) * no + min(ny, no - 1)];
+  }
+  {
+    const int K = a.w[0], Kp = upd(K, 16);
+    for (int i = tid; i < RB * Kp; i += blockDim.x) {
+      const int k = i / RB, r = i % RB;  // rows fastest: XT is written in order
+      const bool in = k < K && r0 + r < nb;
+      const u16 v = in ? f2bf(Xin[(size_t)(idx ? idx[r0 + r] : r0 + r) * K + k]) : (u16)0;
+      cur[r * a.lda + k] = v;
+      if (k < K) a.XT[0][(size_t)k * a.ldr + r0 + r] = v;
+    }
+  }
+  __syncthreads();
+  // four rows of column n to LDS and to the transposed operand
+  auto put = [&](int n, const float* v, u16* out) {
+    ushort4 q;
+    u16* qv = reinterpret_cast<u16*>(&q);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      qv[u] = f2bf(v[u]);
+      nxt[(row0 + u) * a.lda + n] = qv[u];
+    }
+    *reinterpret_cast<ushort4*>(out + (size_t)n * a.ldr + r0 + row0) = q;
+  };
+  float v[4];
+  for (int l = 0; l + 1 < L; ++l) {
+    const int n = tile(a.w[l + 1]) + (lane & 31);
+    const f32x16 acc = reg_product(cur, a.lda, w, upd(a.w[l], 16), fwd(l + 1), upd(a.w[l + 1], 16));
+    const float b0 = bn;
+    bn = bias(l + 1);
+    float4 z;
+    float* zp = reinterpret_cast<float*>(&z);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      zp[u] = acc[u] + b0;
+      const float g = gelu(zp[u]);
+      v[u] = n < a.w[l + 1] && r0 + row0 + u < nb ? g : 0.0f;
+    }
+    zs[l * 512 + tid] = z;
+    put(n, v, a.XT[l + 1]);
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+  {
+    const int l = L - 1;
+    const f32x16 acc = reg_product(cur, a.lda, w, upd(a.w[l], 16), bwd(l), upd(no, 16));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = r0 + row0 + u;
+      const bool in = ny < no && r < nb;
+      const float c = acc[u] + bn;
+      if (in) a.Y[(size_t)r * no + ny] = c;
+      v[u] = in ? 2.0f * (c - t[u]) * scale : 0.0f;
+    }
+    put(ny, v, a.DT[l]);
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+  // dz_{l-1} = (dz_l W_l) * GELU'(z_{l-1}); z was kept by this very lane
+  for (int l = L - 1; l > 0; --l) {
+    const int k = tile(a.w[l]) + (lane & 31), ln = max(l - 1, 1);
+    const f32x16 acc = reg_product(cur, a.lda, w, upd(a.w[l + 1], 16), bwd(ln), upd(a.w[ln + 1], 16));
+    const float4 z = zs[(l - 1) * 512 + tid];
+    const float* zp = reinterpret_cast<const float*>(&z);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float g = acc[u] * gelu_d(zp[u]);
+      v[u] = k < a.w[l] && r0 + row0 + u < nb ? g : 0.0f;
+    }
+    put(k, v, a.DT[l - 1]);
+    __syncthreads();
+    u16* x = cur; cur = nxt; nxt = x;
+  }
+}
+
+// ... and for wider ones, several tiles per wave and layer, pre-activations in Z
 __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, const float* Xin,
                                               const float* Tin, float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 sm[];
   u16 *cur = sm, *nxt = sm + RT * a.lda;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   const int r0 = blockIdx.x * RB, L = a.L;
-  // products in order: forward through the layers, back from the last to the second
-  WReg wr, wn;
-  auto fetch = [&](int p, WReg& w) {
-    if (!REG || p > 2 * L - 2) return;
-    const bool f = p < L;
-    const int l = f ? p : 2 * L - 1 - p;
-    const int cols = upd(f ? a.w[l + 1] : a.w[l], 32), depth = upd(f ? a.w[l] : a.w[l + 1], 16);
-    if (32 * wave < cols) load_tile(w, f ? a.Wp[l] : a.Wt[l], depth, 32 * wave);
-  };
-  fetch(0, wr);
   {
     const int K = a.w[0], Kp = upd(K, 16);
     for (int i = tid; i < RB * Kp; i += blockDim.x) {
@@ -340,7 +437,6 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
     const int K = a.w[l], N = a.w[l + 1], Kp = upd(K, 16), Np = upd(N, 32);
     const bool last = l + 1 == L;
     const float* bias = a.P + a.boff[l];
-    if (REG && 32 * wave >= Np) fetch(l + 1, wn);
     for (int n0 = 32 * wave; n0 < Np; n0 += 32 * nw) {
       const int n = n0 + (lane & 31);
       const bool col = n < N;
@@ -350,9 +446,7 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
 #pragma unroll
         for (int u = 0; u < 4; ++u)
           if (r0 + row0 + u < nb) t[u] = Tin[(size_t)rows[u] * N + n];
-      fetch(l + 1, wn);  // after this product's own loads: waits are in order
-      if (REG) reg_product(cur, a.lda, wr, Kp, acc[0]);
-      else tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
+      tile_product<1>(cur, a.lda, a.Wp[l], Kp, n0, acc);
       ushort4 q;
       u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
@@ -375,14 +469,12 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
       }
       if (col) *reinterpret_cast<ushort4*>((last ? a.DT[l] : a.XT[l + 1]) + (size_t)n * a.ldr + r0 + row0) = q;
     }
-    if (REG) wr = wn;
     __syncthreads();
     u16* x = cur; cur = nxt; nxt = x;
   }
   // dz_{l-1} = (dz_l W_l) * GELU'(z_{l-1}); z was stored by this very lane
   for (int l = L - 1; l > 0; --l) {
     const int K = a.w[l], N = a.w[l + 1], Np = upd(N, 16), Kp = upd(K, 32);
-    if (REG && 32 * wave >= Kp) fetch(2 * L - l, wn);
     for (int k0 = 32 * wave; k0 < Kp; k0 += 32 * nw) {
       const int k = k0 + (lane & 31);
       const bool col = k < K;
@@ -392,9 +484,7 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
         const int r = r0 + row0 + u;
         z[u] = col && r < nb ? a.Z[l - 1][(size_t)r * K + k] : 0.0f;
       }
-      fetch(2 * L - l, wn);
-      if (REG) reg_product(cur, a.lda, wr, Np, acc[0]);
-      else tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
+      tile_product<1>(cur, a.lda, a.Wt[l], Np, k0, acc);
       ushort4 q;
       u16* qv = reinterpret_cast<u16*>(&q);
 #pragma unroll
@@ -405,7 +495,6 @@ __global__ __launch_bounds__(512) void k_rows(Net a, int nb, const int* idx, con
       }
       if (col) *reinterpret_cast<ushort4*>(a.DT[l - 1] + (size_t)k * a.ldr + r0 + row0) = q;
     }
-    if (REG) wr = wn;
     __syncthreads();
     u16* x = cur; cur = nxt; nxt = x;
   }
@@ -727,14 +816,15 @@ void minibatch(tsm_mlp* m, int nb, const int* idx, const float* X, const float* 
   // one a page apart would put every feature into the same cache sets)
   Net net = m->net;
   net.ldr = up(nb, RT);
-  auto rows = [&](auto k) {
+  auto rows = [&](auto k, size_t lds) {
     if (lds > 48 * 1024)
       (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // every row k_update reads (16 a product) is written, zero past the last
     hipLaunchKernelGGL(k, dim3(up(nb, 16) / RB), dim3(512), lds, m->st, net, nb, idx, X, T,
                        1.0f / (float)n);
   };
-  if (net.lda <= 256 + 8) rows(k_rows<true>); else rows(k_rows<false>);
+  if (net.lda <= 256 + 8) rows(k_rows_reg, lds + (size_t)(net.L - 1) * 512 * sizeof(float4));
+  else rows(k_rows, lds);
   const int jobs = m->n_jobs + (n + 255) / 256;
   if (h)
     hipLaunchKernelGGL((k_update<true>), dim3((jobs + 3) / 4), dim3(256), 0, m->st, net, nb, m->jobs,
@@ -864,8 +954,8 @@ extern "C" int tsm_mlp_create(int n_layers, const int* widths, int max_batch,
       const int ni = m->w[l], n1 = m->w[l + 1];
       want(&N.Wp[l], (size_t)up(n1, 32) * up(ni, 16));
       want(&N.Wt[l], (size_t)up(ni, 32) * up(n1, 16));
-      want(&N.XT[l], (size_t)ni * N.ldr);
-      want(&N.DT[l], (size_t)n1 * N.ldr);
+      want(&N.XT[l], (size_t)up(ni, 32) * N.ldr);
+      want(&N.DT[l], (size_t)up(n1, 32) * N.ldr);
       N.woff[l] = (int)m->woff[l];
       N.boff[l] = (int)m->boff[l];
       for (int n = 0; n < n1; n += 32)

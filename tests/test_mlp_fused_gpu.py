@@ -77,3 +77,18 @@ def test_standardised_evaluation_is_the_plain_one(widths, n):
     c, d = rng.standard_normal(widths[-1]), 0.5 + rng.random(widths[-1])
     want = net((u - a) / b).astype(np.float64) * d + c
     assert np.array_equal(net.affine(u, a, b, c, d), want)
+
+
+@pytest.mark.parametrize("width", [256, 257])
+def test_deepest_net(width):
+    """Sixteen layers, the most a net may have, on both sides of the width up to
+    which pre-activations stay on chip: the minibatch kernel's loss is that of the
+    evaluation (the same bits; 60 squares added in FP32, 60 eps = 4e-6)."""
+    widths = [4] + [width] * 15 + [3]
+    print(widths, flush=True)
+    net = MLP(widths, max_batch=32, seed=5)
+    x, t = _data(widths, 20, 2)
+    loss, grad = net.gradient(x, t)
+    assert np.all(np.isfinite(grad)) and np.any(grad != 0.0)
+    want = np.mean((net(x).astype(np.float64) - t) ** 2)
+    np.testing.assert_allclose(loss, want, rtol=2e-5, atol=0)
