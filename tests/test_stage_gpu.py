@@ -1,5 +1,5 @@
 """The stage kernel at the edges of its tables, against the oracle: vertices
-with more neighbours than the eight and sixteen packed items hold, vertices
+with more neighbours than the first chain's eight and a group's seven, vertices
 whose two halo rings do not fit LDS at the wanted tile size (smaller tiles are
 taken), boundary terms beside them, every tile size from the smallest to the
 largest, and runs cut into several calls (the entropy variable kept beside the
