@@ -324,6 +324,10 @@ int tsm_pert(int type, double x, double y, double p, const double* rnd, int n_rn
    sqrt() on the same operands: out[4i..4i+3] = fdiv(a_i, b_i), a_i / b_i,
    fsqrt(a_i), sqrt(a_i). */
 int tsm_check_arith(long n, const double* a, const double* b, double* out);
+/* ... and the functions of about an ulp beside them: out[6i..6i+5] = 1/a_i,
+   1/sqrt(a_i), sqrt(a_i), log(a_i), the library's log(a_i), and the sum of the
+   two minmod slopes minmod(a_i, b_i) + minmod(b_i, b_i) as the TeCNO flux forms it. */
+int tsm_check_math(long n, const double* a, const double* b, double* out);
 
 /* Geometry export in reference order, for parity checks. */
 int tsm_geometry_sizes(tsm_ctx* ctx, int* n_face, int* n_bface);

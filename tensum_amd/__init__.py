@@ -221,6 +221,7 @@ def lib():
         L.tsm_probe_density.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 3
         L.tsm_probe_density_noalloc.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 3
         L.tsm_check_arith.argtypes = [C.c_long] + [C.c_void_p] * 3
+        L.tsm_check_math.argtypes = [C.c_long] + [C.c_void_p] * 3
         L.tsm_enstrophy.argtypes = [C.c_void_p, C.c_int, C.c_void_p]
         L.tsm_global_all.argtypes = [C.c_void_p] + [C.c_void_p] * 2
         L.tsm_mesh_jittered_sizes.argtypes = [C.c_int, C.c_int] + [C.POINTER(C.c_int)] * 5
@@ -344,6 +345,17 @@ def check_arith(a, b):
     b = np.ascontiguousarray(b, dtype=np.float64)
     out = np.empty((a.size, 4))
     _check(lib().tsm_check_arith(a.size, _dptr(a), _dptr(b), _dptr(out)))
+    return out
+
+
+def check_math(a, b):
+    """The kernels' functions of about an ulp: (n, 6) array of 1/a, 1/sqrt(a),
+    sqrt(a), log(a), the device library's log(a), and minmod(a, b) + minmod(b, b)
+    as the TeCNO flux forms it."""
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    b = np.ascontiguousarray(b, dtype=np.float64)
+    out = np.empty((a.size, 6))
+    _check(lib().tsm_check_math(a.size, _dptr(a), _dptr(b), _dptr(out)))
     return out
 
 

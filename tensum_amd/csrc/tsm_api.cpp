@@ -1640,23 +1640,34 @@ extern "C" int tsm_probe_density_noalloc(tsm_ctx* c, int np, const double* px, c
   return TSM_OK;
 }
 
-extern "C" int tsm_check_arith(long n, const double* a, const double* b, double* out) {
+namespace {
+// launch(n, a, b, out, stream) over the operands, m results each
+template <class F>
+int check_operands(long n, const double* a, const double* b, double* out, int m, F&& launch) {
   if (n < 1 || !a || !b || !out) return fail(TSM_E_ARG, "bad argument");
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail(TSM_E_HIP, "no HIP device visible");
   double* d = nullptr;
-  HIP_TRY(hipMalloc(&d, 6 * (size_t)n * sizeof(double)));
+  HIP_TRY(hipMalloc(&d, (size_t)(2 + m) * n * sizeof(double)));
   hipError_t e = hipMemcpy(d, a, 8 * (size_t)n, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(d + n, b, 8 * (size_t)n, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    tsm::launch_check_arith(n, d, d + n, d + 2 * n, nullptr);
+    launch(n, d, d + n, d + 2 * n, nullptr);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipDeviceSynchronize();
-  if (e == hipSuccess) e = hipMemcpy(out, d + 2 * n, 32 * (size_t)n, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(out, d + 2 * n, 8 * (size_t)m * n, hipMemcpyDeviceToHost);
   (void)hipFree(d);
   if (e != hipSuccess) return fail(TSM_E_HIP, hipGetErrorString(e));
   return TSM_OK;
+}
+}  // namespace
+
+extern "C" int tsm_check_arith(long n, const double* a, const double* b, double* out) {
+  return check_operands(n, a, b, out, 4, tsm::launch_check_arith);
+}
+extern "C" int tsm_check_math(long n, const double* a, const double* b, double* out) {
+  return check_operands(n, a, b, out, 6, tsm::launch_check_math);
 }
 
 extern "C" int tsm_global_all(tsm_ctx* c, double* ke, double* ent) {

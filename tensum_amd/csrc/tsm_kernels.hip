@@ -1265,6 +1265,21 @@ void launch_check_arith(long n, const double* a, const double* b, double* out, h
   hipLaunchKernelGGL(k_check_arith, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, a, b, out);
 }
 
+__global__ void k_check_math(long n, const double* a, const double* b, double* out) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double x = a[i], y = b[i];
+  out[6 * i] = frcp(x);
+  out[6 * i + 1] = frsq(x);
+  out[6 * i + 2] = fsqrt3(x);
+  out[6 * i + 3] = flog(x);
+  out[6 * i + 4] = log(x);
+  out[6 * i + 5] = minmod_sum(x, y, y);
+}
+void launch_check_math(long n, const double* a, const double* b, double* out, hipStream_t st) {
+  hipLaunchKernelGGL(k_check_math, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, a, b, out);
+}
+
 void launch_probes(const StageArgs& A, int nv, int np, const int* pc, const double* pw, int S,
                    double* out, hipStream_t st) {
   hipLaunchKernelGGL(k_probes, dim3((np * S + 255) / 256), dim3(256), 0, st, A, nv, np, pc, pw, S, out);

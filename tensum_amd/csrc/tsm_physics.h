@@ -226,6 +226,11 @@ __device__ __forceinline__ double minmod_tvd(double a, double b) {
   if (a > 0.0 && b > 0.0) return fmin(a, b);
   return 0.0;
 }
+// minmod(dl, dz) + minmod(dr, dz): each slope clamped to the interval between 0 and dz
+__device__ __forceinline__ double minmod_sum(double dl, double dr, double dz) {
+  const double lo = fmin(dz, 0.0), hi = fmax(dz, 0.0);
+  return fmax(lo, fmin(hi, dl)) + fmax(lo, fmin(hi, dr));
+}
 __device__ __forceinline__ double minabs(double a, double b) {
   return (fabs(a) < fabs(b)) ? a : b;
 }
@@ -565,10 +570,7 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - ((dl + dr) * (1.0 - K) + (2.0 * dz[i]) * (1.0 + K)) * 0.25;
       } else if (REC == R_MINMOD) {
-        // minmod(d, dz) is d clamped to the interval between 0 and dz
-        const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
-        const double lo = fmin(dz[i], 0.0), hi = fmax(dz[i], 0.0);
-        dZi = dz[i] - 0.5 * (fmax(lo, fmin(hi, dl)) + fmax(lo, fmin(hi, dr)));
+        dZi = dz[i] - 0.5 * minmod_sum(2.0 * gl[i] - dz[i], 2.0 * gr[i] - dz[i], dz[i]);
       } else {
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - limited_slope<REC>(dl, dz[i], 0.0, 0.0) - limited_slope<REC>(dr, dz[i], 0.0, 0.0);
