@@ -226,10 +226,13 @@ __device__ __forceinline__ double minmod_tvd(double a, double b) {
   if (a > 0.0 && b > 0.0) return fmin(a, b);
   return 0.0;
 }
-// minmod(dl, dz) + minmod(dr, dz): each slope clamped to the interval between 0 and dz
+// minmod(dl, dz) + minmod(dr, dz), each the slope clamped to the interval between 0
+// and dz, without branches: both taken with dz's sign, clamped to [0, |dz|] from
+// below first, so that a NaN slope becomes the zero that the branches give (clamped
+// from above first it would become the full jump), and the sign put back.
 __device__ __forceinline__ double minmod_sum(double dl, double dr, double dz) {
-  const double lo = fmin(dz, 0.0), hi = fmax(dz, 0.0);
-  return fmax(lo, fmin(hi, dl)) + fmax(lo, fmin(hi, dr));
+  const double s = copysign(1.0, dz), m = fabs(dz);
+  return s * (fmin(fmax(s * dl, 0.0), m) + fmin(fmax(s * dr, 0.0), m));
 }
 __device__ __forceinline__ double minabs(double a, double b) {
   return (fabs(a) < fabs(b)) ? a : b;
