@@ -738,7 +738,9 @@ extern "C" int tsm_set_state(tsm_ctx* c, int s, const double* prim) {
   tsm::launch_state_put(nv, c->d_perm, in, c->bad, c->W[c->cur] + 4 * off,
                         c->A.W_keep ? c->A.W_keep + 4 * off : nullptr, c->A.ctl + s, c->st);
   tsm::launch_words(sizeof(int), c->bad, bad, c->st);
-  if (!c->tiled) tsm::launch_prim2ent(c->G, c->A, s, c->st);
+  // a refused state leaves these too: under bc_scheme strong they are not those of
+  // the state (the boundary values imposed on it come after them)
+  if (!c->tiled) tsm::launch_prim2ent(c->G, c->A, s, c->st, c->bad);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(c->st));
   const int i = *bad;

@@ -407,7 +407,8 @@ void launch_dt(const DevGeo& G, const StageArgs& A, const StepParams& P, int S, 
 void launch_step_final(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                        int log_slot, hipStream_t st);
 void launch_ssw(const DevGeo& G, const StageArgs& A, int S, hipStream_t st);
-void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st);
+void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st,
+                     const int* bad = nullptr);
 void launch_state_put(int nv, const int* perm, const double* in, int* bad, double* W, double* keep,
                       Ctl* ctl, hipStream_t st);
 void launch_state_get(int nv, const int* perm, const double* W, double* out, hipStream_t st);

@@ -909,7 +909,9 @@ __global__ __launch_bounds__(256) void k_ssw(DevGeo G, StageArgs A) {
 }
 
 // Entropy variables of a freshly set state
-__global__ void k_prim2ent(DevGeo G, StageArgs A, int s) {
+// bad: where a state was refused (not INT_MAX) its sample's variables stay as they are
+__global__ void k_prim2ent(DevGeo G, StageArgs A, int s, const int* bad) {
+  if (bad && *bad != INT_MAX) return;
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= G.nv) return;
   const size_t off = (size_t)s * G.nv;
@@ -1131,8 +1133,8 @@ void launch_ssw(const DevGeo& G, const StageArgs& A, int S, hipStream_t st) {
   hipLaunchKernelGGL(k_ssw_zero, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, G, A);
   hipLaunchKernelGGL(k_ssw, dim3((G.nf + 255) / 256, S), dim3(256), 0, st, G, A);
 }
-void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st) {
-  hipLaunchKernelGGL(k_prim2ent, dim3((G.nv + 255) / 256), dim3(256), 0, st, G, A, s);
+void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st, const int* bad) {
+  hipLaunchKernelGGL(k_prim2ent, dim3((G.nv + 255) / 256), dim3(256), 0, st, G, A, s, bad);
 }
 // Enstrophy partials, 1/2 omega^2 dcarea w per vertex summed per block, with
 // omega = R T (dE[vy].x + v dE[l].x - dE[vx].y - u dE[l].y) from the sample's
