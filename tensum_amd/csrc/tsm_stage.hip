@@ -8,8 +8,9 @@
 // periodic set sums, viscous terms, boundary fluxes and the update.  The last
 // stage also forms the residual-norm partials (src/fv.cc:1801-1879) and the
 // next step's local time step (src/fv.cc:1499-1621) from the new state, so a
-// step needs no separate time-step pass.  No atomics on floating-point values;
-// every sum has one order, whatever the tile size.
+// step needs no separate time-step pass.  No atomics on floating-point values.
+// Every sum that a state depends on has one order, whatever the tile size; the
+// residual norm is a sum over tiles and has one order for each number of tiles.
 //
 // What bounds it: at 1025^2 (KEPES-TeCNO Rusanov, minmod) a stage's FP64
 // issue (0.60 of the rate), LDS (0.36) and HBM traffic (2.8 of 4.9 TB/s) are within
@@ -405,19 +406,24 @@ __device__ __forceinline__ double wave_min(double x) {  // of values up to 1e20
   return wave_fold(x, 1.0e20, [](double a, double b) { return fmin(a, b); });
 }
 
-// The end of a step by one wave, from the partials of nblk blocks of this very
-// launch: they were written through to memory before their blocks counted
-// themselves in, and are read past the caches.
+// The end of a step by one wave, from the partials of nblk blocks: lane i takes
+// those of blocks i, i + 64, ... in that order, then the wave's tree.  Every mesh of
+// up to FOLD_TILES tiles ends its steps so, in the last stage or in a launch of its
+// own: which of the two it is depends on the samples beside this one, its norm does
+// not.  LAUNCH: in the last stage's own launch, where the partials were written
+// through to memory before their blocks counted themselves in and are read past the
+// caches.
 __device__ __forceinline__ double agent_load(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void agent_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams& P, int nblk, int nv,
-                                           const double* dtpart, int log_slot, int s) {
+template <bool LAUNCH>
+__device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams& P, const Ctl& c, int nblk,
+                                           int nv, const double* dtpart, int log_slot, int s) {
   const int lane = threadIdx.x & 63;
-  const Ctl c = A.ctl[s];
+  auto load = [](const double* p) { return LAUNCH ? agent_load(p) : *p; };
   const double* q = A.partial + (size_t)s * nblk * 4;
   const double* dq = dtpart + (size_t)s * nblk;
   double part[4] = {0, 0, 0, 0}, x = 1.0e20;
@@ -427,8 +433,8 @@ __device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams&
     for (int u = 0; u < 8; ++u) {
       const int i = i0 + 64 * u + lane;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) a[u][k] = i < nblk ? agent_load(q + 4 * (size_t)i + k) : 0.0;
-      a[u][4] = i < nblk ? agent_load(dq + i) : 1.0e20;
+      for (int k = 0; k < 4; ++k) a[u][k] = i < nblk ? load(q + 4 * (size_t)i + k) : 0.0;
+      a[u][4] = i < nblk ? load(dq + i) : 1.0e20;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -488,7 +494,7 @@ __device__ __forceinline__ void block_partials(const StageArgs& A, const StepPar
   }
   if (!__builtin_amdgcn_readlane(ends, 63)) return;
   asm volatile("" ::: "memory");
-  final_wave(A, P, nt, nv, dtpart, log_slot, s);
+  final_wave<true>(A, P, A.ctl[s], nt, nv, dtpart, log_slot, s);
   if ((threadIdx.x & 63) == 0)
     __hip_atomic_store(A.arrive + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1058,9 +1064,17 @@ __global__ __launch_bounds__(512, 4) void k_stage_packed(const PackLevel* __rest
 }
 
 // ---------------------------------------------------------------------------
-// end of a step of meshes with more tiles than the stage kernel folds
+// end of a step of contexts with more tiles than the stage kernel folds
 // ---------------------------------------------------------------------------
 namespace {
+// The last stage ends the steps of a context with up to this many tiles over all its
+// samples, which run at once: eight partials a lane of the wave that does it.  A step
+// of the vortex (Roe, minmod) against a launch of its own: 129^2 (150 tiles) 37.7 us
+// against 41.8, 200^2 43.0 / 45.7, 257^2 (541) 53.9 / 54.3, 350^2 63.2 / 62.7.  Where
+// tiles queue for a CU each is held up by the wait for its partials: 32 samples of
+// 257^2 took 1.15 times as long.
+constexpr int FOLD_TILES = 512;
+
 template <int NV>
 __device__ __forceinline__ void bsum(double* v, double* red) {
 #pragma unroll
@@ -1098,6 +1112,10 @@ __device__ __forceinline__ void step_final_body(const StageArgs& A, const StepPa
   __shared__ double red[64];
   const Ctl c = A.ctl[s];
   if (c.done) return;
+  if (nblk <= FOLD_TILES) {
+    if (threadIdx.x < 64) final_wave<false>(A, P, c, nblk, nv, dtpart, log_slot, s);
+    return;
+  }
   double part[4] = {0, 0, 0, 0};
   double x = 1.0e20;
   const double4* q4 = reinterpret_cast<const double4*>(A.partial) + (size_t)s * nblk;
@@ -1137,14 +1155,6 @@ __global__ __launch_bounds__(1024) void k_step_final_packed(const PackLevel* __r
   const PackLevel& L = pk[l];
   step_final_body(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
 }
-
-// The last stage ends the steps of a context with up to this many tiles over all its
-// samples, which run at once: eight partials a lane of the wave that does it.  A step
-// of the vortex (Roe, minmod) against a launch of its own: 129^2 (150 tiles) 37.7 us
-// against 41.8, 200^2 43.0 / 45.7, 257^2 (541) 53.9 / 54.3, 350^2 63.2 / 62.7.  Where
-// tiles queue for a CU each is held up by the wait for its partials: 32 samples of
-// 257^2 took 1.15 times as long.
-constexpr long FOLD_TILES = 512;
 
 // ---------------------------------------------------------------------------
 // launchers
@@ -1245,8 +1255,8 @@ void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const S
 void launch_step_final_tiled(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                              int nblk, const double* dtpart, int log_slot, hipStream_t st) {
   if (A.arrive) return;  // ended by the last stage
-  hipLaunchKernelGGL(k_step_final_tiled, dim3(S), dim3(1024), 0, st, A, P, nblk, G.nv, dtpart,
-                     log_slot);
+  hipLaunchKernelGGL(k_step_final_tiled, dim3(S), dim3(nblk <= FOLD_TILES ? 64 : 1024), 0, st, A, P,
+                     nblk, G.nv, dtpart, log_slot);
 }
 
 // ---------------------------------------------------------------------------
