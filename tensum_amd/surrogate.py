@@ -105,15 +105,19 @@ class MLP:
         return y
 
     def affine(self, u, mu_x, sd_x, mu_y, sd_y):
-        """net((u - mu_x) / sd_x) * sd_y + mu_y in FP64 around the network."""
-        f64 = lambda a: np.ascontiguousarray(a, dtype=np.float64)
+        """net((u - mu_x) / sd_x) * sd_y + mu_y in FP64 around the network.  Rows as
+        the broadcasts give them: a vector is n rows of a one-input network."""
         n_in, n_out = self.widths[0], self.widths[-1]
         u = np.asarray(u, dtype=np.float64)
-        if u.ndim != 2 or u.shape[1] not in (1, n_in):
+        shape = np.broadcast_shapes(u.shape, (n_in,))
+        if np.prod(shape) != shape[0] * n_in:
             raise ValueError(f"inputs of shape {u.shape}, expected (n, {n_in})")
-        u = f64(np.broadcast_to(u, (u.shape[0], n_in)))
-        a = [np.ascontiguousarray(np.broadcast_to(f64(v), (k,)))
-             for v, k in ((mu_x, n_in), (sd_x, n_in), (mu_y, n_out), (sd_y, n_out))]
+        u = np.ascontiguousarray(np.broadcast_to(u, shape)).reshape(shape[0], n_in)
+        try:
+            a = [np.ascontiguousarray(np.broadcast_to(np.asarray(v, np.float64), (1, k)))
+                 for v, k in ((mu_x, n_in), (sd_x, n_in), (mu_y, n_out), (sd_y, n_out))]
+        except ValueError:  # not one of each per column: row by row on the host
+            return self((u - mu_x) / sd_x).astype(np.float64) * sd_y + mu_y
         y = np.empty((u.shape[0], n_out))
         _chk(_mlib().tsm_mlp_forward_affine(self._h, u.shape[0], _p(u), *[_p(v) for v in a], _p(y)))
         return y
