@@ -68,9 +68,9 @@ typedef struct tsm_params {
      the CSR-gather kernels.  Both give the reference's summation order. */
   int kernel_path;
   int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128, or 112 with viscous
-                         terms and gradients);
-                         smaller ones are taken where two halo rings of a tile do
-                         not fit LDS */
+                         terms and gradients); where a tile's slots, faces or two halo
+                         rings in LDS exceed the kernel's limits half as many are tried,
+                         down to 16, then the CSR-gather kernels run (tsm_tile_vertices) */
   int block_grad;     /* checked against the block limits; the stage kernel forms
                          the gradients itself, so no kernel of its own reads it */
   int block_fu;       /* threads per tile of the stage kernel (0: auto) */
@@ -119,6 +119,8 @@ const char* tsm_last_error(void);
 int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_samples,
                tsm_ctx** out);
 void tsm_destroy(tsm_ctx* ctx);
+/* owned vertices per tile in use, 0 with the CSR-gather kernels */
+int tsm_tile_vertices(const tsm_ctx* ctx);
 
 /* Per-sample gamma / gas constant (batched Monte Carlo over material constants;
    the reference can vary only IC/BC expressions per sample, src/perturb.cc). */

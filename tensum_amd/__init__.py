@@ -184,6 +184,7 @@ def lib():
         L.tsm_last_error.restype = C.c_char_p
         L.tsm_create.argtypes = [C.POINTER(TsmMesh), C.POINTER(TsmParams), C.c_int,
                                  C.POINTER(C.c_void_p)]
+        L.tsm_tile_vertices.argtypes = [C.c_void_p]
         L.tsm_destroy.argtypes = [C.c_void_p]
         L.tsm_destroy.restype = None
         for name in ("tsm_set_state", "tsm_get_state", "tsm_residual", "tsm_gradients"):
@@ -465,6 +466,7 @@ class Solver:
         h = C.c_void_p()
         _check(L.tsm_create(C.byref(m), C.byref(self._p), n_samples, C.byref(h)))
         self._h = h
+        self.tile_vertices = int(L.tsm_tile_vertices(h))  # in use; 0: CSR-gather kernels
         self.nv = mesh.n_vertex
         self.n_bface = int(mesh.bface_tag.size)
         self._bface_tag = np.asarray(mesh.bface_tag, dtype=np.int32)

@@ -167,7 +167,7 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
       T.g1ptr.push_back((int)T.g1ent.size());
       T.g1beg.push_back((int)T.g1ptr.size());
     }
-    if ((int)slots.size() > 1023) { msg = "tile exceeds 1023 slots"; return false; }
+    if ((int)slots.size() > 1023) { msg = "tile exceeds 1023 slots"; T.too_large = true; return false; }
     T.max_slots = std::max(T.max_slots, (int)slots.size());
     // local faces in reference order
     std::vector<int> lf;
@@ -175,7 +175,7 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
       for (int f : vfaces[v]) lf.push_back(f);
     std::sort(lf.begin(), lf.end());
     lf.erase(std::unique(lf.begin(), lf.end()), lf.end());
-    if (lf.size() >= (1u << 14)) { msg = "tile exceeds 16383 local faces"; return false; }
+    if (lf.size() >= (1u << 14)) { msg = "tile exceeds 16383 local faces"; T.too_large = true; return false; }
     T.max_faces = std::max(T.max_faces, (int)lf.size());
     std::unordered_map<int, int> lfi;
     for (int k = 0; k < (int)lf.size(); ++k) {

@@ -184,8 +184,9 @@ int validate_params(const tsm_params& p) {
 
 namespace {
 // One attempt at a context, with tiles of tb owned vertices (0: the CSR-gather
-// kernels).  1: the tiles do not fit the stage kernel.
-int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int tb,
+// kernels; -1: the size of params, to which tb is set).  1: a tile holds more slots
+// or faces than the tables address or the stage kernel has LDS or threads for.
+int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int& tb,
                       tsm_ctx** out);
 }  // namespace
 
@@ -199,25 +200,33 @@ extern "C" int tsm_create(const tsm_mesh* mesh, const tsm_params* params, int n_
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
     return fail(TSM_E_HIP, "no HIP device visible");
   // tiled stage kernels: every scheme, Euler or Navier-Stokes, with or without
-  // the Liou fix; strong boundary conditions keep the CSR kernels.  A mesh whose
-  // two halo rings do not fit LDS at the wanted tile size (vertices with
-  // hundreds of cells) takes smaller tiles, and the CSR kernels if none fits.
-  if (params->kernel_path != 0 || params->strong_bc)
-    return create_with_tiles(mesh, params, n_samples, 0, out);
-  // 128 vertices, or 112 where viscous cells share LDS with gradients: 50 KB then,
-  // three tiles per CU instead of two (57 KB).  A no-slip channel with KEPES-TeCNO
-  // Roe and minmod, per step: 257^2 68 us against 86, 400^2 119 against 142, 640^2
-  // 234 against 281; 96 vertices 69, 140, 269.  Euler at 513^2: 128 110 us, 112 112.
-  const bool narrow = params->model == 1 && tsm::stage_has_gradients(params->flux, params->reconstruct);
-  const int want = params->tile_vertices > 0 ? params->tile_vertices : narrow ? 112 : 128;
-  for (int tb = want;; tb /= 2) {
-    rc = create_with_tiles(mesh, params, n_samples, tb < 16 && tb < want ? 0 : tb, out);
-    if (rc != 1) return rc;
+  // the Liou fix; strong boundary conditions keep the CSR kernels.  A mesh with
+  // vertices of so many cells that a tile of the wanted size is too large takes
+  // smaller tiles, and the CSR kernels if none fits.
+  if (params->kernel_path == 0 && !params->strong_bc) {
+    if (params->block_fu > tsm::stage_block_max() || params->block_grad > 512)
+      return fail(TSM_E_ARG, "tiled kernels: block size out of range");
+    int want = -1;
+    if ((rc = create_with_tiles(mesh, params, n_samples, want, out)) != 1) return rc;
+    for (int tb = want / 2; tb >= 16; tb /= 2)
+      if ((rc = create_with_tiles(mesh, params, n_samples, tb, out)) != 1) return rc;
   }
+  int csr = 0;
+  return create_with_tiles(mesh, params, n_samples, csr, out);
 }
 
 namespace {
-int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int tb,
+// Owned vertices per tile where the caller leaves it open: 128, or 112 where viscous
+// cells share LDS with gradients: 50 KB then, three tiles per CU instead of two (57
+// KB).  A no-slip channel with KEPES-TeCNO Roe and minmod, per step: 257^2 68 us
+// against 86, 400^2 119 against 142, 640^2 234 against 281; 96 vertices 69, 140, 269.
+// Euler at 513^2: 128 110 us, 112 112.  A quarter of it has to hold a periodic set.
+int default_tile(const tsm_params& p, size_t largest_set) {
+  if (p.tile_vertices > 0) return p.tile_vertices;
+  return p.model == 1 && tsm::stage_has_gradients(p.flux, p.reconstruct) && largest_set <= 112 / 4 ? 112 : 128;
+}
+
+int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samples, int& tb,
                       tsm_ctx** out) {
   int rc = TSM_OK;
   tsm_ctx* c = new tsm_ctx();
@@ -243,6 +252,14 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     return fail(TSM_E_MESH, "mesh too large for 30-bit face ids");
   }
   // ---- path and vertex numbering -----------------------------------------
+  size_t largest_set = 0;
+  for (const auto& P : g.periodic) largest_set = std::max(largest_set, P.size());
+  if (tb < 0) {
+    tb = default_tile(*params, largest_set);
+  } else if (tb > 0 && largest_set > (size_t)std::max(4, tb / 4)) {
+    delete c;  // a smaller tile than the wanted one that no longer holds a periodic set
+    return 1;
+  }
   c->tiled = tb > 0;
   std::vector<int> perm(nv), inv(nv);
   tsm::TileGeo dev_tg{};   // device-built tile arrays (dev_tiles)
@@ -267,12 +284,14 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
       };
       trc = tsm::build_tiles_device(g, tb, false, c->tiling, dev_tg, dalloc, msg);
       if (trc < 0) { delete c; return fail(trc, "tiling: " + msg); }
+      if (trc == 2) { delete c; return 1; }
     }
     dev_tiles = trc == 0;
     if (!dev_tiles &&
         (!tsm::build_tiles(g, tb, c->tiling, msg, false) || !tsm::validate_tiles(g, c->tiling, msg))) {
+      const bool smaller = c->tiling.too_large;
       delete c;
-      return fail(TSM_E_MESH, "tiling: " + msg);
+      return smaller ? 1 : fail(TSM_E_MESH, "tiling: " + msg);
     }
     perm = c->tiling.perm;
     inv = c->tiling.inv;
@@ -488,10 +507,14 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     tsm::StageTab probe{};
     probe.tb = T.tb; probe.mf = T.max_faces; probe.fu_block = TG.fu_block;
     const int bf = tsm::stage_block(probe);
-    if (bf > tsm::stage_block_max() || bf % 64 || bg > 512 || bg % 64) {
+    if (bf > tsm::stage_block_max()) {  // more faces than its threads take
       delete c;
-      return fail(TSM_E_ARG, "tiled kernels: block size or LDS out of range (blocks " +
-                                 std::to_string(bg) + "/" + std::to_string(bf) + ")");
+      return 1;
+    }
+    if (bf % 64 || bg > 512 || bg % 64) {
+      delete c;
+      return fail(TSM_E_ARG, "tiled kernels: block size out of range (blocks " + std::to_string(bg) + "/" +
+                                 std::to_string(bf) + ")");
     }
 #define UT(field, vec) do { if ((rc = c->upload(&TG.field, vec))) { delete c; return rc; } } while (0)
     if (dev_tiles) {
@@ -590,6 +613,8 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
 }  // namespace
 
 extern "C" void tsm_destroy(tsm_ctx* c) { delete c; }
+
+extern "C" int tsm_tile_vertices(const tsm_ctx* c) { return !c ? -1 : c->tiled ? c->ST.tb : 0; }
 
 namespace {
 // Gives every sample a block of boundary values of its own (they share one

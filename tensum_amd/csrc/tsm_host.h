@@ -76,6 +76,7 @@ struct Tiling {
   // owned, first ring (halo), second ring (halo2); the gradient slots are the
   // first n1 = n_own + first-ring slots.
   bool fused = false;
+  bool too_large = false;            // build_tiles refused: a tile exceeds the slot or face limit
   int max_slots1 = 0;                // largest n1
   std::vector<int> h2beg, halo2;     // second-ring slots
   std::vector<int> g1beg;            // ntiles+1: start of the tile's n1+1 entries in g1ptr
@@ -90,7 +91,7 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
 // the second halo ring: the arrays go straight into
 // device memory from `dalloc` (pointers in TG, with n_gbv); T receives the
 // numbering (perm, inv, vbeg) and the sizes.  0 = built, 1 = left to
-// build_tiles, TSM_E_* with msg.
+// build_tiles, 2 = a tile exceeds the slot or face limit (msg), TSM_E_* with msg.
 struct TileGeo;
 int build_tiles_device(const Geometry& g, int tb, bool ring2, Tiling& T, TileGeo& TG,
                        const std::function<int(void**, size_t)>& dalloc, std::string& msg);

@@ -507,8 +507,8 @@ int build_tiles_device(const Geometry& g, int tb, bool ring2, Tiling& T, TileGeo
   TT(hipMemcpyAsync(h_mx, mx.p, sizeof(h_mx), hipMemcpyDeviceToHost, st));
   TT(hipMemcpyAsync(&h_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
   TT(hipStreamSynchronize(st));
-  if (h_mx[0] > 1023 || (h_bad & 1)) { msg = "tile exceeds 1023 slots"; return TSM_E_MESH; }
-  if (h_mx[1] >= (1 << 14) || (h_bad & 2)) { msg = "tile exceeds 16383 local faces"; return TSM_E_MESH; }
+  if (h_mx[0] > 1023 || (h_bad & 1)) { msg = "tile exceeds 1023 slots"; return 2; }
+  if (h_mx[1] >= (1 << 14) || (h_bad & 2)) { msg = "tile exceeds 16383 local faces"; return 2; }
   const int n_gbv = h_small[3];
   int* d_gbv = nullptr;
   TA(d_gbv, n_gbv);
@@ -589,6 +589,7 @@ extern "C" int tsm_device_tiling_check(const tsm_mesh* mesh, int tile_vertices, 
   tsm::TileGeo TG{};
   const int rc = tsm::build_tiles_device(g, tile_vertices, false, D, TG, dalloc, msg);
   if (rc == 1) return TSM_E_ARG;
+  if (rc == 2) return TSM_E_MESH;
   if (rc != 0) return rc;
   int err = 0;
   long long total = 0;
