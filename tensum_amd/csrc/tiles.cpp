@@ -121,7 +121,6 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
   T.fbeg.assign(1, 0);
   T.bbeg.assign(1, 0);
   T.gptr.assign(nv + 1, 0);
-  T.cptr.assign(nv + 1, 0);
   T.tper.assign(nt, 0);
   T.pinfo.assign(nv, -1);
   std::vector<int> slot(nv, -1);
@@ -196,7 +195,7 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
     std::unordered_map<int, int> lbi;
     for (int k = 0; k < (int)lb.size(); ++k) { lbi[lb[k]] = k; T.tbf.push_back(lb[k]); }
     T.bbeg.push_back((int)T.tbf.size());
-    // gather entries and cell entries per owned vertex
+    // gather entries per owned vertex
     for (int v = b0; v < b1; ++v) {
       int oldv = T.inv[v];
       for (int f : vfaces[v]) {
@@ -206,18 +205,6 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
       }
       for (int b : vbf[v]) T.gent.push_back((uint16_t)(0x4000 | lbi[b]));
       T.gptr[v + 1] = (int)T.gent.size();
-      for (int c : vcells[v]) {
-        uint32_t a = slot[T.perm[g.cell[3 * (size_t)c]]], bb = slot[T.perm[g.cell[3 * (size_t)c + 1]]],
-                 d = slot[T.perm[g.cell[3 * (size_t)c + 2]]];
-        T.cent.push_back(a | (bb << 10) | (d << 20) | ((uint32_t)ccorr[c] << 30));
-        T.cgid.push_back(c);
-      }
-      T.cptr[v + 1] = (int)T.cent.size();
-      if (t >= T.n_periodic_tiles) {
-        bool corr = false;
-        for (int c : vcells[v]) corr = corr || ccorr[c];
-        if (corr) T.gbv.push_back(v);
-      }
     }
     // periodic sets of this tile: consecutive owned slots
     for (int v = b0; v < b1; ++v) {
@@ -272,13 +259,6 @@ bool validate_tiles(const Geometry& g, const Tiling& T, std::string& msg) {
           if (seen_bface) { msg = "gather face after a boundary face"; return false; }
         }
       }
-      for (int k = T.cptr[v]; k < T.cptr[v + 1]; ++k) {
-        const unsigned e = T.cent[k];
-        if ((int)(e & 1023) >= ns || (int)((e >> 10) & 1023) >= ns || (int)((e >> 20) & 1023) >= ns) {
-          msg = "cell slot"; return false;
-        }
-        if (T.cgid[k] < 0 || T.cgid[k] >= g.nc) { msg = "cell id"; return false; }
-      }
       if (T.pinfo[v] >= 0) {
         const int first = T.pinfo[v] >> 8, cnt = T.pinfo[v] & 255;
         if (!T.tper[t] || first + cnt > nown) { msg = "periodic slots"; return false; }
@@ -305,8 +285,6 @@ bool validate_tiles(const Geometry& g, const Tiling& T, std::string& msg) {
       }
     }
   }
-  for (int v : T.gbv)
-    if (v < 0 || v >= nv || v < T.vbeg[T.n_periodic_tiles]) { msg = "boundary gradient vertex"; return false; }
   if (T.fused && ((int)T.h2beg.size() != T.ntiles + 1 || (int)T.g1beg.size() != T.ntiles + 1)) {
     msg = "ring-2 tables"; return false;
   }

@@ -94,12 +94,21 @@ struct tsm_ctx {
   }
   template <class T>
   int alloc(T** p, size_t n) {
-    void* q = nullptr;
-    if (n == 0) n = 1;
-    hipError_t e = hipMalloc(&q, n * sizeof(T));
-    if (e != hipSuccess) return fail(TSM_E_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-    allocs.push_back(q);
-    *p = (T*)q;
+    // small arrays share an allocation: a context has some hundred
+    const size_t b = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+    if (b > shared_left) {
+      void* q = nullptr;
+      const bool own = b > SMALL;
+      hipError_t e = hipMalloc(&q, own ? b : SHARED);
+      if (e != hipSuccess) return fail(TSM_E_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+      allocs.push_back(q);
+      if (own) { *p = (T*)q; return TSM_OK; }
+      shared_at = (char*)q;
+      shared_left = SHARED;
+    }
+    *p = (T*)shared_at;
+    shared_at += b;
+    shared_left -= b;
     return TSM_OK;
   }
   template <class T>
@@ -111,6 +120,31 @@ struct tsm_ctx {
     *dst = d;
     return TSM_OK;
   }
+  // The same for the many arrays of a new context: small ones go in one copy, with
+  // which dst is set (each copy of its own costs some 15 us however small).
+  template <class Ptr, class T>
+  int upload_later(Ptr* dst, const std::vector<T>& src) {
+    static_assert(std::is_same<std::remove_const_t<std::remove_pointer_t<Ptr>>, T>::value, "types");
+    const size_t b = src.size() * sizeof(T);
+    if (b > SMALL) return upload((const T**)dst, src);
+    later.push_back({(const void**)dst, later_bytes.size()});
+    later_bytes.resize(later_bytes.size() + ((std::max<size_t>(b, 1) + 255) & ~(size_t)255));
+    if (b) std::memcpy(later_bytes.data() + later.back().second, src.data(), b);
+    return TSM_OK;
+  }
+  int upload_now() {
+    const char* d = nullptr;
+    if (int rc = upload(&d, later_bytes)) return rc;
+    for (const auto& q : later) *q.first = d + q.second;
+    later.clear();
+    later_bytes.clear();
+    return TSM_OK;
+  }
+  static constexpr size_t SMALL = 64 * 1024, SHARED = 1024 * 1024;
+  char* shared_at = nullptr;
+  size_t shared_left = 0;
+  std::vector<std::pair<const void**, size_t>> later;
+  std::vector<char> later_bytes;
   // the samples' control blocks on the host
   hipError_t read_ctl(std::vector<tsm::Ctl>& q) {
     const size_t n = S * sizeof(tsm::Ctl);
@@ -232,10 +266,13 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   tsm_ctx* c = new tsm_ctx();
   c->P = *params;
   c->S = n_samples;
+  if (hipGetDevice(&c->dev) != hipSuccess) { delete c; return fail(TSM_E_HIP, "hipGetDevice failed"); }
+  hipError_t he = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
+  if (he != hipSuccess) { delete c; return fail(TSM_E_HIP, "hipStreamCreate failed"); }
   std::string msg;
   int grc = 1;  // median duals: geometry on the device unless the host is asked for
   if (params->cell_type == 0 && !params->host_preprocess) {
-    grc = tsm::build_geometry_device(*mesh, c->geo, msg);
+    grc = tsm::build_geometry_device(*mesh, c->geo, c->st, msg);
     if (grc < 0) { delete c; return fail(grc, msg); }
   }
   if (grc == 1 && !tsm::build_geometry(*mesh, params->cell_type, c->geo, msg)) {
@@ -282,7 +319,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
         *p = q;
         return r;
       };
-      trc = tsm::build_tiles_device(g, tb, false, c->tiling, dev_tg, dalloc, msg);
+      trc = tsm::build_tiles_device(g, tb, c->tiling, dev_tg, dalloc, c->st, msg);
       if (trc < 0) { delete c; return fail(trc, "tiling: " + msg); }
       if (trc == 2) { delete c; return 1; }
     }
@@ -299,7 +336,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
     for (int i = 0; i < nv; ++i) perm[i] = inv[i] = i;
   }
   c->perm = perm;
-  if (int e = c->upload(&c->d_perm, perm)) { delete c; return e; }
+  if (int e = c->upload_later(&c->d_perm, perm)) { delete c; return e; }
   if (hipHostMalloc((void**)&c->pin, tsm_ctx::PIN, hipHostMallocDefault) != hipSuccess) {
     delete c;
     return fail(TSM_E_HIP, "hipHostMalloc");
@@ -439,12 +476,9 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   }
   if (vbe.empty()) vbe.push_back(0);
   // ---- device ------------------------------------------------------------
-  if (hipGetDevice(&c->dev) != hipSuccess) { delete c; return fail(TSM_E_HIP, "hipGetDevice failed"); }
-  hipError_t he = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
-  if (he != hipSuccess) { delete c; return fail(TSM_E_HIP, "hipStreamCreate failed"); }
   tsm::DevGeo& G = c->G;
   G.nv = nv; G.nf = nf; G.nb = nb; G.nc = nc;
-#define UP(field, vec) do { if ((rc = c->upload(&G.field, vec))) { delete c; return rc; } } while (0)
+#define UP(field, vec) do { if ((rc = c->upload_later(&G.field, vec))) { delete c; return rc; } } while (0)
   UP(x, xs); UP(y, ys); UP(dcarea, dca); UP(gfact, gfact); UP(weight, wgt);
   UP(carea, g.cell_area);
   UP(fv, fv); UP(fn, fn); UP(vfe_ptr, vfe_ptr); UP(vfe, vfe); UP(vc_ptr, vc_ptr); UP(vc, vc);
@@ -497,9 +531,9 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   if (c->tiled) {
     const tsm::Tiling& T = c->tiling;
     tsm::TileGeo TG{};
-    TG.ntiles = T.ntiles; TG.tb = T.tb; TG.max_slots = T.max_slots; TG.max_faces = T.max_faces;
+    TG.ntiles = T.ntiles; TG.tb = T.tb;
     TG.n_periodic_tiles = T.n_periodic_tiles;
-    TG.n_gbv = dev_tiles ? dev_tg.n_gbv : (int)T.gbv.size();
+    TG.nhalo = dev_tiles ? dev_tg.nhalo : (int)T.halo.size();
     TG.fu_block = std::max(0, params->block_fu);
     // block_grad has had no kernel of its own since the stage kernel forms the
     // gradients; its range is still checked
@@ -516,7 +550,7 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
       return fail(TSM_E_ARG, "tiled kernels: block size out of range (blocks " + std::to_string(bg) + "/" +
                                  std::to_string(bf) + ")");
     }
-#define UT(field, vec) do { if ((rc = c->upload(&TG.field, vec))) { delete c; return rc; } } while (0)
+#define UT(field, vec) do { if ((rc = c->upload_later(&TG.field, vec))) { delete c; return rc; } } while (0)
     if (dev_tiles) {
       TG.vbeg = dev_tg.vbeg; TG.hbeg = dev_tg.hbeg; TG.halo = dev_tg.halo; TG.fbeg = dev_tg.fbeg;
       TG.bbeg = dev_tg.bbeg; TG.tbf = dev_tg.tbf; TG.gptr = dev_tg.gptr;
@@ -534,8 +568,10 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
       *p = q;
       return r;
     };
+    if ((rc = c->upload_now())) { delete c; return rc; }
     rc = tsm::build_stage_tables(c->G, TG, tsm::stage_has_gradients(params->flux, params->reconstruct),
-                                 params->model == 1, wall_cells, c->ST, dalloc, c->st, msg);
+                                 params->model == 1, wall_cells ? (int)vbe.size() : 0, c->ST, dalloc,
+                                 c->st, msg);
     // the static LDS of the kernel and its launches fit beside this much
     if (rc == 0 && tsm::stage_lds(c->ST) > 156 * 1024)
       rc = 1;
@@ -562,14 +598,8 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   if (params->liou_fix) AL(A.ssw, cs);
   AL(A.partial, (size_t)S * std::max(c->nblk_v, c->tiling.ntiles) * 4);
   if (c->tiled) AL(c->dtpart, (size_t)S * c->tiling.ntiles);
-  if (c->tiled && tsm::stage_ends_step(c->tiling.ntiles, S)) {
-    AL(A.arrive, S);
-    if (hipMemset(A.arrive, 0, S * sizeof(int)) != hipSuccess) { delete c; return fail(TSM_E_HIP, "memset"); }
-  }
-  AL(A.ctl, (size_t)S);
   AL(c->bad, 1);
-  double* dg; double* dr; double* dc; double* ts;
-  AL(dg, (size_t)S); AL(dr, (size_t)S); AL(dc, 2 * (size_t)S);
+#undef AL
   // time stamps of an unsteady run (src/fv.cc:50-60); a steady run has none
   // and no final time (src/parameter.cc:250-252)
   const int n_stamps = params->unsteady ? params->n_time_stamps : 1;
@@ -577,19 +607,10 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   std::vector<double> tst(n_stamps + 1);
   double tdt = final_time / n_stamps;
   for (size_t i = 0; i < tst.size(); ++i) tst[i] = i * tdt;
-  AL(ts, tst.size());
-#undef AL
-  HIP_TRY(hipMemcpy(ts, tst.data(), tst.size() * sizeof(double), hipMemcpyHostToDevice));
   c->h_gamma.assign(S, params->gamma);
   c->h_R.assign(S, params->gas_const);
-  HIP_TRY(hipMemcpy(dg, c->h_gamma.data(), S * sizeof(double), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(dr, c->h_R.data(), S * sizeof(double), hipMemcpyHostToDevice));
-  {
-    std::vector<double> gc;  // load_gas
-    for (int k = 0; k < S; ++k) { gc.push_back(1.0 / (params->gamma - 1.0)); gc.push_back(1.0 / params->gamma); }
-    HIP_TRY(hipMemcpy(dc, gc.data(), gc.size() * sizeof(double), hipMemcpyHostToDevice));
-  }
-  A.gamma = dg; A.gasR = dr; A.gasc = dc; A.tstamps = ts;
+  std::vector<double> gc;  // load_gas
+  for (int k = 0; k < S; ++k) { gc.push_back(1.0 / (params->gamma - 1.0)); gc.push_back(1.0 / params->gamma); }
   A.log = nullptr; A.log_cap = 0;
   A.fo = tsm::FluxOpts{params->ev_alpha, params->ev_beta, params->tvb_M, params->nd_active};
   A.vp = tsm::ViscParams{params->mu_ref, params->T_ref, params->T_0, params->omega,
@@ -605,7 +626,12 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
                           params->cfl, (long long)params->max_iter, params->unsteady, n_stamps};
   std::vector<tsm::Ctl> ctl(S);
   for (auto& q : ctl) { q = tsm::Ctl{}; q.res_total = 1e20; q.counter = 1; q.done = 1; }
-  HIP_TRY(hipMemcpy(A.ctl, ctl.data(), S * sizeof(tsm::Ctl), hipMemcpyHostToDevice));
+#define UA(field, vec) do { if ((rc = c->upload_later(&A.field, vec))) { delete c; return rc; } } while (0)
+  UA(tstamps, tst); UA(gamma, c->h_gamma); UA(gasR, c->h_R); UA(gasc, gc); UA(ctl, ctl);
+  const bool folds = c->tiled && tsm::stage_ends_step(c->tiling.ntiles, S);
+  if (folds) UA(arrive, std::vector<int>(S, 0));
+#undef UA
+  if ((rc = c->upload_now())) { delete c; return rc; }
   c->bind_state();
   *out = c;
   return TSM_OK;

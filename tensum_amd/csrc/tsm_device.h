@@ -3,14 +3,47 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <functional>
 #include <string>
+#include <vector>
 
 #include "../../include/tsm.h"
 #include "tsm_physics.h"
 
 namespace tsm {
+
+// Device memory of a build's temporaries: small arrays share an allocation, and all
+// of it is given back at the end.
+class TmpPool {
+ public:
+  template <class T>
+  hipError_t get(T** p, size_t n) {
+    const size_t b = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+    if (b > left_) {
+      void* q = nullptr;
+      const bool own = b > SHARED / 4;
+      const hipError_t e = hipMalloc(&q, own ? b : SHARED);
+      if (e != hipSuccess) return e;
+      blocks_.push_back(q);
+      if (own) { *p = static_cast<T*>(q); return hipSuccess; }
+      at_ = static_cast<char*>(q);
+      left_ = SHARED;
+    }
+    *p = reinterpret_cast<T*>(at_);
+    at_ += b;
+    left_ -= b;
+    return hipSuccess;
+  }
+  ~TmpPool() { for (void* q : blocks_) (void)hipFree(q); }
+
+ private:
+  static constexpr size_t SHARED = 1 << 20;
+  std::vector<void*> blocks_;
+  char* at_ = nullptr;
+  size_t left_ = 0;
+};
 
 // Per-sample loop control, resident in device memory so that whole steps can
 // be queued without a host round trip (src/fv.cc:2230-2395 loop variables).
@@ -62,13 +95,12 @@ struct DevGeo {
 // Tile arrays (device pointers, new vertex ids); the stage kernel's own
 // tables are made from them (StageTab).
 struct TileGeo {
-  int ntiles, tb, max_slots, max_faces;
+  int ntiles, tb;
   int fu_block;              // requested threads per tile (0: smallest that fits)
   int n_periodic_tiles;      // tiles [0, n) hold the periodic sets
-  int n_gbv;                 // vertices with a boundary-corrected cell
-  const int* gbv;            // their ids
-  const int *vbeg, *hbeg, *halo, *fbeg, *bbeg, *tbf, *gptr, *cptr, *cgid, *tper, *pinfo;
-  const unsigned *f_lr, *cent;
+  int nhalo;                 // first-ring slots of all tiles
+  const int *vbeg, *hbeg, *halo, *fbeg, *bbeg, *tbf, *gptr, *tper, *pinfo;
+  const unsigned* f_lr;
   const double* f_n;
   const unsigned short* gent;
 };
@@ -368,8 +400,9 @@ void launch_packed_final(const PackLevel* d, const PackPlan& p, hipStream_t st);
 
 // Stage kernel (tsm_stage.hip) and its tables (tsm_stagetab.hip).
 // build_stage_tables: 0 = built, 1 = the tiles are too large for it (msg),
-// TSM_E_* with msg; memory from dalloc.
-int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, bool walls,
+// TSM_E_* with msg; memory from dalloc.  n_wall: entries of DevGeo::vbe, 0 without
+// wall cells.
+int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, int n_wall,
                        StageTab& S, const std::function<int(void**, size_t)>& dalloc, hipStream_t st,
                        std::string& msg);
 int stage_block(const StageTab& T);

@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "tsm_device.h"
 #include "tsm_host.h"
 
 namespace tsm {
@@ -24,11 +25,15 @@ namespace {
 enum { G_OK = 0, G_FALLBACK = 1, G_BAD_EDGE = 2, G_DUP_BFACE = 3, G_LOOSE_BFACE = 4, G_AREA = 5 };
 
 template <class T>
-struct Dev {  // device array freed on scope exit
+struct Dev {  // device array of the build's pool
   T* p = nullptr;
-  hipError_t alloc(size_t n) { return hipMalloc(&p, (n ? n : 1) * sizeof(T)); }
-  ~Dev() { if (p) (void)hipFree(p); }
 };
+
+// cell of each of the cells' corners
+__global__ void k_cell_of(long long n, int* cell) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) cell[i] = (int)(i / 3);
+}
 
 // Edge keys: boundary faces at positions [0, nb), then cell c's edges
 // (v0,v1), (v1,v2), (v2,v0) at nb + 3c + k.  key = min * nv + max.
@@ -198,7 +203,7 @@ inline int blocks(long long n) { return (int)((n + 255) / 256); }
 
 // 0: built; 1: not handled here (the caller uses the host builder); TSM_E_*
 // with `msg` on a mesh error or a HIP failure.
-int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
+int build_geometry_device(const tsm_mesh& m, Geometry& g, hipStream_t st, std::string& msg) {
   const int nv = m.n_vertex, nc = m.n_cell, nb = m.n_bface;
   if (nv <= 0 || nc <= 0) { msg = "empty mesh"; return TSM_E_MESH; }
   const long long ne = nb + 3LL * nc;
@@ -220,13 +225,11 @@ int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
     bper[i] = bt == TSM_BC_PERIODIC;
   }
 #define GT(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { msg = std::string("device geometry: ") + hipGetErrorString(e_); return TSM_E_HIP; } } while (0)
-  hipStream_t st;
-  GT(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-  struct StreamGuard { hipStream_t s; ~StreamGuard() { (void)hipStreamDestroy(s); } } sg{st};
+  TmpPool pool;
   Dev<double> x, y;
   Dev<int> cv, bv, btag, bp;
-  GT(x.alloc(nv)); GT(y.alloc(nv)); GT(cv.alloc(3 * (size_t)nc)); GT(bv.alloc(2 * (size_t)nb));
-  GT(btag.alloc(nb)); GT(bp.alloc(nb));
+  GT(pool.get(&x.p, nv)); GT(pool.get(&y.p, nv)); GT(pool.get(&cv.p, 3 * (size_t)nc)); GT(pool.get(&bv.p, 2 * (size_t)nb));
+  GT(pool.get(&btag.p, nb)); GT(pool.get(&bp.p, nb));
   GT(hipMemcpyAsync(x.p, m.x, nv * sizeof(double), hipMemcpyHostToDevice, st));
   GT(hipMemcpyAsync(y.p, m.y, nv * sizeof(double), hipMemcpyHostToDevice, st));
   GT(hipMemcpyAsync(cv.p, m.cell_v, 3 * (size_t)nc * sizeof(int), hipMemcpyHostToDevice, st));
@@ -238,9 +241,9 @@ int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
   // ---- faces: sort the edge keys, number the runs ---------------------------
   Dev<unsigned long long> key, key_s;
   Dev<int> pos, pos_s, first, newflag, rank, lcell, rcell, bad;
-  GT(key.alloc(ne)); GT(key_s.alloc(ne)); GT(pos.alloc(ne)); GT(pos_s.alloc(ne));
-  GT(first.alloc(ne)); GT(newflag.alloc(3 * (size_t)nc)); GT(rank.alloc(3 * (size_t)nc));
-  GT(lcell.alloc(ne)); GT(rcell.alloc(ne)); GT(bad.alloc(std::max<long long>(ne, nc)));
+  GT(pool.get(&key.p, ne)); GT(pool.get(&key_s.p, ne)); GT(pool.get(&pos.p, ne)); GT(pool.get(&pos_s.p, ne));
+  GT(pool.get(&first.p, ne)); GT(pool.get(&newflag.p, 3 * (size_t)nc)); GT(pool.get(&rank.p, 3 * (size_t)nc));
+  GT(pool.get(&lcell.p, ne)); GT(pool.get(&rcell.p, ne)); GT(pool.get(&bad.p, std::max<long long>(ne, nc)));
   GT(hipMemsetAsync(newflag.p, 0, 3 * (size_t)nc * sizeof(int), st));
   GT(hipMemsetAsync(bad.p, 0, std::max<long long>(ne, nc) * sizeof(int), st));
   hipLaunchKernelGGL(k_edge_keys, dim3(blocks(ne)), dim3(256), 0, st, nb, nc, (long long)nv, bv.p,
@@ -256,7 +259,7 @@ int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
   while (vbits < 32 && ((unsigned)nv >> vbits)) ++vbits;
   GT(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp4, cv.p, pos.p, pos.p, pos.p, 3 * nc, 0, vbits, st));
   Dev<char> tmp;
-  GT(tmp.alloc(std::max(std::max(tmp_bytes, tmp2), std::max(tmp3, tmp4))));
+  GT(pool.get(&tmp.p, std::max(std::max(tmp_bytes, tmp2), std::max(tmp3, tmp4))));
   const size_t tmp_size = std::max(std::max(tmp_bytes, tmp2), std::max(tmp3, tmp4));
   size_t ts = tmp_size;
   GT(hipcub::DeviceRadixSort::SortPairs(tmp.p, ts, key.p, key_s.p, pos.p, pos_s.p, (int)ne, 0,
@@ -272,12 +275,12 @@ int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
   const int nf = nb + n_new + last_flag;
   Dev<int> fv, ftype, fper, flc, frc, edge_face, slot, nonper, bvo, worst;
   Dev<double> fc, fn, fmeas, bn, bmeas, ccx, ccy, area, mcarea;
-  GT(fv.alloc(2 * (size_t)nf)); GT(ftype.alloc(nf)); GT(fper.alloc(nf)); GT(flc.alloc(nf));
-  GT(frc.alloc(nf)); GT(edge_face.alloc(3 * (size_t)nc)); GT(slot.alloc(3 * (size_t)nc));
-  GT(nonper.alloc(nc)); GT(bvo.alloc(2 * (size_t)nb)); GT(worst.alloc(1));
-  GT(fc.alloc(2 * (size_t)nf)); GT(fn.alloc(2 * (size_t)nf)); GT(fmeas.alloc(nf));
-  GT(bn.alloc(2 * (size_t)nb)); GT(bmeas.alloc(nb)); GT(ccx.alloc(nc)); GT(ccy.alloc(nc));
-  GT(area.alloc(nc)); GT(mcarea.alloc(nv));
+  GT(pool.get(&fv.p, 2 * (size_t)nf)); GT(pool.get(&ftype.p, nf)); GT(pool.get(&fper.p, nf)); GT(pool.get(&flc.p, nf));
+  GT(pool.get(&frc.p, nf)); GT(pool.get(&edge_face.p, 3 * (size_t)nc)); GT(pool.get(&slot.p, 3 * (size_t)nc));
+  GT(pool.get(&nonper.p, nc)); GT(pool.get(&bvo.p, 2 * (size_t)nb)); GT(pool.get(&worst.p, 1));
+  GT(pool.get(&fc.p, 2 * (size_t)nf)); GT(pool.get(&fn.p, 2 * (size_t)nf)); GT(pool.get(&fmeas.p, nf));
+  GT(pool.get(&bn.p, 2 * (size_t)nb)); GT(pool.get(&bmeas.p, nb)); GT(pool.get(&ccx.p, nc)); GT(pool.get(&ccy.p, nc));
+  GT(pool.get(&area.p, nc)); GT(pool.get(&mcarea.p, nv));
   GT(hipMemsetAsync(mcarea.p, 0, nv * sizeof(double), st));
   hipLaunchKernelGGL(k_faces, dim3(blocks(ne)), dim3(256), 0, st, ne, nb, bv.p, btag.p, bp.p, cv.p,
                      first.p, rank.p, lcell.p, rcell.p, fv.p, ftype.p, fper.p, flc.p, frc.p,
@@ -289,15 +292,12 @@ int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg) {
   // vertex areas: (vertex, cell) pairs sorted by vertex, cells kept in order
   {
     Dev<int> cid, vs, cs;
-    GT(cid.alloc(3 * (size_t)nc)); GT(vs.alloc(3 * (size_t)nc)); GT(cs.alloc(3 * (size_t)nc));
-    std::vector<int> h(3 * (size_t)nc);
-    for (long long k = 0; k < 3LL * nc; ++k) h[k] = (int)(k / 3);
-    GT(hipMemcpyAsync(cid.p, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice, st));
+    GT(pool.get(&cid.p, 3 * (size_t)nc)); GT(pool.get(&vs.p, 3 * (size_t)nc)); GT(pool.get(&cs.p, 3 * (size_t)nc));
+    hipLaunchKernelGGL(k_cell_of, dim3(blocks(3LL * nc)), dim3(256), 0, st, 3LL * nc, cid.p);
     ts = tmp_size;
     GT(hipcub::DeviceRadixSort::SortPairs(tmp.p, ts, cv.p, vs.p, cid.p, cs.p, 3 * nc, 0, vbits, st));
     hipLaunchKernelGGL(k_vertex_area, dim3(blocks(3LL * nc)), dim3(256), 0, st, 3 * nc, vs.p, cs.p,
                        area.p, mcarea.p);
-    GT(hipStreamSynchronize(st));
   }
   hipLaunchKernelGGL(k_normals, dim3(blocks(nf)), dim3(256), 0, st, nf, nb, x.p, y.p, ccx.p, ccy.p,
                      fv.p, ftype.p, flc.p, frc.p, fc.p, fn.p, fmeas.p, bvo.p, bn.p, bmeas.p);
@@ -386,7 +386,7 @@ extern "C" int tsm_device_geometry(const tsm_mesh* mesh, int cell_type, int* fv,
   if (!mesh || !nf || !nb || cell_type != 0) return TSM_E_ARG;
   tsm::Geometry g;
   std::string msg;
-  const int rc = tsm::build_geometry_device(*mesh, g, msg);
+  const int rc = tsm::build_geometry_device(*mesh, g, nullptr, msg);
   if (rc == 1) return TSM_E_ARG;
   if (rc != 0) return rc;
   *nf = (int)g.face.size();

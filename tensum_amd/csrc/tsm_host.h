@@ -9,6 +9,8 @@
 
 #include "../../include/tsm.h"
 
+struct ihipStream_t;  // hipStream_t points to it
+
 namespace tsm {
 
 struct Face {
@@ -49,8 +51,9 @@ struct Geometry {
 };
 
 // Median-dual geometry built on the device (tsm_geom.hip), bit-identical to
-// build_geometry: 0 = built, 1 = left to the host builder, else TSM_E_*.
-int build_geometry_device(const tsm_mesh& m, Geometry& g, std::string& msg);
+// build_geometry, by work on stream st: 0 = built, 1 = left to the host builder, else
+// TSM_E_*.
+int build_geometry_device(const tsm_mesh& m, Geometry& g, ihipStream_t* st, std::string& msg);
 
 // Vertex tiling for the LDS-staged kernels (see tiles.cpp).  Vertex ids in
 // every array are the new (tile-contiguous) ids.
@@ -65,12 +68,8 @@ struct Tiling {
   std::vector<int> bbeg, tbf;        // tile boundary faces (global bface ids)
   std::vector<int> gptr;             // nv+1
   std::vector<uint16_t> gent;        // bit15 right end, bit14 bface, low 14 bits local index
-  std::vector<int> cptr;             // nv+1
-  std::vector<uint32_t> cent;        // 3 x 10-bit slots | correction flag << 30
-  std::vector<int> cgid;             // global cell id per cell entry
   std::vector<int> tper;             // tile holds periodic sets
   std::vector<int> pinfo;            // per new vertex: first member slot << 8 | set size, or -1
-  std::vector<int> gbv;              // outside periodic tiles: vertices with a boundary-corrected cell
   // Second halo ring, on request (meshes without periodic sets; the stage kernel's
   // own tables are made on the device from the first ring).  Slots are
   // owned, first ring (halo), second ring (halo2); the gradient slots are the
@@ -89,12 +88,13 @@ bool build_tiles(const Geometry& g, int tb, Tiling& T, std::string& msg, bool ri
 
 // The same tiling built on the device (tsm_tiling.hip) for meshes without
 // the second halo ring: the arrays go straight into
-// device memory from `dalloc` (pointers in TG, with n_gbv); T receives the
+// device memory from `dalloc` (pointers in TG, with nhalo), by work on stream st; T receives the
 // numbering (perm, inv, vbeg) and the sizes.  0 = built, 1 = left to
 // build_tiles, 2 = a tile exceeds the slot or face limit (msg), TSM_E_* with msg.
 struct TileGeo;
-int build_tiles_device(const Geometry& g, int tb, bool ring2, Tiling& T, TileGeo& TG,
-                       const std::function<int(void**, size_t)>& dalloc, std::string& msg);
+int build_tiles_device(const Geometry& g, int tb, Tiling& T, TileGeo& TG,
+                       const std::function<int(void**, size_t)>& dalloc, ihipStream_t* st,
+                       std::string& msg);
 bool validate_tiles(const Geometry& g, const Tiling& T, std::string& msg);
 
 // Builds faces, normals and areas exactly as Grid::preproc does for one

@@ -27,78 +27,72 @@
 namespace tsm {
 namespace {
 
-constexpr unsigned FAN_START = 0x80000000u, FAN_WALL = 0x40000000u, FAN_CLOSED = 0x20000000u,
-                   FAN_V = 0x1fffffffu;
+constexpr unsigned FAN_START = 0x80000000u, FAN_CLOSED = 0x40000000u, FAN_V = 0x3fffffffu;
 
-template <class T>
-struct Tmp {  // device array freed on scope exit
-  T* p = nullptr;
-  hipError_t alloc(size_t n) { return hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)); }
-  ~Tmp() { if (p) (void)hipFree(p); }
-};
 inline unsigned nblk(long long n) { return (unsigned)((std::max(n, 1LL) + 255) / 256); }
 
-// The fan of vertex v: chains of neighbours such that each successive pair
-// (b, d) is a cell (v, b, d) in counter-clockwise order; in a closed chain the
-// last and the first are one too.  A closed ring starts at the vertex's first
-// cell, an open one at the cell without a predecessor.  An entry's wall flag
-// belongs to the cell that ends in it (a closed chain's first entry: the cell
-// from its last).  Returns the entry count and, with out, writes the entries.
-__device__ int fan_of(const DevGeo& G, int v, unsigned char* used, unsigned* out) {
-  const int e0 = G.vc_ptr[v], e1 = G.vc_ptr[v + 1];
-  auto ends = [&](int e, int& b, int& d, int& c) {
-    c = G.vc[e] & 0x7fffffff;
-    const int a0 = G.cv[3 * (size_t)c], a1 = G.cv[3 * (size_t)c + 1], a2 = G.cv[3 * (size_t)c + 2];
-    if (a0 == v) { b = a1; d = a2; }
-    else if (a1 == v) { b = a2; d = a0; }
-    else { b = a0; d = a1; }
-  };
-  for (int e = e0; e < e1; ++e) used[e] = 0;
-  int n = 0, left = e1 - e0;
+// The fan of a vertex with n cells: chains of neighbours such that each successive
+// pair (b, d) is a cell (v, b, d) in counter-clockwise order; in a closed chain the
+// last and the first are one too.  A closed ring starts at the vertex's first cell,
+// an open one at the cell without a predecessor.  b(k), d(k): cell k's pair; used(k)
+// and use(k): the cells taken so far, none at the start.  Returns the entry count, at
+// most two a cell.
+template <class B, class D, class Used, class Use>
+__device__ __forceinline__ int fan_walk(int n, B&& b, D&& d, Used&& used, Use&& use, unsigned* out) {
+  int m = 0, left = n;
   while (left > 0) {
-    int start = -1;
-    for (int e = e0; e < e1; ++e) {
-      if (used[e]) continue;
-      if (start < 0) start = e;
-      int b, d, c, b2, d2, c2;
-      ends(e, b, d, c);
+    int cur = -1;
+    for (int e = 0; e < n; ++e) {
+      if (used(e)) continue;
+      if (cur < 0) cur = e;
+      const int be = b(e);
       bool pred = false;
-      for (int f = e0; f < e1 && !pred; ++f)
-        if (!used[f] && f != e) { ends(f, b2, d2, c2); pred = d2 == b; }
-      if (!pred) { start = e; break; }
+      for (int f = 0; f < n && !pred; ++f) pred = !used(f) && f != e && d(f) == be;
+      if (!pred) { cur = e; break; }
     }
-    int cur = start, b, d, c;
-    ends(cur, b, d, c);
-    const int first = b, n0 = n;
-    if (out) out[n] = (unsigned)b | FAN_START;
-    ++n;
+    const int first = b(cur), m0 = m;
+    unsigned head = (unsigned)first | FAN_START;
+    ++m;
     while (cur >= 0) {
-      used[cur] = 1;
+      use(cur);
       --left;
-      const unsigned wall = G.cnb[c] ? FAN_WALL : 0u;
-      const int from = d;
+      const int from = d(cur);
+      if (from == first) { head |= FAN_CLOSED; break; }  // back where the chain began
+      out[m++] = (unsigned)from;
       cur = -1;
-      if (d == first) {  // back where the chain began
-        if (out) out[n0] |= FAN_CLOSED | wall;
-        break;
-      }
-      if (out) out[n] = (unsigned)d | wall;
-      ++n;
-      for (int f = e0; f < e1; ++f) {
-        if (used[f]) continue;
-        ends(f, b, d, c);
-        if (b == from) { cur = f; break; }
-      }
+      for (int f = 0; f < n && cur < 0; ++f)
+        if (!used(f) && b(f) == from) cur = f;
     }
+    out[m0] = head;
   }
-  return n;
+  return m;
 }
-__global__ void k_fan(DevGeo G, unsigned char* used, const int* ptr, int* cnt, unsigned* fan) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v > G.nv) return;
-  if (v == G.nv) { if (cnt) cnt[v] = 0; return; }
-  const int n = fan_of(G, v, used, fan ? fan + ptr[v] : nullptr);
-  if (cnt) cnt[v] = n;
+// ... of every vertex, at twice the start of its cells.  Bound by the latency of its
+// searches, so the pairs are held in LDS and the taken cells in a register; vertices of
+// more cells than fit read the mesh again instead.
+constexpr int FAN_LDS = 16;
+__global__ __launch_bounds__(64) void k_fan(DevGeo G, unsigned char* used, int* cnt, unsigned* fan) {
+  __shared__ int2 pair[FAN_LDS][64];
+  const int v = blockIdx.x * 64 + threadIdx.x, lane = threadIdx.x;
+  if (v >= G.nv) return;
+  const int e0 = G.vc_ptr[v], n = G.vc_ptr[v + 1] - e0;
+  auto ends = [&](int k) -> int2 {
+    const int c = G.vc[e0 + k] & 0x7fffffff;
+    const int a0 = G.cv[3 * (size_t)c], a1 = G.cv[3 * (size_t)c + 1], a2 = G.cv[3 * (size_t)c + 2];
+    return a0 == v ? make_int2(a1, a2) : (a1 == v ? make_int2(a2, a0) : make_int2(a0, a1));
+  };
+  unsigned* out = fan + 2 * (size_t)e0;
+  if (n <= FAN_LDS) {
+#pragma unroll 4
+    for (int k = 0; k < n; ++k) pair[k][lane] = ends(k);
+    unsigned taken = 0;
+    cnt[v] = fan_walk(n, [&](int k) { return pair[k][lane].x; }, [&](int k) { return pair[k][lane].y; },
+                      [&](int k) { return (taken >> k & 1u) != 0; }, [&](int k) { taken |= 1u << k; }, out);
+  } else {
+    for (int k = 0; k < n; ++k) used[e0 + k] = 0;
+    cnt[v] = fan_walk(n, [&](int k) { return ends(k).x; }, [&](int k) { return ends(k).y; },
+                      [&](int k) { return used[e0 + k] != 0; }, [&](int k) { used[e0 + k] = 1; }, out);
+  }
 }
 
 struct TabIn {
@@ -106,7 +100,7 @@ struct TabIn {
   int nt, grad;
   const int *vbeg, *hbeg, *halo;   // the tiling: owned ranges, first ring
   const int *h2beg, *halo2;        // second ring (null while it is being found)
-  const int *fan_ptr;
+  const int *fan_n;                // entries of each vertex's fan
   const unsigned* fan;
   const int *btbeg, *bt;           // boundary terms (null while they are being found)
 };
@@ -158,9 +152,8 @@ __device__ __forceinline__ int slot_in(const TabIn& T, int t, int u) {
 // The items of a gradient slot: for each member of the vertex's periodic set
 // (the vertex alone without one), a centre entry where the centre is not the
 // slot itself from the start, then the member's fan, then the boundary terms of
-// all members' cells.  f(kind, id, flag, closed): kind 0 neighbour (flag: wall
-// cell; closed: first of a closed chain), 1 centre (flag: the slot's own vertex),
-// 2 boundary term of bface id.
+// all members' cells.  f(kind, id, closed): kind 0 neighbour (closed: first of a
+// closed chain), 1 centre, 2 boundary term of bface id.
 template <class F>
 __device__ void walk_items(const TabIn& T, int v, F&& f) {
   const DevGeo& G = T.G;
@@ -168,54 +161,86 @@ __device__ void walk_items(const TabIn& T, int v, F&& f) {
   const int m0 = p < 0 ? 0 : G.pptr[p], m1 = p < 0 ? 1 : G.pptr[p + 1];
   for (int i = m0; i < m1; ++i) {
     const int m = p < 0 ? v : G.pv[i];
-    if (!(i == m0 && m == v)) f(1, m, m == v, false);
-    for (int e = T.fan_ptr[m]; e < T.fan_ptr[m + 1]; ++e) {
-      const unsigned x = T.fan[e];
-      if ((x & FAN_START) && e > T.fan_ptr[m]) f(1, m, m == v, false);
-      f(0, (int)(x & FAN_V), (x & FAN_WALL) != 0, (x & FAN_CLOSED) != 0);
+    if (!(i == m0 && m == v)) f(1, m, false);
+    const unsigned* fan = T.fan + 2 * (size_t)G.vc_ptr[m];
+    const int n = T.fan_n[m];
+    for (int e = 0; e < n; ++e) {
+      const unsigned x = fan[e];
+      if ((x & FAN_START) && e > 0) f(1, m, false);
+      f(0, (int)(x & FAN_V), (x & FAN_CLOSED) != 0);
     }
   }
   for (int i = m0; i < m1; ++i) {
     const int m = p < 0 ? v : G.pv[i];
     for (int e = G.vc_ptr[m]; e < G.vc_ptr[m + 1]; ++e) {
+      if (G.vc[e] >= 0) continue;  // no bface
       const int c = G.vc[e] & 0x7fffffff;
       for (int z = 0; z < 2; ++z) {
         const int b = G.cbf[2 * (size_t)c + z];
         if (b < 0) break;
-        if (bc_sets_state(G.btype[b])) f(2, b, false, false);
+        if (bc_sets_state(G.btype[b])) f(2, b, false);
       }
     }
   }
 }
 
-// per gradient slot: second-ring candidates, boundary terms
-__global__ void k_gs_count(TabIn T, int nq, int* n2, int* nbt) {
+// Counts of a build, read back together: largest counts of a tile (k_desc, k_be_max),
+// totals, cursors of k_gs_emit, and whether an entry did not fit its bits.
+enum { N_MS, N_MS1, N_MF, N_MBT, N_MWT, N_MC, N_MB, N_BE, N_RING2, N_TERMS, N_OV, N_AT2, N_ATB, N_BAD, N_COUNTS };
+
+// Sum over the block, in its first thread
+__device__ __forceinline__ int block_sum(int x) {
+  __shared__ int part[4];
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
+  __syncthreads();  // the sum before this one has been read
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return part[0] + part[1] + part[2] + part[3];
+}
+// Over the gradient slots: second-ring candidates (corners of first-ring cells: an
+// owned vertex's are all owned or in the first ring), boundary terms, and for each at
+// least as many groups of items as follow its first
+__global__ __launch_bounds__(256) void k_gs_count(TabIn T, int nq, int* ng, int* n) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q > nq) return;
-  int c2 = 0, cb = 0;
+  int c2 = 0, cb = 0, nbr = 0, centres = 0;
   if (q < nq) {
     int t, k, v;
     gs_find(T, q, t, k, v);
-    walk_items(T, v, [&](int kind, int id, bool, bool) {
-      if (kind == 2) ++cb;
-      else if (slot_in(T, t, id) < 0) ++c2;
+    const bool ring = k >= T.vbeg[t + 1] - T.vbeg[t];
+    walk_items(T, v, [&](int kind, int id, bool) {
+      cb += kind == 2;
+      nbr += kind == 0;
+      centres += kind == 1;
+      if (ring && kind != 2 && slot_in(T, t, id) < 0) ++c2;
     });
   }
-  n2[q] = c2; nbt[q] = cb;
+  if (q <= nq) ng[q] = cb == 0 && centres == 0 && nbr <= 8 ? 0 : nbr / 7 + centres + (cb + 6) / 7;
+  c2 = block_sum(c2);
+  cb = block_sum(cb);
+  if (threadIdx.x == 0) {
+    if (c2) atomicAdd(n + N_RING2, c2);
+    if (cb) atomicAdd(n + N_TERMS, cb);
+  }
 }
-__global__ void k_gs_emit(TabIn T, int nq, const int* o2, const int* ob, unsigned long long* k2,
-                          unsigned long long* kb) {
+// their keys, in any order (sorted next)
+__global__ void k_gs_emit(TabIn T, int nq, unsigned long long* k2, unsigned long long* kb, int* n) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= nq) return;
   int t, k, v;
   gs_find(T, q, t, k, v);
-  int a = o2[q], b = ob[q];
-  walk_items(T, v, [&](int kind, int id, bool, bool) {
+  const bool ring = k >= T.vbeg[t + 1] - T.vbeg[t];
+  walk_items(T, v, [&](int kind, int id, bool) {
     const unsigned long long key = ((unsigned long long)(unsigned)t << 32) | (unsigned)id;
-    if (kind == 2) kb[b++] = key;
-    else if (slot_in(T, t, id) < 0) k2[a++] = key;
+    if (kind == 2) kb[atomicAdd(n + N_ATB, 1)] = key;
+    else if (ring && slot_in(T, t, id) < 0) k2[atomicAdd(n + N_AT2, 1)] = key;
   });
 }
+__global__ void k_totals(const int* be, const int* ov, int* n) {
+  n[N_BE] = *be;
+  if (ov) n[N_OV] = *ov;
+}
+// first of the keys at or past each tile; entries to be left out are all ones and
+// sort past them all
 __global__ void k_seg(int n, const unsigned long long* keys, const int* nkeys, int* ptr) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > n) return;
@@ -227,13 +252,16 @@ __global__ void k_seg(int n, const unsigned long long* keys, const int* nkeys, i
   }
   ptr[i] = lo;
 }
-__global__ void k_low(int n, const unsigned long long* keys, int* out) {
+__global__ void k_low(const int* n, const unsigned long long* keys, int* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (int)(unsigned)(keys[i] & 0xffffffffull);
+  if (i < *n) out[i] = (int)(unsigned)(keys[i] & 0xffffffffull);
+}
+__global__ void k_zero_int(int n, int* p) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
 }
 
-// descriptors and the largest counts: mx = slots, gradient slots, local
-// faces, boundary terms, wall terms, viscous cells
+// descriptors and the largest counts
 __global__ void k_desc(TabIn T, const int* fbeg, const int* wtbeg, const int* tcbeg,
                        const unsigned char* special, int4* desc, int* mx) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -243,12 +271,12 @@ __global__ void k_desc(TabIn T, const int* fbeg, const int* wtbeg, const int* tc
   const int nf = fbeg[t + 1] - fbeg[t];
   if (desc) desc[t] = make_int4(T.vbeg[t], nown, n1, nf | (special[t] ? 0x40000000 : 0));
   if (mx) {
-    atomicMax(mx, ns);
-    atomicMax(mx + 1, n1);
-    atomicMax(mx + 2, nf);
-    if (T.btbeg) atomicMax(mx + 3, T.btbeg[t + 1] - T.btbeg[t]);
-    if (wtbeg) atomicMax(mx + 4, wtbeg[t + 1] - wtbeg[t]);
-    if (tcbeg) atomicMax(mx + 5, tcbeg[t + 1] - tcbeg[t]);
+    atomicMax(mx + N_MS, ns);
+    atomicMax(mx + N_MS1, n1);
+    atomicMax(mx + N_MF, nf);
+    if (T.btbeg) atomicMax(mx + N_MBT, T.btbeg[t + 1] - T.btbeg[t]);
+    if (wtbeg) atomicMax(mx + N_MWT, wtbeg[t + 1] - wtbeg[t]);
+    if (tcbeg) atomicMax(mx + N_MC, tcbeg[t + 1] - tcbeg[t]);
   }
 }
 __global__ void k_fill_sid(TabIn T, int ms, int* sid) {
@@ -284,19 +312,16 @@ __device__ __forceinline__ uint4 pack8(const unsigned* w) {
 // the items of each gradient slot (codes in tsm_device.h): the first chain in
 // items if it has up to eight neighbours, everything else in groups (read by tiles
 // marked special only); special[t] is set where a tile has anything but such chains
-// around the slots themselves.  Without ov the groups beyond the first are counted
-// in nov.
-__global__ void k_fill_items(TabIn T, int nq, int ms1, int* nov, const int* ovp, uint4* items,
-                             uint4* items2, int2* item_x, uint4* ov, unsigned char* special,
-                             int* bad) {
+// around the slots themselves.
+__global__ void k_fill_items(TabIn T, int nq, int ms1, const int* ovp, uint4* items, uint4* items2,
+                             int2* item_x, uint4* ov, unsigned char* special, int* bad) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q > nq) return;
-  if (q == nq) { if (nov) nov[q] = 0; return; }
+  if (q >= nq) return;
   int t, k, v;
   gs_find(T, q, t, k, v);
   int first = 0, pos = 0;  // neighbours of the first chain
   bool open = true;
-  walk_items(T, v, [&](int kind, int, bool, bool) {
+  walk_items(T, v, [&](int kind, int, bool) {
     if (kind == 0 && open) ++first;
     else if (!(pos == 0 && kind == 1)) open = false;
     ++pos;
@@ -308,12 +333,12 @@ __global__ void k_fill_items(TabIn T, int nq, int ms1, int* nov, const int* ovp,
   uint4 g0 = pack8(g);
   auto put = [&]() {  // the group is full or the next item needs another
     if (groups == 0) g0 = pack8(g);
-    else if (ov) ov[ovp[q] + groups - 1] = pack8(g);
+    else ov[ovp[q] + groups - 1] = pack8(g);
     ++groups;
     n = 0;
     for (int u = 0; u < 8; ++u) g[u] = SI_END;
   };
-  walk_items(T, v, [&](int kind, int id, bool, bool closed) {
+  walk_items(T, v, [&](int kind, int id, bool closed) {
     if (kind == 2) {
       const int b0 = T.btbeg[t], b1 = T.btbeg[t + 1];
       const int j = find32(T.bt, b0, b1, id) - b0;
@@ -348,20 +373,12 @@ __global__ void k_fill_items(TabIn T, int nq, int ms1, int* nov, const int* ovp,
     ++at;
   });
   if (n > 0) put();
-  if (nov) nov[q] = max(groups - 1, 0);
-  if (!ov) return;
+  if (groups - 1 > ovp[q + 1] - ovp[q]) atomicOr(bad, 1);
   const size_t o = (size_t)t * ms1 + k;
   items[o] = pack8(w);
   items2[o] = g0;
   item_x[o] = make_int2((start & SI_MASK) | (max(groups - 1, 0) << 12), ovp[q]);
   if (groups > 0 || start != k) special[t] = 1;
-}
-__global__ void k_no_items(long long n, uint4* items, uint4* items2, int2* item_x) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const unsigned e = SI_END | (SI_END << 16);
-  items[i] = items2[i] = make_uint4(e, e, e, e);
-  item_x[i] = make_int2(0, 0);
 }
 // boundary entries: per vertex their count, then the entries
 __device__ __forceinline__ int vertex_faces(const int* gptr, const unsigned short* gent, int v) {
@@ -388,7 +405,7 @@ __global__ void k_be_fill(TabIn T, const int* gptr, const unsigned short* gent, 
 }
 __global__ void k_be_max(TabIn T, const int* vbp, int* mx) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < T.nt) atomicMax(mx, vbp[T.vbeg[t + 1]] - vbp[T.vbeg[t]]);
+  if (t < T.nt) atomicMax(mx + N_MB, vbp[T.vbeg[t + 1]] - vbp[T.vbeg[t]]);
 }
 // the first eight gather entries of each vertex
 __global__ void k_ge8(TabIn T, int bf0, const int* gptr, const unsigned short* gent, const int* vbp,
@@ -407,9 +424,9 @@ __global__ void k_ge8(TabIn T, int bf0, const int* gptr, const unsigned short* g
   ge8[v] = pack8(w);
 }
 // boundary terms with their vertices
-__global__ void k_bt4(DevGeo G, int n, const int* bt, int4* out) {
+__global__ void k_bt4(DevGeo G, const int* n, const int* bt, int4* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= *n) return;
   const int b = bt[i];
   out[i] = make_int4(b, G.bv[2 * b], G.bv[2 * b + 1], 0);
 }
@@ -473,43 +490,46 @@ __global__ void k_wall_keys(TabIn T, unsigned long long* keys) {
     keys[e] = ((unsigned long long)(unsigned)t << 32) | ((unsigned)T.G.vbe[e] & 0x7fffffffu);
 }
 __global__ void k_wall_cells(TabIn T, const int* wtbeg, const int* wt, uint4* wcell, int* bad) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T.nt) return;
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= wtbeg[T.nt]) return;
   const DevGeo& G = T.G;
-  for (int j = wtbeg[t]; j < wtbeg[t + 1]; ++j) {
-    const int c = G.blc[wt[j]];
-    int s[3];
-    for (int z = 0; z < 3; ++z) {
-      s[z] = slot_in(T, t, G.cv[3 * (size_t)c + z]);
-      if (s[z] < 0 || s[z] > SI_MASK) { atomicOr(bad, 1); s[z] = 0; }
+  int t = 0, end = T.nt;
+  while (end - t > 1) {
+    const int m = (t + end) >> 1;
+    if (wtbeg[m] <= j) t = m; else end = m;
+  }
+  const int c = G.blc[wt[j]];
+  int s[3];
+  for (int z = 0; z < 3; ++z) {
+    s[z] = slot_in(T, t, G.cv[3 * (size_t)c + z]);
+    if (s[z] < 0 || s[z] > SI_MASK) { atomicOr(bad, 1); s[z] = 0; }
+  }
+  unsigned jt[2] = {0xffffu, 0xffffu};
+  for (int z = 0; z < 2; ++z) {
+    const int b = G.cbf[2 * (size_t)c + z];
+    if (b < 0) break;
+    if (!bc_sets_state(G.btype[b])) continue;
+    jt[z] = (unsigned)z;
+    if (T.grad) {
+      const int k = find32(T.bt, T.btbeg[t], T.btbeg[t + 1], b);
+      if (k >= T.btbeg[t + 1] || T.bt[k] != b) atomicOr(bad, 1);
+      jt[z] = (unsigned)(k - T.btbeg[t]) & 0xffffu;
     }
-    unsigned jt[2] = {0xffffu, 0xffffu};
-    for (int z = 0; z < 2; ++z) {
-      const int b = G.cbf[2 * (size_t)c + z];
-      if (b < 0) break;
-      if (!bc_sets_state(G.btype[b])) continue;
-      jt[z] = (unsigned)z;
-      if (T.grad) {
-        const int k = find32(T.bt, T.btbeg[t], T.btbeg[t + 1], b);
-        if (k >= T.btbeg[t + 1] || T.bt[k] != b) atomicOr(bad, 1);
-        jt[z] = (unsigned)(k - T.btbeg[t]) & 0xffffu;
-      }
+  }
+  uint4* o = wcell + 3 * (size_t)j;
+  o[0] = make_uint4((unsigned)wt[j], (unsigned)s[0] | ((unsigned)s[1] << 16), (unsigned)s[2],
+                    jt[0] | (jt[1] << 16));
+  for (int z = 0; z < 2; ++z) {
+    const int f = G.cwf[2 * c + z];
+    uint4 q = make_uint4(0, 0, 0, 0xffffffffu);
+    if (f >= 0) {
+      const int b = G.cwb[2 * c + z], v0 = G.fv[2 * f], v1 = G.fv[2 * f + 1];
+      if (b > 0x3fffffff) atomicOr(bad, 1);
+      q = make_uint4((unsigned)v0, (unsigned)v1,
+                     (unsigned)b | ((unsigned)bc_end(G, b, v0) << 30) | ((unsigned)bc_end(G, b, v1) << 31),
+                     (unsigned)f);
     }
-    uint4* o = wcell + 3 * (size_t)j;
-    o[0] = make_uint4((unsigned)wt[j], (unsigned)s[0] | ((unsigned)s[1] << 16), (unsigned)s[2],
-                      jt[0] | (jt[1] << 16));
-    for (int z = 0; z < 2; ++z) {
-      const int f = G.cwf[2 * c + z];
-      uint4 q = make_uint4(0, 0, 0, 0xffffffffu);
-      if (f >= 0) {
-        const int b = G.cwb[2 * c + z], v0 = G.fv[2 * f], v1 = G.fv[2 * f + 1];
-        if (b > 0x3fffffff) atomicOr(bad, 1);
-        q = make_uint4((unsigned)v0, (unsigned)v1,
-                       (unsigned)b | ((unsigned)bc_end(G, b, v0) << 30) | ((unsigned)bc_end(G, b, v1) << 31),
-                       (unsigned)f);
-      }
-      o[1 + z] = q;
-    }
+    o[1 + z] = q;
   }
 }
 // per (vertex, bface) in bface order: the tile's wall term, the vertex's corner
@@ -534,180 +554,130 @@ __global__ void k_zero(long long n, unsigned char* p) {
 
 }  // namespace
 
-int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, bool walls,
+int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, int n_wall,
                        StageTab& S, const std::function<int(void**, size_t)>& dalloc, hipStream_t st,
                        std::string& msg) {
 #define TT(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { msg = std::string("stage tables: ") + hipGetErrorString(e_); return TSM_E_HIP; } } while (0)
 #define TA(ptr, n) do { void* q_ = nullptr; int r_ = dalloc(&q_, std::max<size_t>((size_t)(n), 1) * sizeof(*(ptr))); if (r_) { msg = "stage tables: allocation"; return r_; } (ptr) = static_cast<std::remove_reference_t<decltype(ptr)>>(q_); } while (0)
 #define GO(k, n, ...) hipLaunchKernelGGL(k, dim3(nblk(n)), dim3(256), 0, st, __VA_ARGS__)
-  const int nv = G.nv, nt = TG.ntiles;
+  const int nv = G.nv, nt = TG.ntiles, n_inc = 3 * G.nc;
   S = StageTab{};
   S.ntiles = nt; S.tb = TG.tb; S.fu_block = TG.fu_block; S.n_periodic_tiles = TG.n_periodic_tiles;
   S.tper = TG.tper; S.pinfo = TG.pinfo; S.gptr = TG.gptr; S.gent = TG.gent;
-  int nhalo = 0;
-  TT(hipMemcpyAsync(&nhalo, TG.hbeg + nt, sizeof(int), hipMemcpyDeviceToHost, st));
-  TT(hipStreamSynchronize(st));
-  const int nq = nv + (grad ? nhalo : 0);
+  const int nq = nv + (grad ? TG.nhalo : 0);
   TabIn T{};
   T.G = G; T.nt = nt; T.grad = grad ? 1 : 0;
   T.vbeg = TG.vbeg; T.hbeg = TG.hbeg; T.halo = TG.halo;
-  Tmp<char> tmp;
-  size_t tmp_bytes = 0;
+  TmpPool tmp;
   auto scan = [&](const int* in, int* out, int n) -> hipError_t {
     size_t b = 0;
+    char* p = nullptr;
     hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st);
-    if (e == hipSuccess && b > tmp_bytes) {
-      if (tmp.p) (void)hipFree(tmp.p);
-      tmp.p = nullptr;
-      e = tmp.alloc(b);
-      tmp_bytes = e == hipSuccess ? b : 0;
-    }
-    return e == hipSuccess ? hipcub::DeviceScan::ExclusiveSum(tmp.p, b, in, out, n, st) : e;
+    if (e == hipSuccess) e = tmp.get(&p, b);
+    return e == hipSuccess ? hipcub::DeviceScan::ExclusiveSum(p, b, in, out, n, st) : e;
   };
-  // sorted distinct keys: list (low words) and per-tile pointers
-  auto group = [&](Tmp<unsigned long long>& k, int n, int** beg, int** list, int& count) -> int {
-    Tmp<unsigned long long> ks, ku;
-    Tmp<int> nu;
-    TT(ks.alloc(n)); TT(ku.alloc(n)); TT(nu.alloc(1));
-    count = 0;
+  // sorted distinct keys: where each tile's start (beg), their low words (list)
+  auto group = [&](unsigned long long* k, int n, int* beg, int** list) -> int {
+    unsigned long long *ks = nullptr, *ku = nullptr;
+    int* nu = nullptr;
+    TT(tmp.get(&ks, n)); TT(tmp.get(&ku, n)); TT(tmp.get(&nu, 1)); TT(tmp.get(list, n));
     if (n > 0) {
       size_t b1 = 0, b2 = 0;
-      TT(hipcub::DeviceRadixSort::SortKeys(nullptr, b1, k.p, ks.p, n, 0, 64, st));
-      TT(hipcub::DeviceSelect::Unique(nullptr, b2, ks.p, ku.p, nu.p, n, st));
-      Tmp<char> t2;
-      TT(t2.alloc(std::max(b1, b2)));
-      TT(hipcub::DeviceRadixSort::SortKeys(t2.p, b1, k.p, ks.p, n, 0, 64, st));
-      TT(hipcub::DeviceSelect::Unique(t2.p, b2, ks.p, ku.p, nu.p, n, st));
-      TT(hipMemcpyAsync(&count, nu.p, sizeof(int), hipMemcpyDeviceToHost, st));
-      TT(hipStreamSynchronize(st));
+      char* p = nullptr;
+      TT(hipcub::DeviceRadixSort::SortKeys(nullptr, b1, k, ks, n, 0, 64, st));
+      TT(hipcub::DeviceSelect::Unique(nullptr, b2, ks, ku, nu, n, st));
+      TT(tmp.get(&p, std::max(b1, b2)));
+      TT(hipcub::DeviceRadixSort::SortKeys(p, b1, k, ks, n, 0, 64, st));
+      TT(hipcub::DeviceSelect::Unique(p, b2, ks, ku, nu, n, st));
+      GO(k_low, n, nu, ku, *list);
     } else {
-      TT(hipMemcpyAsync(nu.p, &count, sizeof(int), hipMemcpyHostToDevice, st));
-      TT(hipStreamSynchronize(st));
+      GO(k_zero_int, 1, 1, nu);
     }
-    if (count > 0) {  // entries to be left out sort last as all ones
-      unsigned long long last = 0;
-      TT(hipMemcpyAsync(&last, ku.p + count - 1, sizeof(last), hipMemcpyDeviceToHost, st));
-      TT(hipStreamSynchronize(st));
-      if (last == ~0ull) {
-        --count;
-        TT(hipMemcpyAsync(nu.p, &count, sizeof(int), hipMemcpyHostToDevice, st));
-        TT(hipStreamSynchronize(st));
-      }
-    }
-    TA(*beg, nt + 1);
-    TA(*list, count);
-    GO(k_seg, nt + 1, nt, ku.p, nu.p, *beg);
-    if (count > 0) GO(k_low, count, count, ku.p, *list);
-    TT(hipStreamSynchronize(st));
+    GO(k_seg, nt + 1, nt, ku, nu, beg);
     return 0;
   };
-  Tmp<int> mx, bad;
-  TT(mx.alloc(8)); TT(bad.alloc(1));
-  {
-    const int z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    TT(hipMemcpyAsync(mx.p, z, sizeof(z), hipMemcpyHostToDevice, st));
-    TT(hipMemcpyAsync(bad.p, z, sizeof(int), hipMemcpyHostToDevice, st));
-    TT(hipStreamSynchronize(st));
-  }
-  Tmp<unsigned char> special;
-  TT(special.alloc(nt));
-  GO(k_zero, nt, (long long)nt, special.p);
-  Tmp<int> fan_ptr, ovp;
-  Tmp<unsigned> fan;
-  int *h2beg = nullptr, *halo2 = nullptr, *btbeg = nullptr, *bt = nullptr;
+  int *mx = nullptr, h[N_COUNTS];
+  TT(tmp.get(&mx, N_COUNTS));
+  GO(k_zero_int, N_COUNTS, (int)N_COUNTS, mx);
+  int* bad = mx + N_BAD;
+  auto counts = [&]() -> hipError_t {
+    hipError_t e = hipMemcpyAsync(h, mx, sizeof(h), hipMemcpyDeviceToHost, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+  };
+  unsigned char* special = nullptr;
+  TT(tmp.get(&special, nt));
+  GO(k_zero, nt, (long long)nt, special);
+  // ---- boundary entries ---------------------------------------------------------
+  int *becnt = nullptr, *vbp = nullptr;
+  TT(tmp.get(&becnt, nv + 1));
+  TA(vbp, nv + 1);
+  GO(k_be_count, nv + 1, nv, TG.gptr, TG.gent, becnt);
+  TT(scan(becnt, vbp, nv + 1));
+  GO(k_be_max, nt, T, vbp, mx);
+  // ---- fans, second ring and boundary terms ---------------------------------------
+  int *ovp = nullptr, *halo2 = nullptr, *btbeg = nullptr, *bt = nullptr;
   if (grad) {
-    // ---- fans ---------------------------------------------------------------
-    int n_inc = 0;
-    TT(hipMemcpyAsync(&n_inc, G.vc_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
-    Tmp<unsigned char> used;
-    Tmp<int> cnt;
-    TT(used.alloc(n_inc)); TT(cnt.alloc(nv + 1)); TT(fan_ptr.alloc(nv + 1));
-    GO(k_fan, nv + 1, G, used.p, (const int*)nullptr, cnt.p, (unsigned*)nullptr);
-    TT(scan(cnt.p, fan_ptr.p, nv + 1));
-    int nfan = 0;
-    TT(hipMemcpyAsync(&nfan, fan_ptr.p + nv, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
-    TT(fan.alloc(nfan));
-    GO(k_fan, nv + 1, G, used.p, fan_ptr.p, (int*)nullptr, fan.p);
-    T.fan_ptr = fan_ptr.p;
-    T.fan = fan.p;
-    // ---- second ring and boundary terms ---------------------------------------
-    Tmp<int> n2, nb, o2, ob;
-    TT(n2.alloc(nq + 1)); TT(nb.alloc(nq + 1));
-    TT(o2.alloc(nq + 1)); TT(ob.alloc(nq + 1));
-    GO(k_gs_count, nq + 1, T, nq, n2.p, nb.p);
-    TT(scan(n2.p, o2.p, nq + 1));
-    TT(scan(nb.p, ob.p, nq + 1));
-    int c2 = 0, cb = 0;
-    TT(hipMemcpyAsync(&c2, o2.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipMemcpyAsync(&cb, ob.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
+    unsigned char* used = nullptr;
+    int *fan_n = nullptr, *ng = nullptr, *h2beg = nullptr;
+    unsigned* fan = nullptr;
+    TT(tmp.get(&used, n_inc)); TT(tmp.get(&fan_n, nv)); TT(tmp.get(&fan, 2 * (size_t)n_inc));
+    TT(tmp.get(&ng, nq + 1)); TT(tmp.get(&ovp, nq + 1)); TT(tmp.get(&h2beg, nt + 1));
+    TA(btbeg, nt + 1);
+    hipLaunchKernelGGL(k_fan, dim3((nv + 63) / 64), dim3(64), 0, st, G, used, fan_n, fan);
+    T.fan_n = fan_n;
+    T.fan = fan;
+    GO(k_gs_count, nq + 1, T, nq, ng, mx);
+    TT(scan(ng, ovp, nq + 1));
+    GO(k_totals, 1, vbp + nv, ovp + nq, mx);
+    TT(counts());
+    const int c2 = h[N_RING2], cb = h[N_TERMS];
     if (c2 < 0 || cb < 0) { msg = "stage tables: too many entries"; return 1; }
-    Tmp<unsigned long long> k2, kb;
-    TT(k2.alloc(c2)); TT(kb.alloc(cb));
-    GO(k_gs_emit, nq, T, nq, o2.p, ob.p, k2.p, kb.p);
-    int count = 0;
-    if (int r = group(k2, c2, &h2beg, &halo2, count)) return r;
-    if (int r = group(kb, cb, &btbeg, &bt, count)) return r;
+    unsigned long long *k2 = nullptr, *kb = nullptr;
+    TT(tmp.get(&k2, c2)); TT(tmp.get(&kb, cb));
+    GO(k_gs_emit, nq, T, nq, k2, kb, mx);
+    if (int r = group(k2, c2, h2beg, &halo2)) return r;
+    if (int r = group(kb, cb, btbeg, &bt)) return r;
     T.h2beg = h2beg; T.halo2 = halo2; T.btbeg = btbeg; T.bt = bt;
-    // ---- groups of items beyond each slot's first ------------------------------
-    TT(ovp.alloc(nq + 1));
-    GO(k_fill_items, nq + 1, T, nq, 0, n2.p, (const int*)nullptr, (uint4*)nullptr, (uint4*)nullptr,
-       (int2*)nullptr, (uint4*)nullptr, (unsigned char*)nullptr, bad.p);
-    TT(scan(n2.p, ovp.p, nq + 1));
+  } else {
+    GO(k_totals, 1, vbp + nv, (const int*)nullptr, mx);
   }
   // ---- wall terms -------------------------------------------------------------
   int *wtbeg = nullptr, *wt = nullptr;
-  if (walls) {
-    int nvbe = 0, count = 0;
-    TT(hipMemcpyAsync(&nvbe, G.vbe_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
-    Tmp<unsigned long long> k;
-    TT(k.alloc(nvbe));
-    GO(k_wall_keys, nv, T, k.p);
-    if (int r = group(k, nvbe, &wtbeg, &wt, count)) return r;
+  if (n_wall > 0) {
+    unsigned long long* k = nullptr;
+    TT(tmp.get(&k, n_wall));
+    TA(wtbeg, nt + 1);
+    GO(k_wall_keys, nv, T, k);
+    if (int r = group(k, n_wall, wtbeg, &wt)) return r;
     uint4* wcell = nullptr;
     unsigned short* wvent = nullptr;
-    TA(wcell, 3 * (size_t)count);
-    TA(wvent, nvbe);
-    GO(k_wall_cells, nt, T, wtbeg, wt, wcell, bad.p);
-    GO(k_wall_entries, nv, T, wtbeg, wt, wvent, bad.p);
+    TA(wcell, 3 * (size_t)n_wall);
+    TA(wvent, n_wall);
+    GO(k_wall_cells, n_wall, T, wtbeg, wt, wcell, bad);
+    GO(k_wall_entries, nv, T, wtbeg, wt, wvent, bad);
     S.wtbeg = wtbeg; S.wcell = wcell; S.wvent = wvent;
   }
   // ---- viscous cells ----------------------------------------------------------
   int *tcbeg = nullptr, *tc = nullptr;
   if (ns) {
-    int n_inc = 0, count = 0;
-    TT(hipMemcpyAsync(&n_inc, G.vc_ptr + nv, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
-    Tmp<unsigned long long> k;
-    TT(k.alloc(n_inc));
-    GO(k_vcell_keys, nv, T, k.p);
-    if (int r = group(k, n_inc, &tcbeg, &tc, count)) return r;
+    unsigned long long* k = nullptr;
+    TT(tmp.get(&k, n_inc));
+    TT(tmp.get(&tcbeg, nt + 1));
+    GO(k_vcell_keys, nv, T, k);
+    if (int r = group(k, n_inc, tcbeg, &tc)) return r;
     unsigned short* ent = nullptr;
     int* cnt = nullptr;
     uint4* vc8 = nullptr;
     TA(ent, n_inc); TA(cnt, nv); TA(vc8, nv);
-    GO(k_vcell_entries, nv, T, tcbeg, tc, ent, cnt, vc8, bad.p);
+    GO(k_vcell_entries, nv, T, tcbeg, tc, ent, cnt, vc8, bad);
     S.vcent = ent; S.vccnt = cnt; S.vc8 = vc8;
   }
-  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special.p, (int4*)nullptr, mx.p);
-  // ---- boundary entries ---------------------------------------------------------
-  Tmp<int> becnt;
-  int* vbp = nullptr;
-  TT(becnt.alloc(nv + 1));
-  TA(vbp, nv + 1);
-  GO(k_be_count, nv + 1, nv, TG.gptr, TG.gent, becnt.p);
-  TT(scan(becnt.p, vbp, nv + 1));
-  GO(k_be_max, nt, T, vbp, mx.p + 6);
-  int h[8], nbe = 0;
-  TT(hipMemcpyAsync(&nbe, vbp + nv, sizeof(int), hipMemcpyDeviceToHost, st));
-  TT(hipMemcpyAsync(h, mx.p, sizeof(h), hipMemcpyDeviceToHost, st));
-  TT(hipStreamSynchronize(st));
-  S.ms = h[0]; S.ms1 = h[1]; S.mf = h[2]; S.mbt = h[3]; S.mwt = h[4]; S.mc = h[5]; S.mb = h[6];
+  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special, (int4*)nullptr, mx);
+  TT(counts());
+  S.ms = h[N_MS]; S.ms1 = h[N_MS1]; S.mf = h[N_MF]; S.mbt = h[N_MBT]; S.mwt = h[N_MWT]; S.mc = h[N_MC];
+  S.mb = h[N_MB];
   S.bf0 = stage_main_records(S, grad, ns);
-  if (S.ms > SI_MASK) { msg = "stage tables: too many slots"; return 1; }
+  if (S.ms > SI_MASK || h[N_BAD]) { msg = "stage tables: too many slots or entries"; return 1; }
   // ---- padded tables ------------------------------------------------------------
   int* sid = nullptr;
   unsigned* lr = nullptr;
@@ -720,37 +690,30 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, b
   GO(k_fill_faces, (long long)nt * S.mf, nt, S.mf, TG.fbeg, TG.f_lr, TG.f_n, lr, fn);
   GO(k_xy, nv, nv, G.x, G.y, xy);
   int2* be = nullptr;
-  TA(be, nbe);
+  TA(be, h[N_BE]);
   GO(k_be_fill, nv, T, TG.gptr, TG.gent, TG.bbeg, TG.tbf, vbp, be);
-  GO(k_ge8, nv, T, S.bf0, TG.gptr, TG.gent, vbp, ge, bad.p);
+  GO(k_ge8, nv, T, S.bf0, TG.gptr, TG.gent, vbp, ge, bad);
   S.vbp = vbp; S.be = be;
   if (grad) {
-    int nov = 0;
     int2* itx = nullptr;
     uint4* ov = nullptr;
     int4* bt4 = nullptr;
-    int nbt = 0;
-    TT(hipMemcpyAsync(&nbt, btbeg + nt, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipMemcpyAsync(&nov, ovp.p + nq, sizeof(int), hipMemcpyDeviceToHost, st));
-    TT(hipStreamSynchronize(st));
-    TA(it, (size_t)nt * S.ms1); TA(it2, (size_t)nt * S.ms1); TA(itx, (size_t)nt * S.ms1); TA(ov, nov); TA(bt4, nbt);
-    if (nbt > 0) GO(k_bt4, nbt, G, nbt, bt, bt4);
-    GO(k_no_items, (long long)nt * S.ms1, (long long)nt * S.ms1, it, it2, itx);
-    GO(k_fill_items, nq, T, nq, S.ms1, (int*)nullptr, ovp.p, it, it2, itx, ov, special.p, bad.p);
+    TA(it, (size_t)nt * S.ms1); TA(it2, (size_t)nt * S.ms1); TA(itx, (size_t)nt * S.ms1);
+    TA(ov, h[N_OV]); TA(bt4, h[N_TERMS]);
+    if (h[N_TERMS] > 0) GO(k_bt4, h[N_TERMS], G, btbeg + nt, bt, bt4);
+    GO(k_fill_items, nq, T, nq, S.ms1, ovp, it, it2, itx, ov, special, bad);
     S.items = it; S.items2 = it2; S.item_x = itx; S.ov = ov; S.btbeg = btbeg; S.bt = bt4;
   }
   if (ns) {
     unsigned* vcells = nullptr;
     TA(vcells, (size_t)nt * S.mc);
-    GO(k_vcells, (long long)nt * S.mc, T, S.mc, tcbeg, tc, vcells, bad.p);
+    GO(k_vcells, (long long)nt * S.mc, T, S.mc, tcbeg, tc, vcells, bad);
     S.vcells = vcells;
   }
-  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special.p, desc, (int*)nullptr);
-  int hbad = 0;
-  TT(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  GO(k_desc, nt, T, TG.fbeg, wtbeg, tcbeg, special, desc, (int*)nullptr);
   TT(hipGetLastError());
-  TT(hipStreamSynchronize(st));
-  if (hbad) { msg = "stage tables: entry out of range"; return 1; }
+  TT(counts());
+  if (h[N_BAD]) { msg = "stage tables: entry out of range"; return 1; }
   S.desc = desc; S.sid = sid; S.f_lr = lr; S.f_n = fn; S.xy = xy; S.ge8 = ge;
 #undef TT
 #undef TA
