@@ -72,11 +72,6 @@ def measured_traffic(kernel):
 VALU_PEAK_WAVE_INSTR_PER_S = 256 * 2.4e9
 
 
-# Whole-step algorithmic bytes per vertex-stage of an SSP-RK3 step at the
-# 1025^2 size (3 (256 V + 24 E + 12 T) + (40 V + 24 E) divided by 3 V).
-STEP_BYTES_PER_VERTEX_STAGE = 389.2
-
-
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -212,7 +207,7 @@ def main():
     print(f"bench: {args.steps} steps in {wall:.3f} s, {ms_per_step:.3f} ms/step", file=sys.stderr,
           flush=True)
 
-    tiles = T.host_tiling(mesh, prm.tile_vertices or 128,
+    tiles = T.host_tiling(mesh, s.tile_vertices or 128,
                           two_rings=args.workload == "riemann")
     kb = kernel_bytes(nv, nf, nc, tiles)
     if ku["dt_us"] == 0.0:  # tiled path: one kernel per stage
@@ -231,8 +226,9 @@ def main():
                 "algorithmic_bytes_per_launch": kb[dom],
                 "valu_issue_frac": valu_issue_frac(dom, dur_us, args),
                 "kernel_us": {k: round(v, 2) for k, v in ku.items()},
-                "step_frac_at_389B_per_vertex_stage":
-                    round(value * STEP_BYTES_PER_VERTEX_STAGE / (HBM_PEAK_GBS * 1e9), 4)}
+                # the kernels' bytes of a whole step over its time
+                "step_frac": round(sum(kb[k] * (1 if k == "dt" else 3) for k in per_launch)
+                                   / (ms_per_step * 1e-3) / (HBM_PEAK_GBS * 1e9), 4)}
 
     cpu = None
     if not args.no_cpu_baseline:

@@ -18,13 +18,13 @@ from . import Params, Solver, TsmError
 
 TILE_SIZES = (64, 96, 128, 160, 192, 256)
 FU_BLOCKS = (0, 256, 512)      # 0: the smallest block that covers the tile
-GRAD_BLOCKS = (0, 256)
+GRAD_BLOCKS = (0,)             # the stage kernel forms the gradients: nothing launches it
 
 
 def candidates(tiles=TILE_SIZES, fu_blocks=FU_BLOCKS, grad_blocks=GRAD_BLOCKS, separate=True,
                fused=(False,)):
-    """Launch shapes to try; the gradient block only matters for the separate
-    gradient pass, so it is varied only there."""
+    """Launch shapes to try.  block_grad and fused_gradient change no launch; they are
+    varied only where a caller lists values for them."""
     out = []
     for fu in fused:
         for tb in tiles:
@@ -42,7 +42,8 @@ def candidates(tiles=TILE_SIZES, fu_blocks=FU_BLOCKS, grad_blocks=GRAD_BLOCKS, s
 def autotune(mesh, params: Params, state, n_samples=1, steps=10, shapes=None, log=None):
     """Times every launch shape on `mesh` with `state` in every sample and
     returns (best Params, table of (shape, step_us)).  Shapes the kernels
-    cannot take (LDS or block limits) are skipped."""
+    cannot take (block limits, or tiles that tsm_create makes smaller because of
+    LDS or table limits) are skipped."""
     shapes = shapes if shapes is not None else candidates(separate=not params.fused_gradient)
     table = []
     for sh in shapes:
@@ -50,6 +51,10 @@ def autotune(mesh, params: Params, state, n_samples=1, steps=10, shapes=None, lo
         try:
             s = Solver(mesh, prm, n_samples=n_samples)
         except TsmError:
+            continue
+        tiled = prm.kernel_path != "csr" and prm.bc_scheme != "strong"
+        if tiled and prm.tile_vertices > 0 and s.tile_vertices != prm.tile_vertices:
+            s.close()
             continue
         for k in range(n_samples):
             s.set_state(state, k)
