@@ -188,19 +188,30 @@ __device__ void walk_items(const TabIn& T, int v, F&& f) {
 // totals, cursors of k_gs_emit, and whether an entry did not fit its bits.
 enum { N_MS, N_MS1, N_MF, N_MBT, N_MWT, N_MC, N_MB, N_BE, N_RING2, N_TERMS, N_OV, N_AT2, N_ATB, N_BAD, N_COUNTS };
 
-// Sum over the block, in its first thread
-__device__ __forceinline__ int block_sum(int x) {
+// Sum over the threads of the block before this one; total: over all of them
+__device__ __forceinline__ int block_before(int x, int& total) {
   __shared__ int part[4];
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
-  __syncthreads();  // the sum before this one has been read
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int incl = x;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += y;
+  }
+  __syncthreads();  // the sums before these have been read
+  if (lane == 63) part[wave] = incl;
   __syncthreads();
-  return part[0] + part[1] + part[2] + part[3];
+  int before = incl - x;
+  total = 0;
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) before += part[w];
+    total += part[w];
+  }
+  return before;
 }
 // Over the gradient slots: second-ring candidates (corners of first-ring cells: an
 // owned vertex's are all owned or in the first ring), boundary terms, and for each at
 // least as many groups of items as follow its first
-__global__ __launch_bounds__(256) void k_gs_count(TabIn T, int nq, int* ng, int* n) {
+__global__ __launch_bounds__(256) void k_gs_count(TabIn T, int nq, int2* cnt, int* ng, int* n) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   int c2 = 0, cb = 0, nbr = 0, centres = 0;
   if (q < nq) {
@@ -213,26 +224,39 @@ __global__ __launch_bounds__(256) void k_gs_count(TabIn T, int nq, int* ng, int*
       centres += kind == 1;
       if (ring && kind != 2 && slot_in(T, t, id) < 0) ++c2;
     });
+    cnt[q] = make_int2(c2, cb);
   }
   if (q <= nq) ng[q] = cb == 0 && centres == 0 && nbr <= 8 ? 0 : nbr / 7 + centres + (cb + 6) / 7;
-  c2 = block_sum(c2);
-  cb = block_sum(cb);
+  int s2, sb;
+  block_before(c2, s2);
+  block_before(cb, sb);
   if (threadIdx.x == 0) {
-    if (c2) atomicAdd(n + N_RING2, c2);
-    if (cb) atomicAdd(n + N_TERMS, cb);
+    if (s2) atomicAdd(n + N_RING2, s2);
+    if (sb) atomicAdd(n + N_TERMS, sb);
   }
 }
-// their keys, in any order (sorted next)
-__global__ void k_gs_emit(TabIn T, int nq, unsigned long long* k2, unsigned long long* kb, int* n) {
+// their keys, the blocks' in any order (sorted next)
+__global__ __launch_bounds__(256) void k_gs_emit(TabIn T, int nq, const int2* cnt, unsigned long long* k2,
+                                                 unsigned long long* kb, int* n) {
+  __shared__ int base[2];
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
+  const int2 c = q < nq ? cnt[q] : make_int2(0, 0);
+  int s2, sb;
+  int a2 = block_before(c.x, s2), ab = block_before(c.y, sb);
+  if (threadIdx.x == 0) {
+    base[0] = s2 ? atomicAdd(n + N_AT2, s2) : 0;
+    base[1] = sb ? atomicAdd(n + N_ATB, sb) : 0;
+  }
+  __syncthreads();
+  if (c.x + c.y == 0) return;
+  a2 += base[0];
+  ab += base[1];
   int t, k, v;
   gs_find(T, q, t, k, v);
-  const bool ring = k >= T.vbeg[t + 1] - T.vbeg[t];
   walk_items(T, v, [&](int kind, int id, bool) {
     const unsigned long long key = ((unsigned long long)(unsigned)t << 32) | (unsigned)id;
-    if (kind == 2) kb[atomicAdd(n + N_ATB, 1)] = key;
-    else if (ring && slot_in(T, t, id) < 0) k2[atomicAdd(n + N_AT2, 1)] = key;
+    if (kind == 2) kb[ab++] = key;
+    else if (c.x && slot_in(T, t, id) < 0) k2[a2++] = key;
   });
 }
 __global__ void k_totals(const int* be, const int* ov, int* n) {
@@ -621,12 +645,13 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, i
     int *fan_n = nullptr, *ng = nullptr, *h2beg = nullptr;
     unsigned* fan = nullptr;
     TT(tmp.get(&used, n_inc)); TT(tmp.get(&fan_n, nv)); TT(tmp.get(&fan, 2 * (size_t)n_inc));
-    TT(tmp.get(&ng, nq + 1)); TT(tmp.get(&ovp, nq + 1)); TT(tmp.get(&h2beg, nt + 1));
+    int2* gs = nullptr;
+    TT(tmp.get(&ng, nq + 1)); TT(tmp.get(&ovp, nq + 1)); TT(tmp.get(&h2beg, nt + 1)); TT(tmp.get(&gs, nq));
     TA(btbeg, nt + 1);
     hipLaunchKernelGGL(k_fan, dim3((nv + 63) / 64), dim3(64), 0, st, G, used, fan_n, fan);
     T.fan_n = fan_n;
     T.fan = fan;
-    GO(k_gs_count, nq + 1, T, nq, ng, mx);
+    GO(k_gs_count, nq + 1, T, nq, gs, ng, mx);
     TT(scan(ng, ovp, nq + 1));
     GO(k_totals, 1, vbp + nv, ovp + nq, mx);
     TT(counts());
@@ -634,7 +659,7 @@ int build_stage_tables(const DevGeo& G, const TileGeo& TG, bool grad, bool ns, i
     if (c2 < 0 || cb < 0) { msg = "stage tables: too many entries"; return 1; }
     unsigned long long *k2 = nullptr, *kb = nullptr;
     TT(tmp.get(&k2, c2)); TT(tmp.get(&kb, cb));
-    GO(k_gs_emit, nq, T, nq, k2, kb, mx);
+    GO(k_gs_emit, nq, T, nq, gs, k2, kb, mx);
     if (int r = group(k2, c2, h2beg, &halo2)) return r;
     if (int r = group(kb, cb, btbeg, &bt)) return r;
     T.h2beg = h2beg; T.halo2 = halo2; T.btbeg = btbeg; T.bt = bt;
