@@ -65,7 +65,9 @@ typedef struct tsm_params {
   /* Kernel family (no counterpart in the reference): 0 = LDS-tiled stage
      kernels where the configuration allows (every model, scheme and flux
      option except bc_scheme strong), CSR-gather kernels otherwise; 1 = always
-     the CSR-gather kernels.  Both give the reference's summation order. */
+     the CSR-gather kernels.  Both add a vertex's fluxes in the reference's face
+     order; the tiled ones form a gradient from the vertex's neighbours in ring
+     order, the CSR ones cell by cell in the reference's. */
   int kernel_path;
   int tile_vertices;  /* owned vertices per tile of the tiled kernels (0: 128, or 112 with viscous
                          terms and gradients); where a tile's slots, faces or two halo
@@ -357,8 +359,8 @@ int tsm_device_tiling_check(const tsm_mesh* mesh, int tile_vertices, long long* 
                             char* which);
 
 /* Host-only: builds and bounds-checks the vertex tiling of the tiled kernels
-   (two_rings: with the second halo ring of the fused stage kernel, on meshes
-   without periodic sets).  stats[10] = tiles, periodic tiles, max slots, max
+   (two_rings: with the second halo ring that the stage kernel takes where it forms
+   gradients, on meshes without periodic sets).  stats[10] = tiles, periodic tiles, max slots, max
    local faces, first-ring halo entries, local face entries, two rings built,
    second-ring halo entries, gradient cell entries, max gradient slots. */
 int tsm_host_tiling(const tsm_mesh* mesh, int cell_type, int tile_vertices, int two_rings,

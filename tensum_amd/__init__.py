@@ -389,7 +389,7 @@ def _geometry(fn, mesh, cell):
 
 def device_tiling_check(mesh: Mesh, tile_vertices=128):
     """The vertex tiling built on the device against the host's build (median
-    duals without periodic sets): (differing entries over all arrays, name of
+    duals): (differing entries over all arrays, name of
     the first array that differs or "")."""
     m, keep = mesh.to_c()
     n = C.c_longlong(0)

@@ -10,9 +10,7 @@
 //   * per owned vertex, 16-bit gather entries into the local faces, in the
 //     reference's face order (then its non-periodic boundary faces), which is
 //     the summation order of the reference's face-loop scatter
-//     (src/fv.cc:1071-1189);
-//   * per owned vertex, its cells as three packed slot ids (cell vertex order)
-//     for the Green-Gauss gradient (src/fv.cc:887-996).
+//     (src/fv.cc:1071-1189).
 // Periodic sets (src/reduce_residual_periodic.cc) are never split: their
 // members are consecutive owned vertices of one tile, in set order, so the
 // set sums become an in-tile exchange through LDS.  All other vertices are

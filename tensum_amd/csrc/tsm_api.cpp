@@ -1236,8 +1236,8 @@ extern "C" int tsm_run_packed(tsm_ctx** cs, int n, long nsteps, long* done) {
     const tsm_ctx* c = cs[i];
     if (!c) return fail(TSM_E_ARG, "null context in group");
     if (!c->tiled || c->two_rings_asked || c->P.time_scheme != 0 || c->A.ns || c->P.liou_fix)
-      return fail(TSM_E_ARG, "packed steps need Euler SSP-RK3 contexts without the Liou fix on "
-                             "the tiled kernels with a gradient pass of their own");
+      return fail(TSM_E_ARG, "packed steps need Euler SSP-RK3 contexts on the tiled kernels, "
+                             "without the Liou fix and without tile_fused_gradient");
     if (c->P.flux != cs[0]->P.flux || c->P.reconstruct != cs[0]->P.reconstruct)
       return fail(TSM_E_ARG, "packed contexts must share the flux and the reconstruction");
     for (int j = 0; j < i; ++j)

@@ -1,13 +1,17 @@
 // tsm_physics.h -- pointwise gas physics and numerical fluxes, device side.
 //
 // Restates, for 2-D FP64 states (T, u, v, p), the reference's pointwise
-// functions with the same operation order (src/material.h, src/material.cc,
+// functions (src/material.h, src/material.cc,
 // src/kepec.cc, src/kep.cc, src/roe_ec.cc, src/simple_avg.cc,
 // src/kepes_tecno_roe.cc, src/kepes_tecno_rusanov.cc, src/reconstruct.cc,
 // src/limiter.h).  The reference's z components are identically zero in 2-D
 // and every term they contribute is an exact +-0, so they are not carried.
-// Compiled with -ffp-contract=off so that no multiply-add is fused, except in
-// the KEPES-TeCNO flux, which opts in (see there).
+// The operation order is the reference's, without fused multiply-adds
+// (-ffp-contract=off), but for what the stage kernel spends its time on: the
+// KEPES-TeCNO and KEPEC fluxes there fuse multiply-adds and take reciprocals, roots
+// and logarithms of about an ulp (below), face areas do so in every kernel, and
+// divisions by gamma, gamma - 1 and the Prandtl number are multiplications by their
+// reciprocals.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -465,8 +469,7 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
   double vn = vx * unx + vy * uny;
   double vel2 = 0.5 * ((l.u * l.u + l.v * l.v) + (r.u * r.u + r.v * r.v));
 
-  // KEPEC central part with the averages above (identical values to a
-  // separate kepec_flux call).
+  // KEPEC central part with the averages above (as kepec_flux_s forms it)
   Cons F;
   F.m = rho * vn;
   F.mx = unx * p + vx * F.m;
