@@ -61,6 +61,13 @@ struct tsm_ctx {
   // the call's one synchronisation, without copy commands.  Larger answers go
   // through device memory.
   static constexpr size_t PIN = 64 * 1024;
+  // States of up to this much go through it too, behind the words of an answer
+  // (state_off): a copy between the device and pageable memory is staged by the
+  // runtime, 35 to 77 us out for 32 to 135 KB where a kernel and a copy on the host take
+  // 13 to 18; from about 256 KB on the memory is pinned for the copy and the two draw
+  // level (533 KB: 45 and 35).
+  static constexpr size_t PIN_STATE = 512 * 1024;
+  size_t state_off = 0;  // of the state in pin, 0 if it takes the copy
   char* pin = nullptr;
   // input bface b, end point k (bface_v[2b+k]) -> offset of its boundary
   // values in a sample's block of G.bstate; device boundary codes
@@ -337,7 +344,10 @@ int create_with_tiles(const tsm_mesh* mesh, const tsm_params* params, int n_samp
   }
   c->perm = perm;
   if (int e = c->upload_later(&c->d_perm, perm)) { delete c; return e; }
-  if (hipHostMalloc((void**)&c->pin, tsm_ctx::PIN, hipHostMallocDefault) != hipSuccess) {
+  const size_t state_bytes = 4 * (size_t)nv * sizeof(double);
+  if (state_bytes <= tsm_ctx::PIN_STATE) c->state_off = 256;
+  const size_t pin_bytes = std::max(tsm_ctx::PIN, c->state_off ? c->state_off + state_bytes : 0);
+  if (hipHostMalloc((void**)&c->pin, pin_bytes, hipHostMallocDefault) != hipSuccess) {
     delete c;
     return fail(TSM_E_HIP, "hipHostMalloc");
   }
@@ -783,9 +793,16 @@ extern "C" int tsm_set_state(tsm_ctx* c, int s, const double* prim) {
   } else {
     c->csr_ready();
   }
-  double* in = c->W[c->cur == 2 ? 0 : 2];  // free between steps
+  const size_t bytes = 4 * (size_t)nv * sizeof(double);
   int* bad = reinterpret_cast<int*>(c->pin);
-  HIP_TRY(hipMemcpyAsync(in, prim, 4 * (size_t)nv * sizeof(double), hipMemcpyHostToDevice, c->st));
+  double* in;
+  if (c->state_off) {
+    in = reinterpret_cast<double*>(c->pin + c->state_off);
+    std::memcpy(in, prim, bytes);
+  } else {
+    in = c->W[c->cur == 2 ? 0 : 2];  // free between steps
+    HIP_TRY(hipMemcpyAsync(in, prim, bytes, hipMemcpyHostToDevice, c->st));
+  }
   tsm::launch_state_put(nv, c->d_perm, in, c->bad, c->W[c->cur] + 4 * off,
                         c->A.W_keep ? c->A.W_keep + 4 * off : nullptr, c->A.ctl + s, c->st);
   tsm::launch_words(sizeof(int), c->bad, bad, c->st);
@@ -822,11 +839,15 @@ int download_vec(tsm_ctx* c, const double* base, int ncomp, int s, double* out) 
 
 extern "C" int tsm_get_state(tsm_ctx* c, int s, double* prim) {
   if (!c || !prim || s < 0 || s >= c->S) return fail(TSM_E_ARG, "bad argument");
-  double* out = c->W[c->cur == 2 ? 0 : 2];  // free between steps
+  const size_t bytes = 4 * (size_t)c->G.nv * sizeof(double);
+  const bool small = c->state_off > 0;
+  double* out = small ? reinterpret_cast<double*>(c->pin + c->state_off)
+                      : c->W[c->cur == 2 ? 0 : 2];  // free between steps
   tsm::launch_state_get(c->G.nv, c->d_perm, c->W[c->cur] + 4 * (size_t)s * c->G.nv, out, c->st);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(prim, out, 4 * (size_t)c->G.nv * sizeof(double), hipMemcpyDeviceToHost, c->st));
+  if (!small) HIP_TRY(hipMemcpyAsync(prim, out, bytes, hipMemcpyDeviceToHost, c->st));
   HIP_TRY(hipStreamSynchronize(c->st));
+  if (small) std::memcpy(prim, out, bytes);
   return TSM_OK;
 }
 
