@@ -776,10 +776,9 @@ extern "C" int tsm_set_bc_time_expr(tsm_ctx* c, const int* bface_group, int n_gr
 extern "C" int tsm_set_sample_material(tsm_ctx* c, int s, double gamma, double R) {
   if (!c || s < 0 || s >= c->S || !(gamma > 1.0) || !(R > 0.0)) return fail(TSM_E_ARG, "bad argument");
   c->h_gamma[s] = gamma; c->h_R[s] = R;
-  HIP_TRY(hipMemcpy((void*)(c->A.gamma + s), &gamma, sizeof(double), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy((void*)(c->A.gasR + s), &R, sizeof(double), hipMemcpyHostToDevice));
-  const double gc[2] = {1.0 / (gamma - 1.0), 1.0 / gamma};
-  HIP_TRY(hipMemcpy((void*)(c->A.gasc + 2 * s), gc, sizeof(gc), hipMemcpyHostToDevice));
+  tsm::launch_set_gas(c->A, s, tsm::Gas{gamma, R, 1.0 / (gamma - 1.0), 1.0 / gamma}, c->st);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(c->st));
   return TSM_OK;
 }
 

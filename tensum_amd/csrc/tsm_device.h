@@ -445,6 +445,7 @@ void launch_prim2ent(const DevGeo& G, const StageArgs& A, int s, hipStream_t st,
 void launch_state_put(int nv, const int* perm, const double* in, int* bad, double* W, double* keep,
                       Ctl* ctl, hipStream_t st);
 void launch_state_get(int nv, const int* perm, const double* W, double* out, hipStream_t st);
+void launch_set_gas(const StageArgs& A, int s, Gas g, hipStream_t st);
 void launch_words(long bytes, const void* in, void* out, hipStream_t st);
 void launch_all_done(int S, const Ctl* ctl, int* out, hipStream_t st);
 void launch_global(const DevGeo& G, const StageArgs& A, int s, double* out, hipStream_t st);

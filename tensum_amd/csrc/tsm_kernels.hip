@@ -965,6 +965,18 @@ void launch_state_get(int nv, const int* perm, const double* W, double* out, hip
   hipLaunchKernelGGL(k_state_get, dim3((nv + 255) / 256), dim3(256), 0, st, nv, perm,
                      reinterpret_cast<const double4*>(W), reinterpret_cast<double4*>(out));
 }
+// One sample's material constants (three copies to the device took 42 us, two 27;
+// this and its wait 13)
+__global__ void k_set_gas(double* gamma, double* R, double* c, int s, Gas g) {
+  gamma[s] = g.gamma;
+  R[s] = g.R;
+  c[2 * s] = g.ig1;
+  c[2 * s + 1] = g.igam;
+}
+void launch_set_gas(const StageArgs& A, int s, Gas g, hipStream_t st) {
+  hipLaunchKernelGGL(k_set_gas, dim3(1), dim3(1), 0, st, const_cast<double*>(A.gamma),
+                     const_cast<double*>(A.gasR), const_cast<double*>(A.gasc), s, g);
+}
 // A few words to or from host memory in stream order, without a copy command
 __global__ void k_words(long n, const unsigned* in, unsigned* out) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
