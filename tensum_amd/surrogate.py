@@ -109,13 +109,18 @@ class MLP:
         the broadcasts give them: a vector is n rows of a one-input network."""
         n_in, n_out = self.widths[0], self.widths[-1]
         u = np.asarray(u, dtype=np.float64)
-        shape = np.broadcast_shapes(u.shape, (n_in,))
-        if np.prod(shape) != shape[0] * n_in:
-            raise ValueError(f"inputs of shape {u.shape}, expected (n, {n_in})")
-        u = np.ascontiguousarray(np.broadcast_to(u, shape)).reshape(shape[0], n_in)
+        if u.ndim != 2 or u.shape[1] != n_in:
+            shape = np.broadcast_shapes(u.shape, (n_in,))
+            if np.prod(shape) != shape[0] * n_in:
+                raise ValueError(f"inputs of shape {u.shape}, expected (n, {n_in})")
+            u = np.broadcast_to(u, shape).reshape(shape[0], n_in)
+        u = np.ascontiguousarray(u)
+
+        def row(v, k):
+            v = np.asarray(v, np.float64)
+            return np.ascontiguousarray(v if v.shape == (k,) else np.broadcast_to(v, (1, k)))
         try:
-            a = [np.ascontiguousarray(np.broadcast_to(np.asarray(v, np.float64), (1, k)))
-                 for v, k in ((mu_x, n_in), (sd_x, n_in), (mu_y, n_out), (sd_y, n_out))]
+            a = [row(mu_x, n_in), row(sd_x, n_in), row(mu_y, n_out), row(sd_y, n_out)]
         except ValueError:  # not one of each per column: row by row on the host
             return self((u - mu_x) / sd_x).astype(np.float64) * sd_y + mu_y
         y = np.empty((u.shape[0], n_out))
