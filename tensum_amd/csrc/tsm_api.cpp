@@ -777,6 +777,9 @@ extern "C" int tsm_set_sample_material(tsm_ctx* c, int s, double gamma, double R
   if (!c || s < 0 || s >= c->S || !(gamma > 1.0) || !(R > 0.0)) return fail(TSM_E_ARG, "bad argument");
   c->h_gamma[s] = gamma; c->h_R[s] = R;
   tsm::launch_set_gas(c->A, s, tsm::Gas{gamma, R, 1.0 / (gamma - 1.0), 1.0 / gamma}, c->st);
+  c->bind_state();  // the stored entropy variables are those of the old constants
+  if (c->tiled) c->e_valid = false;
+  else tsm::launch_prim2ent(c->G, c->A, s, c->st);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(c->st));
   return TSM_OK;

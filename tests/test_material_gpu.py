@@ -29,3 +29,17 @@ def test_material_set_between_steps(path):
         o.set_state(mid[k])
         o.run(4)
         assert np.array_equal(s.get_state(k), o.get_state())
+
+
+@pytest.mark.parametrize("path", ["auto", "csr"])
+def test_queries_after_a_material(path):
+    m = vortex_mesh(17)
+    base = dict(flux="kepes_tecno_roe", reconstruct="minmod", cfl=0.5, final_time=1e9, kernel_path=path)
+    w = vortex(m.x, m.y)
+    s, o = T.Solver(m, T.Params(**base)), T.Solver(m, T.Params(**base, gamma=1.3, gas_const=0.9))
+    s.set_state(w)
+    o.set_state(w)
+    s.gradients()  # with the old constants
+    s.set_material(0, 1.3, 0.9)
+    assert np.array_equal(s.gradients(), o.gradients())
+    assert np.array_equal(s.residual(), o.residual())
