@@ -329,8 +329,9 @@ int tsm_pert(int type, double x, double y, double p, const double* rnd, int n_rn
    fsqrt(a_i), sqrt(a_i). */
 int tsm_check_arith(long n, const double* a, const double* b, double* out);
 /* ... and the functions of about an ulp beside them: out[6i..6i+5] = 1/a_i,
-   1/sqrt(a_i), sqrt(a_i), log(a_i), the library's log(a_i), and the sum of the
-   two minmod slopes minmod(a_i, b_i) + minmod(b_i, b_i) as the TeCNO flux forms it. */
+   1/sqrt(a_i), sqrt(a_i), log(a_i), the library's log(a_i), and
+   (minmod(2 a_i - b_i, b_i) + minmod(b_i, b_i)) / 2 as the TeCNO flux forms it from
+   the projected gradients a_i and b_i at a face's ends and the jump b_i. */
 int tsm_check_math(long n, const double* a, const double* b, double* out);
 
 /* Geometry export in reference order, for parity checks. */

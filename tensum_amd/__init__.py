@@ -351,8 +351,8 @@ def check_arith(a, b):
 
 def check_math(a, b):
     """The kernels' functions of about an ulp: (n, 6) array of 1/a, 1/sqrt(a),
-    sqrt(a), log(a), the device library's log(a), and minmod(a, b) + minmod(b, b)
-    as the TeCNO flux forms it."""
+    sqrt(a), log(a), the device library's log(a), and (minmod(2a - b, b) +
+    minmod(b, b)) / 2 as the TeCNO flux forms it."""
     a = np.ascontiguousarray(a, dtype=np.float64)
     b = np.ascontiguousarray(b, dtype=np.float64)
     out = np.empty((a.size, 6))

@@ -1288,7 +1288,7 @@ __global__ void k_check_math(long n, const double* a, const double* b, double* o
   out[6 * i + 2] = fsqrt3(x);
   out[6 * i + 3] = flog(x);
   out[6 * i + 4] = log(x);
-  out[6 * i + 5] = minmod_sum(x, y, y);
+  out[6 * i + 5] = minmod_half(x, y, y);
 }
 void launch_check_math(long n, const double* a, const double* b, double* out, hipStream_t st) {
   hipLaunchKernelGGL(k_check_math, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, a, b, out);

@@ -230,13 +230,15 @@ __device__ __forceinline__ double minmod_tvd(double a, double b) {
   if (a > 0.0 && b > 0.0) return fmin(a, b);
   return 0.0;
 }
-// minmod(dl, dz) + minmod(dr, dz), each the slope clamped to the interval between 0
-// and dz, without branches: both taken with dz's sign, clamped to [0, |dz|] from
-// below first, so that a NaN slope becomes the zero that the branches give (clamped
-// from above first it would become the full jump), and the sign put back.
-__device__ __forceinline__ double minmod_sum(double dl, double dr, double dz) {
-  const double s = copysign(1.0, dz), m = fabs(dz);
-  return s * (fmin(fmax(s * dl, 0.0), m) + fmin(fmax(s * dr, 0.0), m));
+// Half of minmod(2 gl - dz, dz) + minmod(2 gr - dz, dz) without branches: the slopes
+// are formed with dz's sign (s dz = |dz|), clamped to [0, |dz|] from below first, so
+// that a NaN slope becomes the zero that the branches give (clamped from above first
+// it would become the full jump), and the sign is put back.
+__device__ __forceinline__ double minmod_half(double gl, double gr, double dz) {
+#pragma clang fp contract(fast)
+  const double s = copysign(2.0, dz), m = fabs(dz);
+  const double a = __builtin_fma(s, gl, -m), b = __builtin_fma(s, gr, -m);
+  return copysign(0.5, dz) * (fmin(fmax(a, 0.0), m) + fmin(fmax(b, 0.0), m));
 }
 __device__ __forceinline__ double minabs(double a, double b) {
   return (fabs(a) < fabs(b)) ? a : b;
@@ -576,7 +578,7 @@ __device__ __forceinline__ Cons tecno_flux(const Gas& g, const FluxOpts& o, doub
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - ((dl + dr) * (1.0 - K) + (2.0 * dz[i]) * (1.0 + K)) * 0.25;
       } else if (REC == R_MINMOD) {
-        dZi = dz[i] - 0.5 * minmod_sum(2.0 * gl[i] - dz[i], 2.0 * gr[i] - dz[i], dz[i]);
+        dZi = dz[i] - minmod_half(gl[i], gr[i], dz[i]);
       } else {
         const double dl = 2.0 * gl[i] - dz[i], dr = 2.0 * gr[i] - dz[i];
         dZi = dz[i] - limited_slope<REC>(dl, dz[i], 0.0, 0.0) - limited_slope<REC>(dr, dz[i], 0.0, 0.0);

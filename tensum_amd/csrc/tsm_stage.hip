@@ -421,9 +421,11 @@ __device__ __forceinline__ void agent_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <bool LAUNCH>
-__device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams& P, const Ctl& c, int nblk,
-                                           int nv, const double* dtpart, int log_slot, int s) {
+__device__ __forceinline__ void final_wave(const StageArgs& A, const StepParams& P, int nblk, int nv,
+                                           const double* dtpart, int log_slot, int s) {
   const int lane = threadIdx.x & 63;
+  const Ctl c = A.ctl[s];
+  if (!LAUNCH && c.done) return;
   auto load = [](const double* p) { return LAUNCH ? agent_load(p) : *p; };
   const double* q = A.partial + (size_t)s * nblk * 4;
   const double* dq = dtpart + (size_t)s * nblk;
@@ -495,7 +497,7 @@ __device__ __forceinline__ void block_partials(const StageArgs& A, const StepPar
   }
   if (!__builtin_amdgcn_readlane(ends, 63)) return;
   asm volatile("" ::: "memory");
-  final_wave<true>(A, P, A.ctl[s], nt, nv, dtpart, log_slot, s);
+  final_wave<true>(A, P, nt, nv, dtpart, log_slot, s);
   if ((threadIdx.x & 63) == 0)
     __hip_atomic_store(A.arrive + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1113,10 +1115,6 @@ __device__ __forceinline__ void step_final_body(const StageArgs& A, const StepPa
   __shared__ double red[64];
   const Ctl c = A.ctl[s];
   if (c.done) return;
-  if (nblk <= FOLD_TILES) {
-    if (threadIdx.x < 64) final_wave<false>(A, P, c, nblk, nv, dtpart, log_slot, s);
-    return;
-  }
   double part[4] = {0, 0, 0, 0};
   double x = 1.0e20;
   const double4* q4 = reinterpret_cast<const double4*>(A.partial) + (size_t)s * nblk;
@@ -1149,12 +1147,18 @@ __global__ __launch_bounds__(1024) void k_step_final_tiled(StageArgs A, StepPara
                                                           int log_slot) {
   step_final_body(A, P, nblk, nv, dtpart, log_slot, blockIdx.x);
 }
+// ... with up to FOLD_TILES tiles
+__global__ __launch_bounds__(64) void k_step_final_wave(StageArgs A, StepParams P, int nblk, int nv,
+                                                        const double* dtpart, int log_slot) {
+  final_wave<false>(A, P, nblk, nv, dtpart, log_slot, blockIdx.x);
+}
 __global__ __launch_bounds__(1024) void k_step_final_packed(const PackLevel* __restrict__ pk, int nl) {
   const int b = blockIdx.x;
   int l = 0;
   while (l + 1 < nl && b >= pk[l + 1].base_final) ++l;
   const PackLevel& L = pk[l];
-  step_final_body(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
+  if (L.T.ntiles > FOLD_TILES) step_final_body(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
+  else if (threadIdx.x < 64) final_wave<false>(L.A, L.P, L.T.ntiles, L.G.nv, L.dtpart, -1, b - L.base_final);
 }
 
 // ---------------------------------------------------------------------------
@@ -1256,8 +1260,10 @@ void launch_stage(int flux, int rec, const DevGeo& G, const StageTab& T, const S
 void launch_step_final_tiled(const DevGeo& G, const StageArgs& A, const StepParams& P, int S,
                              int nblk, const double* dtpart, int log_slot, hipStream_t st) {
   if (A.arrive) return;  // ended by the last stage
-  hipLaunchKernelGGL(k_step_final_tiled, dim3(S), dim3(nblk <= FOLD_TILES ? 64 : 1024), 0, st, A, P,
-                     nblk, G.nv, dtpart, log_slot);
+  if (nblk <= FOLD_TILES)
+    hipLaunchKernelGGL(k_step_final_wave, dim3(S), dim3(64), 0, st, A, P, nblk, G.nv, dtpart, log_slot);
+  else
+    hipLaunchKernelGGL(k_step_final_tiled, dim3(S), dim3(1024), 0, st, A, P, nblk, G.nv, dtpart, log_slot);
 }
 
 // ---------------------------------------------------------------------------

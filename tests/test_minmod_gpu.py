@@ -17,15 +17,19 @@ def _minmod(a, b):
 
 
 def test_minmod_takes_the_branches_values():
+    """(minmod(2a - b, b) + minmod(b, b)) / 2 for gradients a and jumps b: multiples of
+    2^-20, so that 2a - b is exact, and values whose slope is decided by size."""
     rng = np.random.default_rng(7)
-    v = np.concatenate([rng.standard_normal(40), 10.0 ** rng.uniform(-300, 300, 20),
-                        -10.0 ** rng.uniform(-300, 300, 20),
-                        [0.0, -0.0, np.inf, -np.inf, np.nan, 1.7976931348623157e308, -5e-324, 5e-324]])
-    a, b = (x.ravel() for x in np.meshgrid(v, v))
-    keep = ~np.isnan(b)  # with the jump itself NaN the flux is NaN whatever the slope
-    a, b = a[keep], b[keep]
-    with np.errstate(over="ignore"):
-        want = _minmod(a, b) + _minmod(b, b)
+    u = rng.integers(-2 ** 22, 2 ** 22, 300) * 2.0 ** -20
+    big = np.concatenate([s * 10.0 ** rng.uniform(-300, 300, 20) for s in (1, -1)])
+    v = np.concatenate([u, [0.0, -0.0, np.inf, -np.inf, np.nan]])
+    a, b = (x.ravel() for x in np.meshgrid(v, u))
+    a2, b2 = (x.ravel() for x in np.meshgrid(np.concatenate([big, [0.0, np.inf, -np.inf, np.nan, 5e-324]]),
+                                             np.concatenate([big, [0.0, 5e-324, -5e-324]])))
+    far = ~((np.abs(a2) > 1e-3 * np.abs(b2)) & (np.abs(a2) < 1e3 * np.abs(b2)))
+    a, b = np.concatenate([a, a2[far]]), np.concatenate([b, b2[far]])
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = 0.5 * (_minmod(2 * a - b, b) + _minmod(b, b))
     got = T.check_math(a, b)[:, 5]
-    bad = ~((got == want) | (np.isnan(got) & np.isnan(want)))
+    bad = got != want
     assert not bad.any(), list(zip(a[bad], b[bad], got[bad], want[bad]))[:10]
