@@ -13,12 +13,12 @@
 // residual norm is a sum over tiles and has one order for each number of tiles.
 //
 // What bounds it: at 1025^2 (KEPES-TeCNO Rusanov, minmod) a stage's FP64
-// issue (0.62 of the rate), LDS (0.36) and HBM traffic (2.8 of 4.9 TB/s) are within
+// issue (0.60 of the rate), LDS (0.36) and HBM traffic (2.8 of 4.9 TB/s) are within
 // a factor of two of each other, and a tile's phases depend on one another through
 // barriers, so the layout is chosen to keep four tiles per CU in different phases.
-// Under a kernel trace a stage takes 94 us, the last 117 and the launch that ends the
+// Under a kernel trace a stage takes 95 us, the last 117 and the launch that ends the
 // step 10 (with gradients in launches of their own: 98, the last 124, and 58 more a
-// stage); a step by itself 303 us (492).  On small meshes a stage is one tile's chain,
+// stage); a step by itself 301 us (492).  On small meshes a stage is one tile's chain,
 // 10 to 13 us.
 //  - gradients never go through memory.  A second launch and a 64-byte record
 //    per vertex written and read back by every neighbouring tile cost more than
